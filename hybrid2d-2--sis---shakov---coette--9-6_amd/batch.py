@@ -43,8 +43,8 @@ def instances(count: int, seed: int = 20261202, side=(64, 256), nv=(24, 64), kn=
 
 class Batch:
     """A gsis_batch over GsisSolver handles (one precision and flux scheme;
-    the synthetic solves of M1 instances run inside the step's graph, one
-    workgroup each, or after it, one cooperative launch each).  The solvers
+    the synthetic solves of M1 instances run inside the step's graph, a few
+    workgroups each, or after it, one cooperative launch each).  The solvers
     stay usable on their own between batch steps."""
 
     def __init__(self, solvers):

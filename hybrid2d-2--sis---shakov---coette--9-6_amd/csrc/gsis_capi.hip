@@ -411,8 +411,9 @@ struct gsis_batch {
   std::vector<int *> flags;
   int nstrip = 0, nseam = 0, ncellb = 0;
   gsis::NsJob *nsjobs = nullptr;  // device table of the inner loops run in the graph
+  int nns = 0, nsblocks = 0;      // its entries, and the workgroups of their launch
   std::vector<bool> in_graph;     // M1 instance whose synthetic solve is captured
-  // synthetic solves inside the graph (one workgroup each): -1 automatic (when
+  // synthetic solves inside the graph (a gang of workgroups each): -1 automatic (when
   // at least kNsGraphMin instances qualify), 0 never, 1 for every qualifying one
   int ns_graph = -1;
   hipGraph_t graph = nullptr;
@@ -422,10 +423,12 @@ struct gsis_batch {
 
 namespace {
 
-// One workgroup per instance pays off with many instances: measured 3.0x
-// faster than one cooperative launch per instance for 64 instances of side
-// 64-160, 0.6x for 16 of side 48-96, 0.17x for one of side 256.
-constexpr int kNsGraphMin = 32;
+// Cooperative launches of several instances run one after another, the
+// gangs of one launch in the graph beside each other.  Measured, after the
+// graph against inside (cavities, 300 inner iterations): 2 instances of side
+// 64-128 31.2 and 29.8 ms, 4 of side 64-160 118 and 48 ms, 16 of side 64-256
+// 443 and 88 ms, 40 1309 and 204 ms; one instance is the same either way.
+constexpr int kNsGraphMin = 4;
 
 void batch_drop_graph(gsis_batch *b) {
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
@@ -488,6 +491,7 @@ int batch_capture(gsis_batch *b) {
   if (rc) return rc;
   {  // which M1 instances run their inner loop inside the graph
     std::vector<gsis::NsJob> jobs;
+    int nq = 0;
     b->in_graph.assign(b->hs.size(), false);
     for (size_t k = 0; k < b->hs.size(); k++) {
       gsis_handle *h = b->hs[k];
@@ -495,13 +499,17 @@ int batch_capture(gsis_batch *b) {
           !gsis::synthetic_batchable(h->syn))
         continue;
       b->in_graph[k] = true;
-      jobs.push_back(gsis::NsJob{h->d, h->syn});
+      nq++;
+      if (h->syn.nflux > 0) jobs.push_back(gsis::NsJob{h->d, h->syn, 0, 0});  // (else no cell is swept)
     }
-    if (b->ns_graph == 0 || (b->ns_graph < 0 && (int)jobs.size() < kNsGraphMin)) {
+    if (b->ns_graph == 0 || (b->ns_graph < 0 && nq < kNsGraphMin)) {
       b->in_graph.assign(b->hs.size(), false);
       jobs.clear();
     }
+    b->nns = (int)jobs.size();
     if (!jobs.empty()) {
+      b->nsblocks = gsis::synthetic_batch_layout(jobs);
+      if (b->nsblocks < 0) return fail(GSIS_EHIP, gsis::synthetic_error());
       if (!b->nsjobs) {
         void *q = nullptr;
         HIPCHK(hipMalloc(&q, b->hs.size() * sizeof(gsis::NsJob)));
@@ -530,13 +538,15 @@ int batch_capture(gsis_batch *b) {
       gsis::launch_convert(h->d, b->s);
       if (h->p.if_viscous) gsis::launch_hot(h->d, b->s);
     }
-    // the synthetic solves of the M1 instances whose inner loop fits one
-    // workgroup and that use no closure: all in one launch, one workgroup each
-    int nj = 0;
-    for (size_t k = 0; k < b->hs.size(); k++)
-      if (b->in_graph[k]) gsis::synthetic_begin(b->hs[k]->d, b->hs[k]->syn, b->s);
-    for (size_t k = 0; k < b->hs.size(); k++) nj += b->in_graph[k] ? 1 : 0;
-    if (nj > 0) gsis::launch_ns_batch(b->nsjobs, nj, b->s);
+    // the synthetic solves of the M1 instances that use no closure: all in one
+    // launch, a gang of workgroups each
+    for (size_t k = 0; k < b->hs.size(); k++) {
+      if (!b->in_graph[k]) continue;
+      gsis_handle *h = b->hs[k];
+      gsis::synthetic_begin(h->d, h->syn, b->s);
+      if (h->syn.nflux == 0) gsis::synthetic_run(h->d, h->syn, 1, 0x7fffffff, b->s);  // no swept cell
+    }
+    gsis::launch_ns_batch(b->nsjobs, b->nns, b->nsblocks, b->s);
     for (size_t k = 0; k < b->hs.size(); k++)
       if (b->in_graph[k]) gsis::synthetic_finish(b->hs[k]->d, b->hs[k]->syn, b->s);
     const hipError_t e2 = hipStreamEndCapture(b->s, &b->graph);

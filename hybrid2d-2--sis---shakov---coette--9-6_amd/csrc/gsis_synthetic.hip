@@ -11,30 +11,41 @@
 // (src/sub_LU_SGS.f90:4-143).
 //
 // The inner loop is one cooperative launch that iterates on the device until
-// the max |energy residual| drops to ns_tol or ns_maxit is reached:
-//  * flux workgroups (1..nflux) own 16x16-cell tiles of the swept cells
-//    3..n-3.  Per iteration each stages U of its tile plus two halo rings in
-//    LDS, forms the primitives and viscosity, the face fluxes (inviscid,
-//    viscous, HoT), then per cell Res, Lc, Lv, dt and everything the LU-SGS
-//    sweeps need that does not depend on dU, stored by anti-diagonal plane;
-//  * workgroup 0 runs the two sweeps.  Lane j of its wavefronts owns row j,
-//    so one sweep step is one anti-diagonal plane: the forward recursion takes
-//    dU(i-1,j) from the lane's own previous step and dU(i,j-1) from the lane
-//    below (a cross-lane shift; between wavefronts a hand-off through an LDS
-//    ring, no barrier per plane).  The backward pass writes U + dU of each
-//    cell as soon as it is final; the sweeps read the pre-update U from the
-//    records, so the update is the reference's "after both sweeps".  On a
-//    mesh whose swept cells all have the normals (1,0) and (0,1) (checked
-//    on the host at set-up) the sweep skips the normals: DF across an
-//    i-face is dFx, across a j-face dFy.
-// Any order of the cells that respects the sweep dependences gives the same
-// dU, and the planes are visited in the reference's order, so the inner
-// iteration counts are the reference's.  The loop ends by the reference's
-// rule: iteration k+1 runs when max |Res_4| of iteration k exceeds ns_tol and
-// k < ns_maxit.  Every wait between workgroups is bounded; a timeout ends the
-// loop and is reported by the host.
+// the max |energy residual| drops to ns_tol or ns_maxit is reached.  Its
+// recurrence sets its time: dU of a cell needs dU of (i-1,j) and (i,j-1)
+// (forward; (i+1,j) and (i,j+1) backward), so an iteration is two chains of
+// nx+ny-11 plane steps, however many CUs there are.  Everything else is
+// arranged around the chain:
+//  * a sweep workgroup per band of 64 swept rows, each on a CU of its own.  One
+//    wavefront sweeps, a row per lane, a plane per step; the band's edge row
+//    goes to the next band through memory (0.3 us one way on one XCD, which
+//    costs a lag of a few steps per band, not time per step).  The other
+//    wavefronts of the workgroup do what would hold it up: three fetch the
+//    records of coming planes and form what does not depend on dU, one brings
+//    the neighbouring band's values, one keeps the books;
+//  * flux workgroups compute tile after tile what the sweeps need: primitives,
+//    viscosity, face fluxes (inviscid, viscous, HoT), Res, Lc, Lv, dt, stored
+//    by anti-diagonal plane.  A tile of the next iteration is computed as soon
+//    as the backward sweep has passed its cells, and the next forward sweep
+//    starts when the first tiles are done: the decision that there is a next
+//    iteration is taken from the residual before the backward sweep begins.
+// One lane per row and one plane per step give the order of the reference's
+// sweeps, so the inner iteration counts are the reference's.  The loop ends by
+// the reference's rule: iteration k+1 runs when max |Res_4| of iteration k
+// exceeds ns_tol and k < ns_maxit.  Every wait between workgroups is bounded;
+// a timeout ends the loop and is reported by the host.
+//
+// Measured per inner iteration (mesh cells, sweeps of all bands in one
+// workgroup with separate flux phases before): 64^2 102 -> 64 us, 128^2
+// 238 -> 127 us, 256^2 607 -> 258 us; 40 instances of side 64-256 in one
+// launch 4.5 -> 0.42 ms (one workgroup each before).  A plane step takes about
+// 0.2 us, 450-480 cycles, of which the arithmetic alone takes about 400; an
+// iteration adds about 10 us for the turn from the backward to the forward
+// sweep (the flux of the first tile).
+#include <algorithm>
 #include <cstring>
 #include <string>
+#include <vector>
 
 #include "gsis_ns_common.h"
 #include "gsis_synthetic.h"
@@ -47,65 +58,120 @@ std::string g_syn_err;
 
 const char *synthetic_error() { return g_syn_err.c_str(); }
 
-constexpr int kTile = 16;                    // flux tile: kTile x kTile cells
-constexpr int kTW = kTile + 4;               // with two halo rings each side
-constexpr int kTC = kTW * kTW;
-constexpr int kNFace = (kTile + 1) * kTile;  // i-faces (or j-faces) of a tile
-constexpr int kMaxSweepWaves = 16;           // rows <= 1024
-constexpr int kRingMax = 10;                 // sweep hand-off slots per wavefront (at most)
-constexpr int kSlot = 14;                    // doubles per hand-off slot: dU, dFx, dFy, Cbj, Hsj
+// A flux tile: kTI x kTJ cells.  A workgroup's 384 threads take each phase of
+// a tile of 8 x 16 at once (240 cells with halo, 280 faces, 128 cells), so it
+// has the latency of 8 x 8 and less halo; 16 x 16 takes two rounds of faces.
+constexpr int kTI = 8, kTJ = 16;
+constexpr int kCI = kTI + 4, kCJ = kTJ + 4;  // with two halo rings each side
+constexpr int kTC = kCI * kCJ;
+constexpr int kLev = kTJ / kTI;  // tile (a, b) is of level a + kLev b: it holds the planes from 6 + kTI level on
+constexpr int kBand = 64;                    // swept rows of a sweep workgroup, one per lane of its sweep wavefront
+constexpr int kBandTiles = kBand / kTJ;      // tile rows of a band
+constexpr int kMaxBands = 16;                // rows <= 1024
+constexpr int kThreads = 384;                // a workgroup of the inner loop: six wavefronts
+constexpr int kLoaders = 3;                  // wavefronts of a sweep workgroup that fetch records
+constexpr int kGroup = 4;                    // plane steps a loader fetches and hands over at a time
+constexpr int kGroups = 2;                   // groups of prepared records in LDS
+constexpr int kPad = kGroup - 1;             // planes before the first and after the last one that steps store to
+constexpr int kHand = 64;                    // received neighbour values in LDS (a power of two)
 constexpr long long kWaitTicks = 200000000;  // bounded waits: 2 s of the 100 MHz wall clock
+constexpr long long kStartTicks = 12000000000;  // a batched gang's wait for its last workgroup: 120 s
 
-enum { kCtlGo = 1, kCtlErr = 3 };
+// ctl words
+enum { kCtlGo = 1, kCtlErr = 3, kCtlBad = 4, kCtlStop = 5, kCtlLast = 6, kCtlArrived = 7 };
 
-// Sweep records are blocked by (plane, wavefront): block ((p-6)*nw + w) holds
-// the 64 rows 3+64w .. 3+64w+63, field k of row 3+64w+l at (k/2)*128 + 2l + k%2,
-// so each pair of fields of a plane is one contiguous 1 KiB load per
-// wavefront.  Offsets in doubles; the record array stays below 4 GiB
-// (synthetic_init), so byte offsets fit the 32-bit buffer offsets.
-constexpr int kBlk = kNRec * 64;  // doubles per block
-static_assert(kRecRes == 0 && kRecU == 4 && kRecRa == 8 && kRecCbi == 9 && kRecCbj == 10 && kRecHsi == 11 &&
-                  kRecHsj == 12 && kRecRr == 13 && kRecNi == 14 && kRecNj == 16 && kNRec == 18,
-              "the sweep's pair loads and the flux workgroups' pair stores assume this field order");
-__device__ __forceinline__ size_t rec_blk(int p, int w, int nw) { return ((size_t)(p - 6) * nw + w) * kBlk; }
-__device__ __forceinline__ size_t rec_cell(int i, int j, int nw) {  // the cell's first pair
-  const int r = j - 3;
-  return rec_blk(i + j, r >> 6, nw) + 2 * (r & 63);
-}
+// Sweep records are blocked by (plane, band): block ((p-6)*nw + w) holds the
+// 64 rows 3+64w .. 3+64w+63, pair q of row 3+64w+l at q*128 + 2l, so each pair
+// of fields of a plane is one contiguous 1 KiB load per wavefront.  dU*, the
+// updated state and the geometry weights use the same blocks with 2, 2 and
+// geo_pairs pairs.  Every array stays below 2 GiB (synthetic_init), so byte
+// offsets fit the 32-bit buffer offsets.
+constexpr int kBlk = kNRec * 64;      // doubles per block
+constexpr int kBlk4 = 4 * 64;         // the same of dU* and of the updated state
+__host__ __device__ inline int geo_pairs(bool axis) { return axis ? 2 : 6; }
+static_assert(kRecRes == 0 && kRecU == 4 && kRecRa == 8 && kRecCbi == 9 && kRecCbj == 10 && kRecRr == 11 &&
+                  kNRec == 12,
+              "the loaders' pair loads and the flux workgroups' pair stores assume this field order");
+// block and row-in-block of a cell
+__device__ __forceinline__ int blk_of(int i, int j, int nw) { return (i + j - 6) * nw + ((j - 3) >> 6); }
 
-// The record array as a raw buffer; loads and stores through it carry sc1,
-// the cache policy of ld_agent / st_agent, so they are coherent across the
-// device's XCDs.
+// Record, dU*, state and hand-off arrays as raw buffers; loads and stores
+// through them carry sc1, the cache policy of ld_agent / st_agent, so they are
+// coherent across the device's XCDs.
 constexpr int kBufWord3 = 0x00020000;  // gfx9-family descriptor word 3 (raw buffer, stride 0)
 constexpr int kCoherent = 16;          // buffer instruction cache policy: sc1
+constexpr unsigned kOff = 0x80000000u;  // past every buffer's range: a store there is discarded
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
-typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 // Global-memory views of the mesh arrays: loads through them are global
 // loads also where the compiler cannot infer the address space of a Dev
 // field (the flux workgroups' function, the batched kernel's job table)
 typedef const __attribute__((address_space(1))) double gdbl;
 __device__ __forceinline__ gdbl *gp(const double *p) { return (gdbl *)p; }
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rec_rsrc(const SyntheticState &st) {
-  return __builtin_amdgcn_make_buffer_rsrc(st.rec, (short)0, (int)((size_t)st.np * st.nw * kBlk * sizeof(double)),
-                                           kBufWord3);
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_of(double *p, size_t doubles) {
+  return __builtin_amdgcn_make_buffer_rsrc(p, (short)0, (int)(doubles * sizeof(double)), kBufWord3);
 }
-__device__ __forceinline__ void st_pair(__amdgpu_buffer_rsrc_t r, unsigned byte_off, double a, double b) {
-  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, double2{a, b}), r, byte_off, 0, kCoherent);
+__device__ __forceinline__ size_t nblocks(const SyntheticState &st) { return (size_t)st.np * st.nw; }
+// dU* and the updated state have kPad more planes at either end, which the
+// steps of a last group past the band's last plane store to
+__device__ __forceinline__ size_t padded_blocks(const SyntheticState &st) { return (size_t)(st.np + 2 * kPad) * st.nw; }
+__device__ __forceinline__ int pblk_of(int i, int j, int nw) { return (i + j - 6 + kPad) * nw + ((j - 3) >> 6); }
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rec_rsrc(const SyntheticState &st) {
+  return rsrc_of(st.rec, nblocks(st) * kBlk);
+}
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t ub_rsrc(const SyntheticState &st) {
+  return rsrc_of(st.ub, padded_blocks(st) * kBlk4);
+}
+__device__ __forceinline__ void st_pair(__amdgpu_buffer_rsrc_t r, unsigned voff, int soff, double a, double b) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, double2{a, b}), r, voff, soff, kCoherent);
 }
 __device__ __forceinline__ double2 ld_pair(__amdgpu_buffer_rsrc_t r, unsigned voff, int soff) {
   return __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, kCoherent));
 }
+// hand-off slots [2 directions][nw bands][nx-5+kPad][4]: the values that the
+// edge row of a band passes to the next band, in the order they are made (the
+// last kPad are not read).  A slot
+// whose doubles hold kEmpty has not been written: a signalling NaN, which no
+// arithmetic returns, so each double of a slot says by itself whether it is
+// there, and no flag has to follow the data.
+constexpr unsigned long long kEmpty = 0x7FF4A5A5A5A5A5A5ull;
+constexpr unsigned kEmptyHi = (unsigned)(kEmpty >> 32);
+__host__ __device__ inline int hand_len(int nx) { return nx - 5 + kPad; }
+__device__ __forceinline__ double *hand_of(const Dev &d, const SyntheticState &st, bool fwd, int band) {
+  return st.hand + (size_t)((fwd ? 0 : st.nw) + band) * hand_len(d.nx) * 4;
+}
 
-// Every record slot's density field and its reciprocal to 1 (the rest stays
-// zero): the slots of cells that are not swept keep this finite state for good.
-__global__ void k_rec_init(SyntheticState st) {
-  const size_t nslot = (size_t)st.np * st.nw * 64;
+// Every record slot's density and its reciprocal to 1 (the rest stays zero):
+// the slots of cells that are not swept keep this finite state for good.  The
+// geometry that a cell's terms take, which does not change.  Forward: half
+// lengths and normals of the faces towards i+1 and j+1.  Backward: half
+// lengths of the cell's own lower faces, and the normals of the lower faces of
+// (i-1,j) and (i,j-1), which the reference takes there (src/sub_LU_SGS.f90:82-96).
+__global__ void k_rec_init(Dev d, SyntheticState st) {
+  const size_t nslot = nblocks(st) * 64;
   const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= nslot) return;
   const size_t blk = t / 64, l = t % 64;
   st.rec[blk * kBlk + (kRecU / 2) * 128 + 2 * l] = 1.0;
   st.rec[blk * kBlk + (kRecRr / 2) * 128 + 2 * l + 1] = 1.0;
+  const int p = (int)(blk / st.nw) + 6, j = 3 + 64 * (int)(blk % st.nw) + (int)l, i = p - j;
+  if (j > d.ny - 3 || i < 3 || i > d.nx - 3) return;
+  const int gpn = geo_pairs(st.axis), g0 = gidx(d, i, j), gi = gidx(d, i + 1, j), gj = gidx(d, i, j + 1);
+  double2 *g = reinterpret_cast<double2 *>(st.geo + blk * gpn * 128) + l;
+  g[0] = {0.5 * d.si[gi], 0.5 * d.sj[gj]};
+  g[64] = {0.5 * d.si[g0], 0.5 * d.sj[g0]};
+  if (st.axis) return;
+  g[128] = {d.ni1[gi], d.ni2[gi]};
+  g[192] = {d.nj1[gj], d.nj2[gj]};
+  const int hi = gidx(d, i - 1, j), hj = gidx(d, i, j - 1);
+  g[256] = {d.ni1[hi], d.ni2[hi]};
+  g[320] = {d.nj1[hj], d.nj2[hj]};
+}
+
+// every hand-off slot empty, by the threads t, t + nt, ... of a launch
+__device__ void clear_hands(const Dev &d, const SyntheticState &st, size_t t, size_t nt) {
+  const size_t n = (size_t)2 * st.nw * hand_len(d.nx) * 4;
+  for (; t < n; t += nt) st.hand[t] = __longlong_as_double((long long)kEmpty);
 }
 
 // S0 <- S - S0, S00 <- S on interior cells; the kinetic increment added to the
@@ -116,14 +182,17 @@ __global__ void k_ns_prepare(Dev d, SyntheticState st) {
   if (t == 0) {
     st.ctl[kCtlGo] = (1.0 > st.tol && st.maxit > 0) ? 1 : -1;  // the reference starts from res = 1
     st.ctl[kCtlErr] = 0;
+    st.ctl[kCtlBad] = 0;
+    st.ctl[kCtlStop] = 0;
+    st.ctl[kCtlLast] = 0;
+    st.ctl[kCtlArrived] = 0;
     st.iters[0] = 0;
     st.iters[1] = 0;
     st.iters[2] = 0;
   }
-  if (t < st.nflux) {  // per flux workgroup: no iteration done, no T<0.1
-    reinterpret_cast<int *>(st.part + 8 * t)[0] = 0;
-    reinterpret_cast<int *>(st.part + 8 * t)[1] = 0;
-  }
+  if (t < st.ntx * st.nty) st.ready[t] = 0;      // no iteration's fluxes done
+  if (t < st.nw) st.prog[kProgStride * t] = 0;   // no plane of a backward sweep done
+  clear_hands(d, st, t, (size_t)gridDim.x * blockDim.x);
   const int nc = (d.nx - 1) * (d.ny - 1);
   if (t >= nc) return;
   const int i = t % (d.nx - 1) + 1, j = t / (d.nx - 1) + 1;
@@ -190,101 +259,145 @@ __device__ void van_leer(const double ql[4], const double qr[4], double g, doubl
 // comput_DFn (src/sub_LU_SGS.f90:122-143): DF = F.n(U + dU) - F.n(U) on the
 // unit normal (n1, n2).  F.n is linear in n: F.n = Fx n1 + Fy n2 with the
 // Euler fluxes Fx, Fy of the state, so a cell's DF on any normal is
-// (Fx(U+dU) - Fx(U)) n1 + (Fy(U+dU) - Fy(U)) n2.  The sweep forms the two
-// differences once per cell, when its dU is known, and both cells that take
-// it as a neighbour (its i+1 and its j+1 forward, i-1 and j-1 backward)
-// project them on their own normals.  1/rho is shared by the velocities and
-// the pressure (hardware reciprocal and two Newton steps, about 1 ulp).
-__device__ __forceinline__ double rcp_nr(double a) {
-  double r = __builtin_amdgcn_rcp(a);
-  double e = fma(-a, r, 1.0);
-  r = fma(r, e, r);
-  e = fma(-a, r, 1.0);
-  return fma(r, e, r);
-}
-// Fx(u), Fy(u) with r = 1/u[0] as rcp_nr forms it
-__device__ __forceinline__ void fxy_r(const double u[4], double r, double g, double fx[4], double fy[4]) {
-  const double vx = u[1] * r, vy = u[2] * r;
-  const double p = (g - 1.0) * (u[3] - 0.5 * (u[1] * u[1] + u[2] * u[2]) * r);
-  const double e = u[3] + p;
-  fx[0] = u[1];
-  fx[1] = u[1] * vx + p;
-  fx[2] = u[2] * vx;
-  fx[3] = e * vx;
-  fy[0] = u[2];
-  fy[1] = u[1] * vy;
-  fy[2] = u[2] * vy + p;
-  fy[3] = e * vy;
-}
-__device__ __forceinline__ void fxy(const double u[4], double g, double fx[4], double fy[4]) {
-  fxy_r(u, rcp_nr(u[0]), g, fx, fy);
-}
-// DF of state u and increment du on (n1, n2) in the reference's form (the
-// sweep of the launch for more than 256 swept rows carries states)
-__device__ __forceinline__ void dfn(const double u[4], const double du[4], double n1, double n2, double g,
-                                    double df[4]) {
-  double u2[4];
-  for (int m = 0; m < 4; m++) u2[m] = u[m] + du[m];
-  const double r1 = rcp_nr(u[0]), r2 = rcp_nr(u2[0]);
-  const double un1 = (u[1] * n1 + u[2] * n2) * r1;
-  const double p1 = (g - 1.0) * (u[3] - 0.5 * (u[1] * u[1] + u[2] * u[2]) * r1);
-  const double un2 = (u2[1] * n1 + u2[2] * n2) * r2;
-  const double p2 = (g - 1.0) * (u2[3] - 0.5 * (u2[1] * u2[1] + u2[2] * u2[2]) * r2);
-  df[0] = u2[0] * un2 - u[0] * un1;
-  df[1] = (u2[1] * un2 + p2 * n1) - (u[1] * un1 + p1 * n1);
-  df[2] = (u2[2] * un2 + p2 * n2) - (u[2] * un1 + p1 * n2);
-  df[3] = (u2[3] + p2) * un2 - (u[3] + p1) * un1;
-}
+// (Fx(U+dU) - Fx(U)) n1 + (Fy(U+dU) - Fy(U)) n2.  The first components of the
+// two differences are dU(2) and dU(3), and Fx(3) = Fy(2), so five components
+// are left to form.
 
-struct NsShared {
-  // sweep: lane 63 (forward) or lane 0 (backward) of wavefront w hands its
-  // row's values of step s to the neighbouring wavefront in slot s % kRing,
-  // at xw[(w * kRingMax + slot) * kSlot] (first in the struct: slot
-  // addresses then fit the LDS instructions' offset fields)
-  double xw[kMaxSweepWaves * kRingMax * kSlot];
+// 1/a: the hardware reciprocal (23 bits) and one step r(1 + e + e^2), e =
+// 1 - a r, whose error is e^3: about 1 ulp
+__device__ __forceinline__ double rcp_nr(double a) {
+  const double r = __builtin_amdgcn_rcp(a);
+  const double e = fma(-a, r, 1.0);
+  return fma(r, fma(e, e, e), r);
+}
+// velocities, pressure and pressure + energy of a state with r = 1/u[0]
+struct Euler {
+  double vx, vy, p, e;
+  __device__ Euler(const double u[4], double r, double g1) {
+    const double kin = fma(u[1], u[1], u[2] * u[2]);
+    const double ei = fma(-0.5 * kin, r, u[3]);
+    p = g1 * ei;
+    e = fma(g1, ei, u[3]);
+    vx = u[1] * r;
+    vy = u[2] * r;
+  }
+};
+
+// a flux workgroup's tile
+struct FluxShared {
   double U[4][kTC];    // tile + halo
   double pr[5][kTC];   // d, u, v, T, p (comput_duvtpckw)
   double mu[kTC];      // amu_of
-  double fi[4][kNFace];  // i-face fluxes, face (i0+a, j0+b) at b*(kTile+1)+a
-  double fj[4][kNFace];  // j-face fluxes, face (i0+a, j0+b) at b*kTile+a
-  int prog[kMaxSweepWaves];  // steps a wavefront has handed on
-  int cons[kMaxSweepWaves];  // steps whose hand-off a wavefront has taken
-  int abort;                 // a hand-off wait timed out
-  double red[kMaxSweepWaves];
+  double fi[4][(kTI + 1) * kTJ];  // i-face fluxes, face (i0+a, j0+b) at b*(kTI+1)+a
+  double fj[4][kTI * (kTJ + 1)];  // j-face fluxes, face (i0+a, j0+b) at b*kTI+a
+  double red[kThreads / 64];
   int word;
+};
+// a sweep workgroup's records and words (see sweep_pass)
+constexpr int kLdsPairs = 9;  // pairs of a prepared record, without the normals
+template <bool kAxis>
+struct SweepShared {
+  static constexpr int kPairs = kAxis ? kLdsPairs : kLdsPairs + 2;
+  static constexpr int kStep = kPairs * 128;  // doubles of a step's records
+  double ring[kGroups * kGroup][kPairs * 128];  // prepared records, pair q of lane l at q*128 + 2l
+  double hand[kHand + 2][4];         // values received from the neighbouring band; two that stay zero
+  int avail[kGroups];  // 1 + the running number of the group of steps that a ring slot holds
+  int used;            // half groups whose records the sweep has read
+  int hand_n;          // values received
+  int fwd_done, bwd_done;  // iterations whose sweeps are complete, their stores at memory
+  int bgo;             // iterations whose backward sweep may begin
+  int clr;             // iterations after whose backward sweep its hand-off slots are empty again
+  int quit;            // a wait timed out, or the loop has ended
 };
 
 // the tile's cell fields for ns_face_of
 struct TileCells {
-  const NsShared &sh;
-  const Dev &d;
+  const FluxShared &sh;
   int ib, jb;  // cell (ib, jb) is LDS cell 0
-  __device__ int l(int i, int j) const { return (j - jb) * kTW + (i - ib); }
+  __device__ int l(int i, int j) const { return (j - jb) * kCI + (i - ib); }
   __device__ double u(int i, int j) const { return sh.pr[1][l(i, j)]; }
   __device__ double v(int i, int j) const { return sh.pr[2][l(i, j)]; }
   __device__ double T(int i, int j) const { return sh.pr[3][l(i, j)]; }
   __device__ double mu(int i, int j) const { return sh.mu[l(i, j)]; }
+};
+struct MeshCells {
+  const Dev &d;
   __device__ double x1(int i, int j) const { return gp(d.x1)[cidx(d, i, j)]; }
   __device__ double y1(int i, int j) const { return gp(d.y1)[cidx(d, i, j)]; }
 };
 
-// Residual_FVM face flux (src/sub_Residual.f90:68-202, :210-338) of face
-// (i,j), primitives from the tile in LDS
-__device__ void face_flux(const Dev &d, const TileCells &tc, int dir, int i, int j, bool visc, double fl[4]) {
-  const NsShared &sh = tc.sh;
+// What a thread's part of a tile takes from the mesh, read before the wait for
+// the tile's state: a face (threads below kFaceThreads), or kCells cells.
+constexpr int kFaceThreads = kThreads - 64;                 // the last wavefront has the cells
+constexpr int kCells = (kTI * kTJ + 63) / 64;
+static_assert((kTI + 1) * kTJ + kTI * (kTJ + 1) <= kFaceThreads, "a face per thread");
+struct TileGeo {
+  int i0, j0, nci, ncj;
+  int dir, i, j;  // face; dir < 0: none
+  double s, n1, n2, t11, t22, t12, qx, qy;
+  NsMetric m;
+  double vol[kCells], si[kCells], sj[kCells], ni1[kCells], ni2[kCells], nj1[kCells], nj2[kCells];
+};
+// cell t of a tile: threads run along wrapped anti-diagonals, whose cells are
+// consecutive in the blocked arrays
+__device__ __forceinline__ int cell_b(int t) { return t % kTJ; }
+__device__ __forceinline__ int cell_a(int t) { return (t / kTJ - t % kTJ) & (kTI - 1); }
+
+__device__ __forceinline__ void tile_geo(const Dev &d, const SyntheticState &st, int tile, TileGeo &g) {
+  const int tid = threadIdx.x;
+  g.i0 = 3 + (tile % st.ntx) * kTI;
+  g.j0 = 3 + (tile / st.ntx) * kTJ;
+  g.nci = min(kTI, d.nx - 3 - g.i0 + 1);
+  g.ncj = min(kTJ, d.ny - 3 - g.j0 + 1);
+  g.dir = -1;
+  if (tid < kFaceThreads) {
+    const int nfi = (g.nci + 1) * g.ncj, nfj = g.nci * (g.ncj + 1);
+    if (tid >= nfi + nfj) return;
+    g.dir = tid < nfi ? 0 : 1;
+    g.i = g.i0 + (g.dir == 0 ? tid % (g.nci + 1) : (tid - nfi) % g.nci);
+    g.j = g.j0 + (g.dir == 0 ? tid / (g.nci + 1) : (tid - nfi) / g.nci);
+    const int q = gidx(d, g.i, g.j), c = cidx(d, g.i, g.j), N = d.ncell;
+    g.s = gp(g.dir == 0 ? d.si : d.sj)[q];
+    g.n1 = gp(g.dir == 0 ? d.ni1 : d.nj1)[q];
+    g.n2 = gp(g.dir == 0 ? d.ni2 : d.nj2)[q];
+    if (!st.if_viscous) return;
+    gdbl *tg = gp(g.dir == 0 ? d.taoi : d.taoj), *qg = gp(g.dir == 0 ? d.qi : d.qj);
+    g.t11 = tg[c];
+    g.t22 = tg[N + c];
+    g.t12 = tg[2 * N + c];
+    g.qx = qg[c];
+    g.qy = qg[N + c];
+    g.m = ns_metric_of(MeshCells{d}, g.dir, g.i, g.j);
+    return;
+  }
+#pragma unroll
+  for (int r = 0; r < kCells; r++) {
+    const int t = tid - kFaceThreads + 64 * r, i = g.i0 + min(cell_a(t), g.nci - 1), j = g.j0 + min(cell_b(t), g.ncj - 1);
+    const int g0 = gidx(d, i, j), gi = gidx(d, i + 1, j), gj = gidx(d, i, j + 1);
+    g.vol[r] = gp(d.vol)[g0];
+    g.si[r] = 0.5 * (gp(d.si)[g0] + gp(d.si)[gi]);
+    g.ni1[r] = 0.5 * (gp(d.ni1)[g0] + gp(d.ni1)[gi]);
+    g.ni2[r] = 0.5 * (gp(d.ni2)[g0] + gp(d.ni2)[gi]);
+    g.sj[r] = 0.5 * (gp(d.sj)[g0] + gp(d.sj)[gj]);
+    g.nj1[r] = 0.5 * (gp(d.nj1)[g0] + gp(d.nj1)[gj]);
+    g.nj2[r] = 0.5 * (gp(d.nj2)[g0] + gp(d.nj2)[gj]);
+  }
+}
+
+// Residual_FVM face flux (src/sub_Residual.f90:68-202, :210-338) of the
+// thread's face, primitives from the tile in LDS
+__device__ __forceinline__ void face_flux(const Dev &d, const FluxShared &sh, const TileGeo &g, bool visc,
+                                          double fl[4]) {
+  const TileCells tc{sh, g.i0 - 2, g.j0 - 2};
+  const int c0 = tc.l(g.i, g.j), step = g.dir == 0 ? 1 : kCI;
   double ul[4], ur[4];
   for (int m = 0; m < 4; m++) {
-    const double *q = sh.pr[m < 3 ? m : 4];  // d, u, v, p
-    double u1, u2, u3, u4;
-    if (dir == 0) { u1 = q[tc.l(i - 2, j)]; u2 = q[tc.l(i - 1, j)]; u3 = q[tc.l(i, j)]; u4 = q[tc.l(i + 1, j)]; }
-    else { u1 = q[tc.l(i, j - 2)]; u2 = q[tc.l(i, j - 1)]; u3 = q[tc.l(i, j)]; u4 = q[tc.l(i, j + 1)]; }
+    const double *q = sh.pr[m < 3 ? m : 4] + c0;  // d, u, v, p
+    const double u1 = q[-2 * step], u2 = q[-step], u3 = q[0], u4 = q[step];
     ul[m] = u2 + 0.5 * minmod_ns(u2 - u1, u3 - u2);
     ur[m] = u3 - 0.5 * minmod_ns(u3 - u2, u4 - u3);
   }
-  const int g = gidx(d, i, j);
-  double s, n1, n2;
-  if (dir == 0) { s = gp(d.si)[g]; n1 = gp(d.ni1)[g]; n2 = gp(d.ni2)[g]; }
-  else { s = gp(d.sj)[g]; n1 = gp(d.nj1)[g]; n2 = gp(d.nj2)[g]; }
+  const double s = g.s, n1 = g.n1, n2 = g.n2;
   const double ql[4] = {ul[0], ul[1] * n1 + ul[2] * n2, -ul[1] * n2 + ul[2] * n1, ul[3]};
   const double qr[4] = {ur[0], ur[1] * n1 + ur[2] * n2, -ur[1] * n2 + ur[2] * n1, ur[3]};
   double f0[4];
@@ -295,12 +408,9 @@ __device__ void face_flux(const Dev &d, const TileCells &tc, int dir, int i, int
   fl[3] = -f0[3] * s;
   if (!visc) return;
   double o[8];
-  ns_face_of(tc, d, dir, i, j, o);
-  const int N = d.ncell, c = cidx(d, i, j);
-  gdbl *tg = gp(dir == 0 ? d.taoi : d.taoj);
-  gdbl *qg = gp(dir == 0 ? d.qi : d.qj);
-  const double t11 = o[0] + tg[c], t22 = o[1] + tg[N + c], t12 = o[2] + tg[2 * N + c];
-  const double qx = o[4] + qg[c], qy = o[5] + qg[N + c];
+  ns_face_of(tc, d, g.m, g.dir, g.i, g.j, o);
+  const double t11 = o[0] + g.t11, t22 = o[1] + g.t22, t12 = o[2] + g.t12;
+  const double qx = o[4] + g.qx, qy = o[5] + g.qy;
   const double u1 = o[6], v1 = o[7];
   const double e1 = u1 * t11 + v1 * t12 + qx;
   const double e2 = u1 * t12 + v1 * t22 + qy;
@@ -312,503 +422,622 @@ __device__ void face_flux(const Dev &d, const TileCells &tc, int dir, int i, int
 // One tile of Comput_Residual_one_mesh (src/sub_NS_singlegrid.f90:45-114):
 // comput_duvtpckw with its T<0.1 stop, get_viscous, the face fluxes, Res,
 // comput_Lvc, comput_dt and the LU-SGS diagonal (src/sub_LU_SGS.f90:34-36),
-// stored as sweep records.  Returns this tile's max |Res_4| and T<0.1 flag.
-__device__ void flux_tile(const Dev &d, const SyntheticState &st, NsShared &sh, int tile, double &rmax, int &bad) {
-  const int nx = d.nx, ny = d.ny, N = d.ncell;
-  const int tid = threadIdx.x, nt = blockDim.x;
+// stored as sweep records.  Returns the thread's max |Res_4| and T<0.1 flag.
+// The time of a tile is the chain of its phases (state, faces, residual), not
+// their work: the last wavefront forms what the cells need besides the fluxes
+// beside the faces.
+__device__ __forceinline__ void flux_tile(const Dev &d, const SyntheticState &st, FluxShared &sh, const TileGeo &tg,
+                                          bool first, double &rmax, int &bad) {
+  const int nx = d.nx, ny = d.ny, N = d.ncell, i0 = tg.i0, j0 = tg.j0;
+  const int tid = threadIdx.x, nw = st.nw;
   const double g = d.gamma;
   const bool visc = st.if_viscous != 0;
-  const int i0 = 3 + (tile % st.ntx) * kTile, j0 = 3 + (tile / st.ntx) * kTile;
-  const int ilast = min(i0 + kTile - 1, nx - 3), jlast = min(j0 + kTile - 1, ny - 3);
-  const int nci = ilast - i0 + 1, ncj = jlast - j0 + 1;
-  const TileCells tc{sh, d, i0 - 2, j0 - 2};
-  for (int t = tid; t < kTC; t += nt) {
-    const int i = i0 - 2 + t % kTW, j = j0 - 2 + t / kTW;
-    if (i > nx + 1 || j > ny + 1) continue;
-    const int c = cidx(d, i, j);
-    double u[4];
-    for (int m = 0; m < 4; m++) {
-      u[m] = __hip_atomic_load(gp(d.U) + m * N + c, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      sh.U[m][t] = u[m];
-    }
-    const double dd = u[0], uu = u[1] / dd, vv = u[2] / dd;
-    const double T = (u[3] - 0.5 * dd * (uu * uu + vv * vv)) / (d.cv * dd);
-    sh.pr[0][t] = dd;
-    sh.pr[1][t] = uu;
-    sh.pr[2][t] = vv;
-    sh.pr[3][t] = T;
-    sh.pr[4][t] = (1. / (g * d.ma * d.ma)) * dd * T;
-    sh.mu[t] = visc ? 1. / d.re * pow(T, 0.8100000023841858) : 0.0;
-    if (i >= 1 && i <= nx - 1 && j >= 1 && j <= ny - 1 && T < 0.10000000149011612) bad = 1;
-  }
-  __syncthreads();
-  const int nfi = (nci + 1) * ncj, nfj = nci * (ncj + 1);
-  for (int t = tid; t < nfi + nfj; t += nt) {
-    double fl[4];
-    if (t < nfi) {
-      const int a = t % (nci + 1), b = t / (nci + 1);
-      face_flux(d, tc, 0, i0 + a, j0 + b, visc, fl);
-      for (int m = 0; m < 4; m++) sh.fi[m][b * (kTile + 1) + a] = fl[m];
-    } else {
-      const int a = (t - nfi) % nci, b = (t - nfi) / nci;
-      face_flux(d, tc, 1, i0 + a, j0 + b, visc, fl);
-      for (int m = 0; m < 4; m++) sh.fj[m][b * kTile + a] = fl[m];
+  const TileCells tc{sh, i0 - 2, j0 - 2};
+  // U of the loop's start is in the mesh array; later iterations read the
+  // swept cells from the sweeps' blocked array
+  const __amdgpu_buffer_rsrc_t ru = ub_rsrc(st);
+  static_assert(kTC <= kThreads, "a cell with halo per thread");
+  if (tid < kTC) {
+    const int b = tid % kCJ, a = (tid / kCJ + 2 * kCI - b) % kCI;
+    const int i = i0 - 2 + a, j = j0 - 2 + b, l = b * kCI + a;
+    if (i <= nx + 1 && j <= ny + 1) {
+      double u[4];
+      if (!first && i >= 3 && i <= nx - 3 && j >= 3 && j <= ny - 3) {
+        const unsigned o = (unsigned)pblk_of(i, j, nw) * (kBlk4 * 8u) + 16u * ((j - 3) & 63);
+        const double2 u01 = ld_pair(ru, o, 0), u23 = ld_pair(ru, o + 1024u, 0);
+        u[0] = u01.x; u[1] = u01.y; u[2] = u23.x; u[3] = u23.y;
+      } else {
+        const int c = cidx(d, i, j);
+        for (int m = 0; m < 4; m++) u[m] = gp(d.U)[m * N + c];
+      }
+      for (int m = 0; m < 4; m++) sh.U[m][l] = u[m];
+      const double dd = u[0], uu = u[1] / dd, vv = u[2] / dd;
+      const double T = (u[3] - 0.5 * dd * (uu * uu + vv * vv)) / (d.cv * dd);
+      sh.pr[0][l] = dd;
+      sh.pr[1][l] = uu;
+      sh.pr[2][l] = vv;
+      sh.pr[3][l] = T;
+      sh.pr[4][l] = (1. / (g * d.ma * d.ma)) * dd * T;
+      sh.mu[l] = visc ? 1. / d.re * pow(T, 0.8100000023841858) : 0.0;
+      if (i >= 1 && i <= nx - 1 && j >= 1 && j <= ny - 1 && T < 0.10000000149011612) bad = 1;
     }
   }
   __syncthreads();
-  const int nw = st.nw;
   const __amdgpu_buffer_rsrc_t rr = rec_rsrc(st);
-  for (int t = tid; t < nci * ncj; t += nt) {
-    const int a = t % nci, b = t / nci, i = i0 + a, j = j0 + b;
-    double res[4];
-    for (int m = 0; m < 4; m++)
-      res[m] = sh.fi[m][b * (kTile + 1) + a + 1] - sh.fi[m][b * (kTile + 1) + a] + sh.fj[m][(b + 1) * kTile + a] -
-               sh.fj[m][b * kTile + a];
-    rmax = fmax(rmax, fabs(res[3]));
-    // comput_Lvc and comput_dt (src/sub_NS_singlegrid.f90:160-221)
-    const int g0 = gidx(d, i, j), gi = gidx(d, i + 1, j), gj = gidx(d, i, j + 1);
-    gdbl *gvol = gp(d.vol), *gsi = gp(d.si), *gsj = gp(d.sj);
-    gdbl *gni1 = gp(d.ni1), *gni2 = gp(d.ni2), *gnj1 = gp(d.nj1), *gnj2 = gp(d.nj2);
-    const double s0 = gvol[g0];
-    const double si = 0.5 * (gsi[g0] + gsi[gi]);
-    const double ni1 = 0.5 * (gni1[g0] + gni1[gi]), ni2 = 0.5 * (gni2[g0] + gni2[gi]);
-    const double sj = 0.5 * (gsj[g0] + gsj[gj]);
-    const double nj1 = 0.5 * (gnj1[g0] + gnj1[gj]), nj2 = 0.5 * (gnj2[g0] + gnj2[gj]);
-    const int lc = tc.l(i, j);
-    const double uu = sh.pr[1][lc], vv = sh.pr[2][lc];
-    const double uni = uu * ni1 + vv * ni2, unj = uu * nj1 + vv * nj2;
-    const double cc = sqrt(sh.pr[3][lc]) / d.ma;
-    const double lci = (fabs(uni) + cc) * si, lcj = (fabs(unj) + cc) * sj;
-    const double tmp1 = g / sh.pr[0][lc] * (sh.mu[lc] / d.pr + 0.0 / 0.9);
-    const double lvi = visc ? tmp1 * si * si / s0 : 0.0, lvj = visc ? tmp1 * sj * sj / s0 : 0.0;
-    double dt;
-    if (!st.local_dt) dt = d.dt;
-    else {
-      dt = st.cfl * gvol[g0] / (lci + lcj + 1.0 * (lvi + lvj));
-      if (dt > st.dtmax) dt = st.dtmax;
-      if (dt < st.dtmin) dt = st.dtmin;
+  if (tid < kFaceThreads) {
+    if (tg.dir >= 0) {
+      double fl[4];
+      face_flux(d, sh, tg, visc, fl);
+      const int a = tg.i - i0, b = tg.j - j0;
+      if (tg.dir == 0)
+        for (int m = 0; m < 4; m++) sh.fi[m][b * (kTI + 1) + a] = fl[m];
+      else
+        for (int m = 0; m < 4; m++) sh.fj[m][b * kTI + a] = fl[m];
     }
-    double alfa = gvol[g0] / dt + 1.0 * (lci + lcj);
-    if (visc) alfa = alfa + 2.0 * (lvi + lvj);
-    const unsigned o = (unsigned)(rec_cell(i, j, nw) * sizeof(double));
-    st_pair(rr, o + (kRecRes / 2) * 1024, res[0], res[1]);
-    st_pair(rr, o + (kRecRes / 2 + 1) * 1024, res[2], res[3]);
-    st_pair(rr, o + (kRecU / 2) * 1024, sh.U[0][lc], sh.U[1][lc]);
-    st_pair(rr, o + (kRecU / 2 + 1) * 1024, sh.U[2][lc], sh.U[3][lc]);
-    st_pair(rr, o + (kRecRa / 2) * 1024, 1.0 / alfa, 0.5 * lci + lvi);                // ra, cbi
-    // si/2 and sj/2 weigh the forward sweep's terms across the cell's lower
-    // faces; on the first swept column (row) the cell across is not swept and
-    // the term is left out (src/sub_LU_SGS.f90:44-56): a zero weight leaves it
-    // out without a test in the sweep (the backward sweep reads these of cells
-    // i+1, j+1 >= 4 only)
-    const double hsi = i == 3 ? 0.0 : 0.5 * gsi[g0], hsj = j == 3 ? 0.0 : 0.5 * gsj[g0];
-    st_pair(rr, o + (kRecCbj / 2) * 1024, 0.5 * lcj + lvj, hsi);  // cbj, hsi
-    st_pair(rr, o + (kRecHsj / 2) * 1024, hsj, rcp_nr(sh.U[0][lc]));  // hsj, 1/rho
-    st_pair(rr, o + (kRecNi / 2) * 1024, gni1[g0], gni2[g0]);     // ni1, ni2
-    st_pair(rr, o + (kRecNj / 2) * 1024, gnj1[g0], gnj2[g0]);     // nj1, nj2
-  }
-  __syncthreads();  // the next tile reuses the LDS
-}
-
-__device__ __forceinline__ void barrier_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// x of lane l-1 (wave_shr:1) or l+1 (wave_shl:1) of the wavefront; 0 in the
-// lane that has no such neighbour (lane 0, or lane 63)
-__device__ __forceinline__ double lane_shift(double x, bool up) {
-  const unsigned long long b = __double_as_longlong(x);
-  int lo = (int)(unsigned)b, hi = (int)(unsigned)(b >> 32);
-  if (up) {
-    lo = __builtin_amdgcn_mov_dpp(lo, 0x138, 0xf, 0xf, true);
-    hi = __builtin_amdgcn_mov_dpp(hi, 0x138, 0xf, 0xf, true);
   } else {
-    lo = __builtin_amdgcn_mov_dpp(lo, 0x130, 0xf, 0xf, true);
-    hi = __builtin_amdgcn_mov_dpp(hi, 0x130, 0xf, 0xf, true);
+#pragma unroll
+    for (int r = 0; r < kCells; r++) {
+      const int t = tid - kFaceThreads + 64 * r, a = cell_a(t), b = cell_b(t), i = i0 + a, j = j0 + b;
+      if (t >= kTI * kTJ || a >= tg.nci || b >= tg.ncj) continue;
+      // comput_Lvc and comput_dt (src/sub_NS_singlegrid.f90:160-221)
+      const int lc = tc.l(i, j);
+      const double s0 = tg.vol[r], si = tg.si[r], sj = tg.sj[r];
+      const double uu = sh.pr[1][lc], vv = sh.pr[2][lc];
+      const double uni = uu * tg.ni1[r] + vv * tg.ni2[r], unj = uu * tg.nj1[r] + vv * tg.nj2[r];
+      const double cc = sqrt(sh.pr[3][lc]) / d.ma;
+      const double lci = (fabs(uni) + cc) * si, lcj = (fabs(unj) + cc) * sj;
+      const double tmp1 = g / sh.pr[0][lc] * (sh.mu[lc] / d.pr + 0.0 / 0.9);
+      const double lvi = visc ? tmp1 * si * si / s0 : 0.0, lvj = visc ? tmp1 * sj * sj / s0 : 0.0;
+      double dt;
+      if (!st.local_dt) dt = d.dt;
+      else {
+        dt = st.cfl * s0 / (lci + lcj + 1.0 * (lvi + lvj));
+        if (dt > st.dtmax) dt = st.dtmax;
+        if (dt < st.dtmin) dt = st.dtmin;
+      }
+      double alfa = s0 / dt + 1.0 * (lci + lcj);
+      if (visc) alfa = alfa + 2.0 * (lvi + lvj);
+      const unsigned o = (unsigned)blk_of(i, j, nw) * (kBlk * 8u) + 16u * ((j - 3) & 63);
+      st_pair(rr, o + (kRecU / 2) * 1024u, 0, sh.U[0][lc], sh.U[1][lc]);
+      st_pair(rr, o + (kRecU / 2 + 1) * 1024u, 0, sh.U[2][lc], sh.U[3][lc]);
+      st_pair(rr, o + (kRecRa / 2) * 1024u, 0, 1.0 / alfa, 0.5 * lci + lvi);            // ra, cbi
+      st_pair(rr, o + (kRecCbj / 2) * 1024u, 0, 0.5 * lcj + lvj, rcp_nr(sh.U[0][lc]));  // cbj, 1/rho
+    }
   }
-  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
-// the same, with 1.0 in the lane that has no such neighbour (a density)
-__device__ __forceinline__ double lane_shift_rho(double x, bool up) {
-  const unsigned long long b = __double_as_longlong(x), o = __double_as_longlong(1.0);
-  int lo = (int)(unsigned)b, hi = (int)(unsigned)(b >> 32);
-  const int olo = (int)(unsigned)o, ohi = (int)(unsigned)(o >> 32);
-  if (up) {
-    lo = __builtin_amdgcn_update_dpp(olo, lo, 0x138, 0xf, 0xf, false);
-    hi = __builtin_amdgcn_update_dpp(ohi, hi, 0x138, 0xf, 0xf, false);
-  } else {
-    lo = __builtin_amdgcn_update_dpp(olo, lo, 0x130, 0xf, 0xf, false);
-    hi = __builtin_amdgcn_update_dpp(ohi, hi, 0x130, 0xf, 0xf, false);
-  }
-  return __longlong_as_double((long long)(((unsigned long long)(unsigned)hi << 32) | (unsigned)lo));
-}
-
-// One sweep step's record of a lane's own cell (all of it in the forward
-// sweep; the backward sweep leaves res and reads dU* instead).
-struct Rec {
-  double res[4], ra, ni[2], nj[2], hsi, hsj, u[4], cbi, cbj, rr;
-};
-
-// Every lane loads its row's slot of the plane, whether or not the row has a
-// cell there (the slot exists for every row of a sweep wavefront): nine
-// 16-byte loads, one scalar block offset and immediate pair offsets.  On a
-// mesh whose normals are (1,0) and (0,1) (kAxis) the last two pairs, the
-// normals, are not loaded: seven loads.
-template <bool FWD, bool kAxis>
-__device__ __forceinline__ void load_rec(__amdgpu_buffer_rsrc_t rr, int blk_bytes, __amdgpu_buffer_rsrc_t rd,
-                                         int ds_bytes, int lane, Rec &x) {
-  const unsigned v = (unsigned)lane * 16u;
-  auto pr = [&](int q) { return ld_pair(rr, v + (unsigned)q * 1024u, blk_bytes); };
-  double2 r01, r23;
-  if (FWD) {
-    r01 = pr(kRecRes / 2);
-    r23 = pr(kRecRes / 2 + 1);
-  } else {  // dU* was stored by this lane
-    r01 = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rd, v, ds_bytes, 0));
-    r23 = __builtin_bit_cast(double2, __builtin_amdgcn_raw_buffer_load_b128(rd, v + 1024u, ds_bytes, 0));
-  }
-  const double2 u01 = pr(kRecU / 2), u23 = pr(kRecU / 2 + 1), p4 = pr(kRecRa / 2), p5 = pr(kRecCbj / 2),
-                p6 = pr(kRecHsj / 2);
-  x.res[0] = r01.x; x.res[1] = r01.y; x.res[2] = r23.x; x.res[3] = r23.y;
-  x.u[0] = u01.x; x.u[1] = u01.y; x.u[2] = u23.x; x.u[3] = u23.y;
-  x.ra = p4.x; x.cbi = p4.y;
-  x.cbj = p5.x; x.hsi = p5.y;
-  x.hsj = p6.x;
-  x.rr = p6.y;
-  if (!kAxis) {
-    const double2 p7 = pr(kRecNi / 2), p8 = pr(kRecNj / 2);
-    x.ni[0] = p7.x; x.ni[1] = p7.y;
-    x.nj[0] = p8.x; x.nj[1] = p8.y;
+  __syncthreads();
+  if (tid < kTI * kTJ) {
+    const int a = cell_a(tid), b = cell_b(tid), i = i0 + a, j = j0 + b;
+    if (a < tg.nci && b < tg.ncj) {
+      double res[4];
+      for (int m = 0; m < 4; m++)
+        res[m] = sh.fi[m][b * (kTI + 1) + a + 1] - sh.fi[m][b * (kTI + 1) + a] + sh.fj[m][(b + 1) * kTI + a] -
+                 sh.fj[m][b * kTI + a];
+      rmax = fabs(res[3]);
+      const unsigned o = (unsigned)blk_of(i, j, nw) * (kBlk * 8u) + 16u * ((j - 3) & 63);
+      st_pair(rr, o + (kRecRes / 2) * 1024u, 0, res[0], res[1]);
+      st_pair(rr, o + (kRecRes / 2 + 1) * 1024u, 0, res[2], res[3]);
+    }
   }
 }
 
-// LDS words read and written by several wavefronts of the workgroup
+// x of lane l-1 (FWD, wave_shr:1) or l+1 (wave_shl:1) of the wavefront; edge
+// in the lane that has no such neighbour (lane 0, or lane 63)
+template <bool FWD>
+__device__ __forceinline__ double lane_shift(double x, double edge) {
+  const unsigned long long b = __double_as_longlong(x), e = __double_as_longlong(edge);
+  const int lo = (int)(unsigned)b, hi = (int)(unsigned)(b >> 32), el = (int)(unsigned)e, eh = (int)(unsigned)(e >> 32);
+  constexpr int kCtrl = FWD ? 0x138 : 0x130;
+  const int l = __builtin_amdgcn_update_dpp(el, lo, kCtrl, 0xf, 0xf, false);
+  const int h = __builtin_amdgcn_update_dpp(eh, hi, kCtrl, 0xf, 0xf, false);
+  return __longlong_as_double((long long)(((unsigned long long)(unsigned)h << 32) | (unsigned)l));
+}
+
+// LDS words read and written by several wavefronts of a workgroup; values
+// are wavefront-uniform
 __device__ __forceinline__ int lds_get(int *p) { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP); }
 __device__ __forceinline__ void lds_put(int *p, int v) {
-  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  if ((threadIdx.x & 63) == 0) __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
-// x in a vector register: LDS addresses formed from it keep their constant
-// parts in the instructions' offset fields
-__device__ __forceinline__ int in_vgpr(int x) {
-  asm volatile("" : "+v"(x));
-  return x;
-}
-__device__ __forceinline__ void lgkm_wait() { __builtin_amdgcn_s_waitcnt(0xC07F); }  // lgkmcnt(0)
+__device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 __device__ __forceinline__ void mem_order() { asm volatile("" ::: "memory"); }  // no compiler reordering
+__device__ __forceinline__ void vm_wait() {  // this wavefront's stores are at memory
+  mem_order();
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
+  mem_order();
+}
 
-// Waits until the LDS word *p reaches want; bounded by kWaitTicks, after
-// which (or once another wavefront has timed out) it gives up, sets the
-// workgroup's abort word and the error word, and the sweep runs to its end on
-// whatever values it has, so that every wavefront still reaches the barriers.
-__device__ __forceinline__ void wait_lds(int *p, int want, int *abort, int *err) {
-  if (lds_get(p) >= want || lds_get(abort)) return;
-  const long long t0 = wall_clock64();
-  while (lds_get(p) < want && !lds_get(abort)) {
+// A bounded wait's bookkeeping: every 64 polls it looks for the end of the
+// loop (the error word; for the waits of a sweep, the stop word too) and for
+// the time; a timeout sets the error word.
+struct Patience {
+  int *ctl;
+  long long limit, t0 = 0;
+  int n = 0;
+  __device__ explicit Patience(int *c, long long ticks = kWaitTicks) : ctl(c), limit(ticks) {}
+  __device__ bool over(bool stop_too) {
+    if ((++n & 63) != 0) return false;
+    if (uniform(ld_agent(ctl + kCtlErr)) != 0 || (stop_too && uniform(ld_agent(ctl + kCtlStop)) != 0)) return true;
+    if (n == 64) t0 = wall_clock64();
+    if (wall_clock64() - t0 > limit) {
+      st_agent(ctl + kCtlErr, 1);
+      return true;
+    }
+    return false;
+  }
+};
+
+// Waits until the LDS word *p has reached want (in wrapping order); false
+// when the loop has ended instead.
+template <class Sh>
+__device__ bool wait_lds(int *p, int want, Sh &sh, int *ctl) {
+  Patience pt(ctl);
+  while (uniform(lds_get(p)) - want < 0) {
+    if (uniform(lds_get(&sh.quit))) return false;
     __builtin_amdgcn_s_sleep(1);
-    if (wall_clock64() - t0 > kWaitTicks) {
-      lds_put(abort, 1);
-      st_agent(err, 1);
+    if (pt.over(true)) {
+      lds_put(&sh.quit, 1);
+      return false;
     }
+  }
+  mem_order();
+  return true;
+}
+// Waits for the word after iteration k: whether iteration k+1 runs.
+template <class Sh>
+__device__ bool next_iteration(int k, Sh &sh, int *ctl) {
+  Patience pt(ctl);
+  int go;
+  while ((go = uniform(ld_agent(ctl + kCtlGo))) == k) {
+    if (uniform(lds_get(&sh.quit))) return false;
+    __builtin_amdgcn_s_sleep(4);
+    if (pt.over(true)) {
+      lds_put(&sh.quit, 1);
+      return false;
+    }
+  }
+  mem_order();
+  return go == k + 1;
+}
+
+// the plane steps of a band: rows j0 .. j0+rows-1, planes first .. last
+struct Band {
+  int w, j0, rows, first, last, n, groups;
+  int links;  // values handed from band to band in a sweep
+
+  __device__ Band(const Dev &d, int band) : w(band), j0(3 + kBand * band) {
+    rows = min(kBand, d.ny - 3 - j0 + 1);
+    first = j0 + 3;
+    last = d.nx - 3 + j0 + rows - 1;
+    n = last - first + 1;
+    groups = (n + kGroup - 1) / kGroup;
+    links = d.nx - 5;
+  }
+};
+
+// A prepared record of a lane's cell: Res/alfa (forward) or dU* (backward),
+// U, the inverse diagonal, the weights towards the cells that use this one as
+// their neighbour (hi, hj negated in a backward sweep), and those components
+// of the Euler fluxes of U that are not U's own: f = Fx(2), Fx(3) = Fy(2),
+// Fx(4), Fy(3), Fy(4); ni, nj: the normals of the faces towards those cells.
+struct Rec {
+  double r[4], u[4], ra, cbi, cbj, hi, hj, f[5], ni[2], nj[2];
+};
+template <bool kAxis>
+__device__ __forceinline__ void read_rec(const double *slot, int lane, Rec &x) {
+  const double2 *s = reinterpret_cast<const double2 *>(slot) + lane;
+  const double2 a = s[0], b = s[64], c = s[128], e = s[192], f = s[256], g = s[320], h = s[384], k = s[448], l = s[512];
+  x.r[0] = a.x; x.r[1] = a.y; x.r[2] = b.x; x.r[3] = b.y;
+  x.u[0] = c.x; x.u[1] = c.y; x.u[2] = e.x; x.u[3] = e.y;
+  x.ra = f.x; x.cbi = f.y;
+  x.cbj = g.x; x.hi = g.y;
+  x.hj = h.x; x.f[0] = h.y;
+  x.f[1] = k.x; x.f[2] = k.y;
+  x.f[3] = l.x; x.f[4] = l.y;
+  if (!kAxis) {
+    const double2 o = s[576], q = s[640];
+    x.ni[0] = o.x; x.ni[1] = o.y;
+    x.nj[0] = q.x; x.nj[1] = q.y;
   }
 }
 
-// du_LU_SGS_2D (src/sub_LU_SGS.f90:4-113) and the update of cells 3..n-3.
-// Lane j owns row j (j = 3 + thread index); step p visits plane i + j = p.
-// Each step is straight-line code: every lane issues the same loads and
-// stores (a lane without a cell stores out of the buffer's range, which
-// discards the store), so the waits for a record loaded kDepth - 1 steps
-// earlier do not wait for the later ones.  The loop runs a multiple of kDepth steps;
-// the steps after the last plane have no cell in any row.
-// kDepth records in registers: each step's record is loaded at the start of
-// the step kDepth - 1 steps before it is used (the loads come from the
-// device's coherence point, written by other CUs, and go out among the
-// step's arithmetic), which takes (kDepth - 1) * 34 more VGPRs than one
-// record.
+// One sweep of a band by its sweep wavefront: du_LU_SGS_2D
+// (src/sub_LU_SGS.f90:4-113), forward dU* = (Res + dui + duj)/alfa on planes
+// first .. last (:26-69) or backward dU = dU* + (dui + duj)/alfa on planes
+// last .. first (:73-111) and U + dU.  Lane l owns row j0 + l; a step visits
+// one plane.  The off-diagonal term that cell (i,j) adds to (i+1,j) (forward;
+// (i-1,j) backward) stays in the lane, the one for (i,j+1) moves to the next
+// lane, or through memory to the next band:
+//   forward:  dui = 0.5 (DF si(i,j) + Lci(i-1,j) dU) + Lvi(i-1,j) dU      (:44-49)
+//   backward: dui = -0.5 (DF si(i+1,j) - Lci(i+1,j) dU) + Lvi(i+1,j) dU   (:82-86)
+// with DF = F.n(U+dU) - F.n(U) of the neighbour (comput_DFn, :122-143): all
+// of a term's factors belong to the neighbour and to the face between, so the
+// neighbour forms the whole term and four values move, not eleven.  Terms
+// across faces to cells that are not swept (src/sub_LU_SGS.f90:44-56) vanish
+// without a test: the slots of such cells hold U = (1,0,0,0) and zero weights.
 //
-// What a lane carries from one step to the next: its own cell's dU, flux
-// differences dFx, dFy, Cbi and Hsi (the cell is the i-neighbour of the
-// lane's next one), and the j-neighbour row's dU, dFx, dFy, Cbj and Hsj,
-// shifted in from the next lane at the end of the step (in the edge lane:
-// from the neighbouring wavefront, below).  The launch for more than 256
-// swept rows (kDiff false) carries the states U instead and forms DF in the
-// reference's form: with flux differences that launch, held to 128 VGPRs and
-// spilling, gave results off by about 1e-6 on meshes of 294-302 swept rows,
-// varying from run to run, for a reason not found; with states it matches
-// the oracle on every tall mesh tried.
-//
-// Hand-offs between wavefronts (LDS ring of kRing slots per wavefront): the
-// edge lane (63 forward, 0 backward) of wavefront w writes its values of step
-// s in slot s % kRing; prog[w] = s + 1 says slots up to s are written,
-// cons[w] = s + 1 that wavefront w has taken the slots up to s of its
-// neighbour.  No step waits for an LDS round trip in the steady state:
-//  * the words and the neighbour's next slot are read at the end of a step,
-//    one step before they are needed, the slot straight into the edge lane of
-//    the shifted row (first the word, then the slot: the LDS performs a
-//    wavefront's operations in order, so a slot read after a word that says
-//    "written" holds the written values);
-//  * the next step first works on its own i-neighbour, then waits for those
-//    reads (lgkmcnt(0)), publishes prog and cons, and only if the word it read
-//    was too old waits for the neighbour and reads the slot again.  A
-//    wavefront so settles one to two steps behind its neighbour;
-//  * a slot is written only when the word cons read one step earlier says it
-//    has been taken (cons only grows), else after waiting for it.
-//
-// kAxis (with kDiff): every swept cell's normals are ni = (1,0), nj = (0,1),
-// so DF across an i-face is dFx and across a j-face dFy, exactly the values
-// fma(dFy, ni2, dFx ni1) and fma(dFy, nj2, dFx nj1) take there (up to the
-// sign of a zero): the normals are not loaded, a lane hands on dFy of its row
-// and keeps dFx.
-template <bool FWD, int kDepth, bool kDiff, bool kAxis>
-__device__ void sweep_pass(const Dev &d, const SyntheticState &st, NsShared &sh) {
-  static_assert(kDiff || !kAxis, "the axis-aligned form carries flux differences");
-  const int nx = d.nx, ny = d.ny, N = d.ncell, nwr = st.nw;
-  const double g = d.gamma;
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int j = 3 + tid;
-  const int pmin = 6, pmax = nx + ny - 6;
-  const int nstep = pmax - pmin + 1, nstepd = (nstep + kDepth - 1) / kDepth * kDepth;
-  if (w >= nwr) return;  // a wavefront without rows
-  // the wavefront this one takes the neighbouring row from, and the one it
-  // hands its edge row to
-  const int from = FWD ? w - 1 : w + 1, to = FWD ? w + 1 : w - 1;
-  const bool has_from = from >= 0 && from < nwr, has_to = to >= 0 && to < nwr;
-  const bool edge_in = FWD ? lane == 0 : lane == 63, edge_out = FWD ? lane == 63 : lane == 0;
-  constexpr int kRing = 2 * kDepth;  // a multiple of kDepth: no slot index wraps within a group of steps
-  static_assert(kRing <= kRingMax, "hand-off ring");
-  int *abort = &sh.abort, *err = st.ctl + kCtlErr;
-  const int fromc = has_from ? from : w, toc = has_to ? to : w;  // (in range also where unused)
-  int *pw = &sh.prog[in_vgpr(w)], *pfrom = &sh.prog[in_vgpr(fromc)];  // prog of this wavefront, of from
-  int *cw = &sh.cons[in_vgpr(w)], *cto = &sh.cons[in_vgpr(toc)];      // cons of this wavefront, of to
-  // records, dU* (pairs of components, 256 doubles per block) and U as raw buffers
-  const __amdgpu_buffer_rsrc_t rr = rec_rsrc(st);
-  const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(
-      st.dstar, (short)0, (int)((size_t)st.np * nwr * 256 * sizeof(double)), kBufWord3);
-  const __amdgpu_buffer_rsrc_t ru =
-      __builtin_amdgcn_make_buffer_rsrc(d.U, (short)0, (int)((size_t)4 * N * sizeof(double)), kBufWord3);
-  constexpr unsigned kOff = 0x80000000u;  // past every buffer's range: the store is discarded
-  // the plane of step s (clamped to the last one: the steps past it reload it)
-  // as a block index (p - 6) * nw + w
-  auto bidx = [&](int s) {
-    const int q = min(s, nstep - 1);
-    return (FWD ? q : nstep - 1 - q) * nwr + w;
+// What bounds a step is the number of the wavefront's instructions: a lone
+// wavefront issues one in about 5 cycles, of whatever kind, and a step takes
+// about 42 FP64 operations in about 75.  Nothing it executes waits for memory.
+// Records come through LDS, prepared by the loader wavefronts; the
+// neighbouring band's values come through LDS, brought by the receiver; both
+// are read a step before they are used, and the words that say that they are
+// there are looked at once in kGroup steps.  Its only memory instructions are
+// stores, whose completion it waits for once per sweep (and, eight steps
+// late, where it publishes the progress that the flux workgroups follow).
+template <bool FWD, bool kAxis>
+__device__ __forceinline__ bool sweep_pass(const Dev &d, const SyntheticState &st, SweepShared<kAxis> &sh,
+                                           const Band &bd, int k, int &group, int &hseq) {
+  static_assert(kGroup == 4 && kGroups == 2, "the loop below");
+  const int lane = threadIdx.x & 63, nw = st.nw;
+  const double g1 = d.gamma - 1.0;
+  const bool has_from = FWD ? bd.w > 0 : bd.w < nw - 1, has_to = FWD ? bd.w < nw - 1 : bd.w > 0;
+  const int n_in = has_from ? bd.links : 0;
+  int *ctl = st.ctl;
+  const __amdgpu_buffer_rsrc_t rs = rsrc_of(FWD ? st.dstar : st.ub, padded_blocks(st) * kBlk4);
+  const __amdgpu_buffer_rsrc_t rh = rsrc_of(hand_of(d, st, FWD, bd.w), (size_t)hand_len(d.nx) * 4);
+  // the edge row's values go out from the step of its first cell to the last step
+  const unsigned v_out = lane == (FWD ? kBand - 1 : 0) ? 0u : kOff;
+  const int out_from = has_to ? (FWD ? kBand - 1 : bd.rows - 1) : 0x7fffffff;
+  int h_out = 0;
+  // every lane stores every step: a slot without a cell gets zeros (forward) or is not read (backward)
+  constexpr int kBlkBytes = kBlk4 * 8;
+  const unsigned v_st = (unsigned)lane * 16u;
+  int soff = (((FWD ? bd.first : bd.last) - 6 + kPad) * nw + bd.w) * kBlkBytes;  // block of the step's plane
+  const int dsoff = (FWD ? nw : -nw) * kBlkBytes;
+  // of the lane's previous cell: dU, DF across the i-face and their weights; the term for the next lane
+  double du[4] = {0, 0, 0, 0}, fi[4] = {0, 0, 0, 0}, hi = 0.0, cbi = 0.0, to[4] = {0, 0, 0, 0}, t[4];
+  double in0[4], in1[4];  // values from the neighbouring band for the next two steps
+  int hn = 0;
+  // (zeros without a neighbour; past the last value any finite value does, as
+  // the edge lane has no cell there)
+  const double *hands = sh.hand[has_from ? 0 : kHand];
+  const int hmask = has_from ? kHand - 1 : 0;
+  auto fetch_hands = [&](int s) {
+    const double2 *h = reinterpret_cast<const double2 *>(hands + 4 * (s & hmask));
+    const double2 a = h[0], b = h[1], c = h[2], e = h[3];  // kHand is even: no wrap
+    in0[0] = a.x; in0[1] = a.y; in0[2] = b.x; in0[3] = b.y;
+    in1[0] = c.x; in1[1] = c.y; in1[2] = e.x; in1[3] = e.y;
   };
-  auto pof = [&](int s) { return FWD ? pmin + s : pmax - s; };
-  auto act = [&](int s) {
-    const int p = pof(s);
-    return s < nstep && j <= ny - 3 && p - j >= 3 && p - j <= nx - 3;
+  // the word, then the values: LDS performs a wavefront's operations in order
+  auto fetch_next_hands = [&](int s) {
+    hn = lds_get(&sh.hand_n);
+    mem_order();
+    fetch_hands(s);
   };
-  // byte offset of cell (p - j, j) in a component of U, less 8 p
-  const unsigned ucell = (unsigned)(((j + 1) * d.NI + 1 - j) * (int)sizeof(double));
-  // own previous cell (the i-neighbour) and the j-neighbour row, both of the
-  // previous step: dU and the weights, and either the flux differences dFx,
-  // dFy (kDiff) or the state U (cfx, nfx hold U; cfy, nfy unused)
-  double cdu[4], cfx[4], cfy[4], ccbi = 0.0, chsi = 0.0;
-  double ndu[4], nfx[4], nfy[4], ncb = 0.0, nhs = 0.0;
-  for (int m = 0; m < 4; m++) {
-    cdu[m] = cfy[m] = ndu[m] = nfy[m] = 0.0;
-    cfx[m] = nfx[m] = kDiff ? 0.0 : 1.0;
-  }
-  // the neighbour's slot at xb into the edge lane of the j-neighbour row
-  auto read_slot = [&](const double *xb) {
-    if (edge_in) {
-      for (int m = 0; m < 4; m++) {
-        ndu[m] = xb[m];
-        if (!kAxis) nfx[m] = xb[4 + m];
-        if (kDiff) nfy[m] = xb[8 + m];
-      }
-      ncb = xb[12];
-      nhs = xb[13];
-    }
+  auto gather = [&](const double in[4]) {  // the off-diagonal terms of this step's cells
+    for (int m = 0; m < 4; m++) t[m] = fma(hi, fi[m], fma(cbi, du[m], lane_shift<FWD>(to[m], in[m])));
   };
-  auto slot_of = [&](int v, int t) { return (v * kRingMax + t % kRing) * kSlot; };
-  int fprog = 0, fcons = 0;  // prog[from] and cons[to] as read one step earlier
-  Rec r[kDepth];
-#pragma unroll
-  for (int q = 0; q < kDepth - 1; q++) load_rec<FWD, kAxis>(rr, bidx(q) * kBlk * 8, rd, bidx(q) * 2048, lane, r[q]);
-  // block of the loads issued in step s (those of step s + kDepth - 1), moving
-  // by one plane per step and held at the last plane; block of step s
-  const int dbl = FWD ? nwr : -nwr, blim = FWD ? (nstep - 1) * nwr + w : w;
-  int bl = bidx(kDepth - 1), bs = w;
-  // slots of the group of steps s0 .. s0+kDepth-1: xin + kSlot q (from's), xout + kSlot q (this wavefront's)
-  const double *xin = sh.xw;
-  double *xout = sh.xw;
-  auto step = [&](int s, int q, Rec &x) {
-    // the record of step s + kDepth - 1, into the slot step s - 1 has used:
-    // issued first, so that the loads go out among this step's arithmetic
-    load_rec<FWD, kAxis>(rr, bl * (kBlk * 8), rd, bl * 2048, lane, r[(q + kDepth - 1) % kDepth]);
-    bl = FWD ? min(bl + dbl, blim) : max(bl + dbl, blim);
-    const int p = pof(s), i = p - j;
-    const bool on = act(s);
-    // off-diagonal term from the i-neighbour (this lane's previous cell)
-    double dfi[4], dfj[4];
-    if constexpr (kAxis) {
-      for (int m = 0; m < 4; m++) dfi[m] = cfx[m];
-    } else if constexpr (kDiff) {
-      for (int m = 0; m < 4; m++) dfi[m] = fma(cfy[m], x.ni[1], cfx[m] * x.ni[0]);
-    } else {
-      dfn(cfx, cdu, x.ni[0], x.ni[1], g, dfi);
-    }
-    if (s > 0) {
-      lgkm_wait();  // the previous step's slot write and reads are complete
-      if (has_to && lane == 0) lds_put(pw, s);
-      if (has_from) {
-        if (__builtin_amdgcn_readfirstlane(fprog) < s) {  // read too early: wait for slot s-1, read it again
-          wait_lds(pfrom, s, abort, err);
-          mem_order();
-          read_slot(&sh.xw[slot_of(fromc, s - 1)]);
-          lgkm_wait();
-        }
-        if (lane == 0) lds_put(cw, s);
-      }
-    }
-    // off-diagonal term from the j-neighbour
-    if constexpr (kAxis) {
-      for (int m = 0; m < 4; m++) dfj[m] = nfy[m];
-    } else if constexpr (kDiff) {
-      for (int m = 0; m < 4; m++) dfj[m] = fma(nfy[m], x.nj[1], nfx[m] * x.nj[0]);
-    } else {
-      dfn(nfx, ndu, x.nj[0], x.nj[1], g, dfj);
-    }
-    // The terms across faces to cells that are not swept (i = 3, j = 3 forward;
-    // i = nx-3, j = ny-3 backward) vanish without a test: the forward weights
-    // Hsi, Hsj of those cells are zero, and a slot of a cell that is not swept
-    // holds U = (1,0,0,0) and zero weights (written once by k_rec_init, never by
-    // the flux workgroups), so its dU and flux differences stay zero.
-    double du[4];
+  auto step = [&](int s, const Rec &x) {
+    double u[4];
     for (int m = 0; m < 4; m++) {
-      // forward:  dui = 0.5 (DF si(i,j) + Lci(i-1,j) dU) + Lvi(i-1,j) dU      (:44-49)
-      // backward: dui = -0.5 (DF si(i+1,j) - Lci(i+1,j) dU) + Lvi(i+1,j) dU   (:82-86)
-      const double ti = FWD ? fma(x.hsi, dfi[m], ccbi * cdu[m]) : fma(-chsi, dfi[m], ccbi * cdu[m]);
-      const double tj = FWD ? fma(x.hsj, dfj[m], ncb * ndu[m]) : fma(-nhs, dfj[m], ncb * ndu[m]);
-      double a = FWD ? x.res[m] : 0.0;
-      a = a + ti;
-      a = a + tj;
-      du[m] = FWD ? a * x.ra : x.res[m] + a * x.ra;  // backward: x.res holds dU*
+      du[m] = fma(t[m], x.ra, x.r[m]);
+      u[m] = x.u[m] + du[m];
     }
-    // plain stores: dU* is read back by this lane, U is written back to the
-    // device's coherence point by the release fence after the sweep
-    if (FWD) {
-      const unsigned v = on ? (unsigned)lane * 16u : kOff;
-      const int so = bs * 2048;  // bidx(s) where a lane has a cell
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, double2{du[0], du[1]}), rd, v, so, 0);
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, double2{du[2], du[3]}), rd, v + 1024u, so,
-                                             0);
-    } else {
-      const unsigned v = on ? ucell + (unsigned)p * 8u : kOff;
-      for (int m = 0; m < 4; m++)
-        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, x.u[m] + du[m]), ru, v,
-                                              m * N * (int)sizeof(double), 0);
+    const double *q = FWD ? du : u;  // dU* or the updated state
+    st_pair(rs, v_st, soff, q[0], q[1]);
+    st_pair(rs, v_st + 1024u, soff, q[2], q[3]);
+    soff += dsoff;
+    const Euler w(u, rcp_nr(u[0]), g1);
+    const double dx[4] = {du[1], fma(u[1], w.vx, w.p) - x.f[0], fma(u[2], w.vx, -x.f[1]), fma(w.e, w.vx, -x.f[2])};
+    const double dy[4] = {du[2], dx[2], fma(u[2], w.vy, w.p) - x.f[3], fma(w.e, w.vy, -x.f[4])};
+    for (int m = 0; m < 4; m++) {
+      const double fj = kAxis ? dy[m] : fma(dy[m], x.nj[1], dx[m] * x.nj[0]);
+      fi[m] = kAxis ? dx[m] : fma(dy[m], x.ni[1], dx[m] * x.ni[0]);
+      to[m] = fma(x.hj, fj, x.cbj * du[m]);
     }
-    // carry: this cell's dU and flux differences, and the j-neighbour row's
-    // of the next step (zero in the edge lane of a wavefront without a
-    // neighbour, where the term has a zero weight)
-    if constexpr (kDiff) {
-      double u2[4], fx1[4], fy1[4], fx2[4], fy2[4];
-      for (int m = 0; m < 4; m++) {
-        cdu[m] = on ? du[m] : 0.0;
-        u2[m] = x.u[m] + cdu[m];
-      }
-      fxy_r(x.u, x.rr, g, fx1, fy1);  // 1/rho of the record's state from the record
-      fxy(u2, g, fx2, fy2);
-      for (int m = 0; m < 4; m++) {
-        cfx[m] = fx2[m] - fx1[m];
-        cfy[m] = fy2[m] - fy1[m];
-        ndu[m] = lane_shift(cdu[m], FWD);
-        if (!kAxis) nfx[m] = lane_shift(cfx[m], FWD);
-        nfy[m] = lane_shift(cfy[m], FWD);
-      }
-    } else {  // the state (the edge lane of a wavefront without a neighbour gets (1,0,0,0), dU = 0)
-      for (int m = 0; m < 4; m++) {
-        cfx[m] = x.u[m];
-        cdu[m] = on ? du[m] : 0.0;
-        nfx[m] = m == 0 ? lane_shift_rho(cfx[m], FWD) : lane_shift(cfx[m], FWD);
-        ndu[m] = lane_shift(cdu[m], FWD);
-      }
+    hi = x.hi;
+    cbi = x.cbi;
+    if (s >= out_from) {
+      st_pair(rh, v_out, h_out, to[0], to[1]);
+      st_pair(rh, v_out + 16u, h_out, to[2], to[3]);
+      h_out += 32;
     }
-    ccbi = x.cbi;
-    chsi = x.hsi;
-    ncb = lane_shift(x.cbj, FWD);
-    nhs = lane_shift(x.hsj, FWD);
-    if (has_to) {  // hand the edge row on, once slot s % kRing has been taken
-      if (__builtin_amdgcn_readfirstlane(fcons) < s - kRing + 1) {
-        wait_lds(cto, s - kRing + 1, abort, err);
-        mem_order();
-      }
-      if (edge_out) {
-        double *xb = xout + kSlot * q;
-        for (int m = 0; m < 4; m++) {
-          xb[m] = cdu[m];
-          if (!kAxis) xb[4 + m] = cfx[m];
-          if (kDiff) xb[8 + m] = cfy[m];
-        }
-        xb[12] = x.cbj;
-        xb[13] = x.hsj;
-      }
-      mem_order();
-      fcons = lds_get(cto);
-    }
-    if (has_from) {  // for the next step: the word, then the slot of this step
-      mem_order();
-      fprog = lds_get(pfrom);
-      mem_order();
-      read_slot(xin + kSlot * q);
-    }
-    bs += nwr;
   };
-  for (int s = 0; s < nstepd; s += kDepth) {
-    xin = &sh.xw[in_vgpr(slot_of(fromc, s))];
-    xout = &sh.xw[in_vgpr(slot_of(w, s))];
-#pragma unroll
-    for (int q = 0; q < kDepth; q++) step(s + q, q, r[q]);
-  }
-}
-
-// The wavefronts of a pass are coupled only through their hand-offs: a
-// wavefront may run up to 2 kDepth steps ahead of the one that takes its edge row.
-// kDiff: carry flux differences (the launches of 256 threads); the launch of
-// up to 1024 threads carries states (see sweep_pass).  kAxis: the mesh's
-// normals are (1,0) and (0,1) on every swept cell.
-template <int kDepth, bool kDiff = true, bool kAxis = false>
-__device__ void sweep(const Dev &d, const SyntheticState &st, NsShared &sh) {
-  const int tid = threadIdx.x;
-  if (tid < kMaxSweepWaves) { sh.prog[tid] = 0; sh.cons[tid] = 0; }
-  if (tid == 0) sh.abort = 0;
-  barrier_lds();
-  sweep_pass<true, kDepth, kDiff, kAxis>(d, st, sh);  // dU* = (Res + dui + duj)/alfa, planes 6 .. nx+ny-6 (:26-69)
-  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this lane's dU* stores are complete
-  barrier_lds();
-  if (tid < kMaxSweepWaves) { sh.prog[tid] = 0; sh.cons[tid] = 0; }
-  barrier_lds();
-  sweep_pass<false, kDepth, kDiff, kAxis>(d, st, sh);  // dU = dU* + (dui + duj)/alfa, planes nx+ny-6 .. 6 (:73-111), then U + dU
-  // release: the U stores reach the device's coherence point before the
-  // flux workgroups are told to read U (L2 write-back, then vmcnt(0))
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-}
-
-// Polls *p until it reaches want (ge) or equals want or is negative (!ge).
-// Bounded by kWaitTicks of the 100 MHz wall clock; a timeout sets *err.  The
-// flux workgroups wait through a whole sweep, so they poll with long sleeps
-// (SLEEP) to keep their loads off the memory the sweep reads.
-template <int SLEEP>
-__device__ bool wait_until(const int *p, int want, bool ge, int *err) {
-  const long long t0 = wall_clock64();
-  int it = 0, v = ld_agent(p);
-  while (!(ge ? v >= want : (v == want || v < 0))) {
-    __builtin_amdgcn_s_sleep(SLEEP);
-    if ((++it & 15) == 0) {
-      if (ld_agent(err) != 0) return false;
-      if (wall_clock64() - t0 > kWaitTicks) {
-        st_agent(err, 1);
-        return false;
+  Rec x, y;
+  if (!wait_lds(&sh.avail[group & 1], group + 1, sh, ctl)) return false;
+  read_rec<kAxis>(sh.ring[(group & 1) * kGroup], lane, x);
+  mem_order();
+  fetch_next_hands(0);
+  for (int q = 0; q < bd.groups; q++) {
+    const int s = kGroup * q;
+    const double *ring = sh.ring[(group & 1) * kGroup];
+    if (s < n_in) {
+      const int need = hseq + min(s + kGroup, n_in);
+      if (uniform(hn) - need < 0) {  // read too early
+        if (!wait_lds(&sh.hand_n, need, sh, ctl)) return false;
+        fetch_hands(s);
       }
     }
-    v = ld_agent(p);
+    mem_order();
+    read_rec<kAxis>(ring + SweepShared<kAxis>::kStep, lane, y);
+    gather(in0);
+    step(s, x);
+    mem_order();
+    lds_put(&sh.used, 2 * group + 1);  // the first half's records are read, in order
+    read_rec<kAxis>(ring + 2 * SweepShared<kAxis>::kStep, lane, x);
+    gather(in1);
+    fetch_hands(s + 2);
+    step(s + 1, y);
+    mem_order();
+    read_rec<kAxis>(ring + 3 * SweepShared<kAxis>::kStep, lane, y);
+    group++;
+    const int av = lds_get(&sh.avail[group & 1]);
+    gather(in0);
+    step(s + 2, x);
+    mem_order();
+    lds_put(&sh.used, 2 * group);  // all of the group's records
+    if (uniform(av) - (group + 1) < 0 && q + 1 < bd.groups &&
+        !wait_lds(&sh.avail[group & 1], group + 1, sh, ctl))
+      return false;
+    mem_order();
+    read_rec<kAxis>(sh.ring[(group & 1) * kGroup], lane, x);  // (after the last group: not used)
+    gather(in1);
+    fetch_next_hands(s + 4);
+    step(s + 3, y);
+    if (!FWD && (q & 1) != 0) {
+      // at most 16 memory operations (two to four a step) are not complete:
+      // all but the last eight steps are
+      mem_order();
+      __builtin_amdgcn_s_waitcnt(0x4F70);  // vmcnt(16)
+      mem_order();
+      if (lane == 0) st_agent(st.prog + kProgStride * bd.w, ((long long)k << 32) | (s + kGroup - 8));
+    }
   }
+  hseq += n_in;
   return true;
 }
 
+// The sweep wavefront's loop.
+template <bool kAxis>
+__device__ __forceinline__ void sweeper(const Dev &d, const SyntheticState &st, SweepShared<kAxis> &sh, const Band &bd) {
+  int group = 0, hseq = 0;
+  __builtin_amdgcn_s_setprio(3);  // before the workgroup's other wavefront on this SIMD
+  for (int k = st.k0;; k++) {
+    if (k > st.k0 && !wait_lds(&sh.clr, k - 1, sh, st.ctl)) break;
+    if (!sweep_pass<true, kAxis>(d, st, sh, bd, k, group, hseq)) break;
+    vm_wait();
+    lds_put(&sh.fwd_done, k);
+    if (!wait_lds(&sh.bgo, k, sh, st.ctl)) break;
+    if (!sweep_pass<false, kAxis>(d, st, sh, bd, k, group, hseq)) break;
+    vm_wait();
+    if ((threadIdx.x & 63) == 0) st_agent(st.prog + kProgStride * bd.w, ((long long)k << 32) | bd.n);
+    lds_put(&sh.bwd_done, k);
+    if (!next_iteration(k, sh, st.ctl)) break;
+  }
+  lds_put(&sh.quit, 1);
+}
+
+// A loader wavefront (id = 0 .. kLoaders-1): fetches the records of every
+// kLoaders-th group of plane steps into registers, forms what a step needs
+// besides the recurrence (the Euler fluxes of U), and hands them on through
+// LDS when the sweep has read what was there.  The loads in flight are held in this wavefront's registers (kGroup
+// steps of 7 KiB in each of kLoaders wavefronts), so two groups of LDS do.  A
+// forward sweep follows the flux workgroups tile by tile: the records of plane
+// p exist when the tiles of the levels up to (p-6)/kTI in the band's rows are
+// done.
+template <bool kAxis>
+__device__ __forceinline__ void loader(const Dev &d, const SyntheticState &st, SweepShared<kAxis> &sh, const Band &bd,
+                                       int id) {
+  const int lane = threadIdx.x & 63, nw = st.nw;
+  const double g1 = d.gamma - 1.0;
+  constexpr int kGeo = kAxis ? 2 : 6;
+  const __amdgpu_buffer_rsrc_t rr = rec_rsrc(st);
+  const __amdgpu_buffer_rsrc_t rd = rsrc_of(st.dstar, padded_blocks(st) * kBlk4);
+  const __amdgpu_buffer_rsrc_t rg = rsrc_of(st.geo, nblocks(st) * kGeo * 128);
+  const unsigned v = (unsigned)lane * 16u;
+  int gbase = 0;  // groups of the sweeps before this one
+  for (int k = st.k0;; k++) {
+    for (int dir = 0; dir < 2; dir++) {
+      const bool fwd = dir == 0;
+      int level = kLev * kBandTiles * bd.w;  // the tiles of lower levels are done
+      // whether the tiles of group gr are done, as far as one look at each further level says
+      auto look = [&](int gr) -> bool {
+        const int top = min((bd.first + min((gr + 1) * kGroup, bd.n) - 1 - 6) / kTI,
+                            st.ntx - 1 + kLev * (kBandTiles * (bd.w + 1) - 1));
+        for (; level <= top; level++) {
+          const int b = kBandTiles * bd.w + lane, a = level - kLev * b;
+          const bool mine = lane < kBandTiles && b < st.nty && a >= 0 && a < st.ntx;
+          if (__any(mine && ld_agent(st.ready + (mine ? b * st.ntx + a : 0)) < k)) return false;
+        }
+        mem_order();
+        return true;
+      };
+      if (!fwd && !wait_lds(&sh.fwd_done, k, sh, st.ctl)) return;  // dU* is at memory
+      for (int gr = id; gr < bd.groups; gr += kLoaders) {
+        const int s0 = gr * kGroup;
+        if (fwd) {
+          Patience pt(st.ctl);
+          while (!look(gr)) {
+            if (uniform(lds_get(&sh.quit))) return;
+            if (pt.over(true)) {
+              lds_put(&sh.quit, 1);
+              return;
+            }
+          }
+        }
+        double2 q[kGroup][9];
+#pragma unroll
+        for (int t = 0; t < kGroup; t++) {
+          const int s = min(s0 + t, bd.n - 1), p = fwd ? bd.first + s : bd.last - s;
+          const int blk = (p - 6) * nw + bd.w;
+          const __amdgpu_buffer_rsrc_t r0 = fwd ? rr : rd;
+          const int o0 = fwd ? blk * (kBlk * 8) : (blk + kPad * nw) * (kBlk4 * 8);
+          q[t][0] = ld_pair(r0, v, o0);
+          q[t][1] = ld_pair(r0, v + 1024u, o0);
+          for (int m = 2; m < 6; m++) q[t][m] = ld_pair(rr, v + m * 1024u, blk * (kBlk * 8));
+          const int og = blk * (kGeo * 1024);
+          q[t][6] = ld_pair(rg, v + (fwd ? 0u : 1024u), og);
+          if (!kAxis) {
+            q[t][7] = ld_pair(rg, v + (fwd ? 2048u : 4096u), og);
+            q[t][8] = ld_pair(rg, v + (fwd ? 3072u : 5120u), og);
+          }
+        }
+        // while the loads are under way: the tiles of this wavefront's next group
+        if (fwd && gr + kLoaders < bd.groups) (void)look(gr + kLoaders);
+        double f[kGroup][5];
+#pragma unroll
+        for (int t = 0; t < kGroup; t++) {
+          double2 *y = q[t];
+          if (s0 + t >= bd.n) {  // past the last plane: a step without cells
+            y[0] = y[1] = y[3] = y[4] = y[5] = y[6] = {0.0, 0.0};
+            y[2] = {1.0, 0.0};
+            y[5].y = 1.0;
+          }
+          if (fwd) {  // Res to Res/alfa
+            y[0] = {y[0].x * y[4].x, y[0].y * y[4].x};
+            y[1] = {y[1].x * y[4].x, y[1].y * y[4].x};
+          } else {
+            y[6] = {-y[6].x, -y[6].y};
+          }
+          const double u[4] = {y[2].x, y[2].y, y[3].x, y[3].y};
+          const Euler w(u, y[5].y, g1);  // 1/rho of the record's state from the record
+          f[t][0] = fma(u[1], w.vx, w.p);
+          f[t][1] = u[2] * w.vx;
+          f[t][2] = w.e * w.vx;
+          f[t][3] = fma(u[2], w.vy, w.p);
+          f[t][4] = w.e * w.vy;
+        }
+        const int gn = gbase + gr, slot = gn & 1;
+#pragma unroll
+        for (int t = 0; t < kGroup; t++) {
+          // the place of a half group is free when that half of group gn - 2 has been read
+          if (t % 2 == 0 && !wait_lds(&sh.used, 2 * (gn - kGroups) + t / 2 + 1, sh, st.ctl)) return;
+          const double2 *y = q[t];
+          double2 *o = reinterpret_cast<double2 *>(sh.ring[slot * kGroup + t]) + lane;
+          o[0] = y[0];
+          o[64] = y[1];
+          o[128] = y[2];
+          o[192] = y[3];
+          o[256] = y[4];
+          o[320] = {y[5].x, y[6].x};
+          o[384] = {y[6].y, f[t][0]};
+          o[448] = {f[t][1], f[t][2]};
+          o[512] = {f[t][3], f[t][4]};
+          if (!kAxis) {
+            o[576] = y[7];
+            o[640] = y[8];
+          }
+        }
+        mem_order();
+        lds_put(&sh.avail[slot], gn + 1);  // after the records: LDS performs a wavefront's operations in order
+      }
+      gbase += bd.groups;
+    }
+    if (!next_iteration(k, sh, st.ctl)) return;
+  }
+}
+
+// The receiver wavefront: brings the neighbouring band's values from memory
+// to LDS, up to 64 at a time, in order.
+template <bool kAxis>
+__device__ __forceinline__ void receiver(const Dev &d, const SyntheticState &st, SweepShared<kAxis> &sh, const Band &bd) {
+  const int lane = threadIdx.x & 63, nw = st.nw;
+  if (nw == 1) return;
+  int hseq = 0, gbase = 0;
+  for (int k = st.k0;; k++) {
+    for (int dir = 0; dir < 2; dir++, gbase += bd.groups) {
+      const bool fwd = dir == 0;
+      if (fwd ? bd.w == 0 : bd.w == nw - 1) continue;
+      const __amdgpu_buffer_rsrc_t rh =
+          rsrc_of(hand_of(d, st, fwd, fwd ? bd.w - 1 : bd.w + 1), (size_t)hand_len(d.nx) * 4);
+      Patience pt(st.ctl);
+      for (int have = 0; have < bd.links;) {
+        const int at = have + lane;
+        const unsigned v = at < bd.links ? (unsigned)at * 32u : kOff;
+        const double2 a = ld_pair(rh, v, 0), b = ld_pair(rh, v + 16u, 0);
+        auto there = [](double x) { return (unsigned)((unsigned long long)__double_as_longlong(x) >> 32) != kEmptyHi; };
+        const unsigned long long m =
+            __ballot(at < bd.links && there(a.x) && there(a.y) && there(b.x) && there(b.y));
+        int cnt = m == ~0ull ? 64 : __builtin_ctzll(~m);
+        // the sweep has read the values of the steps before kGroup (used / 2 - gbase)
+        cnt = min(cnt, kGroup * ((uniform(lds_get(&sh.used)) >> 1) - gbase) + kHand - have);
+        if (cnt > 0) {
+          if (lane < cnt) {
+            double2 *o = reinterpret_cast<double2 *>(sh.hand[at & (kHand - 1)]);
+            o[0] = a;
+            o[1] = b;
+          }
+          mem_order();
+          have += cnt;
+          lds_put(&sh.hand_n, hseq + have);
+          pt.n = 0;
+        } else {
+          if (uniform(lds_get(&sh.quit))) return;
+          __builtin_amdgcn_s_sleep(1);
+          if (pt.over(true)) {
+            lds_put(&sh.quit, 1);
+            return;
+          }
+        }
+      }
+      hseq += bd.links;
+    }
+    if (!next_iteration(k, sh, st.ctl)) return;
+  }
+}
+
+// The loop's end word: results for the host, then no further iteration.
+__device__ __forceinline__ void end_loop(const SyntheticState &st, int it, int bad, int stopped, int last, double res) {
+  if ((threadIdx.x & 63) != 0) return;
+  st.iters[0] = it;
+  st.iters[1] = bad;
+  st.iters[2] = stopped;
+  reinterpret_cast<double *>(st.iters + 4)[0] = res;  // max |Res_4| of the launch's last iteration
+  st_agent(st.ctl + kCtlLast, last);
+  if (bad) st_agent(st.ctl + kCtlStop, 1);
+}
+
+// A band's fourth helper: empties the hand-off slots that its sweep has read
+// (each direction's during the other direction's sweep, before the band's own
+// sweep of that direction can end, so before they are written again).  In
+// the last band, where the forward sweep ends last and the backward sweep
+// begins, it also decides: a T<0.1 stop before U changes, and whether another
+// iteration runs (src/Hybrid_Sub.f90:99-104).
+template <bool kAxis>
+__device__ __forceinline__ void keeper(const Dev &d, const SyntheticState &st, SweepShared<kAxis> &sh, const Band &bd) {
+  const int lane = threadIdx.x & 63, nw = st.nw;
+  const bool top = bd.w == nw - 1;
+  auto clear = [&](bool fwd) {
+    const int from = fwd ? bd.w - 1 : bd.w + 1;
+    if (from < 0 || from >= nw) return;
+    const __amdgpu_buffer_rsrc_t rh = rsrc_of(hand_of(d, st, fwd, from), (size_t)hand_len(d.nx) * 4);
+    const double e = __longlong_as_double((long long)kEmpty);
+    for (int q = lane; q < 2 * bd.links; q += 64) st_pair(rh, (unsigned)q * 16u, 0, e, e);
+  };
+  for (int k = st.k0;; k++) {
+    if (!wait_lds(&sh.fwd_done, k, sh, st.ctl)) return;
+    clear(true);
+    const int bad = top ? uniform(ld_agent(st.ctl + kCtlBad)) : 0;
+    vm_wait();
+    if (!bad) lds_put(&sh.bgo, k);
+    if (top) {
+      double res = 0.0;
+      for (int t = lane; t < st.ntx * st.nty; t += 64) res = fmax(res, ld_agent(st.tres + t));
+      for (int off = 32; off > 0; off >>= 1) res = fmax(res, __shfl_xor(res, off, 64));
+      bool more = !bad && res > st.tol && k < st.maxit;
+      const bool stopped = more && k >= st.kstop;  // the launch ends here; a later one continues at k + 1
+      if (stopped) more = false;
+      if (!more) {
+        end_loop(st, k, bad, stopped ? 1 : 0, bad ? k - 1 : k, res);
+        vm_wait();
+      }
+      if (lane == 0) st_agent(st.ctl + kCtlGo, more ? k + 1 : -1);
+      if (bad) {
+        lds_put(&sh.quit, 1);
+        return;
+      }
+    }
+    if (!wait_lds(&sh.bwd_done, k, sh, st.ctl)) return;
+    clear(false);
+    vm_wait();
+    lds_put(&sh.clr, k);
+    if (!next_iteration(k, sh, st.ctl)) return;
+  }
+}
+
 // A copy of x with every 32-bit word read once and made wavefront-uniform
-// (scalar registers): x is a function argument passed through the stack,
-// whose fields would otherwise be reloaded per use into vector registers.
+// (scalar registers): the fields of a job in memory would otherwise be
+// reloaded after every store.
 template <typename T>
 __device__ __forceinline__ T uniform_copy(const T &x) {
   static_assert(sizeof(T) % 4 == 0, "word copy");
@@ -820,161 +1049,188 @@ __device__ __forceinline__ T uniform_copy(const T &x) {
   return y;
 }
 
-// The flux workgroups' part of the inner loop.  A separate (not inlined)
-// function: the sweep's registers are then allocated without the flux code's
-// live values, which otherwise push the sweep's scalar registers into
-// spills.  One copy per launch size B, so that each gets the register budget
-// of its kernel's workgroup size (one shared copy is held to 1024 threads).
-// Flux workgroup w reports an iteration in its own slot part[8w..]: its max
-// |Res_4| and T<0.1 flag, then the iteration number once those stores are
-// complete.
-template <int B>
-__device__ __attribute__((noinline)) void ns_flux_role(const Dev d_arg, const SyntheticState st_arg, NsShared &sh) {
-  const Dev d = uniform_copy(d_arg);
-  const SyntheticState st = uniform_copy(st_arg);
+template <bool kAxis>
+__device__ __forceinline__ void sweep_role(const Dev &d, const SyntheticState &st, SweepShared<kAxis> &sh, int band) {
+  for (int t = threadIdx.x; t < (kHand + 2) * 4; t += kThreads) sh.hand[t / 4][t % 4] = 0.0;
+  if (threadIdx.x == 0) {
+    for (int q = 0; q < kGroups; q++) sh.avail[q] = 0;
+    sh.used = sh.hand_n = sh.quit = 0;
+    sh.fwd_done = sh.bwd_done = sh.bgo = sh.clr = st.k0 - 1;
+  }
+  __syncthreads();
+  if (ld_agent(st.ctl + kCtlGo) != st.k0) return;
+  const Band bd(d, uniform(band));
+  const int wave = uniform((int)(threadIdx.x >> 6));
+  // wavefront 4 shares the SIMD of the sweep (0): the one with the least to do
+  if (wave == 0) sweeper<kAxis>(d, st, sh, bd);
+  else if (wave <= kLoaders) loader<kAxis>(d, st, sh, bd, wave - 1);
+  else if (wave == 4) receiver<kAxis>(d, st, sh, bd);
+  else keeper<kAxis>(d, st, sh, bd);
+}
+
+// A flux workgroup (of st.nflux): the fluxes of its tiles, iteration after
+// iteration.  A tile of iteration k+1 is computed as soon as the backward
+// sweep of iteration k has passed every cell that it reads, so the fluxes run
+// beside the sweep, from the last planes to the first; at the end only the
+// first tile's are left, and the forward sweep begins behind them.  When the
+// loop ends the workgroup writes its tiles' U to the mesh array.
+__device__ __forceinline__ void flux_role(const Dev &d, const SyntheticState &st, FluxShared &sh, int wg) {
+  const int tid = threadIdx.x, nx = d.nx, ny = d.ny;
+  const int ntiles = st.ntx * st.nty;
   int *ctl = st.ctl;
-  const int tid = threadIdx.x;
-  const int wg = blockIdx.x - 1, ntiles = st.ntx * st.nty;
-  int *slot = reinterpret_cast<int *>(st.part + 8 * wg);
+  // thread 0: waits until the backward sweep of iteration k has passed the
+  // cells from (ilo, jlo) on in the rows up to jhi
+  auto passed = [&](int k, int ilo, int jlo, int jhi) -> bool {
+    for (int w = (jlo - 3) / kBand; w <= (jhi - 3) / kBand; w++) {
+      const Band bd(d, w);
+      const long long want = ((long long)k << 32) | (bd.last - (ilo + max(jlo, bd.j0)) + 1);
+      Patience pt(ctl);
+      while (ld_agent(st.prog + kProgStride * w) < want) {
+        __builtin_amdgcn_s_sleep(8);
+        if (pt.over(false)) return false;
+      }
+    }
+    return true;
+  };
   for (int k = st.k0;; k++) {
     if (tid == 0) {
-      int go = -1;
-      if (wait_until<60>(ctl + kCtlGo, k, false, ctl + kCtlErr)) go = ld_agent(ctl + kCtlGo);
-      sh.word = go == k ? 1 : 0;
+      Patience pt(ctl);
+      int go;
+      while ((go = ld_agent(ctl + kCtlGo)) != k && go >= 0) {
+        __builtin_amdgcn_s_sleep(32);
+        if (pt.over(false)) { go = -2; break; }
+      }
+      sh.word = go;
     }
     __syncthreads();
-    const int run = sh.word;
+    const int go = sh.word;
     __syncthreads();
-    if (!run) return;
-    double rmax = 0.0;
-    int bad = 0;
-    for (int tile = wg; tile < ntiles; tile += st.nflux) flux_tile(d, st, sh, tile, rmax, bad);
-    // the workgroup's max |Res_4| and T<0.1 flag
-    for (int off = 32; off > 0; off >>= 1) rmax = fmax(rmax, __shfl_down(rmax, off, 64));
-    bad = __syncthreads_or(bad);
-    if ((tid & 63) == 0) sh.red[tid >> 6] = rmax;
-    __syncthreads();
-    if (tid == 0) {
-      double m = sh.red[0];
-      for (int q = 1; q < (int)(blockDim.x >> 6); q++) m = fmax(m, sh.red[q]);
-      st_agent(st.part + 8 * wg + 1, m);
-      st_agent(slot + 1, bad);
+    if (go != k) {
+      if (go != -1) return;
+      break;
     }
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this thread's stores are complete
+    for (int q = ntiles - 1 - wg; q >= 0; q -= st.nflux) {
+      const int tile = uniform(st.order[q]);
+      TileGeo tg;
+      tile_geo(d, st, tile, tg);
+      if (k > st.k0) {
+        if (tid == 0)
+          sh.word = passed(k - 1, max(3, tg.i0 - 2), max(3, tg.j0 - 2), min(ny - 3, tg.j0 + kTJ + 1)) ? 1 : 0;
+        __syncthreads();
+        const int ok = sh.word;
+        __syncthreads();
+        if (!ok) return;
+      }
+      double rmax = 0.0;
+      int bad = 0;
+      flux_tile(d, st, sh, tg, k == st.k0, rmax, bad);
+      // the tile's max |Res_4| and T<0.1 flag, then its iteration number once
+      // every store of the workgroup is complete
+      for (int off = 32; off > 0; off >>= 1) rmax = fmax(rmax, __shfl_down(rmax, off, 64));
+      if ((tid & 63) == 0) sh.red[tid >> 6] = rmax;
+      bad = __syncthreads_or(bad);
+      if (tid == 0) {
+        double m = sh.red[0];
+        for (int e = 1; e < kThreads / 64; e++) m = fmax(m, sh.red[e]);
+        st_agent(st.tres + tile, m);
+        if (bad) st_agent(ctl + kCtlBad, 1);
+      }
+      vm_wait();
+      __syncthreads();
+      if (tid == 0) st_agent(st.ready + tile, k);
+    }
+  }
+  // U of the last complete iteration to the mesh array
+  const int last = uniform(ld_agent(ctl + kCtlLast));
+  if (last < st.k0) return;
+  const __amdgpu_buffer_rsrc_t ru = ub_rsrc(st);
+  for (int q = ntiles - 1 - wg; q >= 0; q -= st.nflux) {
+    const int tile = uniform(st.order[q]);
+    const int i0 = 3 + (tile % st.ntx) * kTI, j0 = 3 + (tile / st.ntx) * kTJ;
+    if (tid == 0) sh.word = passed(last, i0, j0, min(ny - 3, j0 + kTJ - 1)) ? 1 : 0;
     __syncthreads();
-    if (tid == 0) st_agent(slot, k);
+    const int ok = sh.word;
+    __syncthreads();
+    if (!ok) return;
+    for (int t = tid; t < kTI * kTJ; t += kThreads) {
+      const int b = t % kTJ, i = i0 + ((t / kTJ - b) & (kTI - 1)), j = j0 + b;
+      if (i > nx - 3 || j > ny - 3) continue;
+      const unsigned o = (unsigned)pblk_of(i, j, st.nw) * (kBlk4 * 8u) + 16u * ((j - 3) & 63);
+      const double2 u01 = ld_pair(ru, o, 0), u23 = ld_pair(ru, o + 1024u, 0);
+      const int c = cidx(d, i, j), N = d.ncell;
+      d.U[c] = u01.x;
+      d.U[N + c] = u01.y;
+      d.U[2 * N + c] = u23.x;
+      d.U[3 * N + c] = u23.y;
+    }
   }
 }
 
-// The inner loop (src/Hybrid_Sub.f90:99-104): workgroup 0 sweeps, the others
-// compute the fluxes; see the file comment.  kAxis: the sweep of a mesh whose
-// normals are (1,0) and (0,1) on every swept cell (launches of 256 threads).
-template <int B, bool kAxis>
-__global__ void __launch_bounds__(B) k_ns_loop(Dev d, SyntheticState st) {
-  static_assert(B <= 256 || !kAxis, "the axis-aligned sweep carries flux differences");
-  __shared__ NsShared sh;
-  int *ctl = st.ctl;
-  const int tid = threadIdx.x;
-  if (blockIdx.x > 0) {
-    ns_flux_role<B>(d, st, sh);
-    return;
-  }
-  // workgroup 0: the LU-SGS sweeps and the loop control
-  int it = st.k0 - 1, bad = 0, stopped = 0;
-  double res_last = 0.0;
-  if (ld_agent(ctl + kCtlGo) == st.k0) {
-    for (int k = st.k0;; k++) {
-      // every flux workgroup's slot holds k; one lane per workgroup polls
-      int ok = 1;
-      double rmax = 0.0;
-      int b = 0;
-      for (int q = tid; q < st.nflux; q += blockDim.x) {
-        const int *slot = reinterpret_cast<const int *>(st.part + 8 * q);
-        if (!wait_until<1>(slot, k, true, ctl + kCtlErr)) ok = 0;
-        rmax = fmax(rmax, ld_agent(st.part + 8 * q + 1));
-        b |= ld_agent(slot + 1);
-      }
-      ok = __syncthreads_and(ok);
-      b = __syncthreads_or(b);
-      if (!ok) break;  // a wait timed out: end the loop
-      for (int off = 32; off > 0; off >>= 1) rmax = fmax(rmax, __shfl_down(rmax, off, 64));
-      if ((tid & 63) == 0) sh.red[tid >> 6] = rmax;
-      __syncthreads();
-      double res = sh.red[0];
-      for (int q = 1; q < (int)(blockDim.x >> 6); q++) res = fmax(res, sh.red[q]);
-      bad = b;
-      it = k;
-      res_last = res;
-      __syncthreads();
-      if (bad) break;
-      sweep<B <= 256 ? 4 : 3, B <= 256, kAxis>(d, st, sh);  // deeper prefetch where registers allow
-      __syncthreads();
-      bool more = res > st.tol && k < st.maxit;
-      if (more && k >= st.kstop) {  // the launch ends here; a later one continues at k + 1
-        more = false;
-        stopped = 1;
-      }
-      if (tid == 0) st_agent(ctl + kCtlGo, more ? k + 1 : -1);
-      if (!more) break;
-    }
-  }
-  if (tid == 0) {
-    st_agent(ctl + kCtlGo, -1);  // releases the flux workgroups on every exit path
-    st.iters[0] = it;
-    st.iters[1] = bad;
-    st.iters[2] = stopped;
-    reinterpret_cast<double *>(st.iters + 4)[0] = res_last;  // max |Res_4| of the launch's last iteration
-  }
+// LDS of a workgroup of either role
+template <bool kAxis>
+struct LoopShared {
+  static constexpr size_t kBytes =
+      sizeof(SweepShared<kAxis>) > sizeof(FluxShared) ? sizeof(SweepShared<kAxis>) : sizeof(FluxShared);
+};
+
+// Workgroup b of an instance's `blocks`: bands sit at multiples of st.stride,
+// the flux workgroups in between.  With stride 8 the bands of one instance
+// are on one XCD (workgroups go to the eight XCDs in turn), where a hand-off
+// through memory takes 0.30 us one way; between XCDs 0.36-0.49 us.
+template <bool kAxis>
+__device__ __forceinline__ void ns_workgroup(const Dev &d, const SyntheticState &st, int b, char *lds) {
+  const int before = min(st.nw, (b + st.stride - 1) / st.stride);  // bands at workgroups below b
+  if (b % st.stride == 0 && b / st.stride < st.nw)
+    sweep_role<kAxis>(d, st, *reinterpret_cast<SweepShared<kAxis> *>(lds), b / st.stride);
+  else if (b - before < st.nflux)
+    flux_role(d, st, *reinterpret_cast<FluxShared *>(lds), b - before);
 }
 
-// The inner loops of a batch of instances in one launch, one workgroup per
-// instance: the workgroup computes the fluxes of its instance's tiles one
-// after another, then runs the same sweeps, until the reference's rule ends
-// the loop.  No workgroup waits for another, so the launch needs neither
-// co-residency nor host decisions and can be captured in a graph.  The same
-// records and arithmetic as k_ns_loop: the same dU and iteration counts.
-__global__ void __launch_bounds__(256) k_ns_batch(const NsJob *__restrict__ jobs) {
-  __shared__ NsShared sh;
-  const NsJob &J = jobs[blockIdx.x];
-  const Dev &d = J.d;
-  const SyntheticState &st = J.st;
-  const int tid = threadIdx.x;
-  int it = 0, bad = 0;
-  double res_last = 0.0;
-  const bool go = 1.0 > st.tol && st.maxit > 0;  // the reference starts from res = 1
-  if (go && st.rs > 0) {
-    const int ntiles = st.ntx * st.nty;
-    for (int k = 1;; k++) {
-      double rmax = 0.0;
-      int b = 0;
-      for (int tile = 0; tile < ntiles; tile++) flux_tile(d, st, sh, tile, rmax, b);
-      for (int off = 32; off > 0; off >>= 1) rmax = fmax(rmax, __shfl_down(rmax, off, 64));
-      b = __syncthreads_or(b);
-      if ((tid & 63) == 0) sh.red[tid >> 6] = rmax;
-      __syncthreads();
-      double res = sh.red[0];
-      for (int q = 1; q < (int)(blockDim.x >> 6); q++) res = fmax(res, sh.red[q]);
-      it = k;
-      res_last = res;
-      bad = b;
-      __syncthreads();
-      if (bad) break;
-      if (st.axis)
-        sweep<4, true, true>(d, st, sh);
-      else
-        sweep<4>(d, st, sh);
-      __syncthreads();
-      if (!(res > st.tol && k < st.maxit)) break;
+// The inner loop (src/Hybrid_Sub.f90:99-104) of one instance, launched
+// cooperatively (all workgroups resident).
+template <bool kAxis>
+__global__ void __launch_bounds__(kThreads) k_ns_loop(Dev d, SyntheticState st) {
+  __shared__ __align__(16) char lds[LoopShared<kAxis>::kBytes];
+  ns_workgroup<kAxis>(d, st, blockIdx.x, lds);
+}
+
+// The inner loops of a batch of instances in one launch: job J has the
+// workgroups J.wg0 .. J.wg0 + J.blocks - 1, a gang.  The workgroups of a gang
+// wait for each other, so all of them have to be resident: gangs are
+// consecutive and workgroups are dispatched in order, so only the gang at the
+// dispatch front can be incomplete, and it is completed as the gangs before it
+// end (no gang waits for another).  A gang starts once its last workgroup has
+// arrived; that wait alone may take as long as the gangs before it.
+__global__ void __launch_bounds__(kThreads) k_ns_batch(const NsJob *__restrict__ jobs, int njobs) {
+  __shared__ __align__(16) char lds[LoopShared<false>::kBytes];
+  int lo = 0, hi = njobs - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) / 2;
+    if (jobs[mid].wg0 <= (int)blockIdx.x) lo = mid;
+    else hi = mid - 1;
+  }
+  const NsJob &J = jobs[lo];
+  int *word = reinterpret_cast<int *>(lds);
+  if (threadIdx.x == 0) {
+    int *ctl = J.st.ctl;
+    __hip_atomic_fetch_add(ctl + kCtlArrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    Patience pt(ctl, kStartTicks);
+    bool ok = true;
+    while (ok && ld_agent(ctl + kCtlArrived) < J.blocks) {
+      __builtin_amdgcn_s_sleep(32);
+      ok = !pt.over(false);
     }
-  } else if (go) {
-    it = 1;  // no swept cell: one iteration that changes nothing
+    *word = ok ? 1 : 0;
   }
-  if (tid == 0) {
-    st.iters[0] = it;
-    st.iters[1] = bad;
-    st.iters[2] = 0;
-    reinterpret_cast<double *>(st.iters + 4)[0] = res_last;
-  }
+  __syncthreads();
+  const int ok = *word;
+  __syncthreads();
+  if (!ok) return;
+  const int b = (int)blockIdx.x - J.wg0;
+  const Dev d = uniform_copy(J.d);
+  const SyntheticState st = uniform_copy(J.st);
+  if (st.axis) ns_workgroup<true>(d, st, b, lds);
+  else ns_workgroup<false>(d, st, b, lds);
 }
 
 // U0 <- U and the synthetic correction of S on cells 3..n-3 (src/Hybrid_Sub.f90:108-153)
@@ -1003,12 +1259,16 @@ __global__ void k_ns_feedback(Dev d, SyntheticState st) {
 }
 
 // the next launch of the inner loop continues at iteration k0
-__global__ void k_ns_resume(SyntheticState st, int k0) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) {
+__global__ void k_ns_resume(Dev d, SyntheticState st, int k0) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t == 0) {
     st.ctl[kCtlGo] = k0;
+    st.ctl[kCtlBad] = 0;
+    st.ctl[kCtlStop] = 0;
     st.iters[1] = 0;
     st.iters[2] = 0;
   }
+  clear_hands(d, st, t, (size_t)gridDim.x * blockDim.x);
 }
 
 // the degenerate loop of a mesh without swept cells: max |Res_4| over no
@@ -1017,12 +1277,12 @@ __global__ void k_ns_empty(SyntheticState st) {
   if (threadIdx.x == 0 && blockIdx.x == 0) st.iters[0] = st.ctl[kCtlGo] == 1 ? 1 : 0;
 }
 
-// the inner-loop kernel of an instance: 256 or 1024 threads, and for 256 the
-// sweep of an axis-aligned mesh where it is one
 static const void *ns_loop_kernel(const SyntheticState &st) {
-  if (st.block > 256) return reinterpret_cast<const void *>(k_ns_loop<1024, false>);
-  return st.axis ? reinterpret_cast<const void *>(k_ns_loop<256, true>)
-                 : reinterpret_cast<const void *>(k_ns_loop<256, false>);
+  return st.axis ? reinterpret_cast<const void *>(k_ns_loop<true>) : reinterpret_cast<const void *>(k_ns_loop<false>);
+}
+// workgroups of an instance: its bands at multiples of the stride, its flux workgroups between and after them
+static int ns_blocks(const SyntheticState &st) {
+  return std::max(st.stride * (st.nw - 1) + 1, st.nw + st.nflux);
 }
 
 // whether every swept cell (3..nx-3, 3..ny-3) has the face normals ni = (1,0)
@@ -1041,62 +1301,84 @@ int synthetic_init(Dev &d, const gsis_params &p, SyntheticState &st) {
   const size_t N = d.ncell;
   st.rs = d.ny - 5 > 0 && d.nx - 5 > 0 ? d.ny - 5 : 0;
   st.np = st.rs > 0 ? d.nx + d.ny - 11 : 0;
-  if (st.rs > kMaxSweepWaves * 64) {
-    g_syn_err = "synthetic solve: at most " + std::to_string(kMaxSweepWaves * 64 + 5) + " nodes in j";
+  if (st.rs > kMaxBands * kBand) {
+    g_syn_err = "synthetic solve: at most " + std::to_string(kMaxBands * kBand + 5) + " nodes in j";
     return GSIS_EUNSUPPORTED;
   }
-  st.ntx = st.rs > 0 ? (d.nx - 5 + kTile - 1) / kTile : 0;
-  st.nty = st.rs > 0 ? (st.rs + kTile - 1) / kTile : 0;
+  st.ntx = st.rs > 0 ? (d.nx - 5 + kTI - 1) / kTI : 0;
+  st.nty = st.rs > 0 ? (st.rs + kTJ - 1) / kTJ : 0;
   const int ntiles = st.ntx * st.nty;
-  st.block = std::max(256, 64 * ((st.rs + 63) / 64));
-  st.axis = st.block <= 256 && st.rs > 0 && axis_aligned(p, d.nx, d.ny);
+  st.axis = st.rs > 0 && axis_aligned(p, d.nx, d.ny);
+  st.nw = (st.rs + kBand - 1) / kBand;
+  st.stride = 8;
   if (ntiles > 0) {
     int dev = 0, ncu = 0, per = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e == hipSuccess)
-      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, ns_loop_kernel(st), st.block, 0);
+    if (e == hipSuccess) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, ns_loop_kernel(st), kThreads, 0);
     if (e != hipSuccess || per < 1) {
       g_syn_err = std::string("synthetic solve: occupancy query: ") + hipGetErrorString(e) + ", " +
-                  std::to_string(per) + " workgroups of " + std::to_string(st.block) + " threads per CU";
+                  std::to_string(per) + " workgroups of " + std::to_string(kThreads) + " threads per CU";
       return GSIS_EHIP;
     }
-    st.nflux = std::min(ntiles, ncu * per - 1);
-    if (st.nflux < 1) {
+    // one workgroup per CU: the fluxes run beside the sweeps, so more of them
+    // at a time would only share the sweeps' CUs
+    st.nflux = std::min(ntiles, ncu - st.nw);
+    if (st.nflux < 1 || ns_blocks(st) > ncu * per) {
       g_syn_err = "synthetic solve: the inner-loop launch does not fit the device";
       return GSIS_EUNSUPPORTED;
     }
   }
-  st.nw = (st.rs + 63) / 64;
   const size_t nq = (size_t)st.np * st.nw * 64;  // cells of the blocked sweep layout
-  // 32-bit buffer offsets of the records and of U
-  if ((size_t)kNRec * nq * sizeof(double) >= ((size_t)1 << 31) || (size_t)4 * N * sizeof(double) >= ((size_t)1 << 31)) {
+  // 32-bit buffer offsets of the blocked arrays (the largest has 12 doubles
+  // per cell, and the limit leaves room for half as many again) and of U
+  if ((size_t)18 * nq * sizeof(double) >= ((size_t)1 << 31) || (size_t)4 * N * sizeof(double) >= ((size_t)1 << 31)) {
     g_syn_err = "synthetic solve: the mesh is too large for the sweep's buffers (2 GiB)";
     return GSIS_EUNSUPPORTED;
   }
-  const size_t n_dbl = 4 * N + (size_t)kNRec * nq + 4 * nq + 8 * (size_t)std::max(st.nflux, 1);
-  const size_t bytes = n_dbl * 8 + 64;
+  const size_t npad = (size_t)(st.np + 2 * kPad) * st.nw * 64;
+  const size_t n_geo = (size_t)2 * geo_pairs(st.axis) * nq;
+  const size_t n_hand = st.nw > 0 ? (size_t)2 * st.nw * hand_len(d.nx) * 4 : 0;
+  const size_t n_dbl = 4 * N + (size_t)kNRec * nq + 8 * npad + n_geo + n_hand + (size_t)ntiles +
+                       (size_t)kProgStride * std::max(st.nw, 1);
+  const size_t bytes = n_dbl * 8 + 128 + 8 * (size_t)ntiles + 64;
   void *mem = nullptr;
   if (hipMalloc(&mem, bytes) != hipSuccess || hipMemset(mem, 0, bytes) != hipSuccess) {
     g_syn_err = "synthetic solve: device allocation failed";
     return GSIS_EHIP;
   }
-  double *b = reinterpret_cast<double *>(mem);
-  st.s00 = b; b += 4 * N;
+  double *b = reinterpret_cast<double *>(mem);  // every array with pairs starts at a multiple of 16 bytes
   st.rec = b; b += kNRec * nq;
-  st.dstar = b; b += 4 * nq;
-  st.part = b; b += 8 * (size_t)std::max(st.nflux, 1);
+  st.dstar = b; b += 4 * npad;
+  st.ub = b; b += 4 * npad;
+  st.geo = b; b += n_geo;
+  st.hand = b; b += n_hand;
+  st.s00 = b; b += 4 * N;
+  st.prog = reinterpret_cast<long long *>(b); b += (size_t)kProgStride * std::max(st.nw, 1);
+  st.tres = b; b += ntiles;
   st.ctl = reinterpret_cast<int *>(b);
-  st.iters = st.ctl + 8;
+  st.iters = st.ctl + 16;
+  st.ready = st.ctl + 32;
+  st.order = st.ready + ntiles;
   st.mem = mem;
+  auto bail = [&](const char *msg) {
+    (void)hipFree(mem);
+    st.mem = nullptr;
+    g_syn_err = msg;
+    return GSIS_EHIP;
+  };
+  if (ntiles > 0) {  // tiles by level, as the sweeps pass them
+    std::vector<int> order(ntiles);
+    for (int t = 0; t < ntiles; t++) order[t] = t;
+    std::stable_sort(order.begin(), order.end(),
+                     [&](int x, int y) { return x % st.ntx + kLev * (x / st.ntx) < y % st.ntx + kLev * (y / st.ntx); });
+    if (hipMemcpy(st.order, order.data(), sizeof(int) * ntiles, hipMemcpyHostToDevice) != hipSuccess)
+      return bail("synthetic solve: tile order upload failed");
+  }
   if (nq > 0) {
-    hipLaunchKernelGGL(k_rec_init, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, 0, st);
-    if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess) {
-      (void)hipFree(mem);
-      st.mem = nullptr;
-      g_syn_err = "synthetic solve: record initialisation failed";
-      return GSIS_EHIP;
-    }
+    hipLaunchKernelGGL(k_rec_init, dim3((unsigned)((nq + 255) / 256)), dim3(256), 0, 0, d, st);
+    if (hipGetLastError() != hipSuccess || hipDeviceSynchronize() != hipSuccess)
+      return bail("synthetic solve: record initialisation failed");
   }
   st.tol = p.ns_tol;
   st.maxit = p.ns_maxit > 0 ? p.ns_maxit : 100000;
@@ -1115,7 +1397,7 @@ int synthetic_begin(const Dev &d, SyntheticState &st, hipStream_t s) {
     return GSIS_EARG;
   }
   const int nc = (d.nx - 1) * (d.ny - 1);
-  hipLaunchKernelGGL(k_ns_prepare, dim3((std::max(nc, st.nflux) + 255) / 256), dim3(256), 0, s, d, st);
+  hipLaunchKernelGGL(k_ns_prepare, dim3((std::max(nc, st.ntx * st.nty) + 255) / 256), dim3(256), 0, s, d, st);
   return 0;
 }
 
@@ -1124,15 +1406,15 @@ int synthetic_run(const Dev &d, SyntheticState &st, int k0, int kstop, hipStream
     g_syn_err = "synthetic solve: not initialised, or an empty range of inner iterations";
     return GSIS_EARG;
   }
-  if (k0 > 1) hipLaunchKernelGGL(k_ns_resume, dim3(1), dim3(64), 0, s, st, k0);
+  if (k0 > 1) hipLaunchKernelGGL(k_ns_resume, dim3(32), dim3(256), 0, s, d, st, k0);
   if (st.nflux > 0) {
     Dev dd = d;
     SyntheticState ss = st;
     ss.k0 = k0;
     ss.kstop = kstop;
     void *args[] = {&dd, &ss};
-    const hipError_t e = hipLaunchCooperativeKernel(ns_loop_kernel(st),
-                                                    dim3(1 + st.nflux), dim3(st.block), args, 0, s);
+    const hipError_t e =
+        hipLaunchCooperativeKernel(ns_loop_kernel(st), dim3(ns_blocks(st)), dim3(kThreads), args, 0, s);
     if (e != hipSuccess) {
       g_syn_err = std::string("synthetic solve: cooperative launch failed: ") + hipGetErrorString(e);
       return GSIS_EHIP;
@@ -1143,10 +1425,38 @@ int synthetic_run(const Dev &d, SyntheticState &st, int k0, int kstop, hipStream
   return 0;
 }
 
-bool synthetic_batchable(const SyntheticState &st) { return st.on && st.block <= 256; }
+bool synthetic_batchable(const SyntheticState &st) { return st.on && st.rs <= 4 * kBand; }
 
-void launch_ns_batch(const NsJob *djobs, int n, hipStream_t s) {
-  if (n > 0) hipLaunchKernelGGL(k_ns_batch, dim3(n), dim3(256), 0, s, djobs);
+// Flux workgroups per instance: as many tiles each as keep the whole batch
+// resident, but at most kBatchTiles (a tile takes about 4 us, a sweep that
+// its fluxes run beside 50-200 us).
+int synthetic_batch_layout(std::vector<NsJob> &jobs) {
+  constexpr int kBatchTiles = 16;
+  int dev = 0, ncu = 0, per = 0;
+  if (hipGetDevice(&dev) != hipSuccess ||
+      hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+      hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, reinterpret_cast<const void *>(k_ns_batch), kThreads, 0) !=
+          hipSuccess ||
+      per < 1) {
+    g_syn_err = "synthetic solve: occupancy query of the batched launch failed";
+    return -1;
+  }
+  for (int tiles = 1;; tiles++) {
+    int at = 0;
+    for (NsJob &j : jobs) {
+      const int nt = j.st.ntx * j.st.nty;
+      j.st.nflux = (nt + tiles - 1) / tiles;
+      j.st.stride = 8 * (j.st.nw - 1) + 1 <= j.st.nw + j.st.nflux ? 8 : 1;
+      j.wg0 = at;
+      j.blocks = ns_blocks(j.st);
+      at += j.blocks;
+    }
+    if (at <= ncu * per || tiles >= kBatchTiles) return at;
+  }
+}
+
+void launch_ns_batch(const NsJob *djobs, int n, int blocks, hipStream_t s) {
+  if (n > 0) hipLaunchKernelGGL(k_ns_batch, dim3(blocks), dim3(kThreads), 0, s, djobs, n);
 }
 
 void synthetic_finish(const Dev &d, SyntheticState &st, hipStream_t s) {

@@ -315,10 +315,10 @@ int gsis_fill_frd_uniform(gsis_handle *h, const double *g, const double *hv);
  * the step of all instances up to the synthetic solve (S0, kinetic BCs, that
  * launch, moments, DETFPwall, Convert_NS, HoT) is captured once as a hipGraph
  * and replayed per step.  The synthetic solves of instances in mode M1 run
- * either inside the graph, all in one launch with one workgroup per
+ * either inside the graph, all in one launch with a few workgroups per
  * instance, or after the graph, one cooperative launch per instance (the
  * only way for instances with a closure network or more than 256 swept rows).
- * Inside is the default when at least 32 instances qualify; gsis_batch_tune
+ * Inside is the default when at least 4 instances qualify; gsis_batch_tune
  * times the other placement too, gsis_batch_set_ns_graph chooses it.  Both
  * give the same results.  Instances may differ in mesh, velocity grid, gas, walls and mode; they
  * must share precision, flux scheme and device, and fit the
@@ -335,7 +335,7 @@ int gsis_batch_step(gsis_batch *b, int32_t nsteps);
  * choice computes the same step) and reports it with its time per step. */
 int gsis_batch_tune(gsis_batch *b, int32_t steps_per_trial, int32_t *nw, int32_t *order, double *ms_per_step);
 /* Placement of the M1 instances' synthetic solves: -1 automatic (inside the
- * graph when at least 32 instances qualify), 0 after the graph, 1 inside the
+ * graph when at least 4 instances qualify), 0 after the graph, 1 inside the
  * graph for every instance that qualifies; the step is captured again. */
 int gsis_batch_set_ns_graph(gsis_batch *b, int32_t mode);
 /* The number of instances whose synthetic solve runs inside the graph. */
