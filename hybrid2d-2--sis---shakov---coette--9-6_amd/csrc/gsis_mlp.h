@@ -16,32 +16,32 @@ constexpr int kMlpOutPad = 32;                   // output rows padded to one MF
 constexpr int kMlpBatchMax = 8192;               // samples per pass
 
 // rows (outputs) and columns (inputs) of layer l, and its padded row count
-__host__ __device__ inline int mlp_rows(int l) { return l == kMlpLayers - 1 ? kMlpOut : kMlpW; }
-__host__ __device__ inline int mlp_cols(int l) { return l == 0 ? kMlpIn : kMlpW; }
-__host__ __device__ inline int mlp_rows_pad(int l) { return l == kMlpLayers - 1 ? kMlpOutPad : kMlpW; }
+__host__ __device__ constexpr inline int mlp_rows(int l) { return l == kMlpLayers - 1 ? kMlpOut : kMlpW; }
+__host__ __device__ constexpr inline int mlp_cols(int l) { return l == 0 ? kMlpIn : kMlpW; }
+__host__ __device__ constexpr inline int mlp_rows_pad(int l) { return l == kMlpLayers - 1 ? kMlpOutPad : kMlpW; }
 constexpr int kMlpInPad = 32;  // input columns padded to one MFMA block
-__host__ __device__ inline int mlp_cols_pad(int l) { return l == 0 ? kMlpInPad : kMlpW; }
+__host__ __device__ constexpr inline int mlp_cols_pad(int l) { return l == 0 ? kMlpInPad : kMlpW; }
+
+constexpr int kMlpRows = 64;  // samples a workgroup takes
 
 // Device state of one network: FP32 master parameters [W1 b1 W2 b2 ... W5 b5]
 // (W row-major, outputs by inputs), their BF16 copies for the MFMA kernels in
 // both orientations (W and its transpose, rows and columns padded with zeros
-// to whole 32 x 32 blocks), Adam moments, and the work buffers of one batch.
+// to whole 32 x 32 blocks), Adam moments, and what a batch's backward pass
+// leaves for the weight gradients.
 struct MlpDev {
   float *p = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr;  // [nparams]
   unsigned short *w[kMlpLayers] = {}, *wt[kMlpLayers] = {};
   float scale[2 * kMlpIn + 2 * kMlpOut] = {};  // in mean, in std, out mean, out std (host copy)
   float *dscale = nullptr;                     // the same on the device
-  // batch buffers: inputs X0 (+ transpose), per layer pre-activations Z (fp32),
-  // activations H (bf16, + transpose), the GEMM output C (fp32), gradients
-  unsigned short *x0 = nullptr, *x0t = nullptr;
-  float *z[kMlpLayers] = {};
-  unsigned short *h[kMlpLayers] = {}, *ht[kMlpLayers] = {};
-  float *c = nullptr;
-  unsigned short *dz = nullptr, *dzt = nullptr;
-  float *dh = nullptr;
+  // of a batch: inputs of each layer and dZ (bf16, operand order: see MlpTape),
+  // dZ (fp32) [sample][out], dY (fp32) [sample][8], each workgroup's squared error
+  unsigned short *in_t[kMlpLayers] = {}, *dz_t[kMlpLayers] = {};
+  float *dz[kMlpLayers - 1] = {}, *dy = nullptr;
+  double *lpart = nullptr;
   float *xin = nullptr, *yin = nullptr;  // staged samples (raw)
   int *idx = nullptr;                    // batch sample indices
-  double *loss = nullptr;
+  double *loss = nullptr;                // [0] of the last batch, [1] summed over an epoch's batches
   size_t cap = 0;  // samples the staged buffers hold
   hipStream_t s = nullptr;
   int step = 0;  // Adam steps taken
