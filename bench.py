@@ -365,7 +365,7 @@ def main():
     ap.add_argument("--precision", choices=("fp64", "fp32"), default="fp64")
     ap.add_argument("--cpu-steps", type=int, default=1, help="oracle steps of the CPU-baseline sample (0: skip)")
     ap.add_argument("--kernel", choices=("auto", "split", "tiles", "strip16"), default="auto",
-                    help="kinetic kernels: one-pass column-wavefront kernel (auto: 8 columns per workgroup, "
+                    help="kinetic kernels: one-pass column-pair kernel (auto: 16 or 8 columns per workgroup, "
                          "strip16: 16), separate RHS and sweep kernels, or the one-pass velocity-tile walker")
     ap.add_argument("--scheme", choices=("nnd", "weno3", "up1"), default="nnd",
                     help="kinetic flux scheme (the reference's Iflag_scheme 1, 3, 0)")

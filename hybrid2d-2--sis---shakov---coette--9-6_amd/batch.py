@@ -1,5 +1,5 @@
 """Batches of GSIS instances stepped together (gsis_batch_*): one launch of the
-column-wavefront kinetic kernel over every instance's strips per step, the
+column-pair kinetic kernel over every instance's strips per step, the
 whole step of all instances captured once as a hipGraph, and the project's
 autotuner choosing strip width and job order.  No counterpart in the
 reference, which runs one case per process.

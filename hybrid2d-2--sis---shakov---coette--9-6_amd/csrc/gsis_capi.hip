@@ -55,7 +55,7 @@ struct gsis_handle {
   void *FG = nullptr, *FH = nullptr, *slot = nullptr, *RG = nullptr, *RH = nullptr;
   std::vector<void *> allocs;
   double *cpar = nullptr;  // per-cell constants of the fused kinetic kernel
-  gsis::StripBufs strip;   // seam buffers of the column-wavefront kernel
+  gsis::StripBufs strip;   // seam buffer of the column-pair kernel
   int *wall_list = nullptr;
   int nwall = 0;
   double *swall = nullptr;
@@ -98,6 +98,13 @@ int dalloc(gsis_handle *h, P **ptr, size_t bytes) {
   h->allocs.push_back(q);
   *ptr = reinterpret_cast<P *>(q);
   return 0;
+}
+
+// every seam message not written (as before a handle's first step)
+bool strip_clear(gsis_handle *h) {
+  return hipMemsetD32((hipDeviceptr_t)h->strip.msg, (int)gsis::strip_empty_word(h->tsize == 4),
+                      h->strip.msg_elems * h->tsize / 4) == hipSuccess &&
+         hipStreamSynchronize(nullptr) == hipSuccess;
 }
 
 int bc_nk(const gsis_bc &b) { return (b.face == 1 || b.face == 3) ? (b.jend - b.jst + 1) : (b.iend - b.ist + 1); }
@@ -208,7 +215,8 @@ void kinetic(gsis_handle *h) {
     if (sel == GSIS_KERNEL_AUTO || sel == GSIS_KERNEL_STRIP16) {
       h->strip.ev_before = h->timing ? h->ev[2] : nullptr;
       h->strip.ev_after = h->timing ? h->ev[3] : nullptr;
-      ok = gsis::launch_strip<T>(h->d, h->cpar, FG, slot, RG, store, sel == GSIS_KERNEL_STRIP16 ? 16 : 8, h->strip,
+      ok = gsis::launch_strip<T>(h->d, h->cpar, FG, slot, RG, store,
+                                 sel == GSIS_KERNEL_STRIP16 ? 16 : gsis::strip_columns(gsis::strip_blocks(h->d, 16)), h->strip,
                                  h->s);
     }
     if (!ok) {
@@ -407,9 +415,8 @@ struct gsis_batch {
   int nw = 8, order = 0;  // strip width and job order of the captured step
   hipStream_t s = nullptr;
   void *djobs = nullptr;  // device table of StripJob<T>
-  int *epoch = nullptr;   // [0] launch epoch, [1] a seam wait timed out
-  std::vector<int *> flags;
-  int nstrip = 0, nseam = 0, ncellb = 0;
+  int *err = nullptr;     // a seam wait timed out
+  int nstrip = 0, ncellb = 0;
   gsis::NsJob *nsjobs = nullptr;  // device table of the inner loops run in the graph
   int nns = 0, nsblocks = 0;      // its entries, and the workgroups of their launch
   std::vector<bool> in_graph;     // M1 instance whose synthetic solve is captured
@@ -452,7 +459,7 @@ std::vector<int> batch_order(const gsis_batch *b, int order) {
 template <typename T>
 int batch_jobs(gsis_batch *b) {
   std::vector<gsis::StripJob<T>> jobs;
-  int a = 0, c = 0, e = 0;
+  int a = 0, e = 0;
   for (int k : batch_order(b, b->order)) {
     gsis_handle *h = b->hs[k];
     gsis::StripJob<T> j{};
@@ -462,20 +469,15 @@ int batch_jobs(gsis_batch *b) {
     j.R = (T *)h->RG;
     j.slot = (const T *)h->slot;
     j.msg = (T *)h->strip.msg;
-    j.dright = (T *)h->strip.dright;
-    j.flag = b->flags[k];
     j.oflags = h->strip.oflags;
     j.ntiles = (h->d.nv + 63) / 64;
     j.strip0 = a;
-    j.seam0 = c;
     j.cell0 = e;
     a += gsis::strip_blocks(h->d, b->nw);
-    c += gsis::seam_blocks(h->d, b->nw);
     e += gsis::cell_blocks(h->d);
     jobs.push_back(j);
   }
   b->nstrip = a;
-  b->nseam = c;
   b->ncellb = e;
   HIPCHK(hipMemcpy(b->djobs, jobs.data(), jobs.size() * sizeof(jobs[0]), hipMemcpyHostToDevice));
   return 0;
@@ -531,7 +533,7 @@ int batch_capture(gsis_batch *b) {
       phy_boundary<T>(h);
     }
     gsis::launch_strip_batch<T>((const gsis::StripJob<T> *)b->djobs, (int)b->hs.size(), b->nw, b->scheme, b->nstrip,
-                                b->nseam, b->ncellb, b->epoch, b->epoch + 1, b->s);
+                                b->ncellb, b->err, b->s);
     for (gsis_handle *h : b->hs) {
       moments<T>(h);
       if (h->mass_on) gsis::launch_mass_correct(h->d, h->mwork, h->init_mass, b->s);
@@ -590,9 +592,13 @@ int batch_replay(gsis_batch *b, int nsteps) {
     h->tt += nsteps * h->p.dt;
     h->kstep += nsteps;
   }
-  int w[2] = {0, 0};
-  HIPCHK(hipMemcpy(w, b->epoch, sizeof(w), hipMemcpyDeviceToHost));
-  if (w[1]) return fail(GSIS_EHIP, "batch: a wait for a neighbouring strip timed out");
+  int w = 0;
+  HIPCHK(hipMemcpy(&w, b->err, sizeof(w), hipMemcpyDeviceToHost));
+  if (w) {
+    for (gsis_handle *h : b->hs)
+      if (h->strip.msg) (void)strip_clear(h);  // messages nobody received
+    return fail(GSIS_EHIP, "batch: a wait for a neighbouring strip timed out");
+  }
   for (gsis_handle *h : b->hs) {
     const int rc = check_err_flag(h);
     if (rc) return rc;
@@ -701,9 +707,9 @@ int gsis_create(const gsis_params *p, gsis_handle **out) {
       (rc = dalloc(h, &d.taoi, 8 * 4 * N)) || (rc = dalloc(h, &d.taoj, 8 * 4 * N)) ||
       (rc = dalloc(h, &d.qi, 8 * 2 * N)) || (rc = dalloc(h, &d.qj, 8 * 2 * N)) ||
       (rc = dalloc(h, &d.prim, 8 * 5 * N)) || (rc = dalloc(h, &d.res4, 8 * 4 * N)) || (rc = dalloc(h, &d.err, 64)) ||
-      // ny+3 planes of <= 3*1024 constants (k_walk), or kNCellPar per interior cell (k_strip)
+      // ny+3 planes of <= 3*1024 constants (k_walk), or kNCellPar per interior cell and one cell more (k_strip)
       (rc = dalloc(h, &h->cpar, 8 * std::max((size_t)(ny + 3) * 3 * 1024,
-                                             (size_t)(nx - 1) * (ny - 1) * gsis::kNCellPar))) ||
+                                             ((size_t)(nx - 1) * (ny - 1) + 1) * gsis::kNCellPar))) ||
       (rc = dalloc(h, &h->resbuf, 8 * 8)))
     return cleanup(rc);
   {  // Creat_Mesh sets U, U0, U2 to (1,0,0,1) (src/sub_init.f90:159-162)
@@ -757,7 +763,7 @@ int gsis_create(const gsis_params *p, gsis_handle **out) {
       (!wl.empty() && hipMemcpy(h->wall_list, wl.data(), 4 * wl.size(), hipMemcpyHostToDevice) != hipSuccess))
     return cleanup(fail(GSIS_EHIP, "BC table upload failed"));
   d.ovrI1 = o1; d.ovrI3 = o3; d.ovrJ2 = o2; d.ovrJ4 = o4;
-  {  // the same flags as 32-bit words for the column-wavefront kernel's scalar loads
+  {  // the same flags as 32-bit words for the column-pair kernel's scalar loads
     std::vector<int> of(ny + 2 + nx + 2, 0);
     for (int j = 0; j < ny + 2; j++) of[j] = (oi1[j] ? 1 : 0) | (oi3[j] ? 2 : 0);
     for (int i = 0; i < nx + 2; i++) of[ny + 2 + i] = (oj2[i] ? 1 : 0) | (oj4[i] ? 2 : 0);
@@ -772,20 +778,17 @@ int gsis_create(const gsis_params *p, gsis_handle **out) {
   const size_t ns = (size_t)4 * d.L * 2 * d.nv * h->tsize;
   // G plane, H plane and the wall slots in one allocation (the fused kernel
   // addresses all three with 32-bit offsets from one base)
-  if ((rc = dalloc(h, &h->FG, 2 * nf + ns)) || (rc = dalloc(h, &h->RG, 2 * nf))) return cleanup(rc);
+  if ((rc = dalloc(h, &h->FG, 2 * nf + ns + 64)) || (rc = dalloc(h, &h->RG, 2 * nf))) return cleanup(rc);
   h->FH = (char *)h->FG + nf;
   h->slot = (char *)h->FG + 2 * nf;
   h->RH = (char *)h->RG + nf;
-  {  // seam buffers of the column-wavefront kernel, sized for 8 columns per workgroup
+  {  // seam buffer of the column-pair kernel, sized for 8 columns per workgroup
     const size_t rows = gsis::strip_rows(d, 8);
     gsis::StripBufs &sb = h->strip;
     if (rows > 0) {
-      if ((rc = dalloc(h, &sb.msg, rows * 256 * h->tsize)) || (rc = dalloc(h, &sb.dright, rows * 128 * h->tsize)) ||
-          (rc = dalloc(h, &sb.flag, rows * sizeof(int))))
-        return cleanup(rc);
+      if ((rc = dalloc(h, &sb.msg, rows * 256 * h->tsize))) return cleanup(rc);
       sb.msg_elems = rows * 256;
-      sb.dright_elems = rows * 128;
-      sb.flag_elems = rows;
+      if (!strip_clear(h)) return cleanup(fail(GSIS_EHIP, "seam buffer fill failed"));
     }
     sb.err = d.err + 1;
   }
@@ -1132,6 +1135,9 @@ int gsis_batch_create(gsis_handle *const *hs, int32_t n, gsis_batch **out) {
   b->hs.assign(hs, hs + n);
   b->prec = hs[0]->prec;
   b->scheme = hs[0]->d.scheme;
+  long long strips16 = 0;
+  for (int k = 0; k < n; k++) strips16 += gsis::strip_blocks(hs[k]->d, 16);
+  b->nw = gsis::strip_columns(strips16);
   auto bail = [&](int rc) {
     gsis_batch_destroy(b);
     return rc;
@@ -1144,13 +1150,7 @@ int gsis_batch_create(gsis_handle *const *hs, int32_t n, gsis_batch **out) {
   if (hipStreamCreateWithFlags(&b->s, hipStreamNonBlocking) != hipSuccess)
     return bail(fail(GSIS_EHIP, "batch: hipStreamCreate failed"));
   const size_t jb = (size_t)n * std::max(sizeof(gsis::StripJob<double>), sizeof(gsis::StripJob<float>));
-  if (!alloc(&b->djobs, jb) || !alloc((void **)&b->epoch, 64)) return bail(fail(GSIS_EHIP, "batch: allocation failed"));
-  for (int k = 0; k < n; k++) {
-    void *f = nullptr;
-    if (!alloc(&f, std::max<size_t>(gsis::strip_rows(hs[k]->d, 8), 1) * sizeof(int)))
-      return bail(fail(GSIS_EHIP, "batch: allocation failed"));
-    b->flags.push_back((int *)f);
-  }
+  if (!alloc(&b->djobs, jb) || !alloc((void **)&b->err, 64)) return bail(fail(GSIS_EHIP, "batch: allocation failed"));
   const int rc = batch_capture_any(b);
   if (rc) return bail(rc);
   *out = b;

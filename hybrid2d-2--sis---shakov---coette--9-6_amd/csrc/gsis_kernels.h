@@ -29,52 +29,52 @@ constexpr int kNCellPar = 20;  // per-cell constants of the fused kinetic kernel
 // Fused kinetic step over F = [G plane | H plane] (and R likewise); false when
 // the mesh does not fit the fused kernel.
 template <typename T> bool launch_walk(const Dev &d, double *cpar, T *F, const T *slot, T *R, int store_rhs, int tiles, hipStream_t s);
-// Buffers of the column-wavefront kernel (k_strip): seam messages
-// [seam][tile][row][4][64] and the next strip's Delta* [seam][tile][row][2][64]
-// (elements of the working precision), per-row ready flags holding the
-// launch epoch, and a word set when a wait for a flag timed out.
+// Buffers of the column-pair kernel (k_strip): seam messages
+// [seam][tile][row][4][64] (elements of the working precision), every word
+// strip_empty_word() outside a launch, and a word set when a wait for a
+// message timed out.
 struct StripBufs {
-  void *msg = nullptr, *dright = nullptr;
-  int *flag = nullptr, *err = nullptr;
+  void *msg = nullptr;
+  int *err = nullptr;
   // face-override words: ny+2 rows (bit 0 i-face 1, bit 1 i-face nx), then
   // nx+2 columns (bit 0 j-face 1, bit 1 j-face ny)
   const int *oflags = nullptr;
-  size_t msg_elems = 0, dright_elems = 0, flag_elems = 0;
-  int epoch = 0;
+  size_t msg_elems = 0;
   // when set, recorded on the stream just before and after k_strip itself
   hipEvent_t ev_before = nullptr, ev_after = nullptr;
 };
 // seam rows (seam x tile x row) of a mesh with nw columns per workgroup
 size_t strip_rows(const Dev &d, int nw);
-// Column-wavefront kinetic step with nw (8 or 16) columns per workgroup, plus
-// the seam update; false when the mesh or the buffers do not fit.
+// the word a seam message is filled with before its first use
+uint32_t strip_empty_word(bool fp32);
+// Column-pair kinetic step with nw (8 or 16) columns per workgroup; false when
+// the mesh or the buffers do not fit.
 template <typename T> bool launch_strip(const Dev &d, double *cpar, T *F, const T *slot, T *R, int store_rhs, int nw, StripBufs &b, hipStream_t s);
 template <typename T> void launch_res4(const Dev &d, const T *RG, const T *RH, hipStream_t s);
 // One instance of a batched kinetic step: its device state and the first
-// workgroup of its share of each batched launch.  The seam flags are the
-// batch's own (their values are the batch's launch epochs).
+// workgroup of its share of each batched launch.
 template <typename T>
 struct StripJob {
   Dev d;
   const T *cp;  // cell constants in T (k_cellpar), by cell
   T *F, *R;
   const T *slot;
-  T *msg, *dright;
-  int *flag;
+  T *msg;
   const int *oflags;
   int ntiles;
-  int strip0, seam0, cell0;  // first workgroup in the strip, seam and cell-constant launches
+  int strip0, cell0;  // first workgroup in the strip and cell-constant launches
 };
+// columns per workgroup for launches of so many strips of 16 columns
+int strip_columns(long long strips16);
 // workgroups of one job in the batched launches with nw columns per strip workgroup
 int strip_blocks(const Dev &d, int nw);
-int seam_blocks(const Dev &d, int nw);
 int cell_blocks(const Dev &d);
 // the kinetic step of every job (djobs: device table, host copies of the
-// counts): epoch += 1, cell constants, one column-wavefront launch over all
-// jobs' strips (no RHS kept), the seam update; scheme and T shared by all jobs
+// counts): cell constants, one column-pair launch over all jobs' strips (no
+// RHS kept); scheme and T shared by all jobs
 template <typename T>
-void launch_strip_batch(const StripJob<T> *djobs, int njobs, int nw, int scheme, int nstrip, int nseam, int ncellb,
-                        int *epoch, int *werr, hipStream_t s);
+void launch_strip_batch(const StripJob<T> *djobs, int njobs, int nw, int scheme, int nstrip, int ncellb, int *werr,
+                        hipStream_t s);
 // every cell's distribution set to g[v] (G) and h[v] (H), wall slots zero
 template <typename T>
 void launch_fill_uniform(const Dev &d, const double *g, const double *h, T *FG, T *FH, T *slot, hipStream_t s);

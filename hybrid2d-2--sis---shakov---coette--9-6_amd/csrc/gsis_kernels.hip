@@ -625,7 +625,7 @@ __global__ void __launch_bounds__(256) k_sweep(Dev d, int VT, T *FG, T *FH, cons
 // ------------------------------------------------------------------------
 constexpr int kNW = kNCellPar;
 // With pstride = 0 the constants are stored by cell instead, cpar[((j-1)*(nx-1) + i-1)*kNW + k]
-// (the layout of the column-wavefront kernel).
+// (the layout of the column-pair kernel).
 template <typename P>
 __device__ __forceinline__ void cellpar_body(const Dev &d, P *cpar, int pstride, int t) {
   const int ncol = d.nx - 1, nrow = d.ny - 1;
@@ -689,18 +689,6 @@ __device__ __forceinline__ T wflux(int f, int n, int fl, T a, T fm2, T fm1, T f0
   const bool wall = ((fl & 1) && f == 1) || ((fl & 2) && f == n);
   return wall ? a * sv : fx;
 }
-// wflux for the face at index 1 of its direction.  With n >= 5 (checked by
-// gsis_create) neither of wflux's n-1 / n rules can apply, and leaving their
-// comparisons out keeps loop-invariant masks of n out of scalar registers.
-template <int SL, typename T>
-__device__ __forceinline__ T wflux1(int fl, T a, T fm2, T fm1, T f0, T fp1, T sv, T hs) {
-  const T asp = posp(a), asn = negp(a);
-  const T d0 = f0 - fm1;
-  T sl, sr;
-  slopes<SL>(d0, fm1 - fm2, fp1 - f0, sl, sr);
-  const T fx = asp * (fm1 + hs * sl) + asn * (f0 - hs * sr);
-  return (fl & 1) ? a * sv : fx;
-}
 // interior face (no override) of the fused kernel's fast path
 template <int SL, typename T>
 __device__ __forceinline__ T iflux(T a, T fm2, T fm1, T f0, T fp1, T hs) {
@@ -746,7 +734,66 @@ __device__ __forceinline__ double wexp(double x) {
   p = fma(p, r, 1.0);
   return ldexp(p, (int)k);
 }
-__device__ __forceinline__ float wexp(float x) { return expf(x); }
+// exp of two arguments at once, with the coefficients in vector registers
+// where the kernel has the registers to keep them (KEEP: no scalar loads and
+// waits per call) and otherwise loaded once for both; the two Horner chains
+// fill each other's latency.
+template <typename T, bool KEEP>
+struct Exp2 {
+  __device__ __forceinline__ void operator()(T x, T y, T &ex, T &ey) const {
+    ex = expf(x);
+    ey = expf(y);
+  }
+};
+template <bool KEEP>
+struct Exp2<double, KEEP> {
+  double c[12];
+  __device__ __forceinline__ Exp2() {
+    if constexpr (KEEP) {
+      cdptr kc = (cdptr)kExpC;
+#pragma unroll
+      for (int m = 0; m < 12; m++) {
+        c[m] = kc[m];
+        asm volatile("" : "+v"(c[m]));
+      }
+    }
+  }
+  __device__ __forceinline__ void operator()(double x, double y, double &ex, double &ey) const {
+    cdptr kc = (cdptr)kExpC;
+    if constexpr (!KEEP) asm volatile("" : "+s"(kc));
+    x = x < kc[15] ? kc[15] : x;  // below -746 the result underflows to 0 anyway
+    y = y < kc[15] ? kc[15] : y;
+    const double k = rint(x * kc[12]), l = rint(y * kc[12]);
+    double r = fma(k, kc[13], x), t = fma(l, kc[13], y);
+    r = fma(k, kc[14], r);
+    t = fma(l, kc[14], t);
+    double p, q;
+    if constexpr (KEEP) {
+      p = c[0];
+      q = c[0];
+#pragma unroll
+      for (int m = 1; m < 12; m++) {
+        p = fma(p, r, c[m]);
+        q = fma(q, t, c[m]);
+      }
+    } else {
+      p = kc[0];
+      q = kc[0];
+#pragma unroll
+      for (int m = 1; m < 12; m++) {
+        const double a = kc[m];
+        asm("v_fma_f64 %0, %1, %2, %3" : "=v"(p) : "v"(p), "v"(r), "s"(a));
+        asm("v_fma_f64 %0, %1, %2, %3" : "=v"(q) : "v"(q), "v"(t), "s"(a));
+      }
+    }
+    p = fma(p, r, 1.0);
+    q = fma(q, t, 1.0);
+    p = fma(p, r, 1.0);
+    q = fma(q, t, 1.0);
+    ex = ldexp(p, (int)k);
+    ey = ldexp(q, (int)l);
+  }
+};
 // element at a 32-bit byte offset from a uniform base (global_load with an
 // SGPR base and a VGPR offset)
 template <typename T>
@@ -1062,35 +1109,64 @@ __global__ void __launch_bounds__(1024) k_walk(Dev d, const double *cpar, int VT
 }
 
 // ------------------------------------------------------------------------
-// Column-wavefront kinetic step ("strip walker"): the same single pass as
-// k_walk (Shakhov equilibrium, NND fluxes, forward LU-SGS recursion,
-// non-recursive backward pass, update and clamp; src/GKUA_Residual.f90:26-109,
-// 117-469), mapped so that one wavefront owns one mesh column and 64
-// consecutive velocities, with G and H of a velocity in the same lane.  Row,
-// column, wall rules and the 20 cell constants are then wave-uniform (scalar
-// registers and scalar loads), every access to F is one contiguous line per
-// wavefront, and the work that depends only on the cell and the velocity
-// (exp, Shakhov factor, face coefficients, LU-SGS diagonal) is shared by G
-// and H.
+// Column-pair kinetic step: the same single pass as k_walk (Shakhov
+// equilibrium, NND fluxes, forward LU-SGS recursion, non-recursive backward
+// pass, update and clamp; src/GKUA_Residual.f90:26-109,117-469), mapped so
+// that one wavefront owns two neighbouring mesh columns and 64 consecutive
+// velocities, with G and H of a velocity in the same lane.  Row, columns,
+// wall rules and the 20 cell constants are then wave-uniform (scalar registers
+// and scalar loads), every access to F is one contiguous line per wavefront,
+// and the work that depends only on the cell and the velocity (exp, Shakhov
+// factor, face coefficients, LU-SGS diagonal) is shared by G and H.
 //
-// A workgroup holds NW consecutive columns (a strip) of one velocity tile.
-// Wavefront w is at position q = s - w of the tile's sequence at step s
-// (three window-filling virtual rows, then rows 1..ny-1), so the forward
-// recursion's inputs from column i-1 were published one step earlier in LDS;
-// column i finalises position q-2 at the top of step s, using Delta*(i+1, .)
-// published by column i+1 one step earlier.
+// A workgroup holds NC consecutive columns (a strip) of one velocity tile on
+// NC/2 column wavefronts, and three more that do everything which is not
+// arithmetic on a cell:
+// - the loader copies F of the strip's columns and of the two to its right
+//   from memory straight into LDS, two steps ahead of their first use, and
+//   waits for each step's copies by count, so that a step never waits for a
+//   whole memory latency;
+// - the receiver stands for the column left of the strip: it delivers the
+//   face flux, Delta* and F that the first wavefront needs, either computed
+//   from the mesh's left boundary or received from the strip to the left, and
+//   finishes (backward pass, update) the last column of that strip, whose
+//   right neighbour's Delta* only this workgroup has;
+// - the sender passes the last column's flux and Delta* on.
+// The column wavefronts so have no role of their own in a seam, read only LDS
+// and scalars, and wait for no vector memory operation.
 //
-// The strips of a tile form a pipeline across workgroups.  The last column
-// of strip g hands the face flux and Delta* of each row (G and H) to the
-// first column of strip g+1 through a global seam buffer, then raises that
-// row's flag to the launch's epoch; the consumer checks the flag one step
-// before it loads the row.  The grid is strip-major, so a workgroup only
-// waits for one with a lower index, which was dispatched before it: the
-// waits cannot form a cycle.  The waits are bounded; a timeout sets *werr.
-// The last column of a strip is not updated here: its backward pass needs
-// Delta* of the next strip's first column, which k_seam applies after this
-// kernel (the first column stores it in dright).  Until then the column keeps
-// its old values, which are the ones its neighbours read.
+// Column wavefront w is at row r = s - w - 3 at step s (three rows before row
+// 1 fill the window); what wavefront w+1 needs from its left neighbour was
+// published in LDS one step earlier.  Within a wavefront the flux and Delta* of
+// the left column reach the right one in registers.  The left column finishes
+// row r-1 in step r, the right one, which needs Delta* of wavefront w+1, row
+// r-2.
+//
+// Two columns per wavefront because what a wavefront does once per step --
+// addresses, scalar loads, the barrier, publishing, the left face's
+// coefficients -- then serves two cells, and because the two cells' chains fill
+// each other's latency: 344 vector and 123 scalar instructions per two cells
+// (FP64 NND), against 215 and 152 per cell with one column per wavefront, which
+// also held the copies and both seam roles.  Rows r+1 and r+2, the right
+// column's earlier rows and earlier Delta* are read from LDS again instead of
+// being kept, and the step is cut into parts: that fits 130 registers without
+// a spill in the loop (one reload there waits for the stores before it and cost
+// 15% of the kernel).
+//
+// Measured, this kernel against one column per wavefront with a seam-update
+// kernel after it, both included: 128^2 cells x 64^2 velocities FP64 0.77 against
+// 1.04 ms, FP32 0.42 against 0.72; 256^2 x 96^2 FP64 7.4 against 8.8; 101^2 x 37^2
+// WENO3 0.34 against 0.53.  Bound by vector issue: two wavefronts per SIMD
+// (LDS allows no more in FP64) reach 57% of the issue slots, and the kernel
+// runs at 1.96 GHz.  Without its stores it is 12% faster, without its copies 5%.
+//
+// The strips of a tile form a pipeline across workgroups.  A message row is
+// four values per velocity in a slot of its own that holds a signalling NaN
+// (which no arithmetic returns) until it is written; the receiver polls the
+// values themselves and puts the NaN back for the next launch.  The grid is
+// strip-major, so a workgroup only waits for one with a lower index, which was
+// dispatched before it: the waits cannot form a cycle.  They are bounded; a
+// timeout sets *werr.
 // ------------------------------------------------------------------------
 constexpr int kSpinMax = 1 << 20;  // about a second of polling
 
@@ -1106,19 +1182,9 @@ __device__ __forceinline__ void stv(T *base, unsigned voff, T v) {
 }
 
 // Workgroup barrier that orders LDS accesses only.  __syncthreads() also
-// waits for every outstanding vector memory operation (its fence covers the
-// LDS writes of global_load_lds); here the staged copies are read only by the
-// wavefront that issued them, after its own wait, so they stay in flight.
+// waits for every outstanding vector memory operation; here copies and stores
+// stay in flight across it.
 __device__ __forceinline__ void barrier_lds() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// A wavefront-uniform value the compiler must treat as new at this point:
-// everything derived from it is recomputed (a few scalar instructions) rather
-// than hoisted out of the loop and kept in registers.
-template <typename X>
-__device__ __forceinline__ X fresh(X x) {
-  asm volatile("" : "+s"(x));
-  return x;
-}
 
 // 16 bytes per lane from global memory straight into LDS at dst + 16*lane
 // (gfx950 global_load_lds_dwordx4; dst is wavefront-uniform).  The builtin
@@ -1129,356 +1195,621 @@ __device__ __forceinline__ void lds_copy16(const void *src, void *dst) {
   __builtin_amdgcn_global_load_lds(src, dst, 16, 0, 0);
 #endif
 }
+// A wavefront-uniform value the compiler must treat as new at this point: an
+// address formed from it stays a scalar base plus a vector offset instead of
+// becoming a vector address kept across the loop.
+template <typename X>
+__device__ __forceinline__ X fresh(X x) {
+  asm volatile("" : "+s"(x));
+  return x;
+}
+// The same for a lane's value: what was derived from it before is not kept for
+// what is derived from it after.
+template <typename X>
+__device__ __forceinline__ X renew(X x) {
+  asm volatile("" : "+v"(x));
+  return x;
+}
+// wait until at most N vector memory operations are outstanding
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0F70);
+}
 
-// SL: slope rule of the fluxes (0 minmod for NND, 1 WENO3, 2 none: UP1).  At least
-// 4 wavefronts per SIMD (at most 128 VGPRs): with 80 KB of LDS per 8-column
-// workgroup two workgroups share a CU, which the register file must allow.
+// the value of a seam slot that has not been written: signalling NaNs
+template <typename T> struct Seam;
+template <> struct Seam<double> {
+  using U = unsigned long long;
+  static constexpr U kEmpty = 0x7FF4A5A57FF4A5A5ull;
+};
+template <> struct Seam<float> {
+  using U = unsigned;
+  static constexpr U kEmpty = 0x7FA5A5A5u;
+};
 template <typename T>
-using Vec2 = typename std::conditional<std::is_same<T, double>::value, double2, float2>::type;
+__device__ __forceinline__ bool seam_empty(T v) {
+  typename Seam<T>::U u;
+  __builtin_memcpy(&u, &v, sizeof(u));
+  return u == Seam<T>::kEmpty;
+}
 
-// LDS of one workgroup of the column-wavefront kernel (declared by each
-// kernel, so that its addresses are constants of that kernel)
-template <typename T, int NW>
+// LDS of one workgroup (declared by each kernel, so that its addresses are
+// constants of that kernel).  FP64: 144 KB for 16 columns (one workgroup per
+// CU), 80 KB for 8 (two); FP32 half of that.
+template <typename T, int NC>
 struct StripLds {
-  Vec2<T> XG[2][NW][64], XH[2][NW][64];  // (face flux, Delta*) of each column
-  // Values of the next row, copied from global memory straight into LDS
-  // (global_load_lds, 16 bytes per lane) one step ahead, so that no vector
-  // register holds them while they are in flight: per column, slots
-  // 0 F(i, r+2), 1 F(i-1, r), 2 F(i+1, r), 3 F(i+2, r), 4 x-boundary value,
-  // 5 y-boundary value, each the tile's 64 velocities of G then of H.
-  T STG[NW][6][128];
+  // F of the strip's column pairs and of the pair to its right: four row
+  // slots (row + 1) & 3 of 64 velocities of G then of H for each column of the
+  // pair.  A row is used in the two steps from its first use on, and is copied
+  // in the two steps before.
+  T ring[NC / 2 + 1][4][2][128];
+  // what a wavefront publishes for its neighbours in the next step, G then H
+  // of: 0 flux through the right column's right face, 1 Delta* and 2 F of the
+  // right column, 3 Delta* of the left column.  Entry 0 is the column left of
+  // the strip, entry 1 + w wavefront w; entry 0's values 3 hold the wall slot
+  // of the mesh's right boundary.
+  T x[2][NC / 2 + 1][4][128];
 };
 
-template <typename T, int NW, int SL>
-__device__ __forceinline__ void strip_body(StripLds<T, NW> &lds, const Dev &d, const T *__restrict__ cpar,
-                                           T *__restrict__ F, const T *__restrict__ slot, T *__restrict__ R,
-                                           int store_rhs, int ntiles, T *msg, T *dright, int *flag, int epoch,
-                                           int *werr, const int *__restrict__ oflags, int bid) {
-  using T2 = Vec2<T>;
-  constexpr unsigned ES = sizeof(T);
-  auto &XG = lds.XG;
-  auto &XH = lds.XH;
-  auto &STG = lds.STG;
-  constexpr int kPer = 16 / sizeof(T);  // velocities per lane and copy
-  constexpr int kLanes = 64 / kPer;     // lanes per component
-  const int nx = d.nx, ny = d.ny, ncol = nx - 1, nrow = ny - 1, nv = d.nv;
-  const int ngroups = (ncol + NW - 1) / NW;
-  const int LT = nrow + 4;                 // positions: virtual rows -3..0, rows 1..ny-1
-  const int nsteps = (NW - 1) + LT + 2;
-  const int w0 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int g0w = bid / ntiles, tile = bid - g0w * ntiles;
-  const int i0 = g0w * NW + w0 + 1;  // mesh column of this wavefront
-  // Strips early in the pipeline feed all later ones: their wavefronts get
-  // the higher issue priority on a CU they share with later strips.
-  if (g0w == 0) __builtin_amdgcn_s_setprio(3);
-  else if (g0w == 1) __builtin_amdgcn_s_setprio(2);
-  else if (g0w == 2) __builtin_amdgcn_s_setprio(1);
-  if (i0 > ncol) {  // past the last column: keep the workgroup's barriers
-    for (int s = 0; s < nsteps; s++) barrier_lds();
-    return;
+// Flux through one face from the four cells around it; asp, asn: max(a, 0),
+// min(a, 0).  SL: slope rule (0 minmod for NND, 1 WENO3, 2 none: UP1).
+// Fused multiply-adds are written out here and in strip_body, and the compiler
+// forms none of its own: every instantiation (widths, batched) gives the same
+// bits.
+template <int SL, typename T>
+__device__ __forceinline__ T face_flux(T asp, T asn, T fm2, T fm1, T f0, T fp1) {
+#pragma clang fp contract(off)
+  if constexpr (SL == 2) {
+    return fma(asp, fm1, asn * f0);
+  } else {
+    T sl, sr;
+    slopes<SL>(f0 - fm1, fm1 - fm2, fp1 - f0, sl, sr);
+    return fma(asp, fma(T(0.5), sl, fm1), asn * fma(T(-0.5), sr, f0));
   }
-  T vx, vy;
-  {
-    const int vv = min(tile * 64 + (int)(threadIdx.x & 63), nv - 1);
-    vx = T(d.vi[vv % d.nvi]);
-    vy = T(d.vj[vv / d.nvi]);
-  }
-  constexpr T hs = SL == 2 ? T(0) : T(0.5);  // slope factor (0: first-order upwind)
-  // (override words are wavefront-uniform: scalar registers also where the
-  // table's address was itself read from memory, as in the batched kernel)
-  const int cfl0 = __builtin_amdgcn_readfirstlane(oflags[ny + 2 + i0]);  // j-face overrides of column i
-  // Roles, re-derived every step: the first column of strip g > 0 reads the
-  // seam message of strip g-1 (consumer); the last column of a strip that is
-  // not the last writes it (producer) and is updated by k_seam; xlo / xhi:
-  // the mesh's first / last column; xrule: an overridden i-face within reach
-  // of the right face.
-  // byte strides: one cell's velocities, one row of cells, one plane
-  const long long cb = (long long)nv * ES, rb = (long long)d.NI * cb, pb = (long long)d.ncell * cb;
-  char *const Fb0 = reinterpret_cast<char *>(F);
-  char *const Rb0 = reinterpret_cast<char *>(R);
-  const char *const Sb0 = reinterpret_cast<const char *>(slot);
-  // Per-lane offsets are re-derived where they are used, from a copy of the
-  // thread index the compiler cannot see through: keeping them live across
-  // the loop costs more vector registers than the few instructions that
-  // recompute them.
-  // Staged copies: lane l < kLanes copies velocities tile*64 + l*kPer .. +kPer-1
-  // of G, the next kLanes lanes the same of H (one plane, or one slot row,
-  // further).  The last copy of a partial tile is moved back into the
-  // velocity range (those lanes' velocities are not used).
-  auto lane_of = [&]() {
-    unsigned t = threadIdx.x;
-    asm volatile("" : "+v"(t));
-    return (int)(t & 63);
-  };
-  // per-lane byte offsets of a copy: into F (G or H plane) and into the wall slots
-  auto copy_offsets = [&](int l, long long &stF, long long &stS) {
-    const int comp = l / kLanes;
-    const long long pvb = (long long)min(tile * 64 + (l % kLanes) * kPer, nv - kPer) * ES;
-    stF = (comp ? pb : 0ll) + pvb;
-    stS = (comp ? cb : 0ll) + pvb;
-  };
-  auto copy = [&](int w, int k, const char *base, long long st, int l) {
-    if (l < 2 * kLanes) lds_copy16(base + st, &STG[w][k][0]);
-  };
-  T mfg = T(0), mdg = T(0), mfh = T(0), mdh = T(0);  // seam message of row r+1
-  int mflag = 0;                                     // flag of row r+2
-  long long oc = -2 * rb + (long long)(i0 + 1) * cb;  // byte offset of cell (i, r), r = -3
-  constexpr long long kRec = kNW * (long long)sizeof(T);        // bytes of one cell's constants
-  // 32-bit offsets and indices where they fit, to keep scalar registers free
-  int ocp = (-4 * ncol + (i0 - 1)) * (int)kRec;  // cpar byte offset of cell (i, r); used for r >= 1
-  const int ccstep = ncol * (int)kRec;
-  const unsigned sbc = ((unsigned)(g0w > 0 ? g0w - 1 : 0) * ntiles + tile) * (unsigned)nrow;  // seam rows read (row r at sbc + r - 1)
-  const unsigned sbp = ((unsigned)g0w * ntiles + tile) * (unsigned)nrow;                    // seam rows written
-  {
-    const int l = (int)(threadIdx.x & 63);
-    long long stF, stS;
-    copy_offsets(l, stF, stS);
-    copy(w0, 0, Fb0 + oc + 2 * rb, stF, l);  // F(i, -1), the first window value
-  }
-  T g0 = T(0), g1 = T(0), g2 = T(0), g3 = T(0), g4 = T(0);  // G(i, r-2..r+2)
-  T h0 = T(0), h1 = T(0), h2 = T(0), h3 = T(0), h4 = T(0);
-  T gfly = T(0), hfly = T(0);  // flux through the bottom face of the next row
-  T gd_n = T(0), hd_n = T(0), bx_n = T(0), by_n = T(0), gd_o = T(0), hd_o = T(0), bx_o = T(0), by_o = T(0);
-  int flag_due = 0;  // a seam row written in the previous step waits for its flag
-  // The cell constants of the next row are touched one step ahead (one
-  // dword from each 64-byte line of the 160-byte record), so that the
-  // scalar loads of the row's 20 constants hit the scalar cache.
-  int pf0 = 0, pf1 = 0, pf2 = 0, pf3 = 0;
-  // Steps s < w0 and s >= w0 + LT + 2 only keep the workgroup's barriers.
-  // The active steps q = s - w0 = 0 .. LT+1 run five at a time, each given
-  // the five-row windows in rotated order: moving a window down one row
-  // then renames registers instead of copying four values.
-  auto step = [&](int q, T &gA, T &gB, T &gC, T &gD, T &gE, T &hA, T &hB, T &hC, T &hD, T &hE)
-                  __attribute__((always_inline)) {
-    T &g0 = gB, &g1 = gC, &g2 = gD, &g3 = gE, &g4 = gA;  // G(i, r-2..r+2); gA takes the new row
-    T &h0 = hB, &h1 = hC, &h2 = hD, &h3 = hE, &h4 = hA;
-    __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): the previous step's copies, loads and stores are complete
-    // per-wavefront values, re-derived every step (see fresh())
-    const int w = fresh(w0), i = fresh(i0), g = fresh(g0w), cfl = fresh(cfl0);
-    char *const Fb = fresh(Fb0);
-    char *const Rb = fresh(Rb0);
-    const char *const Sb = fresh(Sb0);
-    const bool consumer = w == 0 && g > 0;
-    const bool producer = w == NW - 1 && g < ngroups - 1;
-    const bool xlo = i == 1, xhi = i == ncol;
-    const bool xrule = i == 1 || i >= ncol - 1;
-    const int lane = lane_of();
-    const unsigned voff = (unsigned)min(tile * 64 + lane, nv - 1) * ES, loff = (unsigned)lane * ES;
-    const bool act = tile * 64 + lane < nv;
-    const int s = q + w, r = q - 3;
-    const int buf = s & 1, pbuf = buf ^ 1;
-    if (producer && flag_due) {  // its message stores are complete: publish the row
-      if (lane == 0) st_agent(flag + sbp + (r - 2), epoch);
-      flag_due = 0;
-    }
-    // backward pass + update of row r-2 (src/GKUA_Residual.f90:64-109).  Its
-    // inputs are complete at the top of the step (Delta* of column i+1 was
-    // published in the previous step), and storing early gives the stores a
-    // whole step to complete before the next step's wait.  No wavefront reads
-    // F(i, r-2) after step s-2.
-    const int rf = r - 2;
-    if (rf >= 1 && rf <= nrow && !producer) {
-      T gr = T(0), hr = T(0);
-      if (i < ncol) {
-        gr = XG[pbuf][w + 1][lane].y;
-        hr = XH[pbuf][w + 1][lane].y;
-      }
-      const bool last = rf == nrow;  // Delta*(i, ny) = 0
-      const T gu = gd_o + (bx_o * gr + by_o * (last ? T(0) : gd_n));
-      const T hu = hd_o + (bx_o * hr + by_o * (last ? T(0) : hd_n));
-      T fg = g0 + gu, fh = h0 + hu;
-      if ((double)fg < kClamp) fg = T(kClamp);
-      if ((double)fh < kClamp) fh = T(kClamp);
-      if (act) {
-        stv(reinterpret_cast<T *>(Fb + oc - 2 * rb), voff, fg);
-        stv(reinterpret_cast<T *>(Fb + oc - 2 * rb + pb), voff, fh);
-      }
-    }
-    asm volatile("" ::"s"(pf0), "s"(pf1), "s"(pf2), "s"(pf3));  // the previous step's touches
-    if (r + 1 >= 1 && r + 1 <= nrow) {
-      const int *pc = reinterpret_cast<const int *>(reinterpret_cast<const char *>(cpar) + ocp + ccstep);
-      pf0 = pc[0];
-      pf1 = pc[16];
-      pf2 = pc[kRec > 128 ? 32 : 0];
-      pf3 = pc[kRec / 4 - 1];
-    }
-    const bool real = r >= 1 && r <= nrow;
-    const int rfl = real ? __builtin_amdgcn_readfirstlane(oflags[r]) : 0;  // i-face overrides of row r
-    // the values staged in the previous step for this row
-    // (slots that were not copied for this row hold older values, which are
-    // read here but never used)
-    g4 = STG[w][0][lane];
-    h4 = STG[w][0][64 + lane];
-    const T cgm1 = STG[w][1][lane], chm1 = STG[w][1][64 + lane];
-    const T cgp1 = STG[w][2][lane], chp1 = STG[w][2][64 + lane];
-    const T cgp2 = STG[w][3][lane], chp2 = STG[w][3][64 + lane];
-    const T cgxs = STG[w][4][lane], chxs = STG[w][4][64 + lane];
-    const T cgys = STG[w][5][lane], chys = STG[w][5][64 + lane];
-    const T cmfg = mfg, cmdg = mdg, cmfh = mfh, cmdh = mdh;
-    // row r: equilibrium, fluxes, RHS, forward recursion (src/GKUA_Residual.f90:39-57,117-469)
-    T gd_new = T(0), hd_new = T(0), bx_new = T(0), by_new = T(0);
-    T feqg = T(0), feqh = T(0), axl = T(0), axr = T(0), ayb = T(0), ayt = T(0), ra = T(0);
-    T vinv = T(0), cf = T(0), vol = T(0);
-    if (real) {
-      const T *cc = reinterpret_cast<const T *>(reinterpret_cast<const char *>(cpar) + ocp);
-      {  // Shakhov equilibrium of cell (i,r) (Get_Feq, src/GKUA_Residual.f90:420-469)
-        const T viu = vx - T(cc[4]), vjv = vy - T(cc[5]);
-        const T vij2 = (viu * viu + vjv * vjv) * T(cc[2]);
-        const T fvx = T(cc[1]) * (viu * T(cc[6]) + vjv * T(cc[7]));
-        const T gd = T(cc[0]) * wexp(-vij2);
-        const T b = fvx * (T(2) * vij2 - T(2));
-        // G: gd (1 + phi (2c^2 - 4)); H: (T gd / 2)(1 + phi (2c^2 - 2))
-        feqg = gd * ((T(1) - T(2) * fvx) + b);
-        feqh = ((T(cc[3]) * gd) * T(0.5)) * (T(1) + b);
-      }
-      const T *cc2 = cc;
-      axl = vx * T(cc2[12]) + vy * T(cc2[13]);
-      axr = vx * T(cc2[14]) + vy * T(cc2[15]);
-      ayb = vx * T(cc2[16]) + vy * T(cc2[17]);
-      ayt = vx * T(cc2[18]) + vy * T(cc2[19]);
-      const T alfa = T(cc2[11]) + (posp(axr) - negp(axl) + posp(ayt) - negp(ayb));
-      ra = rcp_pos(alfa);
-      vinv = T(cc2[9]);
-      cf = T(cc2[8]);
-      vol = T(cc2[10]);
-    }
-    // all staged values are in registers before the copies of the next row overwrite them
-    __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0)
-    // copies of the next row rn (one step ahead)
-    const int rn = r + 1;
-    long long stF, stS;
-    copy_offsets(lane, stF, stS);
-    auto slotrow = [&](int face, int pos) { return Sb + (((long long)(face - 1) * d.L + pos) * 2) * cb; };
-    if (rn <= nrow) copy(w, 0, Fb + oc + 3 * rb, stF, lane);
-    if (rn >= 1 && rn <= nrow) {
-      copy(w, 1, Fb + oc + rb - cb, stF, lane);
-      copy(w, 2, Fb + oc + rb + cb, stF, lane);
-      copy(w, 3, Fb + oc + rb + 2 * cb, stF, lane);
-      const int rfn = __builtin_amdgcn_readfirstlane(oflags[rn]);
-      if (xlo) {
-        if (rfn & 1) copy(w, 4, slotrow(1, rn + 1), stS, lane);
-        else copy(w, 4, Fb + oc + rb - 2 * cb, stF, lane);  // ghost cell (-1, rn)
-      } else if (xhi && (rfn & 2)) {
-        copy(w, 4, slotrow(3, rn + 1), stS, lane);
-      }
-      if (rn == 1 && (cfl & 1)) copy(w, 5, slotrow(2, i + 1), stS, lane);
-      else if (rn == nrow && (cfl & 2)) copy(w, 5, slotrow(4, i + 1), stS, lane);
-      if (consumer) {
-        // the flag of row rn was loaded one step ago; wait for it if the
-        // producing strip is behind, then load the row's message
-        const unsigned sr = sbc + (rn - 1);
-        int fv = __builtin_amdgcn_readfirstlane(mflag);
-        if (fv != epoch && __builtin_amdgcn_readfirstlane(ld_agent(werr)) == 0) {
-          int it = 0;
-          do {
-            __builtin_amdgcn_s_sleep(2);
-            fv = __builtin_amdgcn_readfirstlane(ld_agent(flag + sr));
-          } while (fv != epoch && ++it < kSpinMax);
-          if (fv != epoch && lane == 0) st_agent(werr, 1);
-        }
-        const char *m = reinterpret_cast<const char *>(msg + (size_t)sr * 256) + loff;
-        mfg = ld_agent(reinterpret_cast<const T *>(m));
-        mdg = ld_agent(reinterpret_cast<const T *>(m + 64 * ES));
-        mfh = ld_agent(reinterpret_cast<const T *>(m + 128 * ES));
-        mdh = ld_agent(reinterpret_cast<const T *>(m + 192 * ES));
-      }
-    }
-    if (consumer && rn + 1 >= 1 && rn + 1 <= nrow) mflag = ld_agent(flag + sbc + rn);
-    if (real) {
-      const bool first = r == 1;
-      const bool yrule = first || r >= nrow - 1;  // an overridden j-face within reach of the top face
-      // left face: boundary flux, the seam message or column i-1's value
-      T gfl, gdl, hfl, hdl;
-      if (xlo) {
-        gfl = wflux1<SL>(rfl, axl, cgxs, cgm1, g2, cgp1, cgxs, hs);
-        hfl = wflux1<SL>(rfl, axl, chxs, chm1, h2, chp1, chxs, hs);
-        gdl = T(0);
-        hdl = T(0);
-      } else if (w == 0) {
-        gfl = cmfg; gdl = cmdg; hfl = cmfh; hdl = cmdh;
-      } else {
-        const T2 lg = XG[pbuf][w - 1][lane], lh = XH[pbuf][w - 1][lane];
-        gfl = lg.x; gdl = lg.y; hfl = lh.x; hdl = lh.y;
-      }
-      T gfr, hfr, gft, hft, gfb, hfb;
-      if (xrule) {
-        gfr = wflux<SL>(i + 1, nx, rfl, axr, cgm1, g2, cgp1, cgp2, cgxs, hs);
-        hfr = wflux<SL>(i + 1, nx, rfl, axr, chm1, h2, chp1, chp2, chxs, hs);
-      } else {
-        gfr = iflux<SL>(axr, cgm1, g2, cgp1, cgp2, hs);
-        hfr = iflux<SL>(axr, chm1, h2, chp1, chp2, hs);
-      }
-      if (yrule) {
-        gft = wflux<SL>(r + 1, ny, cfl, ayt, g1, g2, g3, g4, cgys, hs);
-        hft = wflux<SL>(r + 1, ny, cfl, ayt, h1, h2, h3, h4, chys, hs);
-      } else {
-        gft = iflux<SL>(ayt, g1, g2, g3, g4, hs);
-        hft = iflux<SL>(ayt, h1, h2, h3, h4, hs);
-      }
-      if (first) {
-        gfb = wflux1<SL>(cfl, ayb, g0, g1, g2, g3, cgys, hs);
-        hfb = wflux1<SL>(cfl, ayb, h0, h1, h2, h3, chys, hs);
-      } else {
-        gfb = gfly;
-        hfb = hfly;
-      }
-      gfly = gft;
-      hfly = hft;
-      const T grr = -(((gfr - gfl) + gft) - gfb) * vinv + cf * (feqg - g2);
-      const T hrr = -(((hfr - hfl) + hft) - hfb) * vinv + cf * (feqh - h2);
-      if (store_rhs && act) {
-        stv(reinterpret_cast<T *>(Rb + oc), voff, grr);
-        stv(reinterpret_cast<T *>(Rb + oc + pb), voff, hrr);
-      }
-      gd_new = (vol * grr + posp(axl) * gdl + posp(ayb) * (first ? T(0) : gd_n)) * ra;
-      hd_new = (vol * hrr + posp(axl) * hdl + posp(ayb) * (first ? T(0) : hd_n)) * ra;
-      XG[buf][w][lane] = T2{gfr, gd_new};
-      XH[buf][w][lane] = T2{hfr, hd_new};
-      bx_new = -negp(axr) * ra;
-      by_new = -negp(ayt) * ra;
-      if (producer) {
-        char *m = reinterpret_cast<char *>(msg + (size_t)(sbp + (r - 1)) * 256) + loff;
-        st_agent(reinterpret_cast<T *>(m), gfr);
-        st_agent(reinterpret_cast<T *>(m + 64 * ES), gd_new);
-        st_agent(reinterpret_cast<T *>(m + 128 * ES), hfr);
-        st_agent(reinterpret_cast<T *>(m + 192 * ES), hd_new);
-        flag_due = 1;
-      }
-      if (consumer) {
-        T *m = dright + (size_t)(sbc + (r - 1)) * 128;
-        stv(m, loff, gd_new);
-        stv(m + 64, loff, hd_new);
-      }
-    }
-    gd_o = gd_n; hd_o = hd_n; bx_o = bx_n; by_o = by_n;
-    gd_n = gd_new; hd_n = hd_new; bx_n = bx_new; by_n = by_new;
-    oc += rb;
-    ocp += ccstep;
-    barrier_lds();
-  };
-  for (int s = 0; s < w0; s++) barrier_lds();
-  for (int q = 0; q < LT + 2; q += 5) {
-    step(q, g0, g1, g2, g3, g4, h0, h1, h2, h3, h4);
-    if (q + 1 < LT + 2) step(q + 1, g1, g2, g3, g4, g0, h1, h2, h3, h4, h0);
-    if (q + 2 < LT + 2) step(q + 2, g2, g3, g4, g0, g1, h2, h3, h4, h0, h1);
-    if (q + 3 < LT + 2) step(q + 3, g3, g4, g0, g1, g2, h3, h4, h0, h1, h2);
-    if (q + 4 < LT + 2) step(q + 4, g4, g0, g1, g2, g3, h4, h0, h1, h2, h3);
-  }
-  for (int s = w0 + LT + 2; s < nsteps; s++) barrier_lds();
-  if (w0 == NW - 1 && g0w < ngroups - 1 && flag_due) {
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    if ((threadIdx.x & 63) == 0) st_agent(flag + sbp + (nrow - 1), epoch);
+}
+// The same under a wall rule (wave-uniform): 1, 2 the face is next to an
+// overridden one, whose side's limiter is dropped; 4 it is overridden, the flux
+// is a * sv (src/GKUA_Residual.f90:200-262).
+template <int SL, typename T>
+__device__ __forceinline__ T face_flux_wall(int rule, T asp, T asn, T fm2, T fm1, T f0, T fp1, T sv) {
+#pragma clang fp contract(off)
+  // (none of the plain flux's intermediate values is kept for this branch)
+  fm1 = renew(fm1);
+  f0 = renew(f0);
+  if (rule & 4) return (asp + asn) * sv;
+  if constexpr (SL == 2) {
+    return fma(asp, fm1, asn * f0);
+  } else {
+    const T d0 = f0 - fm1;
+    T sl, sr;
+    slopes<SL>(d0, fm1 - fm2, fp1 - f0, sl, sr);
+    if (rule & 1) sl = d0;
+    if (rule & 2) sr = d0;
+    return fma(asp, fma(T(0.5), sl, fm1), asn * fma(T(-0.5), sr, f0));
   }
 }
 
-template <typename T, int NW, int SL>
-__global__ void __launch_bounds__(64 * NW, 4) k_strip(Dev d, const T *__restrict__ cpar, T *__restrict__ F,
-                                                 const T *__restrict__ slot, T *__restrict__ R, int store_rhs,
-                                                 int ntiles, T *msg, T *dright, int *flag, int epoch, int *werr,
-                                                 const int *__restrict__ oflags) {
-  __shared__ StripLds<T, NW> lds;
-  strip_body<T, NW, SL>(lds, d, cpar, F, slot, R, store_rhs, ntiles, msg, dright, flag, epoch, werr, oflags,
-                        (int)blockIdx.x);
+template <typename T, int NC, int SL>
+__device__ __forceinline__ void strip_body(StripLds<T, NC> &lds, const Dev &d, const T *__restrict__ cpar_,
+                                           T *__restrict__ F, const T *__restrict__ slot, T *__restrict__ R,
+                                           int store_rhs, int ntiles, T *msg, int *werr,
+                                           const int *__restrict__ oflags_, int bid) {
+#pragma clang fp contract(off)
+  constexpr int NP = NC / 2;
+  constexpr int ES = sizeof(T);
+  constexpr int kRec = kNW * ES;     // bytes of one cell's constants
+  constexpr int kX = 4 * 128;        // elements of one entry of lds.x
+  constexpr int kRing = 4 * 2 * 128; // elements of one pair of lds.ring
+  using U = typename Seam<T>::U;
+  // memory no launch writes while it reads it, at wave-uniform addresses:
+  // read through the scalar cache
+  using CT = const __attribute__((address_space(4))) T *;
+  using CI = const __attribute__((address_space(4))) int *;
+  using GB = __attribute__((address_space(1))) char *;
+  using GT = __attribute__((address_space(1))) T *;
+  const CT cpar = (CT)cpar_;
+  const CI oflags = (CI)oflags_;
+  T *const ring = &lds.ring[0][0][0][0], *const X = &lds.x[0][0][0][0];
+  const int nx = d.nx, ny = d.ny, ncol = nx - 1, nrow = ny - 1, nv = d.nv;
+  const int ngroups = (ncol + NC - 1) / NC;
+  const int nsteps = NP + nrow + 5;
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63;
+  const int g = bid / ntiles, tile = bid - g * ntiles;
+  const int i0 = g * NC + 1;  // the strip's first mesh column
+  // byte strides: one cell's velocities, one row of cells, one plane
+  const long long cb = (long long)nv * ES, rb = (long long)d.NI * cb, pb = (long long)d.ncell * cb;
+  char *const Fb = reinterpret_cast<char *>(F);
+  const char *const Sb = reinterpret_cast<const char *>(slot);
+  const unsigned voff = (unsigned)(tile * 64 + lane) * ES;
+  const bool act = tile * 64 + lane < nv;
+  const size_t seam_row = (size_t)g * ntiles + tile;  // seam rows written: seam_row * nrow + r - 1
+  auto slotrow = [&](int face, int pos) { return Sb + (((long long)(face - 1) * d.L + pos) * 2) * cb; };
+
+  if (wv == NP) {
+    // ---- loader: rows s + 1 - w of pair w at step s, first used at step s + 2
+    constexpr int kPer = 16 / ES;                  // velocities per lane and copy
+    constexpr int kCopies = (NP + 1) * (ES == 8 ? 2 : 1);  // per step (FP32: both columns at once)
+    // lane l copies velocities tile*64 + kPer*(l % (64/kPer)) .. of G, H (and of
+    // the pair's second column in FP32).  A copy that straddles the end of the
+    // velocities reads on into the next cell (those values are not used).
+    const int comp = (lane / (64 / kPer)) & 1, second = ES == 8 ? 0 : lane >> 5;
+    int v0 = tile * 64 + (lane % (64 / kPer)) * kPer;
+    if (v0 >= nv) v0 = tile * 64;
+    const long long stF = (comp ? pb : 0ll) + (long long)v0 * ES, stS = (comp ? cb : 0ll) + (long long)v0 * ES;
+    // lane addresses of row max(s + 1 - w, -1) (at most nrow + 2) of each column
+    // (FP32: of the lane's column of each pair), advanced by a row per step.
+    // Beyond an overridden boundary face lies no cell that is used: the face's
+    // wall slot takes the place of row -1 or nrow + 2.
+    constexpr int kAt = ES == 8 ? 2 : 1;
+    const char *at[NP + 1][kAt];
+    const char *const f0 = Fb + ((long long)(i0 + 1) * cb + stF);  // row -1 of the strip's first column
+    const char *const s2 = slotrow(2, i0 + 1) + stS, *const s4 = slotrow(4, i0 + 1) + stS;
+    const int cmax = ncol + 2 - i0, cin = ncol - i0;  // last column there is, last one that is not a ghost
+    unsigned lo = 0, hi = 0;                          // columns whose bottom / top boundary face is overridden
+    for (int c = 0; c <= min(NC + 1, cin); c++) {
+      const int o = oflags[ny + 2 + i0 + c];
+      lo |= (unsigned)(o & 1) << c;
+      hi |= (unsigned)((o >> 1) & 1) << c;
+    }
+    auto column = [&](int w, int k) { return ES == 8 ? 2 * w + k : 2 * w + second; };
+#pragma unroll
+    for (int w = 0; w <= NP; w++)
+#pragma unroll
+      for (int k = 0; k < kAt; k++) {
+        const int c = column(w, k);
+        at[w][k] = (lo >> c) & 1 ? s2 + c * 2 * cb : f0 + min(c, cmax) * cb;
+      }
+    auto issue = [&](int s) __attribute__((always_inline)) {
+#pragma unroll
+      for (int w = 0; w <= NP; w++) {
+        T *dst = ring + w * kRing + ((s + 2 - w) & 3) * 256;
+#pragma unroll
+        for (int k = 0; k < kAt; k++) lds_copy16(at[w][k], dst + k * 128);
+        const int row = s + 1 - w;
+        if ((unsigned)row <= (unsigned)nrow) {
+#pragma unroll
+          for (int k = 0; k < kAt; k++) at[w][k] += rb;
+        } else if (row == -1) {
+#pragma unroll
+          for (int k = 0; k < kAt; k++) at[w][k] = f0 + (rb + min(column(w, k), cmax) * cb);
+        } else if (row == nrow + 1) {
+#pragma unroll
+          for (int k = 0; k < kAt; k++) at[w][k] = (hi >> column(w, k)) & 1 ? s4 + column(w, k) * 2 * cb : at[w][k] + rb;
+        }
+      }
+    };
+    issue(-2);
+    issue(-1);
+    wait_vm<kCopies>();
+    barrier_lds();
+    for (int s = 0; s < nsteps; s++) {
+      if (s <= nrow + 1 + NP) {
+        issue(s);
+        wait_vm<kCopies>();  // the previous step's copies
+      } else {
+        wait_vm<0>();
+      }
+      barrier_lds();
+    }
+    wait_vm<0>();
+    return;
+  }
+
+  T vx, vy;
+  {
+    const int vv = min(tile * 64 + lane, nv - 1);
+    vx = T(d.vi[vv % d.nvi]);
+    vy = T(d.vj[vv / d.nvi]);
+  }
+
+  if (wv == NP + 1) {
+    // ---- receiver: delivers row s - 2 of the column left of the strip
+    __builtin_amdgcn_s_setprio(3);
+    barrier_lds();
+    const bool left = g == 0;
+    const bool wallr = g == ngroups - 1;     // the right boundary's slots are this strip's to deliver
+    const int wl = (ncol - i0) >> 1;         // the wavefront of the mesh's last column (wallr)
+    const U *const mrow = reinterpret_cast<const U *>(msg) + (left ? 0 : (seam_row - ntiles) * (size_t)nrow * 256) + lane;
+    char *const Fc = Fb + (long long)i0 * cb;  // column i0 - 1, row -1
+    T m0 = T(0), m1 = T(0), m2 = T(0), m3 = T(0), fg = T(0), fh = T(0);  // row s - 2
+    T dg1 = T(0), dh1 = T(0), dg2 = T(0), dh2 = T(0);                    // Delta* of rows s - 3, s - 4
+    T fg1 = T(0), fh1 = T(0), fg2 = T(0), fh2 = T(0);                    // F of rows s - 3, s - 4
+    T wg = T(0), wh = T(0);                                              // right wall slot of row s - 2 - wl
+    for (int s = 0; s < nsteps; s++) {
+      if (act) {
+        T *const xw = X + (s & 1) * (NP + 1) * kX + lane;
+        const T *const xr = X + ((s & 1) ^ 1) * (NP + 1) * kX + lane;
+        const int row = s - 2, rn = row + 1, f = row - 2;
+        T n0 = T(0), n1 = T(0), n2 = T(0), n3 = T(0), nfg = T(0), nfh = T(0), nwg = T(0), nwh = T(0);
+        // the next row's values
+        if (rn >= 1 && rn <= nrow) {
+          const char *fr = Fc + (long long)(rn + 1) * rb;
+          nfg = ldv(reinterpret_cast<const T *>(fr), voff);
+          nfh = ldv(reinterpret_cast<const T *>(fr + pb), voff);
+          if (left) {
+            const bool o = oflags[rn] & 1;
+            const char *sr = o ? slotrow(1, rn + 1) : fr - cb;  // the wall slot, or ghost cell (-1, rn)
+            n0 = ldv(reinterpret_cast<const T *>(sr), voff);
+            n1 = ldv(reinterpret_cast<const T *>(sr + (o ? cb : pb)), voff);
+          } else {
+            const T *m = reinterpret_cast<const T *>(mrow + (size_t)(rn - 1) * 256);
+            n0 = ld_agent(m);
+            n1 = ld_agent(m + 64);
+            n2 = ld_agent(m + 128);
+            n3 = ld_agent(m + 192);
+          }
+        }
+        if (wallr) {
+          const int rw = rn - wl;
+          if (rw >= 1 && rw <= nrow && (oflags[rw] & 2)) {
+            const char *sr = slotrow(3, rw + 1);
+            nwg = ldv(reinterpret_cast<const T *>(sr), voff);
+            nwh = ldv(reinterpret_cast<const T *>(sr + cb), voff);
+          }
+          xw[3 * 128] = wg;
+          xw[3 * 128 + 64] = wh;
+        }
+        if (row >= 1 && row <= nrow) {
+          if (left) {
+            const CT cc = cpar + ((size_t)(row - 1) * ncol) * kNW;
+            const int rfl = oflags[row];
+            const T axl = fma(vx, T(cc[12]), vy * T(cc[13]));
+            const T *rr = ring + ((row + 1) & 3) * 256 + lane;  // F of columns 1 and 2
+            const int rule = rfl & 1 ? 4 : 0;
+            const T xg = face_flux_wall<SL>(rule, posp(axl), negp(axl), m0, fg, rr[0], rr[128], m0);
+            const T xh = face_flux_wall<SL>(rule, posp(axl), negp(axl), m1, fh, rr[64], rr[192], m1);
+            m0 = xg; m2 = xh; m1 = T(0); m3 = T(0);
+          } else {
+            const T *m = reinterpret_cast<const T *>(mrow + (size_t)(row - 1) * 256);
+            if (__any(seam_empty(m0) || seam_empty(m1) || seam_empty(m2) || seam_empty(m3)) &&
+                __builtin_amdgcn_readfirstlane(ld_agent(werr)) == 0) {
+              int it = 0;
+              bool more;
+              do {
+                m0 = ld_agent(m);
+                m1 = ld_agent(m + 64);
+                m2 = ld_agent(m + 128);
+                m3 = ld_agent(m + 192);
+                more = __any(seam_empty(m0) || seam_empty(m1) || seam_empty(m2) || seam_empty(m3));
+              } while (more && ++it < kSpinMax);
+              if (more && lane == 0) st_agent(werr, 1);
+            }
+            U *mw = const_cast<U *>(mrow) + (size_t)(row - 1) * 256;
+            st_agent(mw, Seam<T>::kEmpty);
+            st_agent(mw + 64, Seam<T>::kEmpty);
+            st_agent(mw + 128, Seam<T>::kEmpty);
+            st_agent(mw + 192, Seam<T>::kEmpty);
+          }
+          xw[0] = m0;
+          xw[64] = m2;
+          xw[128] = m1;
+          xw[192] = m3;
+          xw[256] = fg;
+          xw[320] = fh;
+        }
+        if (!left && f >= 1 && f <= nrow) {
+          // backward pass and update of row f (src/GKUA_Residual.f90:64-109):
+          // Delta*(i0, f) was published by wavefront 0 in the previous step
+          const T gr = xr[kX + 3 * 128], hr = xr[kX + 3 * 128 + 64];
+          const CT cc = cpar + ((size_t)(f - 1) * ncol + (i0 - 2)) * kNW;
+          const T axl = fma(vx, T(cc[12]), vy * T(cc[13])), axr = fma(vx, T(cc[14]), vy * T(cc[15]));
+          const T ayb = fma(vx, T(cc[16]), vy * T(cc[17])), ayt = fma(vx, T(cc[18]), vy * T(cc[19]));
+          const T alfa = T(cc[11]) + (posp(axr) - negp(axl) + posp(ayt) - negp(ayb));
+          const T ra = rcp_pos(alfa);
+          const T bx = -negp(axr) * ra, by = -negp(ayt) * ra;
+          T ug = fg2 + (dg2 + fma(bx, gr, by * (f < nrow ? dg1 : T(0))));
+          T uh = fh2 + (dh2 + fma(bx, hr, by * (f < nrow ? dh1 : T(0))));
+          if ((double)ug < kClamp) ug = T(kClamp);
+          if ((double)uh < kClamp) uh = T(kClamp);
+          char *fw = Fc + (long long)(f + 1) * rb;
+          stv(reinterpret_cast<T *>(fw), voff, ug);
+          stv(reinterpret_cast<T *>(fw + pb), voff, uh);
+        }
+        dg2 = dg1; dh2 = dh1; dg1 = m1; dh1 = m3;
+        fg2 = fg1; fh2 = fh1; fg1 = fg; fh1 = fh;
+        m0 = n0; m1 = n1; m2 = n2; m3 = n3; fg = nfg; fh = nfh; wg = nwg; wh = nwh;
+      }
+      barrier_lds();
+    }
+    return;
+  }
+
+  if (wv == NP + 2) {
+    // ---- sender: passes on what the last wavefront published in the previous
+    // step, and touches the cell constants of the step after the next one (one
+    // dword of each 64-byte line), so that the column wavefronts' scalar loads
+    // hit the scalar cache
+    barrier_lds();
+    constexpr int kLines = (2 * kRec + 63) / 64 + 1;  // lines two records can reach into
+    for (int s = 0; s < nsteps; s++) {
+      int t[NP][kLines];
+#pragma unroll
+      for (int w = 0; w < NP; w++) {
+        const int r = min(max(s - w - 1, 1), nrow), iA = min(i0 + 2 * w, ncol - 1);
+        const CI q = (CI)(cpar + ((r - 1) * ncol + (iA - 1)) * kNW);
+        constexpr int last = 2 * kRec / 4 - 1;
+#pragma unroll
+        for (int k = 0; k < kLines; k++) t[w][k] = q[min(16 * k, last)];
+      }
+      const int row = s - NP - 3;
+      if (g < ngroups - 1 && act && row >= 1 && row <= nrow) {
+        const T *const xr = X + (((s & 1) ^ 1) * (NP + 1) + NP) * kX + lane;
+        T *m = msg + (seam_row * nrow + (row - 1)) * 256 + lane;
+        const T a = xr[0], b = xr[128], c = xr[64], e = xr[192];
+        st_agent(m, a);
+        st_agent(m + 64, b);
+        st_agent(m + 128, c);
+        st_agent(m + 192, e);
+      }
+#pragma unroll
+      for (int w = 0; w < NP; w++)
+#pragma unroll
+        for (int k = 0; k < kLines; k++) asm volatile("" ::"s"(t[w][k]));
+      barrier_lds();
+    }
+    return;
+  }
+
+  // ---- column wavefronts
+  const int w = wv, iA = i0 + 2 * w;  // the left mesh column of the pair
+  barrier_lds();
+  if (iA > ncol) {  // past the last column: keep the workgroup's barriers
+    for (int s = 0; s < nsteps; s++) barrier_lds();
+    return;
+  }
+  const bool hasB = iA < ncol;
+  const bool seamB = w == NP - 1 && g < ngroups - 1;  // finished by the next strip's receiver
+  const bool nbrB = iA + 1 < ncol;
+  // overridden i-faces within reach of the pair's right faces
+  const bool xrule = iA == 1 || iA + 1 >= ncol - 1;
+  const int cflA = __builtin_amdgcn_readfirstlane(oflags[ny + 2 + iA]);
+  const int cflB = hasB ? __builtin_amdgcn_readfirstlane(oflags[ny + 3 + iA]) : 0;
+  // the wall rules of the right faces of A (bits 0-2) and B (3-5) where the
+  // mesh's right boundary face is overridden
+  const int rulex = (iA == ncol - 1 ? 2 : iA == ncol ? 4 : 0) | (iA + 1 == ncol - 1 ? 16 : iA + 1 == ncol ? 32 : 0);
+  for (int s = 0; s < w; s++) barrier_lds();
+  const int rg0 = w * kRing + lane;  // own pair's ring; the next pair's is kRing further
+  const int nact = nrow + 6;  // active steps q = s - w
+  CT cc = cpar + (iA - 1) * kNW;  // constants of cell (iA, r), r >= 1
+  const int ccrow = ncol * kNW;   // (a pair without a right column computes on the constants that follow, and drops it)
+  GB fA = (GB)Fb + (rb + (long long)(iA + 1) * cb);  // G of cell (iA, r - 1), r = 1
+  GB fB = (GB)Fb + (long long)(iA + 2) * cb;         // G of cell (iA + 1, r - 2)
+  if (act) {
+    // rows r-1 and r of the left column, r-2, r-1 and r of the right one;
+    // r+1 and r+2 are read from LDS in every step
+    T amg, amh, a0g, a0h, bog, boh, bmg, bmh, b0g, b0h;
+    T fAg, fAh, fBg, fBh;  // fluxes through the bottom faces of row r
+    T ybA, ybB;            // their coefficients
+    // backward coefficients: left column row r-1; right column rows r-1 and r-2,
+    // and its Delta* of row r-2 (row r-1's are read back from LDS)
+    T bxA = T(0), byA = T(0), bxB = T(0), byB = T(0), cxB = T(0), cyB = T(0), eBg = T(0), eBh = T(0);
+    // published values: read and write buffer of the step; the left neighbour's
+    // entry, then the own one, then the right one
+    int xr = ((w & 1) ^ 1) * (NP + 1) * kX + w * kX + lane, xw = (w & 1) * (NP + 1) * kX + w * kX + lane;
+    X[xr + kX + 128] = T(0);
+    X[xr + kX + 192] = T(0);
+    X[xr + kX + 384] = T(0);
+    X[xr + kX + 448] = T(0);
+    // rows -1 .. 2, and the fluxes through the bottom faces of row 1
+    bog = ring[rg0 + 128];
+    boh = ring[rg0 + 192];
+    const T ag = ring[rg0], ah = ring[rg0 + 64];
+    barrier_lds();
+    amg = ring[rg0 + 256];
+    amh = ring[rg0 + 320];
+    bmg = ring[rg0 + 384];
+    bmh = ring[rg0 + 448];
+    barrier_lds();
+    a0g = ring[rg0 + 512];
+    a0h = ring[rg0 + 576];
+    b0g = ring[rg0 + 640];
+    b0h = ring[rg0 + 704];
+    barrier_lds();
+    {
+      const T g2 = ring[rg0 + 768], h2 = ring[rg0 + 832], k2 = ring[rg0 + 896], l2 = ring[rg0 + 960];
+      ybA = fma(vx, T(cc[16]), vy * T(cc[17]));
+      fAg = face_flux_wall<SL>(cflA & 1 ? 4 : 0, posp(ybA), negp(ybA), ag, amg, a0g, g2, ag);
+      fAh = face_flux_wall<SL>(cflA & 1 ? 4 : 0, posp(ybA), negp(ybA), ah, amh, a0h, h2, ah);
+      ybB = fma(vx, T(cc[kNW + 16]), vy * T(cc[kNW + 17]));
+      fBg = face_flux_wall<SL>(cflB & 1 ? 4 : 0, posp(ybB), negp(ybB), bog, bmg, b0g, k2, bog);
+      fBh = face_flux_wall<SL>(cflB & 1 ? 4 : 0, posp(ybB), negp(ybB), boh, bmh, b0h, l2, boh);
+    }
+    barrier_lds();
+    const Exp2<T, (NC == 16)> ex;
+    // backward pass and update of a row (src/GKUA_Residual.f90:64-109) of the
+    // right column (its Delta* in eB; the row above's; the right neighbour's)
+    // and of the left one
+    auto put2 = [&](GB base, T g, T h) __attribute__((always_inline)) {
+      *(GT)(fresh(base) + voff) = g;
+      *(GT)(fresh(base + pb) + voff) = h;
+    };
+    auto put = [&](GB base, T ug, T uh) __attribute__((always_inline)) {
+      if ((double)ug < kClamp) ug = T(kClamp);
+      if ((double)uh < kClamp) uh = T(kClamp);
+      put2(base, ug, uh);
+    };
+    auto finishB = [&](T ng, T nh, int x) __attribute__((always_inline)) {
+      if (hasB && !seamB) {
+        T gr = T(0), hr = T(0);
+        if (nbrB) {
+          gr = X[x + 2 * kX + 384];
+          hr = X[x + 2 * kX + 448];
+        }
+        put(fB, bog + (eBg + fma(cxB, gr, cyB * ng)), boh + (eBh + fma(cxB, hr, cyB * nh)));
+      }
+    };
+    auto finishA = [&](T dg, T dh, T rg, T rh, T ng, T nh) __attribute__((always_inline)) {
+      put(fA, amg + (dg + fma(bxA, rg, byA * ng)), amh + (dh + fma(bxA, rh, byA * nh)));
+    };
+#pragma unroll 1
+    for (int r = 1; r <= nrow; r++) {
+      const int k2 = rg0 + ((r + 3) & 3) * 256, k1 = rg0 + ((r + 2) & 3) * 256, kr = rg0 + kRing + ((r + 1) & 3) * 256;
+      int rules = 0;  // wall rules of the four faces: right of A, of B, top of A, of B
+      if (xrule || r == 1 || r >= nrow - 1) {
+        asm volatile("" ::: "memory");  // (a branch: most rows and columns have none)
+        if (xrule) {
+          const int rf = oflags[r];
+          if ((rf & 1) && iA == 1) rules = 1;
+          if (rf & 2) rules |= rulex;
+        }
+        if (r == 1 || r >= nrow - 1) {
+          const int bit = r == 1 ? 1 : 2, rule = r == 1 ? 1 : r == nrow ? 4 : 2;
+          if (cflA & bit) rules |= rule << 6;
+          if (cflB & bit) rules |= rule << 9;
+        }
+      }
+      const CT cA = cc, cB = cc + kNW;
+      // The step is cut into parts whose values die before the next one's are
+      // read: scheduled as one, it needs more registers than there are.
+      // Fluxes (src/GKUA_Residual.f90:117-418) through the right faces
+      T rAg, rAh, rBg, rBh, tAg, tAh, tBg, tBh;
+      const T xrA = fma(vx, T(cA[14]), vy * T(cA[15])), xrB = fma(vx, T(cB[14]), vy * T(cB[15]));
+      const T xrAp = posp(xrA), xrAn = negp(xrA), xrBp = posp(xrB), xrBn = negp(xrB);
+      {
+        const T e2g = ring[kr], e2h = ring[kr + 64], e3g = ring[kr + 128], e3h = ring[kr + 192];  // F(iA+2, r), F(iA+3, r)
+        const T lfg = X[xr + 256], lfh = X[xr + 320];
+        rAg = face_flux<SL>(xrAp, xrAn, lfg, a0g, b0g, e2g);
+        rAh = face_flux<SL>(xrAp, xrAn, lfh, a0h, b0h, e2h);
+        rBg = face_flux<SL>(xrBp, xrBn, a0g, b0g, e2g, e3g);
+        rBh = face_flux<SL>(xrBp, xrBn, a0h, b0h, e2h, e3h);
+      }
+      const T a1g = ring[k1], a1h = ring[k1 + 64], b1g = ring[k1 + 128], b1h = ring[k1 + 192];
+      __builtin_amdgcn_sched_barrier(0);
+      // through the top faces
+      const T ytA = fma(vx, T(cA[18]), vy * T(cA[19])), ytB = fma(vx, T(cB[18]), vy * T(cB[19]));
+      const T ytAp = posp(ytA), ytAn = negp(ytA), ytBp = posp(ytB), ytBn = negp(ytB);
+      {
+        const T a2g = ring[k2], a2h = ring[k2 + 64], b2g = ring[k2 + 128], b2h = ring[k2 + 192];
+        tAg = face_flux<SL>(ytAp, ytAn, renew(amg), a0g, a1g, a2g);
+        tAh = face_flux<SL>(ytAp, ytAn, renew(amh), a0h, a1h, a2h);
+        tBg = face_flux<SL>(ytBp, ytBn, renew(bmg), b0g, b1g, b2g);
+        tBh = face_flux<SL>(ytBp, ytBn, renew(bmh), b0h, b1h, b2h);
+      }
+      if (rules) {  // next to a wall
+        asm volatile("" ::: "memory");
+        const T a2g = ring[k2], a2h = ring[k2 + 64], b2g = ring[k2 + 128], b2h = ring[k2 + 192];
+        if (rules & 0x1c0) {
+          tAg = face_flux_wall<SL>(rules >> 6, ytAp, ytAn, amg, a0g, a1g, a2g, a2g);
+          tAh = face_flux_wall<SL>(rules >> 6, ytAp, ytAn, amh, a0h, a1h, a2h, a2h);
+        }
+        if (rules & 0xe00) {
+          tBg = face_flux_wall<SL>(rules >> 9, ytBp, ytBn, bmg, b0g, b1g, b2g, b2g);
+          tBh = face_flux_wall<SL>(rules >> 9, ytBp, ytBn, bmh, b0h, b1h, b2h, b2h);
+        }
+        const T wg = X[xr - w * kX + 384], wh = X[xr - w * kX + 448];  // the right wall's slot
+        const T c2g = ring[kr], c2h = ring[kr + 64];
+        if (rules & 7) {
+          rAg = face_flux_wall<SL>(rules, xrAp, xrAn, X[xr + 256], a0g, b0g, c2g, wg);
+          rAh = face_flux_wall<SL>(rules, xrAp, xrAn, X[xr + 320], a0h, b0h, c2h, wh);
+        }
+        if (rules & 0x38) {
+          rBg = face_flux_wall<SL>(rules >> 3, xrBp, xrBn, a0g, b0g, c2g, ring[kr + 128], wg);
+          rBh = face_flux_wall<SL>(rules >> 3, xrBp, xrBn, a0h, b0h, c2h, ring[kr + 192], wh);
+        }
+      }
+      X[xw + kX] = rBg;
+      X[xw + kX + 64] = rBh;
+      X[xw + kX + 256] = b0g;
+      X[xw + kX + 320] = b0h;
+      const T sAg = ((rAg - X[xr]) + tAg) - fAg, sAh = ((rAh - X[xr + 64]) + tAh) - fAh;
+      const T sBg = ((rBg - rAg) + tBg) - fBg, sBh = ((rBh - rAh) + tBh) - fBh;
+      fAg = tAg; fAh = tAh; fBg = tBg; fBh = tBh;
+      __builtin_amdgcn_sched_barrier(0);
+      // equilibrium (Get_Feq, src/GKUA_Residual.f90:420-469) and RHS of both cells
+      T egA, ehA, egB, ehB;
+      {
+        const T ua = vx - T(cA[4]), va = vy - T(cA[5]), ub = vx - T(cB[4]), vb = vy - T(cB[5]);
+        const T wa = fma(ua, ua, va * va) * T(cA[2]), wb = fma(ub, ub, vb * vb) * T(cB[2]);
+        const T fa = T(cA[1]) * fma(ua, T(cA[6]), va * T(cA[7])), fb = T(cB[1]) * fma(ub, T(cB[6]), vb * T(cB[7]));
+        T ga, gb;
+        ex(-wa, -wb, ga, gb);
+        ga *= T(cA[0]);
+        gb *= T(cB[0]);
+        // G: gd (1 + phi (2c^2 - 4)); H: (T gd / 2)(1 + phi (2c^2 - 2))
+        const T ba = fma(T(2), wa, T(-2)), bb = fma(T(2), wb, T(-2));
+        egA = ga * fma(ba, fa, fma(T(-2), fa, T(1)));
+        ehA = ((T(cA[3]) * ga) * T(0.5)) * fma(ba, fa, T(1));
+        egB = gb * fma(bb, fb, fma(T(-2), fb, T(1)));
+        ehB = ((T(cB[3]) * gb) * T(0.5)) * fma(bb, fb, T(1));
+      }
+      const T qAg = fma(T(cA[8]), egA - a0g, -sAg * T(cA[9]));
+      const T qAh = fma(T(cA[8]), ehA - a0h, -sAh * T(cA[9]));
+      const T qBg = fma(T(cB[8]), egB - b0g, -sBg * T(cB[9]));
+      const T qBh = fma(T(cB[8]), ehB - b0h, -sBh * T(cB[9]));
+      __builtin_amdgcn_sched_barrier(0);
+      // LU-SGS diagonals and the forward recursion (:39-57); the bottom
+      // face's coefficient is the top one of the row before
+      const T pAg = X[xr + kX + 384], pAh = X[xr + kX + 448];  // Delta* of row r-1
+      const T pBg = X[xr + kX + 128], pBh = X[xr + kX + 192];
+      const T xlA = fma(vx, T(cA[12]), vy * T(cA[13]));
+      const T raA = rcp_pos(T(cA[11]) + (xrAp - negp(xlA) + ytAp - negp(ybA)));
+      const T raB = rcp_pos(T(cB[11]) + (xrBp - xrAn + ytBp - negp(ybB)));
+      const T nAg = fma(posp(ybA), pAg, fma(T(cA[10]), qAg, posp(xlA) * X[xr + 128])) * raA;
+      const T nAh = fma(posp(ybA), pAh, fma(T(cA[10]), qAh, posp(xlA) * X[xr + 192])) * raA;
+      X[xw + kX + 384] = nAg;
+      X[xw + kX + 448] = nAh;
+      T nBg = fma(posp(ybB), pBg, fma(T(cB[10]), qBg, xrAp * nAg)) * raB;
+      T nBh = fma(posp(ybB), pBh, fma(T(cB[10]), qBh, xrAp * nAh)) * raB;
+      if (!hasB) {
+        nBg = renew(T(0));  // (a branch rather than selects)
+        nBh = renew(T(0));
+      }
+      X[xw + kX + 128] = nBg;
+      X[xw + kX + 192] = nBh;
+      ybA = ytA;
+      ybB = ytB;
+      __builtin_amdgcn_sched_barrier(0);
+      if (r >= 3) finishB(pBg, pBh, xr);
+      if (r >= 2) finishA(pAg, pAh, pBg, pBh, nAg, nAh);
+      if (store_rhs) {
+        const GB rw = (GB)R + (fA - (GB)Fb) + rb;  // cell (iA, r)
+        put2(rw, qAg, qAh);
+        if (hasB) put2(rw + cb, qBg, qBh);
+      }
+      bxA = -xrAn * raA;
+      byA = -ytAn * raA;
+      cxB = bxB;
+      cyB = byB;
+      bxB = -xrBn * raB;
+      byB = -ytBn * raB;
+      eBg = pBg;
+      eBh = pBh;
+      amg = a0g; amh = a0h; a0g = a1g; a0h = a1h;
+      bog = bmg; boh = bmh; bmg = b0g; bmh = b0h; b0g = b1g; b0h = b1h;
+      fA = fresh(fA + rb);
+      fB = fresh(fB + rb);
+      cc += ccrow;
+      const int xt = xr;
+      xr = xw;
+      xw = xt;
+      barrier_lds();
+    }
+    // the two steps after row nrow finish the last rows
+    const T pAg = X[xr + kX + 384], pAh = X[xr + kX + 448], pBg = X[xr + kX + 128], pBh = X[xr + kX + 192];
+    if (nrow >= 2) finishB(pBg, pBh, xr);
+    finishA(pAg, pAh, pBg, pBh, T(0), T(0));
+    barrier_lds();
+    bog = bmg; boh = bmh; cxB = bxB; cyB = byB; eBg = pBg; eBh = pBh;
+    fB += rb;
+    finishB(T(0), T(0), xw);
+    barrier_lds();
+  }
+  for (int s = w + nact; s < nsteps; s++) barrier_lds();
+}
+
+// Wavefronts per SIMD the register file must allow: FP64 one workgroup of 11
+// wavefronts per CU (3 per SIMD, 168 registers) or two of 7 (4, 128); FP32
+// two of 11 (6, 80) or four of 7 (7, 72).
+constexpr int strip_waves(int es, int nc) { return es == 8 ? (nc == 16 ? 3 : 4) : (nc == 16 ? 6 : 7); }
+constexpr int strip_threads(int nc) { return 64 * (nc / 2 + 3); }
+
+template <typename T, int NC, int SL>
+__global__ void __launch_bounds__(strip_threads(NC), strip_waves(sizeof(T), NC))
+    k_strip(Dev d, const T *__restrict__ cpar, T *__restrict__ F, const T *__restrict__ slot, T *__restrict__ R,
+            int store_rhs, int ntiles, T *msg, int *werr, const int *__restrict__ oflags) {
+  __shared__ StripLds<T, NC> lds;
+  strip_body<T, NC, SL>(lds, d, cpar, F, slot, R, store_rhs, ntiles, msg, werr, oflags, (int)blockIdx.x);
 }
 
 // wavefront-uniform copies (scalar registers) of values read from memory
@@ -1503,14 +1834,13 @@ __device__ __forceinline__ int job_of(const J *jobs, int njobs, int b) {
   return __builtin_amdgcn_readfirstlane(lo);
 }
 
-// One launch of the column-wavefront kernel over the strips of every job of a
+// One launch of the column-pair kernel over the strips of every job of a
 // batch (instances of different mesh and velocity grid).  Each job's
 // workgroups are consecutive and strip-major, so a workgroup still waits only
-// for lower-numbered workgroups of its own job.  The launch epoch is read
-// from device memory (a replayed graph increments it in k_batch_epoch).
-template <typename T, int NW, int SL>
-__global__ void __launch_bounds__(64 * NW, 4) k_strip_batch(const StripJob<T> *__restrict__ jobs, int njobs,
-                                                       const int *__restrict__ epoch, int *werr) {
+// for lower-numbered workgroups of its own job.
+template <typename T, int NC, int SL>
+__global__ void __launch_bounds__(strip_threads(NC), strip_waves(sizeof(T), NC))
+    k_strip_batch(const StripJob<T> *__restrict__ jobs, int njobs, int *werr) {
   const int k = job_of<StripJob<T>, &StripJob<T>::strip0>(jobs, njobs, (int)blockIdx.x);
   const StripJob<T> &J = jobs[k];
   // the fields the kernel uses, in scalar registers like kernel arguments
@@ -1524,9 +1854,9 @@ __global__ void __launch_bounds__(64 * NW, 4) k_strip_batch(const StripJob<T> *_
   d.L = uni(J.d.L);
   d.vi = uni(J.d.vi);
   d.vj = uni(J.d.vj);
-  __shared__ StripLds<T, NW> lds;
-  strip_body<T, NW, SL>(lds, d, uni(J.cp), uni(J.F), uni(J.slot), uni(J.R), 0, uni(J.ntiles), uni(J.msg), uni(J.dright),
-                        uni(J.flag), uni(*epoch), werr, uni(J.oflags), (int)blockIdx.x - uni(J.strip0));
+  __shared__ StripLds<T, NC> lds;
+  strip_body<T, NC, SL>(lds, d, uni(J.cp), uni(J.F), uni(J.slot), uni(J.R), 0, uni(J.ntiles), uni(J.msg), werr,
+                        uni(J.oflags), (int)blockIdx.x - uni(J.strip0));
 }
 
 template <typename T>
@@ -1534,64 +1864,6 @@ __global__ void __launch_bounds__(256) k_cellpar_batch(const StripJob<T> *__rest
   const int k = job_of<StripJob<T>, &StripJob<T>::cell0>(jobs, njobs, (int)blockIdx.x);
   const StripJob<T> &J = jobs[k];
   cellpar_body(J.d, const_cast<T *>(J.cp), 0, ((int)blockIdx.x - J.cell0) * 256 + (int)threadIdx.x);
-}
-
-__global__ void k_batch_epoch(int *epoch) {
-  if (threadIdx.x == 0) *epoch += 1;
-}
-
-// Backward pass + update of the last column of every strip but the last
-// (src/GKUA_Residual.f90:64-109): Delta*(i, j) and Delta*(i, j+1) from the
-// seam messages, Delta*(i+1, j) from dright, the coefficients
-// -A^-_x/alfa, -A^-_y/alfa recomputed from the cell constants as k_strip
-// computes them.  One thread per (seam, tile, row, velocity lane).
-template <typename T>
-__device__ __forceinline__ void seam_body(const Dev &d, const T *__restrict__ cpar, T *F, const T *msg,
-                                          const T *dright, int ntiles, int nw, size_t t) {
-  const int lane = (int)(t & 63);
-  const size_t row_id = t >> 6;  // (seam * ntiles + tile) * nrow + r - 1
-  const int ncol = d.nx - 1, nrow = d.ny - 1, nv = d.nv;
-  const int ngroups = (ncol + nw - 1) / nw;
-  if (row_id >= (size_t)(ngroups - 1) * ntiles * nrow) return;
-  const int r = (int)(row_id % nrow) + 1;
-  const int st = (int)(row_id / nrow);
-  const int sg = st / ntiles, tile = st - sg * ntiles;
-  const int i = (sg + 1) * nw;  // last column of strip sg
-  const int v = tile * 64 + lane;
-  if (v >= nv) return;
-  const size_t nf = (size_t)d.ncell * nv;
-  const T vx = T(d.vi[v % d.nvi]), vy = T(d.vj[v / d.nvi]);
-  const T gds = msg[row_id * 256 + 64 + lane], hds = msg[row_id * 256 + 192 + lane];
-  const T gdn = r < nrow ? msg[(row_id + 1) * 256 + 64 + lane] : T(0);  // Delta*(i, j+1), 0 past the last row
-  const T hdn = r < nrow ? msg[(row_id + 1) * 256 + 192 + lane] : T(0);
-  const T gdr = dright[row_id * 128 + lane], hdr = dright[row_id * 128 + 64 + lane];
-  const T *cc = cpar + ((size_t)(r - 1) * ncol + (i - 1)) * kNW;
-  const T axl = vx * T(cc[12]) + vy * T(cc[13]);
-  const T axr = vx * T(cc[14]) + vy * T(cc[15]);
-  const T ayb = vx * T(cc[16]) + vy * T(cc[17]);
-  const T ayt = vx * T(cc[18]) + vy * T(cc[19]);
-  const T alfa = T(cc[11]) + (posp(axr) - negp(axl) + posp(ayt) - negp(ayb));
-  const T ra = rcp_pos(alfa);
-  const T bx = -negp(axr) * ra, by = -negp(ayt) * ra;
-  const size_t o = ((size_t)(r + 1) * d.NI + (size_t)(i + 1)) * nv + v;
-  T fg = F[o] + (gds + (bx * gdr + by * gdn));
-  T fh = F[nf + o] + (hds + (bx * hdr + by * hdn));
-  if ((double)fg < kClamp) fg = T(kClamp);
-  if ((double)fh < kClamp) fh = T(kClamp);
-  F[o] = fg;
-  F[nf + o] = fh;
-}
-template <typename T>
-__global__ void __launch_bounds__(256) k_seam(Dev d, const T *__restrict__ cpar, T *F, const T *msg,
-                                              const T *dright, int ntiles, int nw) {
-  seam_body(d, cpar, F, msg, dright, ntiles, nw, (size_t)blockIdx.x * blockDim.x + threadIdx.x);
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_seam_batch(const StripJob<T> *__restrict__ jobs, int njobs, int nw) {
-  const int k = job_of<StripJob<T>, &StripJob<T>::seam0>(jobs, njobs, (int)blockIdx.x);
-  const StripJob<T> &J = jobs[k];
-  seam_body(J.d, J.cp, J.F, J.msg, J.dright, J.ntiles, nw, (size_t)((int)blockIdx.x - J.seam0) * 256 + threadIdx.x);
 }
 
 // Conserved moments of the stored RHS per interior cell (GaussLegendre_rs,
@@ -2138,68 +2410,61 @@ bool walk_config(const Dev &d, int tiles, int *vt_out, int *k_out, size_t *lds_o
   *lds_out = lds;
   return true;
 }
-// Column-wavefront kernel with NW columns per workgroup, then the seam update.
-template <typename T, int NW>
+// Column-pair kernel with NC columns per workgroup.
+template <typename T, int NC>
 bool launch_strip_nw(const Dev &d, double *cpar, T *F, const T *slot, T *R, int store_rhs, StripBufs &b,
                      hipStream_t s) {
   const int ncol = d.nx - 1, nrow = d.ny - 1;
-  if (ncol < 2 || nrow < 2) return false;
-  const int ngroups = (ncol + NW - 1) / NW, ntiles = (d.nv + 63) / 64;
-  const size_t rows = (size_t)(ngroups - 1) * ntiles * nrow;
-  if (rows * 256 > b.msg_elems || rows * 128 > b.dright_elems || rows > b.flag_elems) return false;
-  const int ncl = ncol * nrow;
+  if (ncol < 2 || nrow < 2 || strip_rows(d, NC) * 256 > b.msg_elems) return false;
+  const int ntiles = (d.nv + 63) / 64, ncl = ncol * nrow;
   // the constants in T: the FP32 kernels read them as single precision
   // without a conversion per use (the same values: each is rounded once)
   T *cp = reinterpret_cast<T *>(cpar);
   hipLaunchKernelGGL(k_cellpar<T>, dim3((ncl + 255) / 256), dim3(256), 0, s, d, cp, 0);
-  b.epoch += 1;
   if (b.ev_before) (void)hipEventRecord(b.ev_before, s);
-  // the WENO3 scheme is a separate instantiation so that the NND / UP1
-  // kernel's register allocation is untouched by the WENO3 weights
+  const dim3 grid(strip_blocks(d, NC)), block(strip_threads(NC));
+  // each flux scheme is a separate instantiation, so that its slopes cost
+  // the others no registers
   if (d.scheme == kSchemeWeno3)
-    hipLaunchKernelGGL((k_strip<T, NW, 1>), dim3(ngroups * ntiles), dim3(64 * NW), 0, s, d, cp, F, slot, R,
-                       store_rhs, ntiles, (T *)b.msg, (T *)b.dright, b.flag, b.epoch, b.err, b.oflags);
+    hipLaunchKernelGGL((k_strip<T, NC, 1>), grid, block, 0, s, d, cp, F, slot, R, store_rhs, ntiles, (T *)b.msg, b.err,
+                       b.oflags);
   else if (d.scheme == 0)  // first-order upwind
-    hipLaunchKernelGGL((k_strip<T, NW, 2>), dim3(ngroups * ntiles), dim3(64 * NW), 0, s, d, cp, F, slot, R,
-                       store_rhs, ntiles, (T *)b.msg, (T *)b.dright, b.flag, b.epoch, b.err, b.oflags);
+    hipLaunchKernelGGL((k_strip<T, NC, 2>), grid, block, 0, s, d, cp, F, slot, R, store_rhs, ntiles, (T *)b.msg, b.err,
+                       b.oflags);
   else
-    hipLaunchKernelGGL((k_strip<T, NW, 0>), dim3(ngroups * ntiles), dim3(64 * NW), 0, s, d, cp, F, slot, R,
-                       store_rhs, ntiles, (T *)b.msg, (T *)b.dright, b.flag, b.epoch, b.err, b.oflags);
+    hipLaunchKernelGGL((k_strip<T, NC, 0>), grid, block, 0, s, d, cp, F, slot, R, store_rhs, ntiles, (T *)b.msg, b.err,
+                       b.oflags);
   if (b.ev_after) (void)hipEventRecord(b.ev_after, s);
-  if (ngroups > 1) {
-    const size_t nthr = rows * 64;
-    hipLaunchKernelGGL(k_seam<T>, dim3((unsigned)((nthr + 255) / 256)), dim3(256), 0, s, d, cp, F,
-                       (const T *)b.msg, (const T *)b.dright, ntiles, NW);
-  }
   return true;
 }
+// Columns per workgroup: 16 where strips of 16 still give every CU a workgroup,
+// else 8, whose shorter pipelines fill more CUs.  Measured, 16 against 8
+// columns: 128^2 x 64^2 (512 strips of 16) 0.86 and 0.89 ms, FP32 0.50 and 0.62,
+// 256^2 x 96^2 (2304) 7.6 and 8.1; 101^2 x 37^2 (154) 0.41 and 0.38, 64^2 x 32^2 (64)
+// 0.22 and 0.18, 12^2 x 24^2 (9) 45 and 41 us.
+int strip_columns(long long strips16) { return strips16 >= 256 ? 16 : 8; }
 int strip_blocks(const Dev &d, int nw) {
   const int ncol = d.nx - 1;
   return (ncol + nw - 1) / nw * ((d.nv + 63) / 64);
 }
-int seam_blocks(const Dev &d, int nw) { return (int)((strip_rows(d, nw) * 64 + 255) / 256); }
 int cell_blocks(const Dev &d) { return ((d.nx - 1) * (d.ny - 1) + 255) / 256; }
 
-template <typename T, int NW>
-void strip_batch_nw(const StripJob<T> *djobs, int njobs, int scheme, int nstrip, int *epoch, int *werr,
-                    hipStream_t s) {
-  if (scheme == kSchemeWeno3)
-    hipLaunchKernelGGL((k_strip_batch<T, NW, 1>), dim3(nstrip), dim3(64 * NW), 0, s, djobs, njobs, epoch, werr);
-  else if (scheme == 0)
-    hipLaunchKernelGGL((k_strip_batch<T, NW, 2>), dim3(nstrip), dim3(64 * NW), 0, s, djobs, njobs, epoch, werr);
-  else
-    hipLaunchKernelGGL((k_strip_batch<T, NW, 0>), dim3(nstrip), dim3(64 * NW), 0, s, djobs, njobs, epoch, werr);
+template <typename T, int NC>
+void strip_batch_nw(const StripJob<T> *djobs, int njobs, int scheme, int nstrip, int *werr, hipStream_t s) {
+  const dim3 grid(nstrip), block(strip_threads(NC));
+  if (scheme == kSchemeWeno3) hipLaunchKernelGGL((k_strip_batch<T, NC, 1>), grid, block, 0, s, djobs, njobs, werr);
+  else if (scheme == 0) hipLaunchKernelGGL((k_strip_batch<T, NC, 2>), grid, block, 0, s, djobs, njobs, werr);
+  else hipLaunchKernelGGL((k_strip_batch<T, NC, 0>), grid, block, 0, s, djobs, njobs, werr);
 }
 
 template <typename T>
-void launch_strip_batch(const StripJob<T> *djobs, int njobs, int nw, int scheme, int nstrip, int nseam, int ncellb,
-                        int *epoch, int *werr, hipStream_t s) {
-  hipLaunchKernelGGL(k_batch_epoch, dim3(1), dim3(64), 0, s, epoch);
+void launch_strip_batch(const StripJob<T> *djobs, int njobs, int nw, int scheme, int nstrip, int ncellb, int *werr,
+                        hipStream_t s) {
   hipLaunchKernelGGL(k_cellpar_batch<T>, dim3(ncellb), dim3(256), 0, s, djobs, njobs);
-  if (nw == 16) strip_batch_nw<T, 16>(djobs, njobs, scheme, nstrip, epoch, werr, s);
-  else strip_batch_nw<T, 8>(djobs, njobs, scheme, nstrip, epoch, werr, s);
-  if (nseam > 0) hipLaunchKernelGGL(k_seam_batch<T>, dim3(nseam), dim3(256), 0, s, djobs, njobs, nw);
+  if (nw == 16) strip_batch_nw<T, 16>(djobs, njobs, scheme, nstrip, werr, s);
+  else strip_batch_nw<T, 8>(djobs, njobs, scheme, nstrip, werr, s);
 }
+uint32_t strip_empty_word(bool fp32) { return fp32 ? Seam<float>::kEmpty : (uint32_t)Seam<double>::kEmpty; }
 
 template <typename T>
 __global__ void k_fill_uniform(Dev d, const double *g, const double *h, T *FG, T *FH, T *slot, size_t nslot) {
@@ -2353,7 +2618,7 @@ void launch_residual(const Dev &d, double *out, hipStream_t s) {
   template void launch_frd_out_chunk<T>(const Dev &, double *, int, int, const T *, const T *, const T *,       \
                                         hipStream_t);                                                           \
   template void launch_frd_in_chunk<T>(const Dev &, const double *, int, int, T *, T *, T *, hipStream_t);    \
-  template void launch_strip_batch<T>(const StripJob<T> *, int, int, int, int, int, int, int *, int *, hipStream_t); \
+  template void launch_strip_batch<T>(const StripJob<T> *, int, int, int, int, int, int *, hipStream_t); \
   template void launch_fill_uniform<T>(const Dev &, const double *, const double *, T *, T *, T *, hipStream_t);
 INST(double)
 INST(float)

@@ -65,10 +65,10 @@ extern "C" {
 #define GSIS_PREC_FP32 1 /* FP32 storage + sweeps, FP64 moments/macro/synthetic */
 
 /* kinetic kernels (gsis_params.split_kernels); every choice gives the same results */
-#define GSIS_KERNEL_AUTO 0    /* one-pass column-wavefront kernel, 8 columns per workgroup, when the mesh fits */
+#define GSIS_KERNEL_AUTO 0    /* one-pass column-pair kernel, 16 or 8 columns per workgroup, when the mesh fits */
 #define GSIS_KERNEL_SPLIT 1   /* separate RHS and LU-SGS sweep kernels */
 #define GSIS_KERNEL_TILES 2   /* one-pass velocity-tile walker (at most 128 cell columns) */
-#define GSIS_KERNEL_STRIP16 3 /* column-wavefront kernel with 16 columns per workgroup */
+#define GSIS_KERNEL_STRIP16 3 /* column-pair kernel with 16 columns per workgroup */
 
 /* One boundary subface, mirrors BC_MSG_TYPE (src/COMMONDATA.f90:34-41) as
  * filled by read_bcin (src/sub_init.f90:266-278).  Node indices are 1-based. */
@@ -311,7 +311,7 @@ int gsis_closure_stats(gsis_handle *h, int64_t *faces, int64_t *accepted, int32_
 int gsis_fill_frd_uniform(gsis_handle *h, const double *g, const double *hv);
 
 /* A batch steps n handles together: the kinetic step of all instances is one
- * launch of the column-wavefront kernel over every instance's strips, and
+ * launch of the column-pair kernel over every instance's strips, and
  * the step of all instances up to the synthetic solve (S0, kinetic BCs, that
  * launch, moments, DETFPwall, Convert_NS, HoT) is captured once as a hipGraph
  * and replayed per step.  The synthetic solves of instances in mode M1 run
@@ -322,7 +322,7 @@ int gsis_fill_frd_uniform(gsis_handle *h, const double *g, const double *hv);
  * times the other placement too, gsis_batch_set_ns_graph chooses it.  Both
  * give the same results.  Instances may differ in mesh, velocity grid, gas, walls and mode; they
  * must share precision, flux scheme and device, and fit the
- * column-wavefront kernel.  A batch step keeps no kinetic RHS (gsis_residual
+ * column-pair kernel.  A batch step keeps no kinetic RHS (gsis_residual
  * reports the last one a gsis_step kept).  The handles must not be stepped
  * on their own while a gsis_batch_step runs; they may be between calls. */
 typedef struct gsis_batch gsis_batch;
