@@ -154,24 +154,38 @@ void phy_boundary(gsis_handle *h) {
   // slot, so they commute with every other BC and go in one launch; far-field
   // and periodic fills (which may share corner ghost cells) keep their order.
   T *FG = (T *)h->FG, *FH = (T *)h->FH, *slot = (T *)h->slot;
-  gsis::WallSet ws{};
+  gsis::BcSet ws{};
   for (const BcDev &b : h->bcd) {
     if (b.code != GSIS_BC_WALL) continue;
     const int nn = (b.face == 1 || b.face == 3) ? (b.jend - b.jst) : (b.iend - b.ist);
     if (nn <= 0) continue;
     if (ws.n == gsis::kMaxWalls) {
       gsis::launch_walls<T>(h->d, ws, FG, FH, slot, h->s);
-      ws = gsis::WallSet{};
+      ws = gsis::BcSet{};
     }
     ws.b[ws.n] = b;
     ws.start[ws.n + 1] = ws.start[ws.n] + nn;
     ws.n++;
   }
   gsis::launch_walls<T>(h->d, ws, FG, FH, slot, h->s);
+  gsis::BcSet ps{};  // periodic subfaces of one direction that follow one another
+  auto flush = [&] {
+    gsis::launch_periodic<T>(h->d, ps, FG, FH, h->s);
+    ps = gsis::BcSet{};
+  };
   for (const BcDev &b : h->bcd) {
-    if (b.code == GSIS_BC_FARFIELD) gsis::launch_farfield<T>(h->d, b, FG, FH, h->s);
-    else if (b.code == GSIS_BC_PERIODIC) gsis::launch_periodic<T>(h->d, b, FG, FH, h->s);
+    if (b.code == GSIS_BC_PERIODIC) {
+      if (ps.n == gsis::kMaxWalls || (ps.n > 0 && (ps.b[0].face - b.face) % 2 != 0)) flush();
+      const int nn = (b.face == 1 || b.face == 3) ? (b.jend - b.jst + 1) : (b.iend - b.ist + 1);
+      ps.b[ps.n] = b;
+      ps.start[ps.n + 1] = ps.start[ps.n] + 2 * nn;
+      ps.n++;
+    } else if (b.code == GSIS_BC_FARFIELD) {
+      flush();
+      gsis::launch_farfield<T>(h->d, b, FG, FH, h->s);
+    }
   }
+  flush();
 }
 
 template <typename T>
@@ -230,6 +244,7 @@ void kinetic(gsis_handle *h) {
     }
     if (h->timing) (void)hipEventRecord(h->ev[0], h->s);
   }
+  gsis::launch_save_s0(h->d, h->s);
   gsis::launch_rhs<T>(h->d, FG, FH, slot, RG, RH, h->s);
   if (h->timing) { (void)hipEventRecord(h->ev[1], h->s); (void)hipEventRecord(h->ev[2], h->s); }
   gsis::launch_sweep<T>(h->d, FG, FH, RG, RH, h->s);
@@ -294,7 +309,6 @@ int synthetic_any(gsis_handle *h) {
 
 template <typename T>
 int one_step(gsis_handle *h) {
-  gsis::launch_save_s0(h->d, h->s);
   phy_boundary<T>(h);
   kinetic<T>(h);
   moments<T>(h, true);
@@ -528,10 +542,7 @@ int batch_capture(gsis_batch *b) {
   }
   hipError_t e = hipStreamBeginCapture(b->s, hipStreamCaptureModeThreadLocal);
   if (e == hipSuccess) {
-    for (gsis_handle *h : b->hs) {
-      gsis::launch_save_s0(h->d, b->s);
-      phy_boundary<T>(h);
-    }
+    for (gsis_handle *h : b->hs) phy_boundary<T>(h);
     gsis::launch_strip_batch<T>((const gsis::StripJob<T> *)b->djobs, (int)b->hs.size(), b->nw, b->scheme, b->nstrip,
                                 b->ncellb, b->err, b->s);
     for (gsis_handle *h : b->hs) {

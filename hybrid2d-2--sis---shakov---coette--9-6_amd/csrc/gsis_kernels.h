@@ -7,17 +7,17 @@ namespace gsis {
 constexpr int kMaxV1 = 512;  // max discrete velocities per direction (LDS tables)
 
 template <typename T> void launch_wall(const Dev &d, const BcDev &b, T *FG, T *FH, T *slot, hipStream_t s);
-// up to kMaxWalls diffuse-wall subfaces launched together; start[k] is the
-// first block of wall k (start[n] = total face nodes)
+// up to kMaxWalls subfaces launched together (diffuse walls; periodic subfaces
+// of one direction); start[k] is the first block of subface k
 constexpr int kMaxWalls = 16;
-struct WallSet {
+struct BcSet {
   int n;
   int start[kMaxWalls + 1];
   BcDev b[kMaxWalls];
 };
-template <typename T> void launch_walls(const Dev &d, const WallSet &ws, T *FG, T *FH, T *slot, hipStream_t s);
+template <typename T> void launch_walls(const Dev &d, const BcSet &ws, T *FG, T *FH, T *slot, hipStream_t s);
 template <typename T> void launch_farfield(const Dev &d, const BcDev &b, T *FG, T *FH, hipStream_t s);
-template <typename T> void launch_periodic(const Dev &d, const BcDev &b, T *FG, T *FH, hipStream_t s);
+template <typename T> void launch_periodic(const Dev &d, const BcSet &bs, T *FG, T *FH, hipStream_t s);
 // inner-face exchange of LAP = 2 layers, FRD(1:2) and S_GKUA(1:10); n1 cells along the face
 template <typename T>
 void launch_inner(const Dev &dd, const BcDev &bd, T *FGd, T *FHd, const Dev &ds, const BcDev &bs, const T *FGs,

@@ -146,13 +146,17 @@ __device__ int block_min_int(int x) {
 // ------------------------------------------------------------------------
 // S0 <- S at the start of the step (src/Hybrid_Sub.f90:29-38)
 // ------------------------------------------------------------------------
+__device__ __forceinline__ void save_s0(const Dev &d, int c) {
+  for (int k = 0; k < 10; k++) d.S0[k * d.ncell + c] = d.S[k * d.ncell + c];
+}
+// (the split path's; the one-pass paths save S0 where they form the cell
+// constants of the same cells: one launch, about 5 us, less per step)
 __global__ void k_save_s0(Dev d) {
   int t = blockIdx.x * blockDim.x + threadIdx.x;
   int ncl = (d.nx - 1) * (d.ny - 1);
   if (t >= ncl) return;
   int i = t % (d.nx - 1) + 1, j = t / (d.nx - 1) + 1;
-  int c = cidx(d, i, j);
-  for (int k = 0; k < 10; k++) d.S0[k * d.ncell + c] = d.S[k * d.ncell + c];
+  save_s0(d, cidx(d, i, j));
 }
 
 // ------------------------------------------------------------------------
@@ -251,7 +255,7 @@ __global__ void k_wall(Dev d, BcDev b, T *FG, T *FH, T *slot) {
 // cells and writes only its own face's slot, so the walls are independent of
 // each other and of the far-field / periodic ghost fills.
 template <typename T>
-__global__ void k_walls(Dev d, WallSet ws, T *FG, T *FH, T *slot) {
+__global__ void k_walls(Dev d, BcSet ws, T *FG, T *FH, T *slot) {
   int w = 0;
   while (w + 1 < ws.n && (int)blockIdx.x >= ws.start[w + 1]) w++;
   wall_node(d, ws.b[w], (int)blockIdx.x - ws.start[w], FG, FH, slot);
@@ -329,9 +333,9 @@ __global__ void k_farfield(Dev d, BcDev b, T *FG, T *FH) {
 // (face node, layer).
 // ------------------------------------------------------------------------
 template <typename T>
-__global__ void k_periodic(Dev d, BcDev b, T *FG, T *FH) {
+__device__ __forceinline__ void periodic_node(const Dev &d, const BcDev &b, int blk, T *FG, T *FH) {
   const int nn = (b.face == 1 || b.face == 3) ? (b.jend - b.jst + 1) : (b.iend - b.ist + 1);
-  const int m = blockIdx.x % nn, k = blockIdx.x / nn + 1;
+  const int m = blk % nn, k = blk / nn + 1;
   int i, j;
   if (b.face == 1 || b.face == 3) { i = b.ist; j = b.jst + m; } else { i = b.ist + m; j = b.jst; }
   int i1, j1, i2, j2;
@@ -346,6 +350,15 @@ __global__ void k_periodic(Dev d, BcDev b, T *FG, T *FH) {
     FG[sb + v] = FG[sa + v];
     FH[sb + v] = FH[sa + v];
   }
+}
+
+// Periodic subfaces of one direction (faces 1 and 3, or 2 and 4) in one launch:
+// each fills ghost layers from cells that none of the others writes.
+template <typename T>
+__global__ void k_periodic(Dev d, BcSet bs, T *FG, T *FH) {
+  int w = 0;
+  while (w + 1 < bs.n && (int)blockIdx.x >= bs.start[w + 1]) w++;
+  periodic_node(d, bs.b[w], (int)blockIdx.x - bs.start[w], FG, FH);
 }
 
 // ------------------------------------------------------------------------
@@ -643,6 +656,7 @@ __device__ __forceinline__ void cellpar_body(const Dev &d, P *cpar, int pstride,
                             d.nj1[g0] * d.sj[g0], d.nj2[g0] * d.sj[g0], d.nj1[gj] * d.sj[gj], d.nj2[gj] * d.sj[gj]};
 #pragma unroll
   for (int k = 0; k < kNW; k++) o[k] = P(vals[k]);
+  save_s0(d, c);
 }
 template <typename P>
 __global__ void k_cellpar(Dev d, P *cpar, int pstride) {
@@ -2106,68 +2120,81 @@ __global__ void k_det_wall(Dev d, const int *list, int n, double *swall) {
   }
 }
 
-// Convert_NS part 1 (src/Hybrid_Sub.f90:221-235): corner extrapolation of S
-// and the NS conservative variables on [0,nx]x[0,ny].
-__global__ void k_convert_u(Dev d) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  const int n1 = d.nx + 1;
-  if (t >= n1 * (d.ny + 1)) return;
-  const int i = t % n1, j = t / n1;
-  const int nx = d.nx, ny = d.ny, N = d.ncell;
-  const int c = cidx(d, i, j);
-  double *S = d.S;
-  int ca = -1, cb = -1, cc = -1;
-  if (i == 0 && j == 0) { ca = cidx(d, 1, 0); cb = cidx(d, 0, 1); cc = cidx(d, 1, 1); }
-  else if (i == nx && j == 0) { ca = cidx(d, nx, 1); cb = cidx(d, nx - 1, 0); cc = cidx(d, nx - 1, 1); }
-  else if (i == 0 && j == ny) { ca = cidx(d, 1, ny); cb = cidx(d, 0, ny - 1); cc = cidx(d, 1, ny - 1); }
-  else if (i == nx && j == ny) { ca = cidx(d, nx - 1, ny); cb = cidx(d, nx, ny - 1); cc = cidx(d, nx - 1, ny - 1); }
-  if (ca >= 0)
-    for (int k = 0; k < 11; k++) S[k * N + c] = S[k * N + ca] + S[k * N + cb] - S[k * N + cc];
-  const double sq = sqrt(2.0 / d.gamma);
-  const double u1 = S[c];
-  const double tu = S[1 * N + c] / d.ma * sq, tv = S[2 * N + c] / d.ma * sq, tt = S[3 * N + c];
-  d.U[0 * N + c] = u1;
-  d.U[1 * N + c] = u1 * tu;
-  d.U[2 * N + c] = u1 * tv;
-  d.U[3 * N + c] = u1 * d.cv * tt + 0.5 * u1 * (tu * tu + tv * tv);
-}
-
-// Convert_NS part 2 (src/Hybrid_Sub.f90:236-239): the four whole-array ghost
-// extrapolations, in order.  Single block.
-__global__ void k_convert_ghost(Dev d) {
-  const int nx = d.nx, ny = d.ny, N = d.ncell;
-  double *U = d.U;
-  for (int ph = 0; ph < 4; ph++) {
-    const int len = (ph < 2) ? (ny + 3) : (nx + 3);
-    for (int t = threadIdx.x; t < 4 * len; t += blockDim.x) {
-      const int m = t % 4, r = t / 4 - 1;  // r in [-1, n+1]
-      int cg, c1, c2;
-      if (ph == 0) { cg = cidx(d, 0, r); c1 = cidx(d, 1, r); c2 = cidx(d, 2, r); }
-      else if (ph == 1) { cg = cidx(d, nx, r); c1 = cidx(d, nx - 1, r); c2 = cidx(d, nx - 2, r); }
-      else if (ph == 2) { cg = cidx(d, r, 0); c1 = cidx(d, r, 1); c2 = cidx(d, r, 2); }
-      else { cg = cidx(d, r, ny); c1 = cidx(d, r, ny - 1); c2 = cidx(d, r, ny - 2); }
-      U[m * N + cg] = 2.0 * U[m * N + c1] - U[m * N + c2];
-    }
-    __syncthreads();
+// NS conservative variables of a cell in [0,nx]x[0,ny] from its S (corners: the
+// extrapolated one), src/Hybrid_Sub.f90:221-235; of any other cell, U as it is.
+// Fused multiply-adds are written out: every thread that needs a cell's value
+// forms the same bits.
+struct Cons { double u[4]; };
+__device__ __forceinline__ Cons cons_of(const Dev &d, int i, int j, bool store) {
+#pragma clang fp contract(off)
+  const int nx = d.nx, ny = d.ny, N = d.ncell, c = cidx(d, i, j);
+  Cons r;
+  if (i < 0 || i > nx || j < 0 || j > ny) {
+    for (int k = 0; k < 4; k++) r.u[k] = d.U[k * N + c];
+    return r;
   }
+  double s[4];
+  if ((i == 0 || i == nx) && (j == 0 || j == ny)) {
+    const int ii = i == 0 ? 1 : nx - 1, jj = j == 0 ? 1 : ny - 1;
+    const int ca = cidx(d, ii, j), cb = cidx(d, i, jj), cc = cidx(d, ii, jj);
+    for (int k = 0; k < 11; k++) {
+      const double x = d.S[k * N + ca] + d.S[k * N + cb] - d.S[k * N + cc];
+      if (k < 4) s[k] = x;
+      if (store) d.S[k * N + c] = x;
+    }
+  } else {
+    for (int k = 0; k < 4; k++) s[k] = d.S[k * N + c];
+  }
+  const double sq = sqrt(2.0 / d.gamma);
+  const double tu = s[1] / d.ma * sq, tv = s[2] / d.ma * sq;
+  r.u[0] = s[0];
+  r.u[1] = s[0] * tu;
+  r.u[2] = s[0] * tv;
+  r.u[3] = fma(s[0] * d.cv, s[3], 0.5 * s[0] * fma(tu, tu, tv * tv));
+  return r;
+}
+__device__ __forceinline__ Cons extrapolate(const Cons &a, const Cons &b) {
+  Cons r;
+  for (int k = 0; k < 4; k++) r.u[k] = fma(2.0, a.u[k], -b.u[k]);
+  return r;
 }
 
-// comput_duvtpckw (src/sub_NS_singlegrid.f90:121-157) over the padded grid,
-// with the T<0.1 stop of interior cells turned into an error flag.
-__global__ void k_prims(Dev d) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
+// Convert_NS (src/Hybrid_Sub.f90:221-239) and comput_duvtpckw
+// (src/sub_NS_singlegrid.f90:121-157), one thread per padded cell: corner
+// extrapolation of S, the conservative variables, the four whole-array ghost
+// extrapolations in their order (columns 0 and nx, then rows 0 and ny, each
+// from the two cells inside it: the thread forms those cells' values itself,
+// at most four of them, so nothing waits for another thread), and the
+// primitive variables, with the T<0.1 stop of interior cells turned into an
+// error flag.  Bound by the latency of its loads: one launch of 10 us where
+// three took 15 (4 x 128 cells).
+__device__ __forceinline__ void convert_cell(const Dev &d, int c) {
   if (c >= d.ncell) return;
-  const int N = d.ncell;
-  const double dd = d.U[c], u = d.U[N + c] / dd, v = d.U[2 * N + c] / dd;
-  const double T = (d.U[3 * N + c] - 0.5 * dd * (u * u + v * v)) / (d.cv * dd);
+  const int nx = d.nx, ny = d.ny, N = d.ncell;
+  const int i = c % d.NI - 1, j = c / d.NI - 1;
+  // a cell after the extrapolation of the columns
+  auto columns = [&](int jj) {
+    if (i == 0) return extrapolate(cons_of(d, 1, jj, false), cons_of(d, 2, jj, false));
+    if (i == nx) return extrapolate(cons_of(d, nx - 1, jj, false), cons_of(d, nx - 2, jj, false));
+    return cons_of(d, i, jj, false);
+  };
+  if ((i == 0 || i == nx) && (j == 0 || j == ny)) (void)cons_of(d, i, j, true);  // S of the corner
+  Cons w;
+  if (j == 0) w = extrapolate(columns(1), columns(2));
+  else if (j == ny) w = extrapolate(columns(ny - 1), columns(ny - 2));
+  else w = columns(j);
+  if ((i >= 0 && i <= nx && j >= 0 && j <= ny) || i == 0 || i == nx || j == 0 || j == ny)
+    for (int k = 0; k < 4; k++) d.U[k * N + c] = w.u[k];
+  const double dd = w.u[0], u = w.u[1] / dd, v = w.u[2] / dd;
+  const double T = (w.u[3] - 0.5 * dd * (u * u + v * v)) / (d.cv * dd);
   d.prim[c] = dd;
   d.prim[N + c] = u;
   d.prim[2 * N + c] = v;
   d.prim[3 * N + c] = T;
   d.prim[4 * N + c] = (1. / (d.gamma * d.ma * d.ma)) * dd * T;
-  const int i = c % d.NI - 1, j = c / d.NI - 1;
-  if (i >= 1 && i <= d.nx - 1 && j >= 1 && j <= d.ny - 1 && T < 0.10000000149011612) atomicOr(d.err, 1);
+  if (i >= 1 && i <= nx - 1 && j >= 1 && j <= ny - 1 && T < 0.10000000149011612) atomicOr(d.err, 1);
 }
+__global__ void k_convert(Dev d) { convert_cell(d, (int)(blockIdx.x * blockDim.x + threadIdx.x)); }
 
 // HoT of Convert_NS (src/Hybrid_Sub.f90:317-349 and :419-448): i-faces
 // (i=1..nx, j=1..ny-1) then j-faces (i=1..nx-1, j=1..ny), one thread each.
@@ -2327,7 +2354,7 @@ void launch_wall(const Dev &d, const BcDev &b, T *FG, T *FH, T *slot, hipStream_
   hipLaunchKernelGGL(k_wall<T>, dim3(nn), dim3(256), 0, s, d, b, FG, FH, slot);
 }
 template <typename T>
-void launch_walls(const Dev &d, const WallSet &ws, T *FG, T *FH, T *slot, hipStream_t s) {
+void launch_walls(const Dev &d, const BcSet &ws, T *FG, T *FH, T *slot, hipStream_t s) {
   if (ws.n <= 0 || ws.start[ws.n] <= 0) return;
   hipLaunchKernelGGL(k_walls<T>, dim3(ws.start[ws.n]), dim3(256), 0, s, d, ws, FG, FH, slot);
 }
@@ -2337,9 +2364,9 @@ void launch_farfield(const Dev &d, const BcDev &b, T *FG, T *FH, hipStream_t s) 
   hipLaunchKernelGGL(k_farfield<T>, dim3(2 * nn), dim3(256), 0, s, d, b, FG, FH);
 }
 template <typename T>
-void launch_periodic(const Dev &d, const BcDev &b, T *FG, T *FH, hipStream_t s) {
-  const int nn = (b.face == 1 || b.face == 3) ? (b.jend - b.jst + 1) : (b.iend - b.ist + 1);
-  hipLaunchKernelGGL(k_periodic<T>, dim3(2 * nn), dim3(256), 0, s, d, b, FG, FH);
+void launch_periodic(const Dev &d, const BcSet &bs, T *FG, T *FH, hipStream_t s) {
+  if (bs.n <= 0) return;
+  hipLaunchKernelGGL(k_periodic<T>, dim3(bs.start[bs.n]), dim3(256), 0, s, d, bs, FG, FH);
 }
 template <typename T>
 void launch_inner(const Dev &dd, const BcDev &bd, T *FGd, T *FHd, const Dev &ds, const BcDev &bs, const T *FGs,
@@ -2551,10 +2578,7 @@ void launch_det_wall(const Dev &d, const int *list, int n, double *swall, hipStr
   hipLaunchKernelGGL(k_det_wall, dim3((n + 127) / 128), dim3(128), 0, s, d, list, n, swall);
 }
 void launch_convert(const Dev &d, hipStream_t s) {
-  const int n = (d.nx + 1) * (d.ny + 1);
-  hipLaunchKernelGGL(k_convert_u, dim3((n + 255) / 256), dim3(256), 0, s, d);
-  hipLaunchKernelGGL(k_convert_ghost, dim3(1), dim3(256), 0, s, d);
-  hipLaunchKernelGGL(k_prims, dim3((d.ncell + 255) / 256), dim3(256), 0, s, d);
+  hipLaunchKernelGGL(k_convert, dim3((d.ncell + 63) / 64), dim3(64), 0, s, d);
 }
 void launch_hot(const Dev &d, hipStream_t s) {
   const int n = d.nx * (d.ny - 1) + (d.nx - 1) * d.ny;
@@ -2604,9 +2628,9 @@ void launch_residual(const Dev &d, double *out, hipStream_t s) {
 
 #define INST(T)                                                                                   \
   template void launch_wall<T>(const Dev &, const BcDev &, T *, T *, T *, hipStream_t);           \
-  template void launch_walls<T>(const Dev &, const WallSet &, T *, T *, T *, hipStream_t);        \
+  template void launch_walls<T>(const Dev &, const BcSet &, T *, T *, T *, hipStream_t);        \
   template void launch_farfield<T>(const Dev &, const BcDev &, T *, T *, hipStream_t);            \
-  template void launch_periodic<T>(const Dev &, const BcDev &, T *, T *, hipStream_t);            \
+  template void launch_periodic<T>(const Dev &, const BcSet &, T *, T *, hipStream_t);            \
   template void launch_inner<T>(const Dev &, const BcDev &, T *, T *, const Dev &, const BcDev &, const T *, \
                                 const T *, int, int, hipStream_t);                                \
   template void launch_rhs<T>(const Dev &, const T *, const T *, const T *, T *, T *, hipStream_t); \
