@@ -147,45 +147,54 @@ int validate(const gsis_params *p) {
   return 0;
 }
 
+// The launches of GKUA_Phy_boundary (src/GKUA_boundary.f90:2-46), which applies
+// the BCs in input order.  Diffuse walls read interior cells and write only
+// their own face slot, so they commute with every other BC and go together;
+// far-field and periodic fills (which may share corner ghost cells) keep
+// their order, periodic subfaces of one direction that follow one another
+// in one launch.
+struct BcLaunches {
+  std::vector<gsis::BcSet> walls;
+  std::vector<std::pair<int, gsis::BcSet>> fills;  // BcJob::kPeriodic or kFarfield, in order
+};
+BcLaunches bc_launches(const gsis_handle *h) {
+  BcLaunches l;
+  auto put = [](gsis::BcSet &w, const BcDev &b, int nn) {
+    w.b[w.n] = b;
+    w.start[w.n + 1] = w.start[w.n] + nn;
+    w.n++;
+  };
+  bool open = false;  // the last fill is a periodic one that the next may join
+  for (const BcDev &b : h->bcd) {
+    const int len = (b.face == 1 || b.face == 3) ? (b.jend - b.jst) : (b.iend - b.ist);
+    if (b.code == GSIS_BC_WALL) {
+      if (len <= 0) continue;
+      if (l.walls.empty() || l.walls.back().n == gsis::kMaxWalls) l.walls.push_back(gsis::BcSet{});
+      put(l.walls.back(), b, len);
+    } else if (b.code == GSIS_BC_PERIODIC) {
+      if (!open || l.fills.back().second.n == gsis::kMaxWalls ||
+          (l.fills.back().second.b[0].face - b.face) % 2 != 0)
+        l.fills.push_back({gsis::BcJob::kPeriodic, gsis::BcSet{}});
+      put(l.fills.back().second, b, 2 * (len + 1));
+      open = true;
+    } else if (b.code == GSIS_BC_FARFIELD) {
+      l.fills.push_back({gsis::BcJob::kFarfield, gsis::BcSet{}});
+      put(l.fills.back().second, b, 2 * (len + 1));
+      open = false;
+    }
+  }
+  return l;
+}
+
 template <typename T>
 void phy_boundary(gsis_handle *h) {
-  // GKUA_Phy_boundary (src/GKUA_boundary.f90:2-46) applies the BCs in input
-  // order.  Diffuse walls read interior cells and write only their own face
-  // slot, so they commute with every other BC and go in one launch; far-field
-  // and periodic fills (which may share corner ghost cells) keep their order.
   T *FG = (T *)h->FG, *FH = (T *)h->FH, *slot = (T *)h->slot;
-  gsis::BcSet ws{};
-  for (const BcDev &b : h->bcd) {
-    if (b.code != GSIS_BC_WALL) continue;
-    const int nn = (b.face == 1 || b.face == 3) ? (b.jend - b.jst) : (b.iend - b.ist);
-    if (nn <= 0) continue;
-    if (ws.n == gsis::kMaxWalls) {
-      gsis::launch_walls<T>(h->d, ws, FG, FH, slot, h->s);
-      ws = gsis::BcSet{};
-    }
-    ws.b[ws.n] = b;
-    ws.start[ws.n + 1] = ws.start[ws.n] + nn;
-    ws.n++;
+  const BcLaunches l = bc_launches(h);
+  for (const gsis::BcSet &w : l.walls) gsis::launch_walls<T>(h->d, w, FG, FH, slot, h->s);
+  for (const auto &f : l.fills) {
+    if (f.first == gsis::BcJob::kPeriodic) gsis::launch_periodic<T>(h->d, f.second, FG, FH, h->s);
+    else gsis::launch_farfield<T>(h->d, f.second.b[0], FG, FH, h->s);
   }
-  gsis::launch_walls<T>(h->d, ws, FG, FH, slot, h->s);
-  gsis::BcSet ps{};  // periodic subfaces of one direction that follow one another
-  auto flush = [&] {
-    gsis::launch_periodic<T>(h->d, ps, FG, FH, h->s);
-    ps = gsis::BcSet{};
-  };
-  for (const BcDev &b : h->bcd) {
-    if (b.code == GSIS_BC_PERIODIC) {
-      if (ps.n == gsis::kMaxWalls || (ps.n > 0 && (ps.b[0].face - b.face) % 2 != 0)) flush();
-      const int nn = (b.face == 1 || b.face == 3) ? (b.jend - b.jst + 1) : (b.iend - b.ist + 1);
-      ps.b[ps.n] = b;
-      ps.start[ps.n + 1] = ps.start[ps.n] + 2 * nn;
-      ps.n++;
-    } else if (b.code == GSIS_BC_FARFIELD) {
-      flush();
-      gsis::launch_farfield<T>(h->d, b, FG, FH, h->s);
-    }
-  }
-  flush();
 }
 
 template <typename T>
@@ -230,7 +239,7 @@ void kinetic(gsis_handle *h) {
       h->strip.ev_before = h->timing ? h->ev[2] : nullptr;
       h->strip.ev_after = h->timing ? h->ev[3] : nullptr;
       ok = gsis::launch_strip<T>(h->d, h->cpar, FG, slot, RG, store,
-                                 sel == GSIS_KERNEL_STRIP16 ? 16 : gsis::strip_columns(gsis::strip_blocks(h->d, 16)), h->strip,
+                                 sel == GSIS_KERNEL_STRIP16 ? 16 : gsis::strip_columns(h->d, gsis::strip_blocks(h->d, 16)), h->strip,
                                  h->s);
     }
     if (!ok) {
@@ -430,7 +439,11 @@ struct gsis_batch {
   hipStream_t s = nullptr;
   void *djobs = nullptr;  // device table of StripJob<T>
   int *err = nullptr;     // a seam wait timed out
-  int nstrip = 0, ncellb = 0;
+  gsis::BatchBlocks nb;                  // jobs and workgroups of the batched launches
+  gsis::BcJob *bcs = nullptr;            // device table of the boundary launches' entries
+  size_t bccap = 0;
+  struct Stage { int first, n, blocks; };
+  std::vector<Stage> stages;             // boundary launches: entries bcs[first..first+n), workgroups
   gsis::NsJob *nsjobs = nullptr;  // device table of the inner loops run in the graph
   int nns = 0, nsblocks = 0;      // its entries, and the workgroups of their launch
   std::vector<bool> in_graph;     // M1 instance whose synthetic solve is captured
@@ -473,33 +486,68 @@ std::vector<int> batch_order(const gsis_batch *b, int order) {
 template <typename T>
 int batch_jobs(gsis_batch *b) {
   std::vector<gsis::StripJob<T>> jobs;
-  int a = 0, e = 0;
-  for (int k : batch_order(b, b->order)) {
-    gsis_handle *h = b->hs[k];
-    gsis::StripJob<T> j{};
-    j.d = h->d;
-    j.cp = reinterpret_cast<const T *>(h->cpar);
-    j.F = (T *)h->FG;
-    j.R = (T *)h->RG;
-    j.slot = (const T *)h->slot;
-    j.msg = (T *)h->strip.msg;
-    j.oflags = h->strip.oflags;
-    j.ntiles = (h->d.nv + 63) / 64;
-    j.strip0 = a;
-    j.cell0 = e;
-    a += gsis::strip_blocks(h->d, b->nw);
-    e += gsis::cell_blocks(h->d);
-    jobs.push_back(j);
-  }
-  b->nstrip = a;
-  b->ncellb = e;
+  // entries of the boundary launches: first every instance's walls and its
+  // first fill, then every instance's second fill, ...
+  std::vector<std::vector<gsis::BcJob>> stages;
+  std::vector<int> blocks;
+  auto enter = [&](size_t stage, int job, int kind, const gsis::BcSet &bs) {
+    if (stages.size() <= stage) {
+      stages.resize(stage + 1);
+      blocks.resize(stage + 1, 0);
+    }
+    gsis::BcJob j{};
+    j.job = job;
+    j.start = blocks[stage];
+    j.kind = kind;
+    j.bs = bs;
+    blocks[stage] += bs.start[bs.n];
+    stages[stage].push_back(j);
+  };
+  b->nb = gsis::BatchBlocks{};
+  const std::vector<int> order = batch_order(b, b->order);
+  for (bool wide : {true, false})
+    for (int k : order) {
+      gsis_handle *h = b->hs[k];
+      if ((b->nw == 16 && h->d.nx - 1 > 8) != wide) continue;  // (strips of 16 would be half empty)
+      gsis::StripJob<T> j{};
+      j.d = h->d;
+      j.cp = reinterpret_cast<const T *>(h->cpar);
+      j.F = (T *)h->FG;
+      j.R = (T *)h->RG;
+      j.slot = (const T *)h->slot;
+      j.msg = (T *)h->strip.msg;
+      j.oflags = h->strip.oflags;
+      j.wall_list = h->wall_list;
+      j.swall = h->swall;
+      j.nwall = h->nwall;
+      j.ntiles = (h->d.nv + 63) / 64;
+      gsis::batch_blocks<T>(j, wide, h->p.if_viscous != 0, b->nb);
+      const BcLaunches l = bc_launches(h);
+      for (const gsis::BcSet &w : l.walls) enter(0, (int)jobs.size(), gsis::BcJob::kWalls, w);
+      for (size_t q = 0; q < l.fills.size(); q++) enter(q, (int)jobs.size(), l.fills[q].first, l.fills[q].second);
+      jobs.push_back(j);
+    }
   HIPCHK(hipMemcpy(b->djobs, jobs.data(), jobs.size() * sizeof(jobs[0]), hipMemcpyHostToDevice));
+  std::vector<gsis::BcJob> all;
+  b->stages.clear();
+  for (size_t q = 0; q < stages.size(); q++) {
+    b->stages.push_back({(int)all.size(), (int)stages[q].size(), blocks[q]});
+    all.insert(all.end(), stages[q].begin(), stages[q].end());
+  }
+  if (all.size() > b->bccap) {  // (the entries are the same at every capture)
+    void *q = nullptr;
+    HIPCHK(hipMalloc(&q, all.size() * sizeof(gsis::BcJob)));
+    b->allocs.push_back(q);
+    b->bcs = reinterpret_cast<gsis::BcJob *>(q);
+    b->bccap = all.size();
+  }
+  if (!all.empty()) HIPCHK(hipMemcpy(b->bcs, all.data(), all.size() * sizeof(gsis::BcJob), hipMemcpyHostToDevice));
   return 0;
 }
 
-// the M0 step of every instance as one graph: per instance S0 <- S and the
-// kinetic BCs, the batched kinetic step, per instance moments + DETFPwall,
-// Convert_NS and the HoT
+// the M0 step of every instance as one graph: kinetic BCs, S0 <- S and the
+// kinetic step, moments + DETFPwall, Convert_NS and the HoT, each launched once
+// for all instances
 template <typename T>
 int batch_capture(gsis_batch *b) {
   batch_drop_graph(b);
@@ -542,15 +590,14 @@ int batch_capture(gsis_batch *b) {
   }
   hipError_t e = hipStreamBeginCapture(b->s, hipStreamCaptureModeThreadLocal);
   if (e == hipSuccess) {
-    for (gsis_handle *h : b->hs) phy_boundary<T>(h);
-    gsis::launch_strip_batch<T>((const gsis::StripJob<T> *)b->djobs, (int)b->hs.size(), b->nw, b->scheme, b->nstrip,
-                                b->ncellb, b->err, b->s);
-    for (gsis_handle *h : b->hs) {
-      moments<T>(h);
+    const auto *jobs = (const gsis::StripJob<T> *)b->djobs;
+    for (const gsis_batch::Stage &st : b->stages)
+      gsis::launch_bc_batch<T>(jobs, b->bcs + st.first, st.n, st.blocks, b->s);
+    gsis::launch_strip_batch<T>(jobs, b->nb, b->scheme, b->err, b->s);
+    gsis::launch_moments_batch<T>(jobs, b->nb, b->s);
+    for (gsis_handle *h : b->hs)
       if (h->mass_on) gsis::launch_mass_correct(h->d, h->mwork, h->init_mass, b->s);
-      gsis::launch_convert(h->d, b->s);
-      if (h->p.if_viscous) gsis::launch_hot(h->d, b->s);
-    }
+    gsis::launch_convert_batch<T>(jobs, b->nb, b->s);
     // the synthetic solves of the M1 instances that use no closure: all in one
     // launch, a gang of workgroups each
     for (size_t k = 0; k < b->hs.size(); k++) {
@@ -1147,8 +1194,9 @@ int gsis_batch_create(gsis_handle *const *hs, int32_t n, gsis_batch **out) {
   b->prec = hs[0]->prec;
   b->scheme = hs[0]->d.scheme;
   long long strips16 = 0;
-  for (int k = 0; k < n; k++) strips16 += gsis::strip_blocks(hs[k]->d, 16);
-  b->nw = gsis::strip_columns(strips16);
+  for (int k = 0; k < n; k++)
+    if (hs[k]->d.nx - 1 > 8) strips16 += gsis::strip_blocks(hs[k]->d, 16);
+  b->nw = strips16 >= gsis::kWideStrips ? 16 : 8;
   auto bail = [&](int rc) {
     gsis_batch_destroy(b);
     return rc;

@@ -51,8 +51,19 @@ uint32_t strip_empty_word(bool fp32);
 // the mesh or the buffers do not fit.
 template <typename T> bool launch_strip(const Dev &d, double *cpar, T *F, const T *slot, T *R, int store_rhs, int nw, StripBufs &b, hipStream_t s);
 template <typename T> void launch_res4(const Dev &d, const T *RG, const T *RH, hipStream_t s);
-// One instance of a batched kinetic step: its device state and the first
-// workgroup of its share of each batched launch.
+// Columns per workgroup: 16 where the mesh has more than 8 and the launch's
+// strips of 16 still give every CU a workgroup, else 8, whose shorter pipelines
+// fill more CUs.  Measured, 16 against 8 columns: 128^2 x 64^2 (512 strips of 16)
+// 0.86 and 0.89 ms, FP32 0.50 and 0.62, 256^2 x 96^2 (2304) 7.6 and 8.1; 101^2 x 37^2
+// (154) 0.41 and 0.38, 64^2 x 32^2 (64) 0.22 and 0.18, 12^2 x 24^2 (9) 45 and 41 us.
+constexpr long long kWideStrips = 256;
+inline int strip_columns(const Dev &d, long long strips16) { return d.nx - 1 > 8 && strips16 >= kWideStrips ? 16 : 8; }
+// workgroups of a mesh's strips with nw columns
+int strip_blocks(const Dev &d, int nw);
+
+// One instance of a batched step: its device state and the first workgroup
+// of its share of each batched launch.  Jobs with strips of 16 columns come
+// before those with 8.
 template <typename T>
 struct StripJob {
   Dev d;
@@ -61,20 +72,34 @@ struct StripJob {
   const T *slot;
   T *msg;
   const int *oflags;
+  const int *wall_list;  // DETFPwall nodes (k_det_wall)
+  double *swall;
+  int nwall;
   int ntiles;
-  int strip0, cell0;  // first workgroup in the strip and cell-constant launches
+  int strip0, cell0, mom0, mom1, det0, conv0, hot0;
 };
-// columns per workgroup for launches of so many strips of 16 columns
-int strip_columns(long long strips16);
-// workgroups of one job in the batched launches with nw columns per strip workgroup
-int strip_blocks(const Dev &d, int nw);
-int cell_blocks(const Dev &d);
-// the kinetic step of every job (djobs: device table, host copies of the
-// counts): cell constants, one column-pair launch over all jobs' strips (no
-// RHS kept); scheme and T shared by all jobs
+// Subfaces of one instance in a batched boundary launch.
+struct BcJob {
+  enum { kWalls, kPeriodic, kFarfield };
+  int job, start, kind;
+  BcSet bs;
+};
+// jobs (the first wide of them with strips of 16 columns) and workgroups of
+// each batched launch
+struct BatchBlocks {
+  int jobs = 0, wide = 0, strip16 = 0, strip8 = 0, cell = 0, mom0 = 0, mom1 = 0, det = 0, conv = 0, hot = 0;
+};
+template <typename T> void batch_blocks(StripJob<T> &j, bool wide, bool hot, BatchBlocks &n);
+// Batched launches over a device table of jobs (scheme and T shared by all):
+// boundary subfaces, S0 + cell constants + one column-pair launch per strip
+// width over all jobs' strips (no RHS kept), moments + DETFPwall, Convert_NS +
+// HoT.
 template <typename T>
-void launch_strip_batch(const StripJob<T> *djobs, int njobs, int nw, int scheme, int nstrip, int ncellb, int *werr,
-                        hipStream_t s);
+void launch_bc_batch(const StripJob<T> *djobs, const BcJob *dbcs, int n, int blocks, hipStream_t s);
+template <typename T>
+void launch_strip_batch(const StripJob<T> *djobs, const BatchBlocks &n, int scheme, int *werr, hipStream_t s);
+template <typename T> void launch_moments_batch(const StripJob<T> *djobs, const BatchBlocks &n, hipStream_t s);
+template <typename T> void launch_convert_batch(const StripJob<T> *djobs, const BatchBlocks &n, hipStream_t s);
 // every cell's distribution set to g[v] (G) and h[v] (H), wall slots zero
 template <typename T>
 void launch_fill_uniform(const Dev &d, const double *g, const double *h, T *FG, T *FH, T *slot, hipStream_t s);

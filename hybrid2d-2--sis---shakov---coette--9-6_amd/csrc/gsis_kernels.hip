@@ -267,9 +267,9 @@ __global__ void k_walls(Dev d, BcSet ws, T *FG, T *FH, T *slot) {
 // One block per (face node, layer k).
 // ------------------------------------------------------------------------
 template <typename T>
-__global__ void k_farfield(Dev d, BcDev b, T *FG, T *FH) {
+__device__ __forceinline__ void farfield_node(const Dev &d, const BcDev &b, int blk, T *FG, T *FH) {
   const int nn = (b.face == 1 || b.face == 3) ? (b.jend - b.jst + 1) : (b.iend - b.ist + 1);
-  const int m = blockIdx.x % nn, k = blockIdx.x / nn + 1;
+  const int m = blk % nn, k = blk / nn + 1;
   int i, j;
   if (b.face == 1 || b.face == 3) { i = b.ist; j = b.jst + m; } else { i = b.ist + m; j = b.jst; }
   int i1, j1, i2, j2;
@@ -326,6 +326,11 @@ __global__ void k_farfield(Dev d, BcDev b, T *FG, T *FH) {
     FG[cf + v] = T(gd);
     FH[cf + v] = T(gd * tt / 2.);
   }
+}
+
+template <typename T>
+__global__ void k_farfield(Dev d, BcDev b, T *FG, T *FH) {
+  farfield_node(d, b, (int)blockIdx.x, FG, FH);
 }
 
 // ------------------------------------------------------------------------
@@ -1826,13 +1831,31 @@ __global__ void __launch_bounds__(strip_threads(NC), strip_waves(sizeof(T), NC))
   strip_body<T, NC, SL>(lds, d, cpar, F, slot, R, store_rhs, ntiles, msg, werr, oflags, (int)blockIdx.x);
 }
 
-// wavefront-uniform copies (scalar registers) of values read from memory
+// wavefront-uniform copies (scalar registers) of values read from memory,
+// pointers as global ones
 __device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
 template <typename P>
 __device__ __forceinline__ P *uni(P *p) {
   const unsigned long long v = reinterpret_cast<unsigned long long>(p);
   const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)v), hi = __builtin_amdgcn_readfirstlane((unsigned)(v >> 32));
-  return reinterpret_cast<P *>(((unsigned long long)hi << 32) | lo);
+  return (P *)(__attribute__((address_space(1))) P *)(((unsigned long long)hi << 32) | lo);
+}
+
+template <typename P>
+__device__ __forceinline__ P *in_global(P *p) {
+  return (P *)(__attribute__((address_space(1))) P *)reinterpret_cast<unsigned long long>(p);
+}
+// an instance's device state with its pointers known to be global ones
+__device__ __forceinline__ Dev dev_of(const Dev &e) {
+  Dev d = e;
+  d.vi = in_global(d.vi); d.vj = in_global(d.vj); d.wi = in_global(d.wi); d.wj = in_global(d.wj);
+  d.rowf = in_global(d.rowf); d.vol = in_global(d.vol); d.si = in_global(d.si); d.sj = in_global(d.sj);
+  d.ni1 = in_global(d.ni1); d.ni2 = in_global(d.ni2); d.nj1 = in_global(d.nj1); d.nj2 = in_global(d.nj2);
+  d.xn = in_global(d.xn); d.yn = in_global(d.yn); d.x1 = in_global(d.x1); d.y1 = in_global(d.y1);
+  d.S = in_global(d.S); d.S0 = in_global(d.S0); d.CF = in_global(d.CF); d.U = in_global(d.U);
+  d.taoi = in_global(d.taoi); d.taoj = in_global(d.taoj); d.qi = in_global(d.qi); d.qj = in_global(d.qj);
+  d.prim = in_global(d.prim); d.err = in_global(d.err);
+  return d;
 }
 
 // the job of workgroup b of a batched launch: the last job whose first
@@ -1877,7 +1900,7 @@ template <typename T>
 __global__ void __launch_bounds__(256) k_cellpar_batch(const StripJob<T> *__restrict__ jobs, int njobs) {
   const int k = job_of<StripJob<T>, &StripJob<T>::cell0>(jobs, njobs, (int)blockIdx.x);
   const StripJob<T> &J = jobs[k];
-  cellpar_body(J.d, const_cast<T *>(J.cp), 0, ((int)blockIdx.x - J.cell0) * 256 + (int)threadIdx.x);
+  cellpar_body(dev_of(J.d), in_global(const_cast<T *>(J.cp)), 0, ((int)blockIdx.x - J.cell0) * 256 + (int)threadIdx.x);
 }
 
 // Conserved moments of the stored RHS per interior cell (GaussLegendre_rs,
@@ -1940,11 +1963,11 @@ __device__ __forceinline__ void buf_st(T v, __amdgpu_buffer_rsrc_t r, unsigned v
 // half of its rows, and combine through LDS: twice the wavefronts shortens the
 // last partial round of the grid.
 template <typename T, bool ONE>
-__global__ void __launch_bounds__(256) k_moments(Dev d, T *__restrict__ FG, T *__restrict__ FH) {
+__device__ __forceinline__ void moments_body(const Dev &d, int blk, T *__restrict__ FG, T *__restrict__ FH) {
   // the wavefront index through readfirstlane, so that the row range below is
   // known to be uniform (scalar row offsets and factors)
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int c = ONE ? blockIdx.x * 2 + (wv >> 1) : blockIdx.x * 4 + wv;
+  const int c = ONE ? blk * 2 + (wv >> 1) : blk * 4 + wv;
   const int half = ONE ? (wv & 1) : 0;
   // whole wavefronts: the reduction below stays wave-uniform; the ONE path
   // returns only after its barrier
@@ -2107,10 +2130,14 @@ __global__ void __launch_bounds__(256) k_moments(Dev d, T *__restrict__ FG, T *_
   }
 }
 
+template <typename T, bool ONE>
+__global__ void __launch_bounds__(256) k_moments(Dev d, T *__restrict__ FG, T *__restrict__ FH) {
+  moments_body<T, ONE>(d, (int)blockIdx.x, FG, FH);
+}
+
 // DETFPwall for every wall/farfield face node (src/GKUA_DETFP_WALL.f90:34-95).
 // list[4*k..]: ghost cell, first cell, second cell, Swall offset.
-__global__ void k_det_wall(Dev d, const int *list, int n, double *swall) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void det_wall_node(const Dev &d, const int *list, int n, double *swall, int t) {
   if (t >= n) return;
   const int cg = list[4 * t], ca = list[4 * t + 1], cb = list[4 * t + 2], so = list[4 * t + 3];
   for (int k = 0; k < 10; k++) {
@@ -2118,6 +2145,10 @@ __global__ void k_det_wall(Dev d, const int *list, int n, double *swall) {
     swall[so + k] = sw;
     d.S[k * d.ncell + cg] = 2.0 * sw - d.S[k * d.ncell + ca];
   }
+}
+
+__global__ void k_det_wall(Dev d, const int *list, int n, double *swall) {
+  det_wall_node(d, list, n, swall, (int)(blockIdx.x * blockDim.x + threadIdx.x));
 }
 
 // NS conservative variables of a cell in [0,nx]x[0,ny] from its S (corners: the
@@ -2198,8 +2229,7 @@ __global__ void k_convert(Dev d) { convert_cell(d, (int)(blockIdx.x * blockDim.x
 
 // HoT of Convert_NS (src/Hybrid_Sub.f90:317-349 and :419-448): i-faces
 // (i=1..nx, j=1..ny-1) then j-faces (i=1..nx-1, j=1..ny), one thread each.
-__global__ void k_hot(Dev d) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void hot_face(const Dev &d, int t) {
   const int nx = d.nx, ny = d.ny, N = d.ncell;
   const int ni = nx * (ny - 1), nj = (nx - 1) * ny;
   if (t >= ni + nj) return;
@@ -2255,6 +2285,55 @@ __global__ void k_hot(Dev d) {
       qg[1 * N + c] = -S[8 * N + cs] * 1.4142135381698608 / ((d.ma * d.ma * d.ma) * pow(d.gamma, 1.5)) - o[5];
     }
   }
+}
+
+__global__ void k_hot(Dev d) { hot_face(d, (int)(blockIdx.x * blockDim.x + threadIdx.x)); }
+
+// ---- the same work over every instance of a batch, one launch each --------
+// A step of n small instances is otherwise some 8n launches of a few
+// microseconds each, one after another (32 instances: 1.5 of 8.9 ms per step).
+// A workgroup finds its instance by its index (job_of) and runs the
+// instance's part as the single launch does.
+template <typename T>
+__global__ void __launch_bounds__(256) k_bc_batch(const StripJob<T> *__restrict__ jobs, const BcJob *__restrict__ bcs,
+                                                  int n) {
+  const BcJob &B = bcs[job_of<BcJob, &BcJob::start>(bcs, n, (int)blockIdx.x)];
+  const StripJob<T> &J = jobs[B.job];
+  const Dev d = dev_of(J.d);
+  T *const FG = in_global(J.F), *const FH = FG + (size_t)d.ncell * d.nv;
+  const int blk = (int)blockIdx.x - B.start;
+  int w = 0;
+  while (w + 1 < B.bs.n && blk >= B.bs.start[w + 1]) w++;
+  const BcDev b = B.bs.b[w];
+  const int k = blk - B.bs.start[w];
+  if (B.kind == BcJob::kWalls) wall_node(d, b, k, FG, FH, in_global(const_cast<T *>(J.slot)));
+  else if (B.kind == BcJob::kPeriodic) periodic_node(d, b, k, FG, FH);
+  else farfield_node(d, b, k, FG, FH);
+}
+template <typename T, bool ONE>
+__global__ void __launch_bounds__(256) k_moments_batch(const StripJob<T> *__restrict__ jobs, int njobs) {
+  const StripJob<T> &J =
+      jobs[ONE ? job_of<StripJob<T>, &StripJob<T>::mom1>(jobs, njobs, (int)blockIdx.x)
+               : job_of<StripJob<T>, &StripJob<T>::mom0>(jobs, njobs, (int)blockIdx.x)];
+  const Dev d = dev_of(J.d);
+  T *const FG = in_global(J.F);
+  moments_body<T, ONE>(d, (int)blockIdx.x - (ONE ? J.mom1 : J.mom0), FG, FG + (size_t)d.ncell * d.nv);
+}
+template <typename T>
+__global__ void __launch_bounds__(64) k_det_wall_batch(const StripJob<T> *__restrict__ jobs, int njobs) {
+  const StripJob<T> &J = jobs[job_of<StripJob<T>, &StripJob<T>::det0>(jobs, njobs, (int)blockIdx.x)];
+  det_wall_node(dev_of(J.d), in_global(J.wall_list), J.nwall, in_global(J.swall),
+                ((int)blockIdx.x - J.det0) * 64 + (int)threadIdx.x);
+}
+template <typename T>
+__global__ void __launch_bounds__(64) k_convert_batch(const StripJob<T> *__restrict__ jobs, int njobs) {
+  const StripJob<T> &J = jobs[job_of<StripJob<T>, &StripJob<T>::conv0>(jobs, njobs, (int)blockIdx.x)];
+  convert_cell(dev_of(J.d), ((int)blockIdx.x - J.conv0) * 64 + (int)threadIdx.x);
+}
+template <typename T>
+__global__ void __launch_bounds__(128) k_hot_batch(const StripJob<T> *__restrict__ jobs, int njobs) {
+  const StripJob<T> &J = jobs[job_of<StripJob<T>, &StripJob<T>::hot0>(jobs, njobs, (int)blockIdx.x)];
+  hot_face(dev_of(J.d), ((int)blockIdx.x - J.hot0) * 128 + (int)threadIdx.x);
 }
 
 // RMS and max over interior cells of the per-cell RHS moments
@@ -2464,20 +2543,16 @@ bool launch_strip_nw(const Dev &d, double *cpar, T *F, const T *slot, T *R, int 
   if (b.ev_after) (void)hipEventRecord(b.ev_after, s);
   return true;
 }
-// Columns per workgroup: 16 where strips of 16 still give every CU a workgroup,
-// else 8, whose shorter pipelines fill more CUs.  Measured, 16 against 8
-// columns: 128^2 x 64^2 (512 strips of 16) 0.86 and 0.89 ms, FP32 0.50 and 0.62,
-// 256^2 x 96^2 (2304) 7.6 and 8.1; 101^2 x 37^2 (154) 0.41 and 0.38, 64^2 x 32^2 (64)
-// 0.22 and 0.18, 12^2 x 24^2 (9) 45 and 41 us.
-int strip_columns(long long strips16) { return strips16 >= 256 ? 16 : 8; }
 int strip_blocks(const Dev &d, int nw) {
   const int ncol = d.nx - 1;
   return (ncol + nw - 1) / nw * ((d.nv + 63) / 64);
 }
-int cell_blocks(const Dev &d) { return ((d.nx - 1) * (d.ny - 1) + 255) / 256; }
+// moments with two wavefronts per cell (one velocity row per pass)
+static bool moments_one(const Dev &d) { return d.nvi > 32 && d.nvi <= 64; }
 
 template <typename T, int NC>
 void strip_batch_nw(const StripJob<T> *djobs, int njobs, int scheme, int nstrip, int *werr, hipStream_t s) {
+  if (nstrip <= 0) return;
   const dim3 grid(nstrip), block(strip_threads(NC));
   if (scheme == kSchemeWeno3) hipLaunchKernelGGL((k_strip_batch<T, NC, 1>), grid, block, 0, s, djobs, njobs, werr);
   else if (scheme == 0) hipLaunchKernelGGL((k_strip_batch<T, NC, 2>), grid, block, 0, s, djobs, njobs, werr);
@@ -2485,11 +2560,46 @@ void strip_batch_nw(const StripJob<T> *djobs, int njobs, int scheme, int nstrip,
 }
 
 template <typename T>
-void launch_strip_batch(const StripJob<T> *djobs, int njobs, int nw, int scheme, int nstrip, int ncellb, int *werr,
-                        hipStream_t s) {
-  hipLaunchKernelGGL(k_cellpar_batch<T>, dim3(ncellb), dim3(256), 0, s, djobs, njobs);
-  if (nw == 16) strip_batch_nw<T, 16>(djobs, njobs, scheme, nstrip, werr, s);
-  else strip_batch_nw<T, 8>(djobs, njobs, scheme, nstrip, werr, s);
+void launch_bc_batch(const StripJob<T> *djobs, const BcJob *dbcs, int n, int blocks, hipStream_t s) {
+  if (blocks > 0) hipLaunchKernelGGL(k_bc_batch<T>, dim3(blocks), dim3(256), 0, s, djobs, dbcs, n);
+}
+template <typename T>
+void launch_strip_batch(const StripJob<T> *djobs, const BatchBlocks &n, int scheme, int *werr, hipStream_t s) {
+  hipLaunchKernelGGL(k_cellpar_batch<T>, dim3(n.cell), dim3(256), 0, s, djobs, n.jobs);
+  strip_batch_nw<T, 16>(djobs, n.wide, scheme, n.strip16, werr, s);
+  strip_batch_nw<T, 8>(djobs + n.wide, n.jobs - n.wide, scheme, n.strip8, werr, s);
+}
+template <typename T>
+void launch_moments_batch(const StripJob<T> *djobs, const BatchBlocks &n, hipStream_t s) {
+  if (n.mom1 > 0) hipLaunchKernelGGL((k_moments_batch<T, true>), dim3(n.mom1), dim3(256), 0, s, djobs, n.jobs);
+  if (n.mom0 > 0) hipLaunchKernelGGL((k_moments_batch<T, false>), dim3(n.mom0), dim3(256), 0, s, djobs, n.jobs);
+  if (n.det > 0) hipLaunchKernelGGL(k_det_wall_batch<T>, dim3(n.det), dim3(64), 0, s, djobs, n.jobs);
+}
+template <typename T>
+void launch_convert_batch(const StripJob<T> *djobs, const BatchBlocks &n, hipStream_t s) {
+  hipLaunchKernelGGL(k_convert_batch<T>, dim3(n.conv), dim3(64), 0, s, djobs, n.jobs);
+  if (n.hot > 0) hipLaunchKernelGGL(k_hot_batch<T>, dim3(n.hot), dim3(128), 0, s, djobs, n.jobs);
+}
+// the next workgroups of each launch to a job of a batch; wide: 16 columns per strip
+template <typename T>
+void batch_blocks(StripJob<T> &j, bool wide, bool hot, BatchBlocks &n) {
+  const Dev &d = j.d;
+  const int one = moments_one(d) ? 1 : 0;
+  j.strip0 = wide ? n.strip16 : n.strip8;
+  j.cell0 = n.cell;
+  j.mom0 = n.mom0;
+  j.mom1 = n.mom1;
+  j.det0 = n.det;
+  j.conv0 = n.conv;
+  j.hot0 = n.hot;
+  (wide ? n.strip16 : n.strip8) += strip_blocks(d, wide ? 16 : 8);
+  n.cell += ((d.nx - 1) * (d.ny - 1) + 255) / 256;
+  (one ? n.mom1 : n.mom0) += one ? (d.ncell + 1) / 2 : (d.ncell + 3) / 4;
+  n.det += (j.nwall + 63) / 64;
+  n.conv += (d.ncell + 63) / 64;
+  if (hot) n.hot += (d.nx * (d.ny - 1) + (d.nx - 1) * d.ny + 127) / 128;
+  n.jobs += 1;
+  n.wide += wide ? 1 : 0;
 }
 uint32_t strip_empty_word(bool fp32) { return fp32 ? Seam<float>::kEmpty : (uint32_t)Seam<double>::kEmpty; }
 
@@ -2550,7 +2660,7 @@ bool launch_walk(const Dev &d, double *cpar, T *F, const T *slot, T *R, int stor
 
 template <typename T>
 void launch_moments(const Dev &d, T *FG, T *FH, hipStream_t s) {
-  if (d.nvi > 32 && d.nvi <= 64)
+  if (moments_one(d))
     hipLaunchKernelGGL((k_moments<T, true>), dim3((d.ncell + 1) / 2), dim3(256), 0, s, d, FG, FH);
   else
     hipLaunchKernelGGL((k_moments<T, false>), dim3((d.ncell + 3) / 4), dim3(256), 0, s, d, FG, FH);
@@ -2642,7 +2752,11 @@ void launch_residual(const Dev &d, double *out, hipStream_t s) {
   template void launch_frd_out_chunk<T>(const Dev &, double *, int, int, const T *, const T *, const T *,       \
                                         hipStream_t);                                                           \
   template void launch_frd_in_chunk<T>(const Dev &, const double *, int, int, T *, T *, T *, hipStream_t);    \
-  template void launch_strip_batch<T>(const StripJob<T> *, int, int, int, int, int, int *, hipStream_t); \
+  template void launch_bc_batch<T>(const StripJob<T> *, const BcJob *, int, int, hipStream_t);                \
+  template void launch_strip_batch<T>(const StripJob<T> *, const BatchBlocks &, int, int *, hipStream_t);     \
+  template void launch_moments_batch<T>(const StripJob<T> *, const BatchBlocks &, hipStream_t);               \
+  template void launch_convert_batch<T>(const StripJob<T> *, const BatchBlocks &, hipStream_t);               \
+  template void batch_blocks<T>(StripJob<T> &, bool, bool, BatchBlocks &);                                    \
   template void launch_fill_uniform<T>(const Dev &, const double *, const double *, T *, T *, T *, hipStream_t);
 INST(double)
 INST(float)
