@@ -87,6 +87,14 @@ struct gsis_handle {
 
 namespace {
 
+// Zeroed memory of a handle.  The clear runs on the null stream, with which the
+// handle's stream does not synchronise: work queued there right after could
+// be cleared again.  gsis_create waits for the null stream once, at its end;
+// later callers wait themselves (null_stream_done).
+int null_stream_done() {
+  const hipError_t e = hipStreamSynchronize(nullptr);
+  return e == hipSuccess ? 0 : fail(GSIS_EHIP, std::string("null stream: ") + hipGetErrorString(e));
+}
 template <typename P>
 int dalloc(gsis_handle *h, P **ptr, size_t bytes) {
   void *q = nullptr;
@@ -854,6 +862,7 @@ int gsis_create(const gsis_params *p, gsis_handle **out) {
     rc = gsis::synthetic_init(h->d, *p, h->syn);
     if (rc) return cleanup(fail(rc, gsis::synthetic_error()));
   }
+  if ((rc = null_stream_done())) return cleanup(rc);
   *out = h;
   return 0;
 }
@@ -888,6 +897,7 @@ int gsis_set_mass_correct(gsis_handle *h, int32_t on) {
   }
   if (!h->mwork) {
     int rc = dalloc(h, &h->mwork, 64);
+    if (!rc) rc = null_stream_done();
     if (rc) return rc;
   }
   gsis::launch_out_mass(h->d, h->mwork, h->s);

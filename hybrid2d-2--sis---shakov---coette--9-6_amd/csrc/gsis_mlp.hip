@@ -411,7 +411,9 @@ template <typename P>
 int malloc_d(MlpDev &d, P **p, size_t bytes) {
   void *q = nullptr;
   if (hipMalloc(&q, std::max(bytes, (size_t)8)) != hipSuccess) return mfail(GSIS_EHIP, "mlp: hipMalloc failed");
-  if (hipMemset(q, 0, std::max(bytes, (size_t)8)) != hipSuccess) return mfail(GSIS_EHIP, "mlp: hipMemset failed");
+  // cleared on the network's own stream, before whatever uses it there
+  if (hipMemsetAsync(q, 0, std::max(bytes, (size_t)8), d.s) != hipSuccess)
+    return mfail(GSIS_EHIP, "mlp: hipMemset failed");
   d.allocs.push_back(q);
   *p = reinterpret_cast<P *>(q);
   return 0;
