@@ -118,6 +118,9 @@ void launch_mass_correct(const Dev &d, double *work, double init, hipStream_t s)
 void launch_det_wall(const Dev &d, const int *list, int n, double *swall, hipStream_t s);
 void launch_convert(const Dev &d, hipStream_t s);
 void launch_hot(const Dev &d, hipStream_t s);
+// ncomp plane-major fields of the padded cells into [ny1][nx1][nf] (zero where there is none)
+void launch_fields_out(const Dev &d, const double *src, int ncomp, int nf, int nx1, int ny1, int o, double *out,
+                       hipStream_t s);
 void launch_residual(const Dev &d, double *out, hipStream_t s);
 
 }  // namespace gsis
