@@ -1164,18 +1164,18 @@ __global__ void __launch_bounds__(1024) k_walk(Dev d, const double *cpar, int VT
 // Two columns per wavefront because what a wavefront does once per step --
 // addresses, scalar loads, the barrier, publishing, the left face's
 // coefficients -- then serves two cells, and because the two cells' chains fill
-// each other's latency: 344 vector and 123 scalar instructions per two cells
-// (FP64 NND), against 215 and 152 per cell with one column per wavefront, which
-// also held the copies and both seam roles.  Rows r+1 and r+2, the right
+// each other's latency: 360 vector and 82 scalar instructions per two cells
+// (FP64 NND, counted over all wavefronts), against 215 and 152 per cell with one
+// column per wavefront.  Rows r+1 and r+2, the right
 // column's earlier rows and earlier Delta* are read from LDS again instead of
 // being kept, and the step is cut into parts: that fits 130 registers without
 // a spill in the loop (one reload there waits for the stores before it and cost
 // 15% of the kernel).
 //
 // Measured, this kernel against one column per wavefront with a seam-update
-// kernel after it, both included: 128^2 cells x 64^2 velocities FP64 0.77 against
-// 1.04 ms, FP32 0.42 against 0.72; 256^2 x 96^2 FP64 7.4 against 8.8; 101^2 x 37^2
-// WENO3 0.34 against 0.53.  Bound by vector issue: two wavefronts per SIMD
+// kernel after it, both included: 128^2 cells x 64^2 velocities FP64 0.74 against
+// 1.01 ms, FP32 0.39 against 0.72; 256^2 x 96^2 FP64 6.3 against 8.8; 101^2 x 37^2
+// WENO3 0.46 against 0.53.  Bound by vector issue: two wavefronts per SIMD
 // (LDS allows no more in FP64) reach 57% of the issue slots, and the kernel
 // runs at 1.96 GHz.  Without its stores it is 12% faster, without its copies 5%.
 //
@@ -2291,7 +2291,7 @@ __global__ void k_hot(Dev d) { hot_face(d, (int)(blockIdx.x * blockDim.x + threa
 
 // ---- the same work over every instance of a batch, one launch each --------
 // A step of n small instances is otherwise some 8n launches of a few
-// microseconds each, one after another (32 instances: 1.5 of 8.9 ms per step).
+// microseconds each, one after another (32 instances: 1.9 of 9.1 ms per step).
 // A workgroup finds its instance by its index (job_of) and runs the
 // instance's part as the single launch does.
 template <typename T>
