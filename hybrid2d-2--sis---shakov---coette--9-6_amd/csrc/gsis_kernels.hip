@@ -146,8 +146,14 @@ __device__ int block_min_int(int x) {
 // ------------------------------------------------------------------------
 // S0 <- S at the start of the step (src/Hybrid_Sub.f90:29-38)
 // ------------------------------------------------------------------------
+// Every load before the first store: a store in between, to memory that the
+// compiler must take to be the same, holds the next load back, and ten waits for
+// memory one after another are 5 us.  (128^2 cells: k_cellpar, which saves S0 too,
+// 6.4 -> 5.1 us, k_det_wall 9.9 -> 6.6.)
 __device__ __forceinline__ void save_s0(const Dev &d, int c) {
-  for (int k = 0; k < 10; k++) d.S0[k * d.ncell + c] = d.S[k * d.ncell + c];
+  double v[10];
+  for (int k = 0; k < 10; k++) v[k] = d.S[k * d.ncell + c];
+  for (int k = 0; k < 10; k++) d.S0[k * d.ncell + c] = v[k];
 }
 // (the split path's; the one-pass paths save S0 where they form the cell
 // constants of the same cells: one launch, about 5 us, less per step)
@@ -659,9 +665,9 @@ __device__ __forceinline__ void cellpar_body(const Dev &d, P *cpar, int pstride,
                             d.S[7 * N + c], d.S[8 * N + c], cf, 1.0 / vol, vol, vol / d.dt + vol * cf,
                             d.ni1[g0] * d.si[g0], d.ni2[g0] * d.si[g0], d.ni1[gi] * d.si[gi], d.ni2[gi] * d.si[gi],
                             d.nj1[g0] * d.sj[g0], d.nj2[g0] * d.sj[g0], d.nj1[gj] * d.sj[gj], d.nj2[gj] * d.sj[gj]};
+  save_s0(d, c);
 #pragma unroll
   for (int k = 0; k < kNW; k++) o[k] = P(vals[k]);
-  save_s0(d, c);
 }
 template <typename P>
 __global__ void k_cellpar(Dev d, P *cpar, int pstride) {
@@ -2140,10 +2146,15 @@ __global__ void __launch_bounds__(256) k_moments(Dev d, T *__restrict__ FG, T *_
 __device__ __forceinline__ void det_wall_node(const Dev &d, const int *list, int n, double *swall, int t) {
   if (t >= n) return;
   const int cg = list[4 * t], ca = list[4 * t + 1], cb = list[4 * t + 2], so = list[4 * t + 3];
+  double a[10], b[10];  // every load before the first store, as in save_s0 (a ghost cell is no node's first or second)
   for (int k = 0; k < 10; k++) {
-    const double sw = (-d.S[k * d.ncell + cb] + 3.0 * d.S[k * d.ncell + ca]) * 0.5;
+    a[k] = d.S[k * d.ncell + ca];
+    b[k] = d.S[k * d.ncell + cb];
+  }
+  for (int k = 0; k < 10; k++) {
+    const double sw = (-b[k] + 3.0 * a[k]) * 0.5;
     swall[so + k] = sw;
-    d.S[k * d.ncell + cg] = 2.0 * sw - d.S[k * d.ncell + ca];
+    d.S[k * d.ncell + cg] = 2.0 * sw - a[k];
   }
 }
 
@@ -2151,37 +2162,39 @@ __global__ void k_det_wall(Dev d, const int *list, int n, double *swall) {
   det_wall_node(d, list, n, swall, (int)(blockIdx.x * blockDim.x + threadIdx.x));
 }
 
-// NS conservative variables of a cell in [0,nx]x[0,ny] from its S (corners: the
-// extrapolated one), src/Hybrid_Sub.f90:221-235; of any other cell, U as it is.
-// Fused multiply-adds are written out: every thread that needs a cell's value
-// forms the same bits.
+// Component k of S extrapolated to a corner of [0,nx]x[0,ny].
+__device__ __forceinline__ double corner_s(const Dev &d, int i, int j, int k) {
+  const int ii = i == 0 ? 1 : d.nx - 1, jj = j == 0 ? 1 : d.ny - 1, o = k * d.ncell;
+  return d.S[o + cidx(d, ii, j)] + d.S[o + cidx(d, i, jj)] - d.S[o + cidx(d, ii, jj)];
+}
+__device__ __forceinline__ bool corner(const Dev &d, int i, int j) {
+  return (i == 0 || i == d.nx) && (j == 0 || j == d.ny);
+}
 struct Cons { double u[4]; };
-__device__ __forceinline__ Cons cons_of(const Dev &d, int i, int j, bool store) {
-#pragma clang fp contract(off)
-  const int nx = d.nx, ny = d.ny, N = d.ncell, c = cidx(d, i, j);
+// What a cell's NS conservative variables are formed from: its S in
+// [0,nx]x[0,ny] (corners: the extrapolated one), U as it is outside.
+__device__ __forceinline__ Cons cons_in(const Dev &d, int i, int j) {
+  const double *src = i < 0 || i > d.nx || j < 0 || j > d.ny ? d.U : d.S;
+  const int c = cidx(d, i, j);
   Cons r;
-  if (i < 0 || i > nx || j < 0 || j > ny) {
-    for (int k = 0; k < 4; k++) r.u[k] = d.U[k * N + c];
-    return r;
-  }
-  double s[4];
-  if ((i == 0 || i == nx) && (j == 0 || j == ny)) {
-    const int ii = i == 0 ? 1 : nx - 1, jj = j == 0 ? 1 : ny - 1;
-    const int ca = cidx(d, ii, j), cb = cidx(d, i, jj), cc = cidx(d, ii, jj);
-    for (int k = 0; k < 11; k++) {
-      const double x = d.S[k * N + ca] + d.S[k * N + cb] - d.S[k * N + cc];
-      if (k < 4) s[k] = x;
-      if (store) d.S[k * N + c] = x;
-    }
-  } else {
-    for (int k = 0; k < 4; k++) s[k] = d.S[k * N + c];
-  }
+  for (int k = 0; k < 4; k++) r.u[k] = src[k * d.ncell + c];
+  return r;
+}
+// The conservative variables (src/Hybrid_Sub.f90:221-235) from that.  Fused
+// multiply-adds are written out: every thread that needs a cell's value forms the
+// same bits.
+__device__ __forceinline__ Cons cons_of(const Dev &d, int i, int j, Cons s) {
+#pragma clang fp contract(off)
+  if (i < 0 || i > d.nx || j < 0 || j > d.ny) return s;
+  if (corner(d, i, j))
+    for (int k = 0; k < 4; k++) s.u[k] = corner_s(d, i, j, k);
   const double sq = sqrt(2.0 / d.gamma);
-  const double tu = s[1] / d.ma * sq, tv = s[2] / d.ma * sq;
-  r.u[0] = s[0];
-  r.u[1] = s[0] * tu;
-  r.u[2] = s[0] * tv;
-  r.u[3] = fma(s[0] * d.cv, s[3], 0.5 * s[0] * fma(tu, tu, tv * tv));
+  const double tu = s.u[1] / d.ma * sq, tv = s.u[2] / d.ma * sq;
+  Cons r;
+  r.u[0] = s.u[0];
+  r.u[1] = s.u[0] * tu;
+  r.u[2] = s.u[0] * tv;
+  r.u[3] = fma(s.u[0] * d.cv, s.u[3], 0.5 * s.u[0] * fma(tu, tu, tv * tv));
   return r;
 }
 __device__ __forceinline__ Cons extrapolate(const Cons &a, const Cons &b) {
@@ -2197,24 +2210,26 @@ __device__ __forceinline__ Cons extrapolate(const Cons &a, const Cons &b) {
 // from the two cells inside it: the thread forms those cells' values itself,
 // at most four of them, so nothing waits for another thread), and the
 // primitive variables, with the T<0.1 stop of interior cells turned into an
-// error flag.  Bound by the latency of its loads: one launch of 10 us where
-// three took 15 (4 x 128 cells).
+// error flag.  Bound by the latency of its loads, so the four cells are loaded
+// together (away from the edges they are one cell) and the corners stored last:
+// 5.0 us at 128^2 cells, 10.4 with a wait for each cell and corner component.
 __device__ __forceinline__ void convert_cell(const Dev &d, int c) {
   if (c >= d.ncell) return;
   const int nx = d.nx, ny = d.ny, N = d.ncell;
   const int i = c % d.NI - 1, j = c / d.NI - 1;
-  // a cell after the extrapolation of the columns
-  auto columns = [&](int jj) {
-    if (i == 0) return extrapolate(cons_of(d, 1, jj, false), cons_of(d, 2, jj, false));
-    if (i == nx) return extrapolate(cons_of(d, nx - 1, jj, false), cons_of(d, nx - 2, jj, false));
-    return cons_of(d, i, jj, false);
-  };
-  if ((i == 0 || i == nx) && (j == 0 || j == ny)) (void)cons_of(d, i, j, true);  // S of the corner
-  Cons w;
-  if (j == 0) w = extrapolate(columns(1), columns(2));
-  else if (j == ny) w = extrapolate(columns(ny - 1), columns(ny - 2));
-  else w = columns(j);
-  if ((i >= 0 && i <= nx && j >= 0 && j <= ny) || i == 0 || i == nx || j == 0 || j == ny)
+  const bool ei = i == 0 || i == nx, ej = j == 0 || j == ny;
+  // the cell of the thread or the first one inside, and the second one
+  const int i1 = i == 0 ? 1 : i == nx ? nx - 1 : i, i2 = i == 0 ? 2 : i == nx ? nx - 2 : i;
+  const int j1 = j == 0 ? 1 : j == ny ? ny - 1 : j, j2 = j == 0 ? 2 : j == ny ? ny - 2 : j;
+  const Cons s11 = cons_in(d, i1, j1), s21 = cons_in(d, i2, j1), s12 = cons_in(d, i1, j2), s22 = cons_in(d, i2, j2);
+  Cons w = cons_of(d, i1, j1, s11);
+  if (ei) w = extrapolate(w, cons_of(d, i2, j1, s21));
+  if (ej) {
+    Cons x = cons_of(d, i1, j2, s12);
+    if (ei) x = extrapolate(x, cons_of(d, i2, j2, s22));
+    w = extrapolate(w, x);
+  }
+  if ((i >= 0 && i <= nx && j >= 0 && j <= ny) || ei || ej)
     for (int k = 0; k < 4; k++) d.U[k * N + c] = w.u[k];
   const double dd = w.u[0], u = w.u[1] / dd, v = w.u[2] / dd;
   const double T = (w.u[3] - 0.5 * dd * (u * u + v * v)) / (d.cv * dd);
@@ -2224,66 +2239,55 @@ __device__ __forceinline__ void convert_cell(const Dev &d, int c) {
   d.prim[3 * N + c] = T;
   d.prim[4 * N + c] = (1. / (d.gamma * d.ma * d.ma)) * dd * T;
   if (i >= 1 && i <= nx - 1 && j >= 1 && j <= ny - 1 && T < 0.10000000149011612) atomicOr(d.err, 1);
+  if (ei && ej) {  // S of the corner
+    double x[11];
+    for (int k = 0; k < 11; k++) x[k] = corner_s(d, i, j, k);
+    for (int k = 0; k < 11; k++) d.S[k * N + c] = x[k];
+  }
 }
 __global__ void k_convert(Dev d) { convert_cell(d, (int)(blockIdx.x * blockDim.x + threadIdx.x)); }
 
 // HoT of Convert_NS (src/Hybrid_Sub.f90:317-349 and :419-448): i-faces
 // (i=1..nx, j=1..ny-1) then j-faces (i=1..nx-1, j=1..ny), one thread each.
+// The S of both cells is loaded before anything is stored (see save_s0): 7.1 us at
+// 128^2 cells, 8.3 with loads between the stores.
 __device__ __forceinline__ void hot_face(const Dev &d, int t) {
   const int nx = d.nx, ny = d.ny, N = d.ncell;
   const int ni = nx * (ny - 1), nj = (nx - 1) * ny;
   if (t >= ni + nj) return;
-  const double *S = d.S;
+  const int dir = t < ni ? 0 : 1, tt = dir ? t - ni : t, row = dir ? nx - 1 : nx;
+  const int i = tt % row + 1, j = tt / row + 1;
+  const int c = cidx(d, i, j), cm = dir ? cidx(d, i, j - 1) : cidx(d, i - 1, j);
+  const bool first = (dir ? j : i) == 1, last = dir ? j == ny : i == nx;
+  double a[6], b[6];  // components 4..9 of the face's two cells
+  for (int k = 0; k < 6; k++) {
+    a[k] = d.S[(4 + k) * N + c];
+    b[k] = d.S[(4 + k) * N + cm];
+  }
   const double gm2 = d.gamma * (d.ma * d.ma);
-  // 1.4142135381698608 is sqrt(2.0) evaluated in REAL(4), as the reference does
+  const double qs = (d.ma * d.ma * d.ma) * pow(d.gamma, 1.5);
   double o[8];
-  if (t < ni) {
-    const int i = t % nx + 1, j = t / nx + 1;
-    ns_face(d, 0, i, j, o);
-    const int c = cidx(d, i, j), cm = cidx(d, i - 1, j);
-    double *tg = d.taoi, *qg = d.qi;
-    if (i != 1 && i != nx) {
-      const double tmp = (S[4 * N + c] + S[5 * N + c] + S[9 * N + c] + S[4 * N + cm] + S[5 * N + cm] + S[9 * N + cm]) / 6.0;
-      tg[0 * N + c] = -((S[4 * N + c] + S[4 * N + cm]) / 2.0 - tmp) / gm2 - o[0];
-      tg[1 * N + c] = -((S[5 * N + c] + S[5 * N + cm]) / 2.0 - tmp) / gm2 - o[1];
-      tg[2 * N + c] = -(S[6 * N + c] + S[6 * N + cm]) / 2.0 / gm2 - o[2];
-      tg[3 * N + c] = -((S[9 * N + c] + S[9 * N + cm]) / 2.0 - tmp) / gm2 - o[3];
-      qg[0 * N + c] = -(S[7 * N + cm] + S[7 * N + c]) / 2.0 * 1.4142135381698608 / ((d.ma * d.ma * d.ma) * pow(d.gamma, 1.5)) - o[4];
-      qg[1 * N + c] = -(S[8 * N + cm] + S[8 * N + c]) / 2.0 * 1.4142135381698608 / ((d.ma * d.ma * d.ma) * pow(d.gamma, 1.5)) - o[5];
-    } else {
-      const int cs = (i == 1) ? c : cm;
-      const double tmp = (S[4 * N + cs] + S[5 * N + cs] + S[9 * N + cs]) / 3.0;
-      tg[0 * N + c] = -(S[4 * N + cs] - tmp) / gm2 - o[0];
-      tg[1 * N + c] = -(S[5 * N + cs] - tmp) / gm2 - o[1];
-      tg[2 * N + c] = -S[6 * N + cs] / gm2 - o[2];
-      tg[3 * N + c] = -(S[9 * N + cs] - tmp) / gm2 - o[3];
-      qg[0 * N + c] = -S[7 * N + cs] * 1.4142135381698608 / ((d.ma * d.ma * d.ma) * pow(d.gamma, 1.5)) - o[4];
-      qg[1 * N + c] = -S[8 * N + cs] * 1.4142135381698608 / ((d.ma * d.ma * d.ma) * pow(d.gamma, 1.5)) - o[5];
-    }
+  ns_face(d, dir, i, j, o);
+  double *tg = dir ? d.taoj : d.taoi, *qg = dir ? d.qj : d.qi;
+  // 1.4142135381698608 is sqrt(2.0) evaluated in REAL(4), as the reference does
+  if (!first && !last) {
+    const double tmp = (a[0] + a[1] + a[5] + b[0] + b[1] + b[5]) / 6.0;
+    tg[0 * N + c] = -((a[0] + b[0]) / 2.0 - tmp) / gm2 - o[0];
+    tg[1 * N + c] = -((a[1] + b[1]) / 2.0 - tmp) / gm2 - o[1];
+    tg[2 * N + c] = -(a[2] + b[2]) / 2.0 / gm2 - o[2];
+    tg[3 * N + c] = -((a[5] + b[5]) / 2.0 - tmp) / gm2 - o[3];
+    qg[0 * N + c] = -(b[3] + a[3]) / 2.0 * 1.4142135381698608 / qs - o[4];
+    qg[1 * N + c] = -(b[4] + a[4]) / 2.0 * 1.4142135381698608 / qs - o[5];
   } else {
-    const int tt = t - ni;
-    const int i = tt % (nx - 1) + 1, j = tt / (nx - 1) + 1;
-    ns_face(d, 1, i, j, o);
-    const int c = cidx(d, i, j), cm = cidx(d, i, j - 1);
-    double *tg = d.taoj, *qg = d.qj;
-    if (j != 1 && j != ny) {
-      const double tmp = (S[4 * N + c] + S[5 * N + c] + S[9 * N + c] + S[4 * N + cm] + S[5 * N + cm] + S[9 * N + cm]) / 6.0;
-      tg[0 * N + c] = -((S[4 * N + c] + S[4 * N + cm]) / 2.0 - tmp) / gm2 - o[0];
-      tg[1 * N + c] = -((S[5 * N + c] + S[5 * N + cm]) / 2.0 - tmp) / gm2 - o[1];
-      tg[2 * N + c] = -(S[6 * N + c] + S[6 * N + cm]) / 2.0 / gm2 - o[2];
-      tg[3 * N + c] = -((S[9 * N + c] + S[9 * N + cm]) / 2.0 - tmp) / gm2 - o[3];
-      qg[0 * N + c] = -(S[7 * N + cm] + S[7 * N + c]) / 2.0 * 1.4142135381698608 / ((d.ma * d.ma * d.ma) * pow(d.gamma, 1.5)) - o[4];
-      qg[1 * N + c] = -(S[8 * N + cm] + S[8 * N + c]) / 2.0 * 1.4142135381698608 / ((d.ma * d.ma * d.ma) * pow(d.gamma, 1.5)) - o[5];
-    } else {
-      const int cs = (j == 1) ? c : cm;
-      const double tmp = (S[4 * N + cs] + S[5 * N + cs] + S[9 * N + cs]) / 3.0;
-      tg[0 * N + c] = -(S[4 * N + cs] - tmp) / gm2 - o[0];
-      tg[1 * N + c] = -(S[5 * N + cs] - tmp) / gm2 - o[1];
-      tg[2 * N + c] = -S[6 * N + cs] / gm2 - o[2];
-      tg[3 * N + c] = -(S[9 * N + cs] - tmp) / gm2 - o[3];
-      qg[0 * N + c] = -S[7 * N + cs] * 1.4142135381698608 / ((d.ma * d.ma * d.ma) * pow(d.gamma, 1.5)) - o[4];
-      qg[1 * N + c] = -S[8 * N + cs] * 1.4142135381698608 / ((d.ma * d.ma * d.ma) * pow(d.gamma, 1.5)) - o[5];
-    }
+    double e[6];  // the inner cell's
+    for (int k = 0; k < 6; k++) e[k] = first ? a[k] : b[k];
+    const double tmp = (e[0] + e[1] + e[5]) / 3.0;
+    tg[0 * N + c] = -(e[0] - tmp) / gm2 - o[0];
+    tg[1 * N + c] = -(e[1] - tmp) / gm2 - o[1];
+    tg[2 * N + c] = -e[2] / gm2 - o[2];
+    tg[3 * N + c] = -(e[5] - tmp) / gm2 - o[3];
+    qg[0 * N + c] = -e[3] * 1.4142135381698608 / qs - o[4];
+    qg[1 * N + c] = -e[4] * 1.4142135381698608 / qs - o[5];
   }
 }
 
