@@ -173,6 +173,12 @@ __global__ void k_save_s0(Dev d) {
 // One block per face node (the last node of the face is skipped, as in the
 // reference's icheck/jcheck test).
 // ------------------------------------------------------------------------
+// Bound by memory where the faces fill the chip, by latency where they do not:
+// a thread loads four velocities' values before it stores any (see save_s0), and
+// the first pass stores the outgoing ones only, the second the rest.  128^2 cells
+// x 64^2 velocities FP64: 26 us, 34 with one velocity at a time and the incoming
+// ones stored twice.
+constexpr int kWallAhead = 4;
 template <typename T>
 __device__ void wall_node(const Dev &d, const BcDev &b, int kk, T *FG, T *FH, T *slot) {
   int i, j, px, py, px1, py1, pos;
@@ -187,14 +193,18 @@ __device__ void wall_node(const Dev &d, const BcDev &b, int kk, T *FG, T *FH, T 
   const size_t c0 = (size_t)cidx(d, px, py) * d.nv, c1 = (size_t)cidx(d, px1, py1) * d.nv;
   const double tw = d.twall;
   // exp(-|c|^2/Tw) = exp(-cx^2/Tw) exp(-cy^2/Tw): nvi + nvj exponentials per
-  // face node, in LDS
-  __shared__ double ex[kMaxV1], ey[kMaxV1];
+  // face node, in LDS with the velocities and weights
+  __shared__ double ex[kMaxV1], ey[kMaxV1], sx[kMaxV1], sy[kMaxV1], wx[kMaxV1], wy[kMaxV1];
   for (int k = threadIdx.x; k < d.nvi; k += blockDim.x) {
     const double cx = d.vi[k] - b.uw;
+    wx[k] = d.wi[k];
+    sx[k] = cx;
     ex[k] = exp(-(cx * cx) / tw);
   }
   for (int k = threadIdx.x; k < d.nvj; k += blockDim.x) {
     const double cy = d.vj[k] - b.vw;
+    wy[k] = d.wj[k];
+    sy[k] = cy;
     ey[k] = exp(-(cy * cy) / tw);
   }
   __syncthreads();
@@ -204,31 +214,44 @@ __device__ void wall_node(const Dev &d, const BcDev &b, int kk, T *FG, T *FH, T 
   int first_in = 0x7fffffff;
   {
     int iv = (int)threadIdx.x % d.nvi, jv = (int)threadIdx.x / d.nvi;
-    for (int v = threadIdx.x; v < d.nv; v += blockDim.x) {
-      T outg, outh;
-      {
-        T f1 = FG[c0 + v], f2 = FG[c1 + v];
-        T t = (-f2 + T(3) * f1) * T(0.5);
-        if (t <= T(0)) t = f1;
-        if (t >= T(1.5) * f1) t = T(1.5) * f1;
-        outg = t;
-        f1 = FH[c0 + v]; f2 = FH[c1 + v];
-        t = (-f2 + T(3) * f1) * T(0.5);
-        if (t <= T(0)) t = f1;
-        if (t >= T(1.5) * f1) t = T(1.5) * f1;
-        outh = t;
+    for (int v0 = threadIdx.x; v0 < d.nv; v0 += kWallAhead * blockDim.x) {
+      T f[kWallAhead][4];
+#pragma unroll
+      for (int q = 0; q < kWallAhead; q++) {
+        const int v = min(v0 + q * (int)blockDim.x, d.nv - 1);
+        f[q][0] = FG[c0 + v];
+        f[q][1] = FG[c1 + v];
+        f[q][2] = FH[c0 + v];
+        f[q][3] = FH[c1 + v];
       }
-      slot[slot_idx(d, b.face, pos, 0, v)] = outg;
-      slot[slot_idx(d, b.face, pos, 1, v)] = outh;
-      const double w = d.wi[iv] * d.wj[jv];
-      const double cx = d.vi[iv] - b.uw, cy = d.vj[jv] - b.vw;
-      const double vnw = (cx * swnx + cy * swny) * st;
-      const double vnn = (vnw - fabs(vnw)) / 2.;
-      acc[0] += w * (vnn * (double)outg);
-      acc[1] += w * ((vnw + fabs(vnw)) / 2. * (ex[iv] * ey[jv]) / (kPi * tw));
-      if (vnw >= 0.0) first_in = min(first_in, v);
-      iv += di; jv += dj;
-      if (iv >= d.nvi) { iv -= d.nvi; jv += 1; }
+#pragma unroll
+      for (int q = 0; q < kWallAhead; q++) {
+        const int v = v0 + q * (int)blockDim.x;
+        if (v < d.nv) {
+          T out[2];
+#pragma unroll
+          for (int ird = 0; ird < 2; ird++) {
+            const T f1 = f[q][2 * ird], f2 = f[q][2 * ird + 1];
+            T t = (-f2 + T(3) * f1) * T(0.5);
+            if (t <= T(0)) t = f1;
+            if (t >= T(1.5) * f1) t = T(1.5) * f1;
+            out[ird] = t;
+          }
+          const double w = wx[iv] * wy[jv];
+          const double vnw = (sx[iv] * swnx + sy[jv] * swny) * st;
+          const double vnn = (vnw - fabs(vnw)) / 2.;
+          acc[0] += w * (vnn * (double)out[0]);
+          acc[1] += w * ((vnw + fabs(vnw)) / 2. * (ex[iv] * ey[jv]) / (kPi * tw));
+          if (vnw >= 0.0) {
+            first_in = min(first_in, v);
+          } else {
+            slot[slot_idx(d, b.face, pos, 0, v)] = out[0];
+            slot[slot_idx(d, b.face, pos, 1, v)] = out[1];
+          }
+          iv += di; jv += dj;
+          if (iv >= d.nvi) { iv -= d.nvi; jv += 1; }
+        }
+      }
     }
   }
   block_sum<2>(acc);
@@ -237,8 +260,7 @@ __device__ void wall_node(const Dev &d, const BcDev &b, int kk, T *FG, T *FH, T 
   {
     int iv = (int)threadIdx.x % d.nvi, jv = (int)threadIdx.x / d.nvi;
     for (int v = threadIdx.x; v < d.nv; v += blockDim.x) {
-      const double cx = d.vi[iv] - b.uw, cy = d.vj[jv] - b.vw;
-      const double vnw = (cx * swnx + cy * swny) * st;
+      const double vnw = (sx[iv] * swnx + sy[jv] * swny) * st;
       if (vnw >= 0.0) {
         // the reference clamps a negative wall density only after its first use
         // (src/GKUA_wall_functions.f90:52-54)
