@@ -549,7 +549,8 @@ int gsis_mlp_create(gsis_mlp **out) {
   }
   for (int k = 0; k < kMlpIn; k++) d.scale[kMlpIn + k] = 1.0f;
   for (int k = 0; k < kMlpOut; k++) d.scale[2 * kMlpIn + kMlpOut + k] = 1.0f;
-  if (hipMemcpy(d.dscale, d.scale, sizeof(d.scale), hipMemcpyHostToDevice) != hipSuccess)
+  // on the network's stream, behind the clear of the same memory
+  if (hipMemcpyAsync(d.dscale, d.scale, sizeof(d.scale), hipMemcpyHostToDevice, d.s) != hipSuccess)
     return bail(mfail(GSIS_EHIP, "mlp: scaling upload failed"));
   pack(d);
   if ((rc = sync(d))) return bail(rc);
