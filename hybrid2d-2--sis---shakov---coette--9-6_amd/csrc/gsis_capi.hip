@@ -110,20 +110,57 @@ int dalloc(gsis_handle *h, P **ptr, size_t bytes) {
   return 0;
 }
 
-// Device memory to the caller's, after what the handle's stream holds.  Short
-// reads go through pinned memory of the handle's own: 100 KB take 12 us there,
-// 53 us straight into pageable memory.  Long ones go in pieces of 960 KB, the
-// longest that the runtime does not pin page by page: 1.03 MB 60 against 81 us,
-// 6 MB 314 against 362.
-constexpr size_t kPinBytes = (size_t)64 << 10, kPieceBytes = (size_t)960 << 10;
+// Device memory to the caller's, after what the handle's stream holds, with one
+// wait for several reads.  A read of up to 512 KB goes through pinned memory of
+// the handle's own: the runtime's copies into pageable memory take 27 us at 16 KB,
+// 47 at 64 KB and 84 at 160 KB, and 29-43 from 190 to 512 KB if it knows the
+// pages (pinning new ones takes about 200); through pinned memory it is 15, 22, 26
+// and 27-40.  Longer ones go in pieces of 960 KB, the longest that the runtime
+// does not pin page by page: 1.03 MB 60 against 81 us, 6 MB 314 against 362.
+// All fields of 30 x 30 cells: 91 us, 234 with a wait per field and pinned memory
+// up to 64 KB only; 60 x 60: 158, 266; 100 x 100: 299, 382.
+constexpr size_t kShortRead = (size_t)512 << 10, kPinBytes = (size_t)1024 << 10, kPieceBytes = (size_t)960 << 10;
+struct Reads {
+  gsis_handle *h;
+  size_t used = 0;  // of the pinned memory
+  int n = 0;
+  struct { void *dst; size_t at, bytes; } short_[16];
+  explicit Reads(gsis_handle *handle) : h(handle) {}
+  // a place of the pinned memory for what goes to dst; nullptr: a long read
+  char *place(void *dst, size_t bytes, int *rc) {
+    *rc = 0;
+    if (!h->pin || bytes > kShortRead) return nullptr;
+    if ((used + bytes > kPinBytes || n == 16) && (*rc = wait())) return nullptr;
+    short_[n++] = {dst, used, bytes};
+    char *at = h->pin + used;
+    used += (bytes + 63) / 64 * 64;
+    return at;
+  }
+  int add(void *dst, const void *src, size_t bytes) {
+    int rc;
+    char *at = place(dst, bytes, &rc);
+    if (rc) return rc;
+    if (at) {
+      HIPCHK(hipMemcpyAsync(at, src, bytes, hipMemcpyDeviceToHost, h->s));
+      return 0;
+    }
+    for (size_t o = 0; o < bytes; o += kPieceBytes)
+      HIPCHK(hipMemcpyAsync((char *)dst + o, (const char *)src + o, std::min(kPieceBytes, bytes - o),
+                            hipMemcpyDeviceToHost, h->s));
+    return 0;
+  }
+  int wait() {
+    HIPCHK(hipStreamSynchronize(h->s));
+    for (int k = 0; k < n; k++) std::memcpy(short_[k].dst, h->pin + short_[k].at, short_[k].bytes);
+    used = 0;
+    n = 0;
+    return 0;
+  }
+};
 int fetch(gsis_handle *h, void *dst, const void *src, size_t bytes) {
-  const bool pinned = h->pin && bytes <= kPinBytes;
-  for (size_t o = 0; o < bytes; o += kPieceBytes)
-    HIPCHK(hipMemcpyAsync((pinned ? h->pin : (char *)dst) + o, (const char *)src + o, std::min(kPieceBytes, bytes - o),
-                          hipMemcpyDeviceToHost, h->s));
-  HIPCHK(hipStreamSynchronize(h->s));
-  if (pinned) std::memcpy(dst, h->pin, bytes);
-  return 0;
+  Reads r(h);
+  const int rc = r.add(dst, src, bytes);
+  return rc ? rc : r.wait();
 }
 
 // every seam message not written (as before a handle's first step)
@@ -1063,9 +1100,14 @@ int gsis_download_macro(gsis_handle *h, double *s, double *s0, double *cf, doubl
   const size_t N = d.ncell;
   int rc = check_err_flag(h);
   // the caller's layout is formed on the device, in the handle's stage
+  Reads reads(h);
   auto get = [&](const double *dev, int ncomp, int nf, int nx1, int ny1, int o, double *out) -> int {
-    gsis::launch_fields_out(d, dev, ncomp, nf, nx1, ny1, o, h->stage, h->s);
-    return fetch(h, out, h->stage, sizeof(double) * nf * nx1 * ny1);
+    const size_t bytes = sizeof(double) * nf * nx1 * ny1;
+    int e;
+    double *at = reinterpret_cast<double *>(reads.place(out, bytes, &e));
+    if (e) return e;
+    gsis::launch_fields_out(d, dev, ncomp, nf, nx1, ny1, o, at ? at : h->stage, h->s);
+    return at ? 0 : reads.add(out, h->stage, bytes);
   };
   auto get_s = [&](const double *dev, int ncomp, double *out) {
     return get(dev, ncomp, 11, d.nx + 7, d.ny + 7, 2, out);
@@ -1074,13 +1116,14 @@ int gsis_download_macro(gsis_handle *h, double *s, double *s0, double *cf, doubl
   int r2 = 0;
   if (s && (r2 = get_s(d.S, 11, s))) return r2;
   if (s0 && (r2 = get_s(d.S0, 10, s0))) return r2;
-  if (cf) HIPCHK(hipMemcpy(cf, d.CF, 8 * N, hipMemcpyDeviceToHost));
+  if (cf && (r2 = reads.add(cf, d.CF, 8 * N))) return r2;
   if (u && (r2 = get_v(d.U, 4, u))) return r2;
   if (taonsi_g && (r2 = get_v(d.taoi, 4, taonsi_g))) return r2;
   if (taonsj_g && (r2 = get_v(d.taoj, 4, taonsj_g))) return r2;
   if (qi_g && (r2 = get_v(d.qi, 2, qi_g))) return r2;
   if (qj_g && (r2 = get_v(d.qj, 2, qj_g))) return r2;
-  if (swall && h->swall_len > 0) HIPCHK(hipMemcpy(swall, h->swall, 8 * (size_t)h->swall_len, hipMemcpyDeviceToHost));
+  if (swall && h->swall_len > 0 && (r2 = reads.add(swall, h->swall, 8 * (size_t)h->swall_len))) return r2;
+  if ((r2 = reads.wait())) return r2;
   return rc;
 }
 

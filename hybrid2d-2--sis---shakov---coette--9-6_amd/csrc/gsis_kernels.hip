@@ -2763,10 +2763,10 @@ void launch_mass_correct(const Dev &d, double *work, double init, hipStream_t s)
 }
 // Macroscopic fields as the caller's arrays hold them: nf components per cell,
 // consecutive, over nx1 x ny1 cells of which the padded cell (-1,-1) is the
-// cell (o,o), zero elsewhere and beyond the ncomp components there are.  The
-// host then copies once into the caller's array; it used to copy a plane-major
-// array, clear the caller's and scatter into it (256 x 256 cells, 11 components:
-// 0.98 -> 0.42 ms).
+// cell (o,o), zero elsewhere and beyond the ncomp components there are; out may
+// be pinned host memory.  The host then copies once into the caller's array; it
+// used to copy a plane-major array, clear the caller's and scatter into it
+// (256 x 256 cells, 11 components: 0.98 -> 0.42 ms).
 __global__ void __launch_bounds__(256) k_fields_out(Dev d, const double *__restrict__ src, int ncomp, int nf, int nx1,
                                                     int ny1, int o, double *__restrict__ out) {
   const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x, q = t / nf;

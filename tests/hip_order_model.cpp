@@ -6,7 +6,8 @@
 //    to have ended, also writes;
 //  * launches whose workgroups wait for each other (the synthetic solve's inner
 //    loops) that another such launch may run beside;
-//  * fills captured into a graph.
+//  * fills captured into a graph;
+// and notes the shortest copy to host memory that is not pinned.
 // Loaded with RTLD_GLOBAL before the library, so that it takes the runtime's place.
 #include <sys/mman.h>
 
@@ -40,6 +41,8 @@ std::vector<Done> gangs;
 std::vector<Launch> launches;
 std::map<const void *, std::string> kernels;
 std::map<void *, size_t> sizes;
+std::map<char *, size_t> pinned;
+size_t shortest_pageable = SIZE_MAX;
 int races = 0, beside = 0, captured_fills = 0, cus = 256;
 struct Config { Dim3 g, b; size_t sh; void *s; };
 thread_local Config config;
@@ -87,6 +90,7 @@ int model_races() { return races; }
 int model_beside() { return beside; }
 int model_captured_fills() { return captured_fills; }
 void model_set_cus(int n) { cus = n; }
+size_t model_shortest_pageable_read() { return shortest_pageable; }
 // launches of the kernels whose name contains part; the last one's workgroups
 int model_launches(const char *part, int *workgroups) {
   int n = 0;
@@ -127,14 +131,19 @@ int hipFree(void *p) {
   munmap(p, sizes[p]);
   return 0;
 }
-int hipHostMalloc(void **p, size_t n, unsigned) { *p = malloc(n); return 0; }
-int hipHostFree(void *p) { free(p); return 0; }
+int hipHostMalloc(void **p, size_t n, unsigned) { LOCK; *p = malloc(n); pinned[(char *)*p] = n; return 0; }
+int hipHostFree(void *p) { LOCK; pinned.erase((char *)p); free(p); return 0; }
 int hipMemset(void *p, int, size_t n) { LOCK; write(p, n, nullptr); return 0; }
 int hipMemsetD32(void *p, int, size_t n) { LOCK; write(p, 4 * n, nullptr); return 0; }
 int hipMemsetAsync(void *p, int, size_t n, void *s) { LOCK; write(p, n, s); return 0; }
 static int copy(void *dst, size_t n, int kind, const void *s) {
   LOCK;
-  if (kind == 2) { memset(dst, 0, n); (void)issue(s); }  // to the host: zeros
+  if (kind == 2) {  // to the host: zeros
+    auto p = pinned.upper_bound((char *)dst);
+    if (p == pinned.begin() || (char *)dst + n > (--p)->first + p->second) shortest_pageable = std::min(shortest_pageable, n);
+    memset(dst, 0, n);
+    (void)issue(s);
+  }
   else write(dst, n, s);
   return 0;
 }

@@ -50,3 +50,18 @@ net.train(x, x[:, :5], 1, 64)
 print(model.model_races())
 """)
     assert out == ["0", "0"]
+
+
+@pytest.mark.parametrize("cells", [6, 19, 20, 30, 40, 58])
+def test_short_reads_go_through_pinned_memory(run, cells):
+    """The runtime's own way into pageable memory takes up to three times as long between 64 and 190 KB."""
+    out = run(f"""
+from gsis_amd import solver
+s = solver.GsisSolver(g.cases.cavity_case({cells}, 6, kn=0.2))
+s.macro()
+s.counters()
+model.model_shortest_pageable_read.restype = ctypes.c_size_t
+print(model.model_shortest_pageable_read(), model.model_races())
+""")
+    assert int(out[0]) > 190 << 10
+    assert out[1] == "0"
