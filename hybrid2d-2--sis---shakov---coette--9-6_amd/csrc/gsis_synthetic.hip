@@ -1427,9 +1427,12 @@ int synthetic_run(const Dev &d, SyntheticState &st, int k0, int kstop, hipStream
 
 bool synthetic_batchable(const SyntheticState &st) { return st.on && st.rs <= 4 * kBand; }
 
-// Flux workgroups per instance: as many tiles each as keep the whole batch
-// resident, but at most kBatchTiles (a tile takes about 4 us, a sweep that
-// its fluxes run beside 50-200 us).
+// Flux workgroups per instance: the fewest tiles each with which the whole batch
+// is resident at once, but at most kBatchTiles (a tile takes about 4 us, a sweep
+// that its fluxes run beside 50-200 us); beyond that the last gangs start when
+// earlier ones have ended.  A gang has at most half of the device's workgroups,
+// however many tiles its mesh has: it has to be resident as a whole, and what
+// other streams run beside it has to find room on every XCD while it gathers.
 int synthetic_batch_layout(std::vector<NsJob> &jobs) {
   constexpr int kBatchTiles = 16;
   int dev = 0, ncu = 0, per = 0;
@@ -1441,11 +1444,12 @@ int synthetic_batch_layout(std::vector<NsJob> &jobs) {
     g_syn_err = "synthetic solve: occupancy query of the batched launch failed";
     return -1;
   }
+  const int most = ncu * per / 2;  // workgroups of a gang
   for (int tiles = 1;; tiles++) {
     int at = 0;
     for (NsJob &j : jobs) {
       const int nt = j.st.ntx * j.st.nty;
-      j.st.nflux = (nt + tiles - 1) / tiles;
+      j.st.nflux = std::max(1, std::min((nt + tiles - 1) / tiles, most - j.st.nw));
       j.st.stride = 8 * (j.st.nw - 1) + 1 <= j.st.nw + j.st.nflux ? 8 : 1;
       j.wg0 = at;
       j.blocks = ns_blocks(j.st);

@@ -65,3 +65,43 @@ print(model.model_shortest_pageable_read(), model.model_races())
 """)
     assert int(out[0]) > 190 << 10
     assert out[1] == "0"
+
+
+BATCH = """
+import importlib, math
+import numpy as np
+from gsis_amd import solver
+batch = importlib.import_module("gsis_amd.batch")
+def box(cells_i, cells_j, bent=False):
+    c = g.cases
+    nx, ny = cells_i + 1, cells_j + 1
+    x, y = np.meshgrid(np.linspace(0.0, 1.0, nx), np.linspace(0.0, 1.0, ny), indexing="ij")
+    if bent:
+        x, y = x + 0.2 * y, y + 0.03 * np.sin(math.pi * x)
+    bcs = [c.BC(2, 1, nx, 1, 1, -2), c.BC(3, nx, nx, 1, ny, -2), c.BC(4, 1, nx, ny, ny, -2, 0.1, 0.0),
+           c.BC(1, 1, 1, 1, ny, -2)]
+    v, w = c.sinh_velocity_grid(4, 6.0)
+    return c.Case("box", c.build_mesh(x, y, bcs), bcs, v, w, v.copy(), w.copy(), c.constants_from_kn(0.1, dt=0.05), "rest")
+def gang(case):
+    s = solver.GsisSolver(case, mode=1)
+    b = batch.Batch([s])
+    b.set_ns_graph(1)
+    n = ctypes.c_int()
+    print(b.ns_graph(), model.model_launches(b"k_ns_batch", ctypes.byref(n)) > 0, n.value)
+"""
+
+
+@pytest.mark.parametrize("cus", [256, 64, 32])
+def test_a_batched_instance_never_needs_more_workgroups_than_fit_beside_others(run, cus):
+    """The workgroups of an instance in a batched launch wait for each other, so all have to be
+    resident: at most half of the device's, at any size of the mesh."""
+    out = run(BATCH + f"""
+model.model_set_cus({cus})
+for i, j in ((5, 5), (64, 64), (128, 69), (700, 260), (2100, 260), (4700, 100), (12, 260)):
+    gang(box(i, j, i % 3 == 0))
+""")
+    rows = [out[k:k + 3] for k in range(0, len(out), 3)]
+    assert len(rows) == 7
+    for in_graph, launched, workgroups in rows:
+        assert (in_graph, launched) == ("1", "True")
+        assert 1 < int(workgroups) <= cus // 2
