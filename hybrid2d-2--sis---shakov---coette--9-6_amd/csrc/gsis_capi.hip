@@ -698,7 +698,8 @@ int batch_replay(gsis_batch *b, int nsteps) {
     m1 = m1 || (b->hs[q]->p.mode == GSIS_MODE_M1 && !b->in_graph[q]);
   }
   for (int k = 0; k < nsteps; k++) {
-    HIPCHK(hipGraphLaunch(b->exec, b->s));
+    auto launch = [&] { return hipGraphLaunch(b->exec, b->s); };
+    HIPCHK(b->nns > 0 ? gsis::ns_turn(b->s, launch) : launch());
     if (!m1) continue;
     // the synthetic solve of each other M1 instance after the captured part
     // of its step (a cooperative launch, or the closure's host-side loop)

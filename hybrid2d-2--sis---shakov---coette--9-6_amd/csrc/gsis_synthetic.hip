@@ -44,6 +44,8 @@
 // sweep (the flux of the first tile).
 #include <algorithm>
 #include <cstring>
+#include <functional>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -1196,11 +1198,14 @@ __global__ void __launch_bounds__(kThreads) k_ns_loop(Dev d, SyntheticState st) 
 
 // The inner loops of a batch of instances in one launch: job J has the
 // workgroups J.wg0 .. J.wg0 + J.blocks - 1, a gang.  The workgroups of a gang
-// wait for each other, so all of them have to be resident: gangs are
-// consecutive and workgroups are dispatched in order, so only the gang at the
-// dispatch front can be incomplete, and it is completed as the gangs before it
-// end (no gang waits for another).  A gang starts once its last workgroup has
-// arrived; that wait alone may take as long as the gangs before it.
+// wait for each other, so all of them have to be resident.  Workgroups go to the
+// eight XCDs in turn and each XCD starts its share in order, so of the first gang
+// that is not complete a missing workgroup waits only for lower-numbered ones of
+// its XCD: those of earlier gangs, which are complete and end, and its own
+// gang's, which leave room (synthetic_batch_layout: at most half of the device's
+// workgroups).  The launch has no such launch beside it (ns_turn).  A gang
+// starts once its last workgroup has arrived; that wait alone may take as long
+// as the gangs before it.
 __global__ void __launch_bounds__(kThreads) k_ns_batch(const NsJob *__restrict__ jobs, int njobs) {
   __shared__ __align__(16) char lds[LoopShared<false>::kBytes];
   int lo = 0, hi = njobs - 1;
@@ -1269,6 +1274,33 @@ __global__ void k_ns_resume(Dev d, SyntheticState st, int k0) {
     st.iters[2] = 0;
   }
   clear_hands(d, st, t, (size_t)gridDim.x * blockDim.x);
+}
+
+// Launches whose workgroups wait for each other (k_ns_loop, k_ns_batch) take turns
+// on a device, whatever streams and threads they come from: two that gather at
+// the same time could each hold workgroup slots that the other needs, until the
+// waits run out.  A launch's stream waits for the launch before it; nothing waits
+// on the host.  Other kernels run beside them.
+namespace {
+struct Turn {
+  std::mutex mu;
+  hipEvent_t last = nullptr;  // recorded behind the device's last such launch
+};
+constexpr int kMaxDevices = 64;
+Turn g_turn[kMaxDevices];
+}  // namespace
+hipError_t ns_turn(hipStream_t s, const std::function<hipError_t()> &launch) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
+  Turn &t = g_turn[dev];
+  std::lock_guard<std::mutex> lock(t.mu);
+  if (t.last) e = hipStreamWaitEvent(s, t.last, 0);
+  else e = hipEventCreateWithFlags(&t.last, hipEventDisableTiming);
+  if (e == hipSuccess) e = launch();
+  if (e == hipSuccess) e = hipEventRecord(t.last, s);
+  return e;
 }
 
 // the degenerate loop of a mesh without swept cells: max |Res_4| over no
@@ -1413,8 +1445,9 @@ int synthetic_run(const Dev &d, SyntheticState &st, int k0, int kstop, hipStream
     ss.k0 = k0;
     ss.kstop = kstop;
     void *args[] = {&dd, &ss};
-    const hipError_t e =
-        hipLaunchCooperativeKernel(ns_loop_kernel(st), dim3(ns_blocks(st)), dim3(kThreads), args, 0, s);
+    const hipError_t e = ns_turn(s, [&] {
+      return hipLaunchCooperativeKernel(ns_loop_kernel(st), dim3(ns_blocks(st)), dim3(kThreads), args, 0, s);
+    });
     if (e != hipSuccess) {
       g_syn_err = std::string("synthetic solve: cooperative launch failed: ") + hipGetErrorString(e);
       return GSIS_EHIP;

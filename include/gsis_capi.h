@@ -324,7 +324,12 @@ int gsis_fill_frd_uniform(gsis_handle *h, const double *g, const double *hv);
  * must share precision, flux scheme and device, and fit the
  * column-pair kernel.  A batch step keeps no kinetic RHS (gsis_residual
  * reports the last one a gsis_step kept).  The handles must not be stepped
- * on their own while a gsis_batch_step runs; they may be between calls. */
+ * on their own while a gsis_batch_step runs; they may be between calls.
+ * Batches and handles may step on different threads at the same time: the
+ * launches whose workgroups wait for each other (the synthetic solves, of a
+ * handle or of a batch) then take turns on the device.  Those of another
+ * process on the same GPU are not ordered with them: give each process a GPU of
+ * its own. */
 typedef struct gsis_batch gsis_batch;
 int gsis_batch_create(gsis_handle *const *hs, int32_t n, gsis_batch **out);
 int gsis_batch_step(gsis_batch *b, int32_t nsteps);

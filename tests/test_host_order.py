@@ -105,3 +105,28 @@ for i, j in ((5, 5), (64, 64), (128, 69), (700, 260), (2100, 260), (4700, 100), 
     for in_graph, launched, workgroups in rows:
         assert (in_graph, launched) == ("1", "True")
         assert 1 < int(workgroups) <= cus // 2
+
+
+def test_launches_whose_workgroups_wait_for_each_other_take_turns(run):
+    """A handle's inner loop and a batch's gangs, on streams and threads of their own: no two may run
+    at once, as each could hold workgroup slots that the other waits for."""
+    out = run(BATCH + """
+import threading
+def handle(n):
+    return solver.GsisSolver(box(n, n + 1), mode=1, kstep_show=1 << 30)
+a, b = handle(20), handle(30)
+for _ in range(3):
+    a.step(1)
+    b.step(2)
+print(model.model_beside())
+both = [batch.Batch([handle(10 + k) for k in range(4)]) for _ in range(2)]
+assert all(x.ns_graph() == 4 for x in both)
+a.step(1)
+both[0].step(1)
+print(model.model_beside())
+ts = [threading.Thread(target=x.step, args=(500,)) for x in both + [a]]
+for t in ts: t.start()
+for t in ts: t.join()
+print(model.model_beside(), model.model_captured_fills(), model.model_races())
+""")
+    assert out == ["0", "0", "0", "0", "0"]
