@@ -518,6 +518,7 @@ struct gsis_batch {
   int ns_graph = -1;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
+  hipEvent_t done[2] = {};  // the ends of the last two steps queued
   std::vector<void *> allocs;
 };
 
@@ -698,8 +699,15 @@ int batch_replay(gsis_batch *b, int nsteps) {
     m1 = m1 || (b->hs[q]->p.mode == GSIS_MODE_M1 && !b->in_graph[q]);
   }
   for (int k = 0; k < nsteps; k++) {
-    auto launch = [&] { return hipGraphLaunch(b->exec, b->s); };
-    HIPCHK(b->nns > 0 ? gsis::ns_turn(b->s, launch) : launch());
+    if (b->nns == 0) {
+      HIPCHK(hipGraphLaunch(b->exec, b->s));
+    } else {
+      // at most two steps queued: others that take turns with them (ns_turn) wait
+      // for what is queued, and a step of milliseconds is enough to queue the next behind
+      if (k >= 2) HIPCHK(hipEventSynchronize(b->done[k & 1]));
+      HIPCHK(gsis::ns_turn(b->s, [&] { return hipGraphLaunch(b->exec, b->s); }));
+      HIPCHK(hipEventRecord(b->done[k & 1], b->s));
+    }
     if (!m1) continue;
     // the synthetic solve of each other M1 instance after the captured part
     // of its step (a cooperative launch, or the closure's host-side loop)
@@ -1276,6 +1284,9 @@ int gsis_batch_create(gsis_handle *const *hs, int32_t n, gsis_batch **out) {
   };
   if (hipStreamCreateWithFlags(&b->s, hipStreamNonBlocking) != hipSuccess)
     return bail(fail(GSIS_EHIP, "batch: hipStreamCreate failed"));
+  for (hipEvent_t &e : b->done)
+    if (hipEventCreateWithFlags(&e, hipEventDisableTiming) != hipSuccess)
+      return bail(fail(GSIS_EHIP, "batch: hipEventCreate failed"));
   const size_t jb = (size_t)n * std::max(sizeof(gsis::StripJob<double>), sizeof(gsis::StripJob<float>));
   if (!alloc(&b->djobs, jb) || !alloc((void **)&b->err, 64)) return bail(fail(GSIS_EHIP, "batch: allocation failed"));
   const int rc = batch_capture_any(b);
@@ -1378,6 +1389,8 @@ int gsis_batch_destroy(gsis_batch *b) {
   if (b->s) (void)hipStreamSynchronize(b->s);
   batch_drop_graph(b);
   for (void *q : b->allocs) (void)hipFree(q);
+  for (hipEvent_t e : b->done)
+    if (e) (void)hipEventDestroy(e);
   if (b->s) (void)hipStreamDestroy(b->s);
   delete b;
   return 0;

@@ -43,7 +43,7 @@ std::map<const void *, std::string> kernels;
 std::map<void *, size_t> sizes;
 std::map<char *, size_t> pinned;
 size_t shortest_pageable = SIZE_MAX;
-int races = 0, beside = 0, captured_fills = 0, cus = 256;
+int races = 0, beside = 0, captured_fills = 0, queued = 0, cus = 256;
 struct Config { Dim3 g, b; size_t sh; void *s; };
 thread_local Config config;
 
@@ -69,8 +69,12 @@ void write(void *dst, size_t n, const void *s) {
 }
 void gang(const void *s) {
   const Done me = issue(s);
-  for (const Done &g : gangs)
+  int ahead = 1;
+  for (const Done &g : gangs) {
     if (!ended_before(g, me)) beside++;
+    ahead += host[g.stream] < g.op;
+  }
+  queued = std::max(queued, ahead);
   gangs.push_back(me);
 }
 void launch(const void *f, Dim3 g, const void *s) {
@@ -89,6 +93,7 @@ extern "C" {
 int model_races() { return races; }
 int model_beside() { return beside; }
 int model_captured_fills() { return captured_fills; }
+int model_queued() { return queued; }  // of those launches, the most that the host did not know to have ended
 void model_set_cus(int n) { cus = n; }
 size_t model_shortest_pageable_read() { return shortest_pageable; }
 // launches of the kernels whose name contains part; the last one's workgroups

@@ -130,3 +130,15 @@ for t in ts: t.join()
 print(model.model_beside(), model.model_captured_fills(), model.model_races())
 """)
     assert out == ["0", "0", "0", "0", "0"]
+
+
+def test_a_batch_leaves_turns_to_others(run):
+    """A batch's call of many steps queues two at a time, so that another thread's solve waits for
+    two steps and not for all of them."""
+    out = run(BATCH + """
+b = batch.Batch([solver.GsisSolver(box(10 + k, 12), mode=1, kstep_show=1 << 30) for k in range(4)])
+b.step(50)
+b.step(1)
+print(b.ns_graph(), model.model_queued())
+""")
+    assert out[0] == "4" and 1 <= int(out[1]) <= 2
