@@ -583,6 +583,7 @@ int batch_jobs(gsis_batch *b) {
       j.R = (T *)h->RG;
       j.slot = (const T *)h->slot;
       j.msg = (T *)h->strip.msg;
+      j.next = h->strip.next;
       j.oflags = h->strip.oflags;
       j.wall_list = h->wall_list;
       j.swall = h->swall;
@@ -926,6 +927,7 @@ int gsis_create(const gsis_params *p, gsis_handle **out) {
       if (!strip_clear(h)) return cleanup(fail(GSIS_EHIP, "seam buffer fill failed"));
     }
     sb.err = d.err + 1;
+    if ((rc = dalloc(h, &sb.next, gsis::strip_counters(d) * sizeof(int)))) return cleanup(rc);
   }
   if (p->mode == GSIS_MODE_M1) {
     rc = gsis::synthetic_init(h->d, *p, h->syn);

@@ -49,7 +49,7 @@ struct Dev {
   double *qi, *qj;      // [2][ncell]
   double *prim;  // [5][ncell]: d, u, v, T, p  (comput_duvtpckw)
   double *res4;  // [4][ncell]: velocity moments of the kinetic RHS per cell
-  int *err;      // [0]: T<0.1 flag
+  int *err;      // [0]: T<0.1 flag, [1]: a strip's wait timed out
   const uint8_t *ovrI1, *ovrI3;  // per row j: wall/farfield override on i-face 1 / nx
   const uint8_t *ovrJ2, *ovrJ4;  // per column i: override on j-face 1 / ny
 };

@@ -31,11 +31,13 @@ constexpr int kNCellPar = 20;  // per-cell constants of the fused kinetic kernel
 template <typename T> bool launch_walk(const Dev &d, double *cpar, T *F, const T *slot, T *R, int store_rhs, int tiles, hipStream_t s);
 // Buffers of the column-pair kernel (k_strip): seam messages
 // [seam][tile][row][4][64] (elements of the working precision), every word
-// strip_empty_word() outside a launch, and a word set when a wait for a
-// message timed out.
+// strip_empty_word() outside a launch, a word set when a wait for a message timed
+// out, and a counter per tile (strip_counters of them) that the tile's workgroups
+// draw their strips from.
+constexpr int kNextStride = 16;  // words from one tile's counter to the next
 struct StripBufs {
   void *msg = nullptr;
-  int *err = nullptr;
+  int *err = nullptr, *next = nullptr;
   // face-override words: ny+2 rows (bit 0 i-face 1, bit 1 i-face nx), then
   // nx+2 columns (bit 0 j-face 1, bit 1 j-face ny)
   const int *oflags = nullptr;
@@ -45,6 +47,7 @@ struct StripBufs {
 };
 // seam rows (seam x tile x row) of a mesh with nw columns per workgroup
 size_t strip_rows(const Dev &d, int nw);
+inline size_t strip_counters(const Dev &d) { return (size_t)((d.nv + 63) / 64) * kNextStride; }
 // the word a seam message is filled with before its first use
 uint32_t strip_empty_word(bool fp32);
 // Column-pair kinetic step with nw (8 or 16) columns per workgroup; false when
@@ -71,6 +74,7 @@ struct StripJob {
   T *F, *R;
   const T *slot;
   T *msg;
+  int *next;
   const int *oflags;
   const int *wall_list;  // DETFPwall nodes (k_det_wall)
   double *swall;

@@ -691,8 +691,15 @@ __device__ __forceinline__ void cellpar_body(const Dev &d, P *cpar, int pstride,
 #pragma unroll
   for (int k = 0; k < kNW; k++) o[k] = P(vals[k]);
 }
+// the counters of the column-pair launch that follows (draw_strip) to zero, by a
+// launch's or a job's first workgroup
+__device__ __forceinline__ void clear_next(int *next, int ntiles) {
+  for (int t = threadIdx.x; t < ntiles; t += blockDim.x) next[kNextStride * t] = 0;
+}
+// next: those counters, if such a launch follows
 template <typename P>
-__global__ void k_cellpar(Dev d, P *cpar, int pstride) {
+__global__ void k_cellpar(Dev d, P *cpar, int pstride, int *next, int ntiles) {
+  if (next && blockIdx.x == 0) clear_next(next, ntiles);
   cellpar_body(d, cpar, pstride, (int)(blockIdx.x * blockDim.x + threadIdx.x));
 }
 
@@ -1210,10 +1217,14 @@ __global__ void __launch_bounds__(1024) k_walk(Dev d, const double *cpar, int VT
 // The strips of a tile form a pipeline across workgroups.  A message row is
 // four values per velocity in a slot of its own that holds a signalling NaN
 // (which no arithmetic returns) until it is written; the receiver polls the
-// values themselves and puts the NaN back for the next launch.  The grid is
-// strip-major, so a workgroup only waits for one with a lower index, which was
-// dispatched before it: the waits cannot form a cycle.  They are bounded; a
-// timeout sets *werr.
+// values themselves and puts the NaN back for the next launch.  A workgroup's
+// tile comes from its index, its strip from the order in which the tile's
+// workgroups start (draw_strip), so a workgroup only waits for ones that have
+// started: the waits cannot form a cycle, whatever else is on the device.  (The
+// order of the indices does not give that: the XCDs start their shares of a
+// launch independently, so beside another stream's kernel whose workgroups wait
+// for each other too a lower index could be left queued behind that kernel.)
+// The waits are bounded; a timeout sets *werr.
 // ------------------------------------------------------------------------
 constexpr int kSpinMax = 1 << 20;  // about a second of polling
 
@@ -1280,6 +1291,24 @@ __device__ __forceinline__ bool seam_empty(T v) {
   return u == Seam<T>::kEmpty;
 }
 
+// The strip of this workgroup of tile `tile`: one more than that of the tile's
+// workgroup that drew before it.  Its index's strip g it gets if the lower ones
+// draw within some 30 us, as they do on a device of its own: the index order puts
+// the workgroups that share a CU at the end of the pipelines (drawn in the order
+// of arrival alone, 39 columns x 60^2 velocities took 6% longer).  next: a counter
+// per tile, each in a line of its own, zero before the launch; word: LDS that is
+// not written before the workgroup's next barrier.
+constexpr int kDrawPolls = 32;
+__device__ __forceinline__ int draw_strip(int *next, int tile, int g, int *word) {
+  if (threadIdx.x == 0) {
+    int *p = next + kNextStride * tile;
+    for (int n = 0; n < kDrawPolls && ld_agent(p) < g; n++) __builtin_amdgcn_s_sleep(1);
+    *word = __hip_atomic_fetch_add(p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  barrier_lds();
+  return __builtin_amdgcn_readfirstlane(*word);
+}
+
 // LDS of one workgroup (declared by each kernel, so that its addresses are
 // constants of that kernel).  FP64: 144 KB for 16 columns (one workgroup per
 // CU), 80 KB for 8 (two); FP32 half of that.
@@ -1340,7 +1369,7 @@ template <typename T, int NC, int SL>
 __device__ __forceinline__ void strip_body(StripLds<T, NC> &lds, const Dev &d, const T *__restrict__ cpar_,
                                            T *__restrict__ F, const T *__restrict__ slot, T *__restrict__ R,
                                            int store_rhs, int ntiles, T *msg, int *werr,
-                                           const int *__restrict__ oflags_, int bid) {
+                                           const int *__restrict__ oflags_, int *next, int bid) {
 #pragma clang fp contract(off)
   constexpr int NP = NC / 2;
   constexpr int ES = sizeof(T);
@@ -1362,7 +1391,9 @@ __device__ __forceinline__ void strip_body(StripLds<T, NC> &lds, const Dev &d, c
   const int nsteps = NP + nrow + 5;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = threadIdx.x & 63;
-  const int g = bid / ntiles, tile = bid - g * ntiles;
+  int g = bid / ntiles;
+  const int tile = bid - g * ntiles;
+  if (ngroups > 1) g = draw_strip(next, tile, g, reinterpret_cast<int *>(&lds.x));
   const int i0 = g * NC + 1;  // the strip's first mesh column
   // byte strides: one cell's velocities, one row of cells, one plane
   const long long cb = (long long)nv * ES, rb = (long long)d.NI * cb, pb = (long long)d.ncell * cb;
@@ -1854,9 +1885,9 @@ constexpr int strip_threads(int nc) { return 64 * (nc / 2 + 3); }
 template <typename T, int NC, int SL>
 __global__ void __launch_bounds__(strip_threads(NC), strip_waves(sizeof(T), NC))
     k_strip(Dev d, const T *__restrict__ cpar, T *__restrict__ F, const T *__restrict__ slot, T *__restrict__ R,
-            int store_rhs, int ntiles, T *msg, int *werr, const int *__restrict__ oflags) {
+            int store_rhs, int ntiles, T *msg, int *werr, int *next, const int *__restrict__ oflags) {
   __shared__ StripLds<T, NC> lds;
-  strip_body<T, NC, SL>(lds, d, cpar, F, slot, R, store_rhs, ntiles, msg, werr, oflags, (int)blockIdx.x);
+  strip_body<T, NC, SL>(lds, d, cpar, F, slot, R, store_rhs, ntiles, msg, werr, oflags, next, (int)blockIdx.x);
 }
 
 // wavefront-uniform copies (scalar registers) of values read from memory,
@@ -1900,12 +1931,12 @@ __device__ __forceinline__ int job_of(const J *jobs, int njobs, int b) {
 }
 
 // One launch of the column-pair kernel over the strips of every job of a
-// batch (instances of different mesh and velocity grid).  Each job's
-// workgroups are consecutive and strip-major, so a workgroup still waits only
-// for lower-numbered workgroups of its own job.
+// batch (instances of different mesh and velocity grid).  Each job's workgroups
+// are consecutive and strip-major.
 template <typename T, int NC, int SL>
 __global__ void __launch_bounds__(strip_threads(NC), strip_waves(sizeof(T), NC))
     k_strip_batch(const StripJob<T> *__restrict__ jobs, int njobs, int *werr) {
+  __shared__ StripLds<T, NC> lds;
   const int k = job_of<StripJob<T>, &StripJob<T>::strip0>(jobs, njobs, (int)blockIdx.x);
   const StripJob<T> &J = jobs[k];
   // the fields the kernel uses, in scalar registers like kernel arguments
@@ -1919,15 +1950,15 @@ __global__ void __launch_bounds__(strip_threads(NC), strip_waves(sizeof(T), NC))
   d.L = uni(J.d.L);
   d.vi = uni(J.d.vi);
   d.vj = uni(J.d.vj);
-  __shared__ StripLds<T, NC> lds;
   strip_body<T, NC, SL>(lds, d, uni(J.cp), uni(J.F), uni(J.slot), uni(J.R), 0, uni(J.ntiles), uni(J.msg), werr,
-                        uni(J.oflags), (int)blockIdx.x - uni(J.strip0));
+                        uni(J.oflags), uni(J.next), (int)blockIdx.x - uni(J.strip0));
 }
 
 template <typename T>
 __global__ void __launch_bounds__(256) k_cellpar_batch(const StripJob<T> *__restrict__ jobs, int njobs) {
   const int k = job_of<StripJob<T>, &StripJob<T>::cell0>(jobs, njobs, (int)blockIdx.x);
   const StripJob<T> &J = jobs[k];
+  if ((int)blockIdx.x == J.cell0) clear_next(in_global(J.next), J.ntiles);
   cellpar_body(dev_of(J.d), in_global(const_cast<T *>(J.cp)), 0, ((int)blockIdx.x - J.cell0) * 256 + (int)threadIdx.x);
 }
 
@@ -2555,20 +2586,20 @@ bool launch_strip_nw(const Dev &d, double *cpar, T *F, const T *slot, T *R, int 
   // the constants in T: the FP32 kernels read them as single precision
   // without a conversion per use (the same values: each is rounded once)
   T *cp = reinterpret_cast<T *>(cpar);
-  hipLaunchKernelGGL(k_cellpar<T>, dim3((ncl + 255) / 256), dim3(256), 0, s, d, cp, 0);
+  hipLaunchKernelGGL(k_cellpar<T>, dim3((ncl + 255) / 256), dim3(256), 0, s, d, cp, 0, b.next, ntiles);
   if (b.ev_before) (void)hipEventRecord(b.ev_before, s);
   const dim3 grid(strip_blocks(d, NC)), block(strip_threads(NC));
   // each flux scheme is a separate instantiation, so that its slopes cost
   // the others no registers
   if (d.scheme == kSchemeWeno3)
     hipLaunchKernelGGL((k_strip<T, NC, 1>), grid, block, 0, s, d, cp, F, slot, R, store_rhs, ntiles, (T *)b.msg, b.err,
-                       b.oflags);
+                       b.next, b.oflags);
   else if (d.scheme == 0)  // first-order upwind
     hipLaunchKernelGGL((k_strip<T, NC, 2>), grid, block, 0, s, d, cp, F, slot, R, store_rhs, ntiles, (T *)b.msg, b.err,
-                       b.oflags);
+                       b.next, b.oflags);
   else
     hipLaunchKernelGGL((k_strip<T, NC, 0>), grid, block, 0, s, d, cp, F, slot, R, store_rhs, ntiles, (T *)b.msg, b.err,
-                       b.oflags);
+                       b.next, b.oflags);
   if (b.ev_after) (void)hipEventRecord(b.ev_after, s);
   return true;
 }
@@ -2674,7 +2705,8 @@ bool launch_walk(const Dev &d, double *cpar, T *F, const T *slot, T *R, int stor
   const size_t slot_bytes = (size_t)8 * d.L * d.nv * sizeof(T);
   if (so < (ptrdiff_t)(2 * (size_t)d.ncell * d.nv * sizeof(T)) || (size_t)so + slot_bytes > 4294967295u) return false;
   const int ncl = (d.nx - 1) * (d.ny - 1);
-  hipLaunchKernelGGL(k_cellpar<double>, dim3((ncl + 255) / 256), dim3(256), 0, s, d, cpar, 3 * vt * (d.nx - 1));
+  hipLaunchKernelGGL(k_cellpar<double>, dim3((ncl + 255) / 256), dim3(256), 0, s, d, cpar, 3 * vt * (d.nx - 1),
+                     (int *)nullptr, 0);
   const int ntiles = 2 * ((d.nv + vt - 1) / vt);
   const int nb = (ntiles + K - 1) / K;
   const unsigned planeb = (unsigned)((size_t)d.ncell * d.nv * sizeof(T));
