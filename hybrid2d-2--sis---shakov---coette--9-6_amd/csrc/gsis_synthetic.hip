@@ -1362,13 +1362,15 @@ int synthetic_init(Dev &d, const gsis_params &p, SyntheticState &st) {
     }
   }
   const size_t nq = (size_t)st.np * st.nw * 64;  // cells of the blocked sweep layout
-  // 32-bit buffer offsets of the blocked arrays (the largest has 12 doubles
-  // per cell, and the limit leaves room for half as many again) and of U
-  if ((size_t)18 * nq * sizeof(double) >= ((size_t)1 << 31) || (size_t)4 * N * sizeof(double) >= ((size_t)1 << 31)) {
+  // 32-bit buffer offsets of the blocked arrays and of U; the largest blocked ones
+  // are the records and, with normals, the geometry (the padded ones have 4
+  // doubles a cell and kPad planes more at either end)
+  const size_t npad = (size_t)(st.np + 2 * kPad) * st.nw * 64;
+  if (std::max({kNRec * nq, 2 * geo_pairs(st.axis) * nq, 4 * npad}) * sizeof(double) >= ((size_t)1 << 31) ||
+      (size_t)4 * N * sizeof(double) >= ((size_t)1 << 31)) {
     g_syn_err = "synthetic solve: the mesh is too large for the sweep's buffers (2 GiB)";
     return GSIS_EUNSUPPORTED;
   }
-  const size_t npad = (size_t)(st.np + 2 * kPad) * st.nw * 64;
   const size_t n_geo = (size_t)2 * geo_pairs(st.axis) * nq;
   const size_t n_hand = st.nw > 0 ? (size_t)2 * st.nw * hand_len(d.nx) * 4 : 0;
   const size_t n_dbl = 4 * N + (size_t)kNRec * nq + 8 * npad + n_geo + n_hand + (size_t)ntiles +

@@ -142,3 +142,19 @@ b.step(1)
 print(b.ns_graph(), model.model_queued())
 """)
     assert out[0] == "4" and 1 <= int(out[1]) <= 2
+
+
+@pytest.mark.parametrize("bent", [False, True], ids=["axis", "bent"])
+def test_the_largest_meshes_of_the_synthetic_solve(run, bent):
+    """Refused is what does not fit the 32-bit offsets into the sweep's arrays: 12 doubles for each of 64
+    rows of a plane, nx - 5 planes in a single band of one row, below 2 GiB up to nx = 349530."""
+    out = run(BATCH + f"""
+for nx in (349530, 349531):
+    q = box(nx - 1, 5, {bent})
+    try:
+        solver.GsisSolver(q, mode=1).close()
+        print("taken")
+    except g.capi.GsisError as e:
+        print("2 GiB" in str(e) and "refused")
+""")
+    assert out == ["taken", "refused"]
