@@ -1356,6 +1356,7 @@ int synthetic_init(Dev &d, const gsis_params &p, SyntheticState &st) {
     // one workgroup per CU: the fluxes run beside the sweeps, so more of them
     // at a time would only share the sweeps' CUs
     st.nflux = std::min(ntiles, ncu - st.nw);
+    if (ns_blocks(st) > ncu * per) st.stride = 1;  // (a device of few CUs: bands next to each other)
     if (st.nflux < 1 || ns_blocks(st) > ncu * per) {
       g_syn_err = "synthetic solve: the inner-loop launch does not fit the device";
       return GSIS_EUNSUPPORTED;

@@ -158,3 +158,19 @@ for nx in (349530, 349531):
         print("2 GiB" in str(e) and "refused")
 """)
     assert out == ["taken", "refused"]
+
+
+@pytest.mark.parametrize("cus", [256, 64, 32])
+def test_many_bands_on_few_cus(run, cus):
+    """The bands of an instance are spread over every eighth workgroup only where the device has the CUs."""
+    out = run(BATCH + f"""
+model.model_set_cus({cus})
+n = ctypes.c_int()
+for j in (260, 330, 1028):
+    s = solver.GsisSolver(box(20, j), mode=1, kstep_show=1 << 30)
+    s.step(1)
+    model.model_launches(b"k_ns_loop", ctypes.byref(n))
+    print(n.value)
+    s.close()
+""")
+    assert len(out) == 3 and all(1 < int(n) <= cus for n in out)
