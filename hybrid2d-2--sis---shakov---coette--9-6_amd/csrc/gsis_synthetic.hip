@@ -51,6 +51,7 @@
 
 #include "gsis_ns_common.h"
 #include "gsis_synthetic.h"
+#include "gsis_wait.h"
 
 namespace gsis {
 
@@ -77,7 +78,8 @@ constexpr int kGroups = 2;                   // groups of prepared records in LD
 constexpr int kPad = kGroup - 1;             // planes before the first and after the last one that steps store to
 constexpr int kHand = 64;                    // received neighbour values in LDS (a power of two)
 constexpr long long kWaitTicks = 200000000;  // bounded waits: 2 s of the 100 MHz wall clock
-constexpr long long kStartTicks = 12000000000;  // a batched gang's wait for its last workgroup: 120 s
+// a batched gang's wait for its last workgroup: 120 s without an iteration of an earlier gang
+constexpr long long kStartTicks = 12000000000;
 
 // ctl words
 enum { kCtlGo = 1, kCtlErr = 3, kCtlBad = 4, kCtlStop = 5, kCtlLast = 6, kCtlArrived = 7 };
@@ -553,14 +555,14 @@ __device__ __forceinline__ void vm_wait() {  // this wavefront's stores are at m
 // the time; a timeout sets the error word.
 struct Patience {
   int *ctl;
-  long long limit, t0 = 0;
+  long long t0 = 0;
   int n = 0;
-  __device__ explicit Patience(int *c, long long ticks = kWaitTicks) : ctl(c), limit(ticks) {}
+  __device__ explicit Patience(int *c) : ctl(c) {}
   __device__ bool over(bool stop_too) {
     if ((++n & 63) != 0) return false;
     if (uniform(ld_agent(ctl + kCtlErr)) != 0 || (stop_too && uniform(ld_agent(ctl + kCtlStop)) != 0)) return true;
     if (n == 64) t0 = wall_clock64();
-    if (wall_clock64() - t0 > limit) {
+    if (wall_clock64() - t0 > kWaitTicks) {
       st_agent(ctl + kCtlErr, 1);
       return true;
     }
@@ -1204,8 +1206,8 @@ __global__ void __launch_bounds__(kThreads) k_ns_loop(Dev d, SyntheticState st) 
 // its XCD: those of earlier gangs, which are complete and end, and its own
 // gang's, which leave room (synthetic_batch_layout: at most half of the device's
 // workgroups).  The launch has no such launch beside it (ns_turn).  A gang
-// starts once its last workgroup has arrived; that wait alone may take as long
-// as the gangs before it.
+// starts once its last workgroup has arrived; that wait alone takes as long as
+// gangs before it do, and is bounded by the time in which none of them goes on.
 __global__ void __launch_bounds__(kThreads) k_ns_batch(const NsJob *__restrict__ jobs, int njobs) {
   __shared__ __align__(16) char lds[LoopShared<false>::kBytes];
   int lo = 0, hi = njobs - 1;
@@ -1216,16 +1218,26 @@ __global__ void __launch_bounds__(kThreads) k_ns_batch(const NsJob *__restrict__
   }
   const NsJob &J = jobs[lo];
   int *word = reinterpret_cast<int *>(lds);
-  if (threadIdx.x == 0) {
+  if (threadIdx.x < 64) {
     int *ctl = J.st.ctl;
-    __hip_atomic_fetch_add(ctl + kCtlArrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    Patience pt(ctl, kStartTicks);
+    if (threadIdx.x == 0) __hip_atomic_fetch_add(ctl + kCtlArrived, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    StallLimit limit(kStartTicks);
     bool ok = true;
-    while (ok && ld_agent(ctl + kCtlArrived) < J.blocks) {
+    for (int n = 1; ok && uniform(ld_agent(ctl + kCtlArrived)) < J.blocks; n++) {
       __builtin_amdgcn_s_sleep(32);
-      ok = !pt.over(false);
+      if ((n & 63) != 0) continue;
+      // the earlier gangs' iterations
+      long long sum = 0;
+      for (int q = threadIdx.x; q < lo; q += 64) sum += ld_agent(jobs[q].st.ctl + kCtlGo);
+      for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
+      if (uniform(ld_agent(ctl + kCtlErr)) != 0) {
+        ok = false;
+      } else if (limit.over(sum, wall_clock64())) {
+        st_agent(ctl + kCtlErr, 1);
+        ok = false;
+      }
     }
-    *word = ok ? 1 : 0;
+    if (threadIdx.x == 0) *word = ok ? 1 : 0;
   }
   __syncthreads();
   const int ok = *word;
