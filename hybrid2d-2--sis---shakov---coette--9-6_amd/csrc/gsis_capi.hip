@@ -1263,7 +1263,7 @@ int gsis_batch_create(gsis_handle *const *hs, int32_t n, gsis_batch **out) {
     if (h->prec != hs[0]->prec || h->d.scheme != hs[0]->d.scheme || h->dev != hs[0]->dev)
       return fail(GSIS_EARG, "batch: instances must share precision, flux scheme and device");
     if (h->d.nx - 1 < 2 || h->d.ny - 1 < 2 || gsis::strip_rows(h->d, 8) * 256 > h->strip.msg_elems)
-      return fail(GSIS_EUNSUPPORTED, "batch: instance " + std::to_string(k) + " does not fit the column-wavefront kernel");
+      return fail(GSIS_EUNSUPPORTED, "batch: instance " + std::to_string(k) + " does not fit the column-pair kernel");
     for (int m = 0; m < k; m++)
       if (hs[m] == h) return fail(GSIS_EARG, "batch: a handle is listed twice");
   }

@@ -6,7 +6,6 @@ namespace gsis {
 
 constexpr int kMaxV1 = 512;  // max discrete velocities per direction (LDS tables)
 
-template <typename T> void launch_wall(const Dev &d, const BcDev &b, T *FG, T *FH, T *slot, hipStream_t s);
 // up to kMaxWalls subfaces launched together (diffuse walls; periodic subfaces
 // of one direction); start[k] is the first block of subface k
 constexpr int kMaxWalls = 16;

@@ -275,10 +275,6 @@ __device__ void wall_node(const Dev &d, const BcDev &b, int kk, T *FG, T *FH, T 
   }
 }
 
-template <typename T>
-__global__ void k_wall(Dev d, BcDev b, T *FG, T *FH, T *slot) {
-  wall_node(d, b, blockIdx.x, FG, FH, slot);
-}
 // All diffuse walls of the block in one launch: a wall reads only interior
 // cells and writes only its own face's slot, so the walls are independent of
 // each other and of the far-field / periodic ghost fills.
@@ -2220,12 +2216,10 @@ __device__ __forceinline__ double corner_s(const Dev &d, int i, int j, int k) {
   const int ii = i == 0 ? 1 : d.nx - 1, jj = j == 0 ? 1 : d.ny - 1, o = k * d.ncell;
   return d.S[o + cidx(d, ii, j)] + d.S[o + cidx(d, i, jj)] - d.S[o + cidx(d, ii, jj)];
 }
-__device__ __forceinline__ bool corner(const Dev &d, int i, int j) {
-  return (i == 0 || i == d.nx) && (j == 0 || j == d.ny);
-}
 struct Cons { double u[4]; };
 // What a cell's NS conservative variables are formed from: its S in
-// [0,nx]x[0,ny] (corners: the extrapolated one), U as it is outside.
+// [0,nx]x[0,ny], U as it is outside.  (Of a corner no value is formed: the ghost
+// extrapolations replace it.)
 __device__ __forceinline__ Cons cons_in(const Dev &d, int i, int j) {
   const double *src = i < 0 || i > d.nx || j < 0 || j > d.ny ? d.U : d.S;
   const int c = cidx(d, i, j);
@@ -2239,8 +2233,6 @@ __device__ __forceinline__ Cons cons_in(const Dev &d, int i, int j) {
 __device__ __forceinline__ Cons cons_of(const Dev &d, int i, int j, Cons s) {
 #pragma clang fp contract(off)
   if (i < 0 || i > d.nx || j < 0 || j > d.ny) return s;
-  if (corner(d, i, j))
-    for (int k = 0; k < 4; k++) s.u[k] = corner_s(d, i, j, k);
   const double sq = sqrt(2.0 / d.gamma);
   const double tu = s.u[1] / d.ma * sq, tv = s.u[2] / d.ma * sq;
   Cons r;
@@ -2486,12 +2478,6 @@ __global__ void k_frd_in_chunk(Dev d, const double *stage, int v0, int nvc, T *F
 // ------------------------------------------------------------------------
 // launchers
 // ------------------------------------------------------------------------
-template <typename T>
-void launch_wall(const Dev &d, const BcDev &b, T *FG, T *FH, T *slot, hipStream_t s) {
-  const int nn = (b.face == 1 || b.face == 3) ? (b.jend - b.jst) : (b.iend - b.ist);
-  if (nn <= 0) return;
-  hipLaunchKernelGGL(k_wall<T>, dim3(nn), dim3(256), 0, s, d, b, FG, FH, slot);
-}
 template <typename T>
 void launch_walls(const Dev &d, const BcSet &ws, T *FG, T *FH, T *slot, hipStream_t s) {
   if (ws.n <= 0 || ws.start[ws.n] <= 0) return;
@@ -2818,7 +2804,6 @@ void launch_residual(const Dev &d, double *out, hipStream_t s) {
 }
 
 #define INST(T)                                                                                   \
-  template void launch_wall<T>(const Dev &, const BcDev &, T *, T *, T *, hipStream_t);           \
   template void launch_walls<T>(const Dev &, const BcSet &, T *, T *, T *, hipStream_t);        \
   template void launch_farfield<T>(const Dev &, const BcDev &, T *, T *, hipStream_t);            \
   template void launch_periodic<T>(const Dev &, const BcSet &, T *, T *, hipStream_t);            \

@@ -97,7 +97,6 @@ struct MlpTape {
 };
 typedef short bf16x8 __attribute__((ext_vector_type(8)));
 
-template <bool TRAIN>
 struct MlpShared {
   unsigned short f[kMlpRows * kLdF];  // H of the last layer, or dZ
   unsigned short x[kMlpRows * kLdX];  // inputs
@@ -139,7 +138,7 @@ __device__ __forceinline__ f32x16 mm(const unsigned short *a, const Operands<K> 
 template <bool TRAIN>
 __global__ void __launch_bounds__(kMlpThreads) k_mlp_pass(MlpNet net, const float *x, const int *idx, int n, float *y,
                                                           const float *target, MlpTape tape) {
-  __shared__ __align__(16) MlpShared<TRAIN> sh;
+  __shared__ __align__(16) MlpShared sh;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int r = lane & 31, h = lane >> 5, kq = 4 * h;
   const int nb = wave & 3, rb = wave >> 2;  // this wavefront's feature block and sample block
