@@ -1298,8 +1298,16 @@ constexpr int kDrawPolls = 32;
 __device__ __forceinline__ int draw_strip(int *next, int tile, int g, int *word) {
   if (threadIdx.x == 0) {
     int *p = next + kNextStride * tile;
-    for (int n = 0; n < kDrawPolls && ld_agent(p) < g; n++) __builtin_amdgcn_s_sleep(1);
-    *word = __hip_atomic_fetch_add(p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    int at = g;  // the counter; if it has come to g, one exchange does
+    if (!__hip_atomic_compare_exchange_strong(p, &at, g + 1, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_AGENT)) {
+      for (int n = 0; n < kDrawPolls && at < g; n++) {
+        __builtin_amdgcn_s_sleep(1);
+        at = ld_agent(p);
+      }
+      at = __hip_atomic_fetch_add(p, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    *word = at;
   }
   barrier_lds();
   return __builtin_amdgcn_readfirstlane(*word);
