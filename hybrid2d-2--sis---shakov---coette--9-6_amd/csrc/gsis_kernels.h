@@ -56,8 +56,9 @@ template <typename T> void launch_res4(const Dev &d, const T *RG, const T *RH, h
 // Columns per workgroup: 16 where the mesh has more than 8 and the launch's
 // strips of 16 still give every CU a workgroup, else 8, whose shorter pipelines
 // fill more CUs.  Measured, 16 against 8 columns: 128^2 x 64^2 (512 strips of 16)
-// 0.86 and 0.89 ms, FP32 0.50 and 0.62, 256^2 x 96^2 (2304) 7.6 and 8.1; 101^2 x 37^2
-// (154) 0.41 and 0.38, 64^2 x 32^2 (64) 0.22 and 0.18, 12^2 x 24^2 (9) 45 and 41 us.
+// 0.73 and 0.74 ms, FP32 0.39 and 0.49, 256^2 x 96^2 (2304) 6.1 and 6.6; 96^2 x 48^2
+// (216) 0.342 and 0.336, 101^2 x 37^2 (154) 0.35 and 0.33, 64^2 x 32^2 (64) 0.21 and
+// 0.17, 12^2 x 24^2 (9) 43 and 39 us.
 constexpr long long kWideStrips = 256;
 inline int strip_columns(const Dev &d, long long strips16) { return d.nx - 1 > 8 && strips16 >= kWideStrips ? 16 : 8; }
 // workgroups of a mesh's strips with nw columns

@@ -1195,7 +1195,7 @@ __global__ void __launch_bounds__(1024) k_walk(Dev d, const double *cpar, int VT
 // Two columns per wavefront because what a wavefront does once per step --
 // addresses, scalar loads, the barrier, publishing, the left face's
 // coefficients -- then serves two cells, and because the two cells' chains fill
-// each other's latency: 360 vector and 82 scalar instructions per two cells
+// each other's latency: 364 vector and 81 scalar instructions per two cells
 // (FP64 NND, counted over all wavefronts), against 215 and 152 per cell with one
 // column per wavefront.  Rows r+1 and r+2, the right
 // column's earlier rows and earlier Delta* are read from LDS again instead of
@@ -1205,8 +1205,8 @@ __global__ void __launch_bounds__(1024) k_walk(Dev d, const double *cpar, int VT
 //
 // Measured, this kernel against one column per wavefront with a seam-update
 // kernel after it, both included: 128^2 cells x 64^2 velocities FP64 0.74 against
-// 1.01 ms, FP32 0.39 against 0.72; 256^2 x 96^2 FP64 6.3 against 8.8; 101^2 x 37^2
-// WENO3 0.46 against 0.53.  Bound by vector issue: two wavefronts per SIMD
+// 1.01 ms, FP32 0.39 against 0.72; 256^2 x 96^2 FP64 6.2 against 8.8; 101^2 x 37^2
+// WENO3 0.42 against 0.53.  Bound by vector issue: two wavefronts per SIMD
 // (LDS allows no more in FP64) reach 57% of the issue slots, and the kernel
 // runs at 1.96 GHz.  Without its stores it is 12% faster, without its copies 5%.
 //

@@ -37,11 +37,12 @@
 //
 // Measured per inner iteration (mesh cells, sweeps of all bands in one
 // workgroup with separate flux phases before): 64^2 102 -> 64 us, 128^2
-// 238 -> 127 us, 256^2 607 -> 258 us; 40 instances of side 64-256 in one
-// launch 4.5 -> 0.42 ms (one workgroup each before).  A plane step takes about
-// 0.2 us, 450-480 cycles, of which the arithmetic alone takes about 400; an
-// iteration adds about 10 us for the turn from the backward to the forward
-// sweep (the flux of the first tile).
+// 238 -> 127 us, 256^2 607 -> 255-266 us; 40 instances of side 64-256 in one
+// launch 4.5 -> 0.42 ms (one workgroup each before).  Between these meshes (234,
+// 490 and 1002 plane steps) a step costs 0.25 us, and an iteration 6 us besides.
+// A step of which everything it waits for is there already takes 0.2 us (450-480
+// cycles, about 400 of them the arithmetic): a fifth of the step in the loop is
+// waiting that has not been told apart.
 #include <algorithm>
 #include <cstring>
 #include <functional>
