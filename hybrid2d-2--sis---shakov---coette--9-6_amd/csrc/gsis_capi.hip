@@ -47,6 +47,10 @@ struct gsis_handle {
   gsis_params p{};
   std::vector<gsis_bc> bc;
   std::vector<BcDev> bcd;
+  struct BcLaunches {
+    std::vector<gsis::BcSet> walls;
+    std::vector<std::pair<int, gsis::BcSet>> fills;  // BcJob::kPeriodic or kFarfield, in order
+  } bcl;  // a step's boundary launches
   Dev d{};
   hipStream_t s = nullptr;
   int dev = 0;  // device current at gsis_create
@@ -216,12 +220,8 @@ int validate(const gsis_params *p) {
 // far-field and periodic fills (which may share corner ghost cells) keep
 // their order, periodic subfaces of one direction that follow one another
 // in one launch.
-struct BcLaunches {
-  std::vector<gsis::BcSet> walls;
-  std::vector<std::pair<int, gsis::BcSet>> fills;  // BcJob::kPeriodic or kFarfield, in order
-};
-BcLaunches bc_launches(const gsis_handle *h) {
-  BcLaunches l;
+gsis_handle::BcLaunches bc_launches(const gsis_handle *h) {
+  gsis_handle::BcLaunches l;
   auto put = [](gsis::BcSet &w, const BcDev &b, int nn) {
     w.b[w.n] = b;
     w.start[w.n + 1] = w.start[w.n] + nn;
@@ -252,7 +252,7 @@ BcLaunches bc_launches(const gsis_handle *h) {
 template <typename T>
 void phy_boundary(gsis_handle *h) {
   T *FG = (T *)h->FG, *FH = (T *)h->FH, *slot = (T *)h->slot;
-  const BcLaunches l = bc_launches(h);
+  const auto &l = h->bcl;
   for (const gsis::BcSet &w : l.walls) gsis::launch_walls<T>(h->d, w, FG, FH, slot, h->s);
   for (const auto &f : l.fills) {
     if (f.first == gsis::BcJob::kPeriodic) gsis::launch_periodic<T>(h->d, f.second, FG, FH, h->s);
@@ -590,7 +590,7 @@ int batch_jobs(gsis_batch *b) {
       j.nwall = h->nwall;
       j.ntiles = (h->d.nv + 63) / 64;
       gsis::batch_blocks<T>(j, wide, h->p.if_viscous != 0, b->nb);
-      const BcLaunches l = bc_launches(h);
+      const auto &l = h->bcl;
       for (const gsis::BcSet &w : l.walls) enter(0, (int)jobs.size(), gsis::BcJob::kWalls, w);
       for (size_t q = 0; q < l.fills.size(); q++) enter(q, (int)jobs.size(), l.fills[q].first, l.fills[q].second);
       jobs.push_back(j);
@@ -703,10 +703,15 @@ int batch_replay(gsis_batch *b, int nsteps) {
     if (b->nns == 0) {
       HIPCHK(hipGraphLaunch(b->exec, b->s));
     } else {
-      // at most two steps queued: others that take turns with them (ns_turn) wait
+      // at most two steps queued: others that take turns with them (NsTurn) wait
       // for what is queued, and a step of milliseconds is enough to queue the next behind
       if (k >= 2) HIPCHK(hipEventSynchronize(b->done[k & 1]));
-      HIPCHK(gsis::ns_turn(b->s, [&] { return hipGraphLaunch(b->exec, b->s); }));
+      {
+        gsis::NsTurn turn;
+        HIPCHK(turn.begin(b->s));
+        HIPCHK(hipGraphLaunch(b->exec, b->s));
+        HIPCHK(turn.end());
+      }
       HIPCHK(hipEventRecord(b->done[k & 1], b->s));
     }
     if (!m1) continue;
@@ -885,6 +890,7 @@ int gsis_create(const gsis_params *p, gsis_handle **out) {
     }
     h->bcd.push_back(bd);
   }
+  h->bcl = bc_launches(h);
   h->swall_len = soff;
   h->nwall = (int)wl.size() / 4;
   uint8_t *o1, *o3, *o2, *o4;

@@ -1,6 +1,6 @@
 // gsis_synthetic.h -- synthetic NS solve of mode M1 (src/Hybrid_Sub.f90:45-153).
 #pragma once
-#include <functional>
+#include <mutex>
 #include <vector>
 
 #include "../../include/gsis_capi.h"
@@ -87,10 +87,18 @@ int synthetic_batch_layout(std::vector<NsJob> &jobs);
 // the inner loops of n instances with swept cells (device table djobs, after
 // synthetic_batch_layout), between their synthetic_begin and synthetic_finish
 void launch_ns_batch(const NsJob *djobs, int n, int blocks, hipStream_t s);
-// makes a launch on stream s (a graph's that holds launch_ns_batch, say) that
-// starts when the device's last launch of an inner loop has ended, and that the
-// next one waits for
-hipError_t ns_turn(hipStream_t s, const std::function<hipError_t()> &launch);
+// The turn of a launch of inner loops (a graph's that holds launch_ns_batch, say):
+// begin, the launch, end.  It starts when the device's last such launch has
+// ended, and the next one waits for it.
+struct NsTurn {
+  hipError_t begin(hipStream_t stream);
+  hipError_t end();
+
+ private:
+  std::unique_lock<std::mutex> lock;  // held while the launch is queued
+  int dev = 0;
+  hipStream_t s = nullptr;
+};
 void synthetic_free(SyntheticState &st);
 const char *synthetic_error();
 

@@ -45,7 +45,6 @@
 // waiting that has not been told apart.
 #include <algorithm>
 #include <cstring>
-#include <functional>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -1206,7 +1205,7 @@ __global__ void __launch_bounds__(kThreads) k_ns_loop(Dev d, SyntheticState st) 
 // that is not complete a missing workgroup waits only for lower-numbered ones of
 // its XCD: those of earlier gangs, which are complete and end, and its own
 // gang's, which leave room (synthetic_batch_layout: at most half of the device's
-// workgroups).  The launch has no such launch beside it (ns_turn).  A gang
+// workgroups).  The launch has no such launch beside it (NsTurn).  A gang
 // starts once its last workgroup has arrived; that wait alone takes as long as
 // gangs before it do, and is bounded by the time in which none of them goes on.
 __global__ void __launch_bounds__(kThreads) k_ns_batch(const NsJob *__restrict__ jobs, int njobs) {
@@ -1295,26 +1294,22 @@ __global__ void k_ns_resume(Dev d, SyntheticState st, int k0) {
 // waits run out.  A launch's stream waits for the launch before it; nothing waits
 // on the host.  Other kernels run beside them.
 namespace {
-struct Turn {
+constexpr int kMaxDevices = 64;
+struct {
   std::mutex mu;
   hipEvent_t last = nullptr;  // recorded behind the device's last such launch
-};
-constexpr int kMaxDevices = 64;
-Turn g_turn[kMaxDevices];
+} g_turn[kMaxDevices];
 }  // namespace
-hipError_t ns_turn(hipStream_t s, const std::function<hipError_t()> &launch) {
-  int dev = 0;
-  hipError_t e = hipGetDevice(&dev);
+hipError_t NsTurn::begin(hipStream_t stream) {
+  const hipError_t e = hipGetDevice(&dev);
   if (e != hipSuccess) return e;
   if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
-  Turn &t = g_turn[dev];
-  std::lock_guard<std::mutex> lock(t.mu);
-  if (t.last) e = hipStreamWaitEvent(s, t.last, 0);
-  else e = hipEventCreateWithFlags(&t.last, hipEventDisableTiming);
-  if (e == hipSuccess) e = launch();
-  if (e == hipSuccess) e = hipEventRecord(t.last, s);
-  return e;
+  s = stream;
+  lock = std::unique_lock<std::mutex>(g_turn[dev].mu);
+  hipEvent_t &last = g_turn[dev].last;
+  return last ? hipStreamWaitEvent(s, last, 0) : hipEventCreateWithFlags(&last, hipEventDisableTiming);
 }
+hipError_t NsTurn::end() { return hipEventRecord(g_turn[dev].last, s); }
 
 // the degenerate loop of a mesh without swept cells: max |Res_4| over no
 // cells is 0, so the reference runs one iteration that changes nothing
@@ -1461,9 +1456,11 @@ int synthetic_run(const Dev &d, SyntheticState &st, int k0, int kstop, hipStream
     ss.k0 = k0;
     ss.kstop = kstop;
     void *args[] = {&dd, &ss};
-    const hipError_t e = ns_turn(s, [&] {
-      return hipLaunchCooperativeKernel(ns_loop_kernel(st), dim3(ns_blocks(st)), dim3(kThreads), args, 0, s);
-    });
+    NsTurn turn;
+    hipError_t e = turn.begin(s);
+    if (e == hipSuccess)
+      e = hipLaunchCooperativeKernel(ns_loop_kernel(st), dim3(ns_blocks(st)), dim3(kThreads), args, 0, s);
+    if (e == hipSuccess) e = turn.end();
     if (e != hipSuccess) {
       g_syn_err = std::string("synthetic solve: cooperative launch failed: ") + hipGetErrorString(e);
       return GSIS_EHIP;

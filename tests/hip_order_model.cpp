@@ -7,17 +7,21 @@
 //  * launches whose workgroups wait for each other (the synthetic solve's inner
 //    loops) that another such launch may run beside;
 //  * fills captured into a graph;
-// and notes the shortest copy to host memory that is not pinned.
+// and notes the shortest copy to host memory that is not pinned, and what the
+// library itself allocates on the host.
 // Loaded with RTLD_GLOBAL before the library, so that it takes the runtime's place.
+#include <dlfcn.h>
 #include <sys/mman.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -86,10 +90,22 @@ void launch(const void *f, Dim3 g, const void *s) {
   else (void)issue(s);
 }
 }  // namespace
+// allocations of host memory by the library's own code
+static std::atomic<long> own_allocations{0};
+__attribute__((noinline)) void *operator new(size_t n) {
+  Dl_info info;
+  if (dladdr(__builtin_return_address(0), &info) && info.dli_fname && strstr(info.dli_fname, "libgsis")) own_allocations++;
+  if (void *p = malloc(n ? n : 1)) return p;
+  throw std::bad_alloc();
+}
+void operator delete(void *p) noexcept { free(p); }
+void operator delete(void *p, size_t) noexcept { free(p); }
+
 #define LOCK std::lock_guard<std::recursive_mutex> lock(mu)
 
 extern "C" {
 // ---- the account
+long model_own_allocations() { return own_allocations; }
 int model_races() { return races; }
 int model_beside() { return beside; }
 int model_captured_fills() { return captured_fills; }

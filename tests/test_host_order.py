@@ -174,3 +174,19 @@ for j in (260, 330, 1028):
     s.close()
 """)
     assert len(out) == 3 and all(1 < int(n) <= cus for n in out)
+
+
+def test_a_step_allocates_nothing_on_the_host(run):
+    """What a step launches is laid out when its handle is made: an allocation that failed in a step
+    would throw through its C entry."""
+    out = run(BATCH + """
+model.model_own_allocations.restype = ctypes.c_long
+hs = [solver.GsisSolver(c, mode=m, kstep_show=1 << 30)
+      for c, m in ((box(12, 9), 0), (box(12, 9, True), 1), (g.cases.couette_case(ny_cells=9, nx_cells=6, nv=6), 0))]
+n = model.model_own_allocations()
+for h in hs:
+    h.step(3)
+    h.counters()
+print(n > 0, model.model_own_allocations() - n)
+""")
+    assert out == ["True", "0"]
