@@ -852,7 +852,10 @@ int gsis_create(const gsis_params *p, gsis_handle **out) {
       (rc = dalloc(h, &h->resbuf, 8 * (16 + (size_t)11 * (nx + 7) * (ny + 7)))))
     return cleanup(rc);
   h->stage = h->resbuf + 16;
-  if (hipHostMalloc((void **)&h->pin, kPinBytes, hipHostMallocDefault) != hipSuccess) h->pin = nullptr;  // (reads are pageable then)
+  if (hipHostMalloc((void **)&h->pin, kPinBytes, hipHostMallocDefault) != hipSuccess) {
+    h->pin = nullptr;         // reads are pageable then
+    (void)hipGetLastError();  // and no later call reports this
+  }
   {  // Creat_Mesh sets U, U0, U2 to (1,0,0,1) (src/sub_init.f90:159-162)
     std::vector<double> u(4 * N, 0.0);
     for (size_t c = 0; c < N; c++) { u[c] = 1.0; u[3 * N + c] = 1.0; }

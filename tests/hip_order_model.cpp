@@ -50,6 +50,8 @@ size_t shortest_pageable = SIZE_MAX;
 int races = 0, beside = 0, captured_fills = 0, queued = 0, cus = 256;
 struct Config { Dim3 g, b; size_t sh; void *s; };
 thread_local Config config;
+thread_local int last_error = 0;  // (of a call that failed, until it is asked for)
+bool no_pinned = false;
 
 Done issue(const void *s) {
   Stream &q = streams[s];
@@ -111,6 +113,7 @@ int model_beside() { return beside; }
 int model_captured_fills() { return captured_fills; }
 int model_queued() { return queued; }  // of those launches, the most that the host did not know to have ended
 void model_set_cus(int n) { cus = n; }
+void model_no_pinned_memory() { no_pinned = true; }
 size_t model_shortest_pageable_read() { return shortest_pageable; }
 // launches of the kernels whose name contains part; the last one's workgroups
 int model_launches(const char *part, int *workgroups) {
@@ -135,7 +138,7 @@ int hipDeviceGetAttribute(int *v, int, int) { *v = cus; return 0; }  // (asked f
 int hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, int, size_t) { *n = 1; return 0; }
 int hipFuncSetAttribute(const void *, int, int) { return 0; }
 const char *hipGetErrorString(int) { return "error of the model"; }
-int hipGetLastError() { return 0; }
+int hipGetLastError() { const int e = last_error; last_error = 0; return e; }
 int hipGetSymbolAddress(void **, const void *) { return 1; }
 int hipMalloc(void **p, size_t n) {  // an address range that nothing reads or writes
   LOCK;
@@ -152,7 +155,7 @@ int hipFree(void *p) {
   munmap(p, sizes[p]);
   return 0;
 }
-int hipHostMalloc(void **p, size_t n, unsigned) { LOCK; *p = malloc(n); pinned[(char *)*p] = n; return 0; }
+int hipHostMalloc(void **p, size_t n, unsigned) { LOCK; if (no_pinned) return last_error = 2; *p = malloc(n); pinned[(char *)*p] = n; return 0; }
 int hipHostFree(void *p) { LOCK; pinned.erase((char *)p); free(p); return 0; }
 int hipMemset(void *p, int, size_t n) { LOCK; write(p, n, nullptr); return 0; }
 int hipMemsetD32(void *p, int, size_t n) { LOCK; write(p, 4 * n, nullptr); return 0; }

@@ -190,3 +190,16 @@ for h in hs:
 print(n > 0, model.model_own_allocations() - n)
 """)
     assert out == ["True", "0"]
+
+
+def test_a_handle_without_pinned_memory(run):
+    """Pinned memory that cannot be had is no error: reads go into pageable memory, steps run."""
+    out = run(BATCH + """
+model.model_no_pinned_memory()
+s = solver.GsisSolver(box(12, 9), mode=1, kstep_show=1 << 30)
+s.step(2)
+s.macro()
+model.model_shortest_pageable_read.restype = ctypes.c_size_t
+print(s.counters()[0], model.model_shortest_pageable_read())
+""")
+    assert out == ["2", "8"]
